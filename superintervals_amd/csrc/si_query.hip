@@ -17,7 +17,8 @@
 //     one query; when it finishes, the lane takes the next query from a pool of 64
 //     the wave grabs from the tile's LDS counter, so lanes stay busy however uneven
 //     the hit counts are.  counts[q] / offsets are written in input order.
-//  3. Fill: the same kernel writes each query's positions at its CSR offset.
+//  3. Fill: a sweep over the query starts writes each query's positions at its CSR offset
+//     (si_sweep.h); the walk kernel of the count does on an index with start > end intervals.
 //
 // The walk is the reference's backward superset walk taken one aligned 64-byte line of
 // ends at a time.  In the line [b0, b0 + W) holding the current position cur, every
@@ -380,7 +381,7 @@ int plan_impl(const siIndex* ix, const S* qs, const S* qe, size_t nq, void* plan
     // guaranteed run): through the search tree when the index has one
     const bool learned = g_tune.ub_learned && ix->learned;
     const bool tree = !learned && g_tune.ub_tree && ix->ub.d_top && ix->n > 0;
-    const bool with_lb = range_skip_on(ix);
+    const bool with_lb = ix->n_inverted == 0;   // (whatever range_skip says: a fill may run under another setting)
     // with both trees of the same shape the bound search also finds each query's rank-form
     // count, which the offsets and count passes then take from the plan
     const bool with_rank = tree && rank_exact(ix) && ix->eb.d_top && ix->eb.nlv == ix->ub.nlv &&
@@ -1338,7 +1339,8 @@ __global__ __launch_bounds__(Q_THREADS) void k_walk_heavy(IndexView<S> ix_arg, T
         const bool lead = __builtin_amdgcn_readfirstlane(he.lead) != 0;
         uint32_t left = __builtin_amdgcn_readfirstlane(he.left);   // fill modes: hits still expected
         uint64_t acc = he.acc;
-        const uint64_t oend = (MODE != W_COUNT) ? min(offsets[q + 1], cap) : 0;
+        // (never below acc: offsets that decrease give an empty room, not a wrapped one)
+        const uint64_t oend = (MODE != W_COUNT) ? max(min(offsets[q + 1], cap), acc) : 0;
         wave_walk<S, MODE>(ix, td, ub, lv, lane, s, cur, top, lead, acc, oend, left, out_idx, vals, out_val);
         if (MODE == W_COUNT) {
             // every lane stores the same value (no lane-dependent branch in the loop)
@@ -1349,6 +1351,8 @@ __global__ __launch_bounds__(Q_THREADS) void k_walk_heavy(IndexView<S> ix_arg, T
         }
     }
 }
+
+#include "si_sweep.h"
 
 // ============================================================================
 // One query, one wave (the single-query host calls)
@@ -1849,22 +1853,19 @@ void walk_shape(size_t nq, uint32_t* tile, uint32_t* ntiles, unsigned* grid) {
     *grid = (unsigned)std::max<size_t>(1, std::min<size_t>(resident, *ntiles));
 }
 
+// Queries per wave of the sweep: enough waves to fill the chip (32 a CU; 16 and 64 a CU
+// measured within 8 % of it either way), at most SW_CHUNK.
+inline uint32_t sweep_chunk(size_t nq, int cus) {
+    const size_t waves = (size_t)cus * 32u;
+    return (uint32_t)std::min<size_t>(SW_CHUNK, (nq + waves - 1) / waves);
+}
+
 template <typename S, int MODE>
 int launch_walk(const siIndex* ix, void* plan, size_t nq, uint32_t* counts, uint64_t* counts64,
                 const uint64_t* offsets, uint32_t* out_idx, int32_t* out_val, hipStream_t st,
                 uint64_t cap = ~0ull) {
     if (nq == 0) return SI_OK;
     PlanView<S> pv = plan_view<S>(plan, nq);
-    uint32_t tile = 0, ntiles = 0;
-    unsigned grid = 0;
-    walk_shape<S, MODE>(nq, &tile, &ntiles, &grid);
-    k_walk_counters_reset<<<1, 64, 0, st>>>(pv.counter);
-    LAUNCH_CHECK();
-    k_walk<S, MODE><<<grid, T_THREADS, 0, st>>>(
-        ix->view<S>(), pv, (uint32_t)nq, tile, ntiles, g_tune.lane_steps, range_skip_on(ix), pv.counter, counts,
-        counts64, offsets, out_idx, ix->d_values, out_val, cap, nullptr, MultiTiles{nullptr, nullptr, nullptr, 0u});
-    LAUNCH_CHECK();
-    // parked (heavy) walks: one wave each, resident grid, exits at once when none were parked
     static int cus = 0;
     if (cus == 0) {
         int dev = 0;
@@ -1872,6 +1873,30 @@ int launch_walk(const siIndex* ix, void* plan, size_t nq, uint32_t* counts, uint
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         cus = std::max(cus, 1);
     }
+    k_walk_counters_reset<<<1, 64, 0, st>>>(pv.counter);
+    LAUNCH_CHECK();
+    bool swept = false;
+    if constexpr (MODE != W_COUNT) {
+        // the sweep answers every query of an index without start > end; the line walk is for the
+        // others (the run [lower_bound, upper_bound] may hold misses there) and for range_skip = 0
+        swept = range_skip_on(ix);
+        if (swept) {
+            const uint32_t chunk = sweep_chunk(nq, cus);
+            k_sweep<S, MODE><<<grid_for(nq, chunk * SW_WAVES), SW_THREADS, 0, st>>>(
+                ix->view<S>(), ix->tree<S>(), pv, (uint32_t)nq, chunk, offsets,
+                MODE == W_VALUES ? (uint32_t*)out_val : out_idx, ix->d_values, cap);
+        }
+    }
+    if (!swept) {
+        uint32_t tile = 0, ntiles = 0;
+        unsigned grid = 0;
+        walk_shape<S, MODE>(nq, &tile, &ntiles, &grid);
+        k_walk<S, MODE><<<grid, T_THREADS, 0, st>>>(
+            ix->view<S>(), pv, (uint32_t)nq, tile, ntiles, g_tune.lane_steps, range_skip_on(ix), pv.counter, counts,
+            counts64, offsets, out_idx, ix->d_values, out_val, cap, nullptr, MultiTiles{nullptr, nullptr, nullptr, 0u});
+    }
+    LAUNCH_CHECK();
+    // parked (heavy) walks: one wave each, resident grid, exits at once when none were parked
     IndexView<S> hv = ix->view<S>();
     LongView<S> lv = long_view_of<S>(ix);
     if (!g_tune.heavy_ends32) { hv.ends32 = nullptr; lv.ends32 = nullptr; }

@@ -1,0 +1,533 @@
+// si_sweep.h -- the fill pass as a sweep over query starts (included by si_query.hip).
+//
+// A query's hits are the run [lower_bound(s), upper_bound(e)], every position of which
+// starts inside the query, and, below it, the positions p < lower_bound(s) with ends[p] >= s:
+// the intervals that hold the point s.  That second set changes little between queries with
+// neighbouring starts, so a wave takes a chunk of the plan's queries, orders them by start and
+// carries the set along as a list in registers instead of walking down from every query:
+//
+//   window  the 64 positions [wbase, wbase + 64) that hold lower_bound - 1, one per lane;
+//   list    the positions below wbase whose end reached the chunk's current start when they
+//           were last looked at, ascending, at most SW_CAP of them, four registers per lane.
+//
+// A query then costs one compare and ballot per register and one store per register with
+// hits, each covering consecutive output slots; its run is written 64 values a store.  When
+// the starts leave the window, the survivors of list and window are packed together through
+// LDS and the next line of ends becomes the window; a chunk's first query, and a query more
+// than SW_GAP lines past the window, collects its list through the max tree (the lines with
+// an end that reaches s, highest first).
+//
+// Where many queries with few hits share a window (SW_FEW), each lane answers its own: the
+// wave goes through the window's and the list's entries once for all of them.
+//
+// What bounds it: on 10M int32 intervals x 10M queries (122 hits a query) it issues 33 vector
+// and 39 scalar instructions a query, where the line walk with its shared emission chunks
+// issued 140 and 62, and takes 2.44 ms (3.65 ms before), 2.0 TB/s of positions.  What is left is
+// the writes: lists of 488 bytes that start anywhere leave two lines partly written each (the
+// same segments aligned to 256 bytes are written in 0.8 ms by a kernel that does nothing else,
+// unaligned in 1.8 ms).  100K queries on 10M: 66 us (143), 1M: 276 us (656), 4096: 14 us (111);
+// 3M queries with 1.2 hits each on 100K intervals: 108 us (116).
+//
+// A query is left to the wave-cooperative kernel (k_walk_heavy), which continues below the
+// run, when more than SW_CAP intervals hold its start, and when it ends below its own start's
+// lower bound (start > end).
+#pragma once
+
+constexpr int SW_THREADS = 256;
+constexpr int SW_WAVES = SW_THREADS / WAVE;
+constexpr int SW_REGS = 4;                        // list registers per lane
+constexpr uint32_t SW_CAP = SW_REGS * WAVE;       // entries of a list
+constexpr uint32_t SW_CHUNK = 256;                // most queries of a wave
+constexpr uint32_t SW_GAP = 8;                    // lines walked one by one before a list is collected anew
+
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// A value that is the same in every lane, in a scalar register (the compiler takes values that
+// leave a loop with ballots for lane-dependent ones; what they steer would then run on masks).
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+
+__device__ __forceinline__ int32_t read_lane(int32_t v, uint32_t l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ uint32_t read_lane(uint32_t v, uint32_t l) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, l);
+}
+__device__ __forceinline__ uint64_t read_lane(uint64_t v, uint32_t l) {
+    return (uint64_t)read_lane((uint32_t)(v >> 32), l) << 32 | read_lane((uint32_t)v, l);
+}
+__device__ __forceinline__ int64_t read_lane(int64_t v, uint32_t l) { return (int64_t)read_lane((uint64_t)v, l); }
+
+// Ascending bitonic sort of 64 * NR keys, element r * 64 + lane in k[r].
+template <int NR>
+__device__ __forceinline__ void wave_sort(uint32_t (&k)[NR], int lane) {
+#pragma unroll
+    for (int K = 2; K <= WAVE * NR; K <<= 1) {
+#pragma unroll
+        for (int J = K >> 1; J >= 1; J >>= 1) {
+            if (J >= WAVE) {
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    const int p = r | (J / WAVE);
+                    if (p != r) {
+                        const bool up = ((r * WAVE) & K) == 0;
+                        const uint32_t lo = min(k[r], k[p]), hi = max(k[r], k[p]);
+                        k[r] = up ? lo : hi;
+                        k[p] = up ? hi : lo;
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < NR; ++r) {
+                    const uint32_t o = __shfl_xor(k[r], J, WAVE);
+                    const bool up = ((r * WAVE + lane) & K) == 0, first = (lane & J) == 0;
+                    k[r] = (up == first) ? min(k[r], o) : max(k[r], o);
+                }
+            }
+        }
+    }
+}
+
+// The positions below line `line0` (64 positions a line) with an end >= s, descending, at
+// l_end / l_pay[0 .. n); returns n, or a number above SW_CAP when there are more (the entries
+// are then incomplete).  The payload is the position, or its value.
+template <typename S, bool VALUES>
+__device__ __forceinline__ uint32_t collect_holding(const S* __restrict__ ends, const int32_t* __restrict__ vals,
+                                                    const TreeDesc<S>& td, uint32_t line0, S s, int lane,
+                                                    S* __restrict__ l_end, uint32_t* __restrict__ l_pay) {
+    constexpr uint32_t NL = 4;   // lines with hits fetched per round trip
+    if (line0 == 0u || td.nlev < 2) return 0u;
+    const uint32_t hi_line = line0 - 1u;
+    uint32_t g1 = hi_line & ~63u, n = 0;
+    uint64_t rem = group_mask(td, g1, s, lane) & mask_upto(hi_line - g1);
+    while (true) {
+        if (rem == 0) {
+            if (g1 == 0u) break;
+            const uint32_t l = prev_line(td, g1, 0u, s, lane);
+            if (l == NONE) break;
+            g1 = l & ~63u;
+            rem = group_mask(td, g1, s, lane) & mask_upto(l - g1);
+            continue;
+        }
+        const uint32_t nv = min((uint32_t)__popcll(rem), NL);
+        uint32_t pay[NL];
+        S e[NL];
+#pragma unroll
+        for (uint32_t j = 0; j < NL; ++j) {
+            const uint32_t b = rem ? 63u - (uint32_t)__builtin_clzll(rem) : 0u;
+            if (rem) rem &= ~(1ull << b);
+            const uint32_t p = (g1 + b) * 64u + 63u - (uint32_t)lane;   // (past the last line: the group's first, unused)
+            e[j] = ends[p];
+            pay[j] = VALUES ? (uint32_t)vals[p] : p;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < NL; ++j) {
+            const bool h = j < nv && e[j] >= s;
+            const uint64_t m = __builtin_amdgcn_ballot_w64(h);
+            const uint32_t cnt = (uint32_t)__popcll(m);
+            if (n + cnt > SW_CAP) return n + cnt;   // wave-uniform
+            if (h) {
+                const uint32_t slot = n + lanes_below(m);
+                l_end[slot] = e[j];
+                l_pay[slot] = pay[j];
+            }
+            n += cnt;
+        }
+    }
+    return n;
+}
+
+// The queries of one sweep group as its lanes hold them, and the list they are answered from.
+template <typename S>
+struct SweepGroup {
+    S s;                 // query start
+    uint32_t ub, lb;     // upper_bound of the end, lower_bound of the start
+    uint64_t at;         // address of the query's first output slot
+    uint32_t room;       // output slots it may write
+    uint32_t found;      // its hits, written as they are found
+};
+
+// Answers the group's queries `todo` (a lane each): their run, then, with NB >= 0, the hits in
+// the window (we, wp: position wbase + 63 - lane) and in the first NB list registers.  Every
+// store goes through a buffer resource over the query's own slots, so slots past its room and
+// lanes without a hit (offset 0xFFFFFFFF) are dropped by the hardware.
+//
+// Everything the loop reads is waited for before it: a load still in flight at the loop's head
+// would put a wait for all memory operations, the stores of the query before included, into
+// every turn of the loop.
+template <typename S, int MODE, int NB>
+__device__ __forceinline__ void sweep_emit(SweepGroup<S>& g, uint64_t todo, int lane, uint32_t wbase, S& we, uint32_t& wp,
+                                           S (&le)[SW_REGS], uint32_t (&lp)[SW_REGS],
+                                           const int32_t* __restrict__ vals) {
+    constexpr bool VALUES = MODE == W_VALUES;
+    constexpr int NL = NB > 0 ? NB : 0;
+    const uint32_t lane4 = (uint32_t)lane * 4u;
+    asm volatile("" : "+v"(g.s), "+v"(g.ub), "+v"(g.lb), "+v"(g.at), "+v"(g.room));
+    if (NB >= 0) {
+        asm volatile("" : "+v"(we), "+v"(wp));
+#pragma unroll
+        for (int r = 0; r < NL; ++r) asm volatile("" : "+v"(le[r]), "+v"(lp[r]));
+    }
+    while (todo) {
+        const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+        todo &= todo - 1ull;
+        const uint32_t ub = read_lane(g.ub, j), lb = read_lane(g.lb, j);
+        uint32_t room = read_lane(g.room, j);
+        uint64_t at = read_lane(g.at, j);
+        uint64_t mw = 0, ml[NL + 1];
+        uint32_t lead = ub + 1u - lb, total = lead;   // (NONE + 1 = 0)
+        if (NB >= 0) {
+            const S s = read_lane(g.s, j);
+            const uint32_t d = (0u - lb) & 63u;   // window lanes from d on are below lb
+            mw = __builtin_amdgcn_ballot_w64(we >= s) & (~0ull << d);
+            total += (uint32_t)__popcll(mw);
+#pragma unroll
+            for (int r = 0; r < NL; ++r) {
+                ml[r] = __builtin_amdgcn_ballot_w64(le[r] >= s);   // (lanes past the list hold the smallest value)
+                total += (uint32_t)__popcll(ml[r]);
+            }
+            if (MODE == W_VECTOR) {
+                // the leading run: [lb, ub] and the positions right below it that are hits
+                const uint64_t miss = ~mw & (~0ull << d);
+                if (miss) {
+                    const uint32_t z = (uint32_t)__builtin_ctzll(miss);
+                    lead += z - d;
+                    mw &= ~0ull << z;
+                } else {
+                    lead += 64u - d;
+                    mw = 0;
+                    bool on = true;   // every position down to wbase is a hit: on into the list
+#pragma unroll
+                    for (int r = 0; r < NL; ++r) {
+                        if (on) {
+                            const uint64_t out_of = ~(ml[r] & __builtin_amdgcn_ballot_w64(
+                                                                  lp[r] == wbase - 1u - (uint32_t)(r * WAVE + lane)));
+                            if (out_of) {
+                                const uint32_t z = (uint32_t)__builtin_ctzll(out_of);
+                                lead += z;
+                                ml[r] &= ~0ull << z;
+                                on = false;
+                            } else {
+                                lead += 64u;
+                                ml[r] = 0;
+                            }
+                        }
+                    }
+                }
+            }
+        }
+        g.found = (uint32_t)lane == j ? total : g.found;
+        // the (leading) run
+        uint32_t p = (MODE == W_VECTOR) ? ub + 1u - lead + (uint32_t)lane : ub - (uint32_t)lane;
+        uint32_t w = min(lead, room);
+        if (w >= 8u * WAVE) {
+            global_u32* o = reinterpret_cast<global_u32*>((uintptr_t)at);
+            for (; w >= (uint32_t)WAVE; w -= WAVE) {
+                o[(uint32_t)lane] = VALUES ? (uint32_t)vals[p] : p;
+                o += WAVE;
+                p += (MODE == W_VECTOR) ? (uint32_t)WAVE : 0u - (uint32_t)WAVE;
+            }
+            const uint32_t done = (min(lead, room)) - w;
+            at += (uint64_t)done * 4u;
+            lead -= done;
+            room -= done;
+        }
+        // (at most 2^28 slots: everything below is within a few thousand of `at`)
+        {
+            const __amdgpu_buffer_rsrc_t rs =
+                __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at), (short)0, (int)(w * 4u), 0x00020000);
+            for (uint32_t x = 0; x < w; x += WAVE) {
+                // (lanes past the run read a value too: position 0's)
+                const uint32_t v = VALUES ? (uint32_t)vals[x + (uint32_t)lane < w ? p : 0u] : p;
+                __builtin_amdgcn_raw_buffer_store_b32(v, rs, lane4 + x * 4u, 0, 0);
+                p += (MODE == W_VECTOR) ? (uint32_t)WAVE : 0u - (uint32_t)WAVE;
+            }
+        }
+        if (NB >= 0) {
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                reinterpret_cast<void*>(at), (short)0, (int)(min(room, 1u << 28) * 4u), 0x00020000);
+            uint32_t k = lead;
+            auto put = [&](uint64_t mask, uint32_t pay) {
+                const uint32_t off = (lanes_below(mask) << 2) + k * 4u;
+                __builtin_amdgcn_raw_buffer_store_b32(pay, rs, __builtin_amdgcn_inverse_ballot_w64(mask) ? off : 0xFFFFFFFFu,
+                                                      0, 0);
+                k += (uint32_t)__popcll(mask);
+            };
+            if (w == lead) {   // (else the room ended inside the run)
+                put(mw, wp);
+#pragma unroll
+                for (int r = 0; r < NL; ++r) put(ml[r], lp[r]);
+            }
+        }
+    }
+}
+
+// Queries with at most this many hits are answered a lane each, when enough of them share a
+// window (sweep_lanes).
+constexpr uint32_t SW_FEW = 16;
+
+// Answers the queries `todo` a lane each: every lane writes its own run, then the wave goes
+// through the window's and the list's entries that reach `from` once, highest first, and each
+// lane takes those that reach its start.
+template <typename S, int MODE, bool LIST>
+__device__ __forceinline__ void sweep_lanes(SweepGroup<S>& g, uint64_t todo, int lane, uint32_t wbase, S from, const S& we,
+                                            const uint32_t& wp, const S (&le)[SW_REGS], const uint32_t (&lp)[SW_REGS],
+                                            uint32_t A, const int32_t* __restrict__ vals) {
+    constexpr bool VALUES = MODE == W_VALUES;
+    const bool mine = __builtin_amdgcn_inverse_ballot_w64(todo);
+    const uint32_t c = mine ? g.ub + 1u - g.lb : 0u;
+    const uint32_t d = (0u - g.lb) & 63u;   // window lanes from d on are below lb
+    // the window's entries below the largest lb
+    uint64_t cw = 0;
+    if (LIST) cw = __builtin_amdgcn_ballot_w64(we >= from) & (~0ull << ((0u - uniform(wave_max(mine ? g.lb : 0u))) & 63u));
+    // f(entry's end, payload, whether it lies below the lane's lb), highest position first
+    auto entries = [&](auto&& f) {
+        if (!LIST) return;
+        for (uint64_t m = cw; m; m &= m - 1ull) {
+            const uint32_t i = (uint32_t)__builtin_ctzll(m);
+            f(read_lane(we, i), read_lane(wp, i), i >= d);
+        }
+#pragma unroll
+        for (int r = 0; r < SW_REGS; ++r) {
+            if (A <= (uint32_t)(r * WAVE)) break;
+            uint64_t m = __builtin_amdgcn_ballot_w64(le[r] >= from && (uint32_t)(r * WAVE + lane) < A);
+            for (; m; m &= m - 1ull) {
+                const uint32_t i = (uint32_t)__builtin_ctzll(m);
+                f(read_lane(le[r], i), read_lane(lp[r], i), true);
+            }
+        }
+    };
+    uint32_t lead = c;
+    if (MODE == W_VECTOR)   // the leading run: [lb, ub] and the positions right below it that are hits
+        entries([&](S e, uint32_t p, bool below) { lead += (mine && below && e >= g.s && p == g.ub - lead) ? 1u : 0u; });
+    global_u32* const o = reinterpret_cast<global_u32*>((uintptr_t)g.at);
+    for (uint32_t x = 0; __builtin_amdgcn_ballot_w64(x < lead); ++x) {
+        const uint32_t p = (MODE == W_VECTOR) ? g.ub + 1u - lead + x : g.ub - x;
+        if (x < min(lead, g.room)) o[x] = VALUES ? (uint32_t)vals[p] : p;
+    }
+    uint32_t k = lead;
+    entries([&](S e, uint32_t p, bool below) {
+        // (in vector order the entries of the leading run, above ub - lead, are written already)
+        const bool h = mine && below && e >= g.s && (MODE != W_VECTOR || p < g.ub + 1u - lead);
+        if (h && k < g.room) o[k] = p;
+        k += h ? 1u : 0u;
+    });
+    g.found = mine ? k : g.found;
+}
+
+// One wave per chunk of `chunk` consecutive sorted queries (see above).  MODE: W_DESC,
+// W_VECTOR or W_VALUES; out: the positions or values as 32-bit words; only slots below cap
+// and inside a query's segment [offsets[q], offsets[q + 1]) are written.  Queries left to the
+// wave-cooperative kernel go to the plan's heavy list, their run already written (not in
+// vector order, where the run is part of the leading run).
+template <typename S, int MODE>
+__global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<S> td, PlanView<S> pv, uint32_t nq,
+                                                      uint32_t chunk, const uint64_t* __restrict__ offsets,
+                                                      uint32_t* __restrict__ out, const int32_t* __restrict__ vals,
+                                                      uint64_t cap) {
+    constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
+    constexpr bool VALUES = MODE == W_VALUES;
+    __shared__ S s_end[SW_WAVES][SW_CAP];
+    __shared__ uint32_t s_pay[SW_WAVES][SW_CAP];
+    __shared__ uint32_t s_key[SW_WAVES][SW_CHUNK];
+    const int lane = lane_id();
+    const uint32_t wv = uniform(threadIdx.x / WAVE);
+    S* const l_end = s_end[wv];
+    uint32_t* const l_pay = s_pay[wv];
+    uint32_t* const l_key = s_key[wv];
+    const uint64_t t0w = (uint64_t)(blockIdx.x * (uint32_t)SW_WAVES + wv) * chunk;
+    if (t0w >= nq) return;
+    const uint32_t t0 = (uint32_t)t0w;
+    const uint32_t m = min(chunk, nq - t0);   // this wave's queries
+
+    // ---- the chunk's queries in the order of their starts: keys (start - smallest) >> sh in
+    // 24 bits, query in 8
+    S smin;
+    uint32_t sh = 0;
+    {
+        S sv[SW_REGS];
+        S lo = pv.s[t0], hi = lo;
+        uint32_t off_line = 0;   // a query whose window is not the first one's
+        const uint32_t line0 = (uniform(pv.lb[t0]) - 1u) & ~63u;
+#pragma unroll
+        for (int r = 0; r < SW_REGS; ++r) {
+            const uint32_t i = (uint32_t)(r * WAVE + lane);
+            sv[r] = (i < m) ? pv.s[t0 + i] : lo;
+            off_line |= ((i < m) ? (pv.lb[t0 + i] - 1u) & ~63u : line0) ^ line0;
+        }
+#pragma unroll
+        for (int r = 0; r < SW_REGS; ++r) {
+            lo = min(lo, sv[r]);
+            hi = max(hi, sv[r]);
+        }
+        hi = wave_max(hi);
+        // (~v reverses the order of a signed type without overflow)
+        lo = (S)~wave_max((S)~lo);
+        smin = lo;
+        uint32_t key[SW_REGS];
+        if (__builtin_amdgcn_ballot_w64(off_line != 0u) == 0ull) {
+            // one window for all: no order is needed
+#pragma unroll
+            for (int r = 0; r < SW_REGS; ++r) key[r] = (uint32_t)(r * WAVE + lane);
+        } else {
+            const uint64_t span = (uint64_t)hi - (uint64_t)lo;
+            const uint32_t bits = span ? 64u - (uint32_t)__builtin_clzll(span) : 0u;
+            sh = uniform(bits > 24u ? bits - 24u : 0u);
+#pragma unroll
+            for (int r = 0; r < SW_REGS; ++r) {
+                const uint32_t i = (uint32_t)(r * WAVE + lane);
+                key[r] = (i < m) ? (uint32_t)(((uint64_t)sv[r] - (uint64_t)lo) >> sh) << 8 | i : 0xFFFFFFFFu;
+            }
+            if (m > (uint32_t)WAVE) {
+                wave_sort<SW_REGS>(key, lane);
+            } else if (m > 1u) {
+                uint32_t k1[1] = {key[0]};
+                wave_sort<1>(k1, lane);
+                key[0] = k1[0];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < SW_REGS; ++r) l_key[r * WAVE + lane] = key[r];
+        wave_lds_sync();
+    }
+
+    // ---- sweep
+    uint32_t lp[SW_REGS] = {0u, 0u, 0u, 0u};   // list: payloads and ends, A entries, descending
+    S le[SW_REGS] = {SMIN, SMIN, SMIN, SMIN};
+    uint32_t A = 0, wbase = NONE;               // wbase NONE: no list yet
+    S we = SMIN;                                // window: ends and payloads
+    uint32_t wp = 0, full = 0;                  // full: a list outgrew SW_CAP, the chunk's other queries are left too
+    bool bad = false;
+
+    // the packed entries l_end / l_pay[0 .. n) as the list
+    auto take_list = [&](uint32_t n) {
+        wave_lds_sync();
+        A = n;
+#pragma unroll
+        for (int r = 0; r < SW_REGS; ++r) {
+            const uint32_t i = (uint32_t)(r * WAVE + lane);
+            le[r] = (i < n) ? l_end[i] : SMIN;
+            lp[r] = (i < n) ? l_pay[i] : 0u;
+        }
+        wave_lds_sync();
+    };
+    auto load_window = [&]() {
+        const uint32_t p = wbase + 63u - (uint32_t)lane;
+        we = ix.ends[p];
+        wp = VALUES ? (uint32_t)vals[p] : p;
+    };
+
+    for (uint32_t g0 = 0; g0 < m; g0 += WAVE) {
+        // 64 queries in start order, one per lane
+        const bool mine = g0 + (uint32_t)lane < m;
+        const uint32_t gkey = l_key[min(g0 + (uint32_t)lane, m - 1u)];
+        const uint32_t gk = t0 + (gkey & 255u);
+        const uint32_t gq = pv.q[gk];
+        SweepGroup<S> g;
+        g.ub = pv.idx[gk];
+        g.lb = pv.lb[gk];
+        g.s = pv.s[gk];
+        const uint64_t go0 = offsets[gq], go1 = offsets[gq + 1];
+        const uint32_t gcnt = (uint32_t)(go1 - go0);
+        const uint64_t go = min(go0, cap), goe = min(go1, cap);
+        g.room = goe > go ? (uint32_t)min(goe - go, (uint64_t)0xFFFFFFFFu) : 0u;
+        g.at = (uint64_t)(uintptr_t)(out + go);
+        g.found = 0;
+        const uint32_t gline = (g.lb - 1u) & ~63u;
+        const bool ordered = g.lb <= g.ub + 1u;   // else start > end, with starts between the two
+        // queries whose hits all lie in their run, then those the list serves
+        const uint64_t runs = __builtin_amdgcn_ballot_w64(mine && ordered && g.lb == 0u);
+        uint64_t todo = __builtin_amdgcn_ballot_w64(mine && ordered && g.lb != 0u);
+        uint64_t left = __builtin_amdgcn_ballot_w64(mine && !ordered && g.ub != NONE);
+        const uint64_t few = __builtin_amdgcn_ballot_w64(mine && ordered && gcnt <= SW_FEW && g.ub + 1u - g.lb <= SW_FEW);
+        if (runs) {
+            const uint64_t rf = (uint32_t)__popcll(runs & few) >= 8u ? runs & few : 0ull;
+            if (rf) sweep_lanes<S, MODE, false>(g, rf, lane, 0u, smin, we, wp, le, lp, 0u, vals);
+            if (runs & ~rf) sweep_emit<S, MODE, -1>(g, runs & ~rf, lane, 0u, we, wp, le, lp, vals);
+        }
+        while (todo) {
+            if (full) {
+                if (MODE != W_VECTOR) sweep_emit<S, MODE, -1>(g, todo, lane, 0u, we, wp, le, lp, vals);
+                left |= todo;
+                break;
+            }
+            // the next query in start order, and all that share its window
+            const uint32_t j = (uint32_t)__builtin_ctzll(todo);
+            const uint32_t line = read_lane(gline, j);
+            if (line != wbase) {
+                // no start of the chunk's queries from here on is below this
+                const S from = (S)((uint64_t)smin + ((uint64_t)(read_lane(gkey, j) >> 8) << sh));
+                if (wbase == NONE || line < wbase || line - wbase > SW_GAP * 64u) {
+                    wbase = line;
+                    load_window();
+                    const uint32_t n =
+                        uniform(collect_holding<S, VALUES>(ix.ends, vals, td, line >> 6, from, lane, l_end, l_pay));
+                    if (n > SW_CAP) full = 1u;
+                    else take_list(n);
+                } else {
+                    do {
+                        // survivors of the window, then of the list, packed
+                        const uint64_t bw = __builtin_amdgcn_ballot_w64(we >= from);
+                        uint64_t bl[SW_REGS];
+                        uint32_t n = (uint32_t)__popcll(bw), at = n;
+#pragma unroll
+                        for (int r = 0; r < SW_REGS; ++r) {
+                            // (lanes past the list hold SMIN, which a from of SMIN would keep)
+                            bl[r] = __builtin_amdgcn_ballot_w64(le[r] >= from && (uint32_t)(r * WAVE + lane) < A);
+                            n += (uint32_t)__popcll(bl[r]);
+                        }
+                        if (n > SW_CAP) {
+                            full = 1u;
+                            break;
+                        }
+                        if (__builtin_amdgcn_inverse_ballot_w64(bw)) {
+                            l_end[lanes_below(bw)] = we;
+                            l_pay[lanes_below(bw)] = wp;
+                        }
+#pragma unroll
+                        for (int r = 0; r < SW_REGS; ++r) {
+                            if (__builtin_amdgcn_inverse_ballot_w64(bl[r])) {
+                                l_end[at + lanes_below(bl[r])] = le[r];
+                                l_pay[at + lanes_below(bl[r])] = lp[r];
+                            }
+                            at += (uint32_t)__popcll(bl[r]);
+                        }
+                        wbase += 64u;
+                        load_window();
+                        take_list(n);
+                    } while (wbase < line);
+                }
+                if (full) continue;
+            }
+            uint64_t same = todo & __builtin_amdgcn_ballot_w64(gline == wbase);
+            todo &= ~same;
+            // a query answered by the whole wave costs about 70 instructions, an entry that every lane looks at 20
+            const uint64_t sf = same & few;
+            const S low = (S)((uint64_t)smin + ((uint64_t)(read_lane(gkey, j) >> 8) << sh));   // no start is below
+            if ((uint32_t)__popcll(sf) * 3u >= (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(we >= low)) + A + SW_FEW) {
+                sweep_lanes<S, MODE, true>(g, sf, lane, wbase, low, we, wp, le, lp, A, vals);
+                same &= ~sf;
+                if (same == 0) continue;
+            }
+            if (A == 0u) sweep_emit<S, MODE, 0>(g, same, lane, wbase, we, wp, le, lp, vals);
+            else if (A <= (uint32_t)WAVE) sweep_emit<S, MODE, 1>(g, same, lane, wbase, we, wp, le, lp, vals);
+            else if (A <= 2u * WAVE) sweep_emit<S, MODE, 2>(g, same, lane, wbase, we, wp, le, lp, vals);
+            else sweep_emit<S, MODE, SW_REGS>(g, same, lane, wbase, we, wp, le, lp, vals);
+        }
+        const bool leave = (left >> lane) & 1ull;
+        bad |= mine && !leave && g.found != gcnt;
+        if (leave) {
+            // (per lane, outside every wave-wide step; the run [lb, ub] is written, but for the vector order)
+            const uint32_t c = ordered && MODE != W_VECTOR ? g.ub + 1u - g.lb : 0u;
+            HeavyEntry he;
+            he.k = gk;
+            he.cur = ordered ? g.lb - 1u : g.ub;
+            he.top = g.ub;
+            he.lead = MODE == W_VECTOR ? 1u : 0u;
+            he.acc = go + min(c, g.room);
+            he.left = gcnt - c;
+            he.pad = 0u;
+            pv.heavy[atomicAdd(&pv.counter[1], 1u)] = he;
+        }
+    }
+    if (bad) atomicOr(&pv.counter[3], 1u);   // a query's hits differ from its offsets
+}

@@ -1159,3 +1159,45 @@ def test_output_offsets_beyond_2_31(sia):
         assert bool((rows == row.to(torch.int32).to(dev)).all()), order
     del rows, idx
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n,nq,depth", [(1, 3, 1), (63, 64, 5), (64, 65, 64), (129, 257, 130), (5000, 1, 255),
+                                        (5000, 1023, 256), (5000, 1025, 257), (70_000, 70_001, 40),
+                                        (300_000, 4096, 300), (40_000, 300_000, 600), (100_000, 400_000, 1),
+                                        (3000, 400_000, 3)])
+def test_sweep_fill(sia, orc, dtype, n, nq, depth):
+    """The fill's sweep over query starts: lists of about `depth` intervals holding a point
+    (255, 256, 257 and more: around and past what the sweep keeps in registers), batches that
+    give a wave one query, part of a register and several, starts close together, in clusters
+    far apart and at the ends of the coordinate range, queries with start > end, and queries
+    past every interval; both orders and the values equal the oracle's."""
+    print(f"[gpu] sweep fill dtype={np.dtype(dtype).name} n={n} nq={nq} depth={depth}", flush=True)
+    rng = np.random.default_rng(n + nq + depth)
+    info = np.iinfo(dtype)
+    step = 7
+    s = np.sort(rng.integers(0, step * n + 1, n))
+    # lengths: exactly depth / step positions for most, a few long ones, a stretch of dense starts
+    e = s + np.where(rng.random(n) < 0.02, rng.integers(1, 50 * step * depth + 2, n), rng.integers(1, 2 * step * depth + 2, n))
+    e[: n // 50] += step * n // 3
+    qs = rng.integers(-50, step * n + 500, nq)
+    far = rng.random(nq)
+    qs = np.where(far < 0.05, rng.integers(step * n // 2, step * n // 2 + 40, nq), qs)
+    qe = qs + np.where(rng.random(nq) < 0.9, rng.integers(0, 40 * step, nq), rng.integers(-30 * step, 200 * step, nq))
+    qs[-1], qe[-1] = info.min, info.max
+    qs[0] = info.min if nq > 1 else qs[0]
+    if nq > 3:
+        qs[1], qe[1] = info.max, info.max
+        qs[2], qe[2] = info.max, info.min
+    s, e, qs, qe = (x.astype(dtype) for x in (s, e, qs, qe))
+    vals = (np.arange(n, dtype=np.int64) * 7 % 1_000_003).astype(np.int32)
+    ix = _dev_index(sia, s, e, vals)
+    oix = orc.build_index(s, e, vals)
+    for order, mode in (("desc", 0), ("vector", 1)):
+        off, idx = ix.search(qs, qe, order=order)
+        ooff, oidx = orc.search_batch(oix, qs, qe, mode=mode)
+        assert np.array_equal(off, ooff) and np.array_equal(idx.astype(np.int64), oidx), order
+    off, v = ix.search(qs, qe, values=True)
+    ooff, oidx = orc.search_batch(oix, qs, qe, mode=0)
+    assert np.array_equal(v, oix["data"][oidx])
+    ix.close()
