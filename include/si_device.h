@@ -87,6 +87,11 @@ void siIndexDestroy(siIndex* ix);
 int siIndexBuild(siIndex* ix, const void* starts, const void* ends, const int32_t* values,
                  size_t n, int start_sorted, int end_sorted, int on_device, void* stream);
 
+/* As siIndexBuild, but a flag below 0 is found on the device from the intervals in the given
+ * order, as add() would have left it (superintervals.hpp:95-105). */
+int siIndexBuildDetect(siIndex* ix, const void* starts, const void* ends, const int32_t* values,
+                       size_t n, int start_sorted, int end_sorted, int on_device, void* stream);
+
 /* Number of intervals in the built index (0 before the first build). */
 size_t siIndexSize(const siIndex* ix);
 

@@ -126,17 +126,15 @@ class DeviceIndex:
                 values = np.ascontiguousarray(values, dtype=np.int32)
         if len(starts) != len(ends):
             raise ValueError("starts and ends must have the same length")
-        if start_sorted is None or end_sorted is None:
-            if on_dev:
-                ss, es = add_flags(starts.cpu().numpy(), ends.cpu().numpy())
-            else:
-                ss, es = add_flags(starts, ends)
-            start_sorted = ss if start_sorted is None else start_sorted
-            end_sorted = es if end_sorted is None else end_sorted
+        detect = start_sorted is None or end_sorted is None
+        if detect and on_dev:   # found on the device; what the current stream still writes is waited for
+            import torch
+            torch.cuda.current_stream(starts.device).synchronize()
         n = len(starts)
-        N.check(N.lib.siIndexBuild(self._h, _ptr(starts), _ptr(ends), _ptr(values), n,
-                                   int(bool(start_sorted)), int(bool(end_sorted)), int(on_dev),
-                                   _stream_of(stream)), "siIndexBuild")
+        N.check(N.lib.siIndexBuildDetect(self._h, _ptr(starts), _ptr(ends), _ptr(values), n,
+                                         -1 if start_sorted is None else int(bool(start_sorted)),
+                                         -1 if end_sorted is None else int(bool(end_sorted)), int(on_dev),
+                                         _stream_of(stream)), "siIndexBuildDetect")
         self.n = n
         return self
 

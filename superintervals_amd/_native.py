@@ -48,6 +48,7 @@ _SIGS = {
     "siIndexCreate": (_vp, [_i]),
     "siIndexDestroy": (None, [_vp]),
     "siIndexBuild": (_i, [_vp, _vp, _vp, _vp, _sz, _i, _i, _i, _vp]),
+    "siIndexBuildDetect": (_i, [_vp, _vp, _vp, _vp, _sz, _i, _i, _i, _vp]),
     "siIndexSize": (_sz, [_vp]),
     "siIndexCoordBytes": (_i, [_vp]),
     "siIndexDownload": (_i, [_vp, _vp, _vp, _vp, _vp, _vp]),

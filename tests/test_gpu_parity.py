@@ -1201,3 +1201,55 @@ def test_sweep_fill(sia, orc, dtype, n, nq, depth):
     ooff, oidx = orc.search_batch(oix, qs, qe, mode=0)
     assert np.array_equal(v, oix["data"][oidx])
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [1, 2, 3, 64, 2047, 2048, 2049, 300_001])
+def test_build_finds_add_flags(sia, orc, dtype, n):
+    """The build finds the add() flags of intervals in the given order (on the device) as
+    add_flags does on the host: sorted inputs, one break or one rising tie at the first, the last
+    and a middle place, a tie after a break (which the flags do not see), extreme coordinates,
+    host arrays and device tensors; the permutation equals that of a build given add_flags'."""
+    import torch
+    print(f"[gpu] add flags dtype={np.dtype(dtype).name} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    info = np.iinfo(dtype)
+    s0 = np.sort(rng.integers(0, 4 * n, n)).astype(dtype)
+    e0 = (s0 + rng.integers(0, 50, n)).astype(dtype)
+    o = np.lexsort((-e0.astype(np.int64), s0))
+    s0, e0 = s0[o], e0[o]
+    cases = [(s0, e0)]
+    for k in sorted({0, n // 2, n - 2} & set(range(n - 1))):
+        s, e = s0.copy(), e0.copy()
+        s[k] = info.max                      # a break after k
+        cases.append((s, e))
+        s, e = s0.copy(), e0.copy()
+        s[k + 1:] = np.maximum(s[k + 1:], s[k] + 5)
+        s[k + 1] = s[k]
+        e[k], e[k + 1] = info.min, info.max  # a rising tie at k
+        cases.append((s, e))
+        s2 = s.copy()
+        s2[0] = info.max                     # the same after a break at 0
+        cases.append((s2, e))
+    ix, ref = sia.DeviceIndex(dtype), sia.DeviceIndex(dtype)
+    for s, e in cases:
+        ss, es = sia.add_flags(s, e) if dtype == np.int32 else (
+            bool((s[1:] >= s[:-1]).all()), _end_sorted(s, e))
+        want = ref.build(s, e, None, ss, es).download()
+        ts, te = torch.from_numpy(s).cuda(), torch.from_numpy(e).cuda()
+        for a, b in ((s, e), (ts, te)):
+            got = ix.build(a, b).download()
+            assert all(np.array_equal(got[k], want[k]) for k in ("starts", "ends", "perm", "branch"))
+        assert np.array_equal(ix.build(ts, te, None, start_sorted=ss).download()["perm"], want["perm"])
+    ix.close()
+    ref.close()
+
+
+def _end_sorted(s, e):
+    """add()'s end flag by comparisons (add_flags subtracts, which wraps at the int64 limits)."""
+    for k in range(s.size - 1):
+        if s[k + 1] < s[k]:
+            return True
+        if s[k + 1] == s[k] and e[k + 1] > e[k]:
+            return False
+    return True
