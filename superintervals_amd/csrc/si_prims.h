@@ -218,7 +218,7 @@ int device_excl_scan(const TI* in, size_t n, TO* out, TO* total, TO* ws, hipStre
 }
 
 // ============================================================================
-// Radix sort: stable LSD over 64-bit keys with a 32-bit payload
+// Radix sort: stable LSD over 32- or 64-bit keys, with a 32-bit payload or none
 // ============================================================================
 constexpr int RS_THREADS = 256;
 // 2048-item tiles: the scatter's LDS (keys, payloads, digit starts: 25 KB) lets six
@@ -234,7 +234,8 @@ constexpr int RS_BINS = 256;
 // each thread loads its RS_ROUNDS keys of a tile before counting them.  A digit equal in
 // every lane of a wave (the case this pass looks for) is added once by one lane; others
 // by one LDS atomic per lane.
-__global__ __launch_bounds__(RS_THREADS) void k_rs_hist8(const uint64_t* __restrict__ keys, size_t n, int dlo,
+template <typename K>
+__global__ __launch_bounds__(RS_THREADS) void k_rs_hist8(const K* __restrict__ keys, size_t n, int dlo,
                                                           int dhi, uint32_t* __restrict__ hist8 /*[8][256]*/) {
     __shared__ uint32_t h[8][RS_BINS];
     for (int k = threadIdx.x; k < 8 * RS_BINS; k += RS_THREADS) (&h[0][0])[k] = 0;
@@ -243,11 +244,11 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist8(const uint64_t* __restr
     for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const size_t base = t * RS_TILE;
         const uint32_t tile_n = (uint32_t)min((size_t)RS_TILE, n - base);
-        uint64_t key[RS_ROUNDS];
+        K key[RS_ROUNDS];
 #pragma unroll
         for (int r = 0; r < RS_ROUNDS; ++r) {
             const uint32_t li = (uint32_t)r * RS_THREADS + threadIdx.x;
-            key[r] = li < tile_n ? keys[base + li] : 0ull;
+            key[r] = li < tile_n ? keys[base + li] : (K)0;
         }
 #pragma unroll
         for (int r = 0; r < RS_ROUNDS; ++r) {
@@ -272,10 +273,17 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_hist8(const uint64_t* __restr
     }
 }
 
+// A pass's digit of a key.  flip = 0x80 on the top digit sorts the raw bits of signed numbers.
+template <typename K>
+__device__ __forceinline__ uint32_t rs_digit(K key, int shift, uint32_t flip) {
+    return ((uint32_t)(key >> shift) & 255u) ^ flip;
+}
+
 // Per-tile digit counts, digit-major: th[d * ntiles + tile].  A digit equal across a wave
 // is added once, from one lane.
-__global__ __launch_bounds__(RS_THREADS) void k_rs_tile_hist(const uint64_t* __restrict__ keys,
-                                                             size_t n, int shift,
+template <typename K>
+__global__ __launch_bounds__(RS_THREADS) void k_rs_tile_hist(const K* __restrict__ keys,
+                                                             size_t n, int shift, uint32_t flip,
                                                              uint32_t* __restrict__ th,
                                                              uint32_t ntiles) {
     __shared__ uint32_t h[RS_BINS];
@@ -288,7 +296,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_tile_hist(const uint64_t* __r
         const bool valid = i < n;
         const uint64_t vm = __builtin_amdgcn_ballot_w64(valid);
         if (vm == 0ull) continue;   // wave-uniform
-        const uint32_t digit = valid ? (uint32_t)(keys[i] >> shift) & 255u : 0u;
+        const uint32_t digit = valid ? rs_digit(keys[i], shift, flip) : 0u;
         const uint32_t d0 = __builtin_amdgcn_readfirstlane(digit);   // lane 0's: valid whenever any is
         if (__builtin_amdgcn_ballot_w64(valid && digit == d0) == vm) {
             if (lane_id() == 0) atomicAdd(&h[d0], (uint32_t)__popcll(vm));
@@ -308,7 +316,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_tile_hist(const uint64_t* __r
 // per digit over the 32 (round, wave) entries turns those numbers into each entry's start.
 // s_c (RS_ROUNDS * 4 rows of RS_BINS 16-bit counts) must be free on entry; it is free
 // again once every thread has passed a barrier after the call.
-__device__ __forceinline__ uint32_t rs_rank_tile(const uint64_t (&key)[RS_ROUNDS], uint32_t tile_n, int shift,
+template <typename K>
+__device__ __forceinline__ uint32_t rs_rank_tile(const K (&key)[RS_ROUNDS], uint32_t tile_n, int shift, uint32_t flip,
                                                  uint16_t (*s_c)[RS_BINS], uint32_t (&off)[RS_ROUNDS]) {
     const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
     uint32_t* const s_c32 = reinterpret_cast<uint32_t*>(&s_c[0][0]);
@@ -319,7 +328,7 @@ __device__ __forceinline__ uint32_t rs_rank_tile(const uint64_t (&key)[RS_ROUNDS
 #pragma unroll
     for (int r = 0; r < RS_ROUNDS; ++r) {
         const bool valid = (uint32_t)r * RS_THREADS + tid < tile_n;
-        const uint32_t digit = (uint32_t)(key[r] >> shift) & 255u;
+        const uint32_t digit = rs_digit(key[r], shift, flip);
         uint64_t peers = __builtin_amdgcn_ballot_w64(valid);
 #pragma unroll
         for (int b = 0; b < 8; ++b) {
@@ -340,7 +349,7 @@ __device__ __forceinline__ uint32_t rs_rank_tile(const uint64_t (&key)[RS_ROUNDS
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < RS_ROUNDS; ++r) off[r] += s_c[r * 4 + w][(uint32_t)(key[r] >> shift) & 255u];
+    for (int r = 0; r < RS_ROUNDS; ++r) off[r] += s_c[r * 4 + w][rs_digit(key[r], shift, flip)];
     return run;
 }
 
@@ -355,18 +364,25 @@ struct ArrayOut {
     }
 };
 
+// The sort's buffer of a sort without payload.
+template <typename K>
+struct KeyOut {
+    K* __restrict__ k;
+    __device__ __forceinline__ void put(size_t dst, K key, uint32_t) const { k[dst] = key; }
+};
+
 // Stable scatter of one tile (tile-major digit offsets from the scan of the per-tile digit
 // counts): the tile is ranked in registers, staged in LDS in digit order and written out so
 // equal digits land contiguously.
-template <class Out>
+template <class Out, typename K = uint64_t, bool VALS = true>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
-    const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin, Out out, size_t n, int shift,
+    const K* __restrict__ kin, const uint32_t* __restrict__ vin, Out out, size_t n, int shift, uint32_t flip,
     const uint32_t* __restrict__ th_base, uint32_t ntiles) {
     __shared__ union {
         uint16_t c[RS_ROUNDS * 4][RS_BINS];
-        uint64_t key[RS_TILE];
+        K key[RS_TILE];
     } s_u;
-    __shared__ uint32_t s_val[RS_TILE];
+    __shared__ uint32_t s_val[VALS ? RS_TILE : 1];
     __shared__ uint32_t s_dstart[RS_BINS];
     __shared__ uint32_t s_w[4];
 
@@ -374,24 +390,24 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     const uint32_t tile = blockIdx.x;
     const size_t base = (size_t)tile * RS_TILE;
     const uint32_t tile_n = (uint32_t)min((size_t)RS_TILE, n - base);
-    uint64_t key[RS_ROUNDS];
+    K key[RS_ROUNDS];
     uint32_t val[RS_ROUNDS], off[RS_ROUNDS];
 #pragma unroll
     for (int r = 0; r < RS_ROUNDS; ++r) {
         const uint32_t li = (uint32_t)r * RS_THREADS + tid;
-        key[r] = li < tile_n ? kin[base + li] : 0ull;
-        val[r] = li < tile_n ? vin[base + li] : 0u;
+        key[r] = li < tile_n ? kin[base + li] : (K)0;
+        val[r] = VALS && li < tile_n ? vin[base + li] : 0u;
     }
-    const uint32_t cnt = rs_rank_tile(key, tile_n, shift, s_u.c, off);
+    const uint32_t cnt = rs_rank_tile(key, tile_n, shift, flip, s_u.c, off);
     uint32_t tot;
     s_dstart[tid] = block_excl_scan256<uint32_t>(cnt, s_w, &tot);   // its barriers free s_u.c
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < RS_ROUNDS; ++r) {
         if ((uint32_t)r * RS_THREADS + tid < tile_n) {
-            const uint32_t slot = s_dstart[(uint32_t)(key[r] >> shift) & 255u] + off[r];
+            const uint32_t slot = s_dstart[rs_digit(key[r], shift, flip)] + off[r];
             s_u.key[slot] = key[r];
-            s_val[slot] = val[r];
+            if (VALS) s_val[slot] = val[r];
         }
     }
     __syncthreads();
@@ -399,10 +415,10 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     for (int r = 0; r < RS_ROUNDS; ++r) {
         const uint32_t slot = (uint32_t)r * RS_THREADS + tid;
         if (slot < tile_n) {
-            const uint64_t k = s_u.key[slot];
-            const uint32_t digit = (uint32_t)(k >> shift) & 255u;
+            const K k = s_u.key[slot];
+            const uint32_t digit = rs_digit(k, shift, flip);
             const size_t dst = (size_t)th_base[(size_t)digit * ntiles + tile] + (slot - s_dstart[digit]);
-            out.put(dst, k, s_val[slot]);
+            out.put(dst, k, VALS ? s_val[slot] : 0u);
         }
     }
 }
@@ -445,12 +461,62 @@ __global__ void k_zero_u64(uint64_t* __restrict__ p, size_t n) {
     if (i < n) p[i] = 0;
 }
 
+// Histograms of key digits [dlo, dhi) of n > 0 keys, read back into h8 ([8][256], zeroed by
+// the caller; synchronises the stream).
+template <typename K>
+int rs_digit_hist(const K* keys, size_t n, int dlo, int dhi, const RsTemp& tmp, uint32_t* h8, hipStream_t st) {
+    k_zero_u32<<<grid_for(8 * RS_BINS, 256), 256, 0, st>>>(tmp.hist8, 8 * RS_BINS);
+    LAUNCH_CHECK();
+    const unsigned hb = (unsigned)std::min<size_t>(rs_ntiles(n), 1024);
+    k_rs_hist8<K><<<hb, RS_THREADS, 0, st>>>(keys, n, dlo, dhi, tmp.hist8);
+    LAUNCH_CHECK();
+    HIP_TRY(hipMemcpyAsync(h8, tmp.hist8, 8 * RS_BINS * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    return SI_OK;
+}
+
+// True when digit d is equal for all n keys.
+inline bool rs_digit_constant(const uint32_t* h8, int d, size_t n) {
+    for (int b = 0; b < RS_BINS; ++b)
+        if (h8[d * RS_BINS + b] == n) return true;
+    return false;
+}
+
+// Ascending sort of n signed numbers given by their raw bits, by the digits d with run[d] (the
+// others are equal for all of them; at least one must be set): in -> out, through the buffers
+// k0 and k1.  in is not written; out may not be in, k0 or k1.
+template <typename K>
+int radix_sort_signed(const K* in, K* k0, K* k1, K* out, size_t n, const bool (&run)[8], const RsTemp& tmp,
+                      hipStream_t st) {
+    const uint32_t ntiles = (uint32_t)rs_ntiles(n);
+    int last_d = -1;
+    for (int d = 0; d < (int)sizeof(K); ++d)
+        if (run[d]) last_d = d;
+    const K* src = in;
+    for (int d = 0; d <= last_d; ++d) {
+        if (!run[d]) continue;
+        const uint32_t flip = (d == (int)sizeof(K) - 1) ? 0x80u : 0u;
+        K* const dst = (d == last_d) ? out : k0;
+        k_rs_tile_hist<K><<<ntiles, RS_THREADS, 0, st>>>(src, n, 8 * d, flip, tmp.th, ntiles);
+        LAUNCH_CHECK();
+        const int rc = device_excl_scan<uint32_t, uint32_t>(tmp.th, (size_t)ntiles * RS_BINS, tmp.tb, nullptr, tmp.ws, st);
+        if (rc != SI_OK) return rc;
+        k_rs_scatter<KeyOut<K>, K, false><<<ntiles, RS_THREADS, 0, st>>>(src, nullptr, KeyOut<K>{dst}, n, 8 * d, flip,
+                                                                         tmp.tb, ntiles);
+        LAUNCH_CHECK();
+        src = dst;
+        std::swap(k0, k1);
+    }
+    return SI_OK;
+}
+
 // Stable sort of (keys, vals) by key digits [digit_lo, digit_hi) (8-bit digits,
 // least significant first).  Digits that are equal for every key are skipped, which
 // needs one host read-back of the digit histograms; skip_constant = false sorts every
 // digit in [digit_lo, digit_hi) with no read-back, so the sort can be captured in a graph.
 // tmp comes from rs_temp_carve.  On return *keys_sorted / *vals_sorted point at whichever
 // buffer holds the result.
+// known_hist (optional, [8][256]): the keys' digit histograms, when the caller has read them back.
 // With last (optional), the last pass run writes the sorted items through it instead of
 // into the buffers, and *last_written says whether one ran; only if none ran are the
 // items in *keys_sorted / *vals_sorted.
@@ -458,21 +524,18 @@ template <class LastOut = ArrayOut>
 int radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n,
                      int digit_lo, int digit_hi, const RsTemp& tmp, uint64_t** keys_sorted,
                      uint32_t** vals_sorted, hipStream_t st, bool skip_constant = true,
-                     const LastOut* last = nullptr, bool* last_written = nullptr) {
+                     const LastOut* last = nullptr, bool* last_written = nullptr,
+                     const uint32_t* known_hist = nullptr) {
     if (last_written) *last_written = false;
     *keys_sorted = k0;
     *vals_sorted = v0;
     if (n < 2) return SI_OK;
-    uint32_t h8[8 * RS_BINS] = {0};
-    if (skip_constant) {
-        k_zero_u32<<<grid_for(8 * RS_BINS, 256), 256, 0, st>>>(tmp.hist8, 8 * RS_BINS);
-        LAUNCH_CHECK();
-        const unsigned hb = (unsigned)std::min<size_t>(rs_ntiles(n), 1024);
-        k_rs_hist8<<<hb, RS_THREADS, 0, st>>>(k0, n, digit_lo, digit_hi, tmp.hist8);
-        LAUNCH_CHECK();
-        HIP_TRY(hipMemcpyAsync(h8, tmp.hist8, sizeof(h8), hipMemcpyDeviceToHost, st));
-        HIP_TRY(hipStreamSynchronize(st));
+    uint32_t h[8 * RS_BINS] = {0};
+    if (skip_constant && !known_hist) {
+        const int rc = rs_digit_hist(k0, n, digit_lo, digit_hi, tmp, h, st);
+        if (rc != SI_OK) return rc;
     }
+    const uint32_t* const h8 = known_hist ? known_hist : h;
 
     const uint32_t ntiles = (uint32_t)rs_ntiles(n);
     const size_t nth = (size_t)ntiles * RS_BINS;
@@ -481,24 +544,22 @@ int radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, siz
     bool sort_digit[8] = {false};   // the digits sorted: all but those constant over the keys
     int last_d = -1;
     for (int d = digit_lo; d < digit_hi; ++d) {
-        bool constant = false;
-        for (int b = 0; skip_constant && b < RS_BINS; ++b)
-            if (h8[d * RS_BINS + b] == n) { constant = true; break; }
-        sort_digit[d] = !constant;
-        if (!constant) last_d = d;
+        sort_digit[d] = !(skip_constant && rs_digit_constant(h8, d, n));
+        if (sort_digit[d]) last_d = d;
     }
     for (int d = digit_lo; d < digit_hi; ++d) {
         if (!sort_digit[d]) continue;
         const int shift = 8 * d;
-        k_rs_tile_hist<<<ntiles, RS_THREADS, 0, st>>>(ka, n, shift, tmp.th, ntiles);
+        k_rs_tile_hist<uint64_t><<<ntiles, RS_THREADS, 0, st>>>(ka, n, shift, 0u, tmp.th, ntiles);
         LAUNCH_CHECK();
         int rc = device_excl_scan<uint32_t, uint32_t>(tmp.th, nth, tmp.tb, nullptr, tmp.ws, st);
         if (rc != SI_OK) return rc;
         if (last && d == last_d) {
-            k_rs_scatter<LastOut><<<ntiles, RS_THREADS, 0, st>>>(ka, va, *last, n, shift, tmp.tb, ntiles);
+            k_rs_scatter<LastOut><<<ntiles, RS_THREADS, 0, st>>>(ka, va, *last, n, shift, 0u, tmp.tb, ntiles);
             if (last_written) *last_written = true;
         } else {
-            k_rs_scatter<ArrayOut><<<ntiles, RS_THREADS, 0, st>>>(ka, va, ArrayOut{kb, vb}, n, shift, tmp.tb, ntiles);
+            k_rs_scatter<ArrayOut><<<ntiles, RS_THREADS, 0, st>>>(ka, va, ArrayOut{kb, vb}, n, shift, 0u, tmp.tb,
+                                                                    ntiles);
         }
         LAUNCH_CHECK();
         std::swap(ka, kb);

@@ -1253,3 +1253,86 @@ def _end_sorted(s, e):
         if s[k + 1] == s[k] and e[k + 1] > e[k]:
             return False
     return True
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [1, 2, 15, 16, 17, 63, 64, 65, 255, 256, 257, 4097, 70_001])
+def test_build_shapes_of_ends(sia, orc, dtype, n):
+    """The build against the oracle (sorted arrays, permutation, branch, payload) at the edges of
+    the 16-ary max tree's groups and levels, for ends that rise (every branch open to the left,
+    none found), fall (each branch the neighbour), are equal, saw-tooth over groups, reach back
+    to one far position, hold the type's extremes, and for starts in runs of equal values: of up
+    to 32 (mended in place) and longer (sorted by both coordinates), all equal, with equal pairs;
+    presorted or not."""
+    print(f"[gpu] build shapes dtype={np.dtype(dtype).name} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    info = np.iinfo(dtype)
+    i = np.arange(n, dtype=np.int64)
+    shapes = {
+        "rising": (i * 3, i * 3 + 1), "falling": (i, 2 * n - i), "equal ends": (i, np.full(n, n)),
+        "saw": (i, i + (16 - i % 16) * 5), "back": (i, np.where(i == n // 3, 10 * n, i)),
+        "runs": (i // 32, rng.integers(0, 40, n)), "runs of 33": (i // 33, rng.integers(0, 40, n)),
+        "one start": (np.zeros(n, np.int64), rng.integers(0, 10, n)),
+        "pairs": (rng.integers(0, n // 4 + 1, n), rng.integers(-5, 5, n)),
+        "random": (rng.integers(0, 10 * n, n), rng.integers(0, 10 * n, n)),
+    }
+    ends = np.array([info.min, info.max, info.max - 1, info.min + 1, 0], dtype=np.int64)
+    shapes["extremes"] = (rng.choice(ends, n), rng.choice(ends, n))
+    from superintervals_amd import autotune
+    ix = sia.DeviceIndex(dtype)
+    saved = autotune.current()
+    try:
+        for name, (s, e) in shapes.items():
+            for shuffled in (False, True):
+                o = rng.permutation(n) if shuffled else i
+                a, b = s[o].astype(dtype), e[o].astype(dtype)
+                autotune.apply(saved)
+                got = ix.build(a, b, i.astype(np.int32)).download(values=True)
+                want = orc.build_index(a, b, i.astype(np.int32))
+                for key in ("starts", "ends", "branch"):
+                    assert np.array_equal(got[key], want[key]), (name, shuffled, key)
+                assert np.array_equal(got["values"], want["data"]), (name, shuffled)
+                assert np.array_equal(got["perm"], want["data"]), (name, shuffled)
+                # the line walk reads the exits
+                q = np.concatenate([a[:50], b[:50], rng.integers(0, 10 * n, 50).astype(dtype)])
+                autotune.apply({"count_rank": 0, "range_skip": 0})
+                assert np.array_equal(ix.count(q, q), orc.count_batch(want, q, q)), (name, shuffled)
+    finally:
+        autotune.apply(saved)
+    ix.close()
+
+
+def test_builds_from_threads_keep_their_blocks(sia, orc):
+    """Indexes built, rebuilt (larger, smaller, empty) and destroyed from several threads at once,
+    on streams of their own: every index stays what its own intervals give (the device blocks
+    that builds pass on to one another never serve two at a time)."""
+    import threading
+    import torch
+    print("[gpu] builds from threads", flush=True)
+    errors = []
+
+    def work(seed):
+        try:
+            rng = np.random.default_rng(seed)
+            st = torch.cuda.Stream()
+            live = []
+            for k, n in enumerate((70_000, 500, 90_000, 0, 66_000, 120_000)):
+                s = rng.integers(0, 1_000_000, n).astype(np.int32)
+                e = (s + rng.integers(0, 3000, n)).astype(np.int32)
+                ix = live.pop()[0] if k % 2 and live else sia.DeviceIndex(np.int32)
+                live.append((ix.build(s, e, stream=st), orc.build_index(s, e)))
+                for a, want in live:
+                    got = a.download()
+                    for key in ("starts", "ends", "branch"):
+                        assert np.array_equal(got[key], want[key]), (seed, k, key)
+            for a, _ in live:
+                a.close()
+        except BaseException as x:   # noqa: B902
+            errors.append(x)
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors[0]
