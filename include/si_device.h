@@ -130,7 +130,7 @@ double siIndexLastBuildMs(const siIndex* ix);
  *                  count descend 64-ary trees of first keys (top level of at most 4096
  *                  keys in Eytzinger order in LDS, then one 64-key node per level) over
  *                  the starts / the sorted ends; 0: plain halving
- *   "plan_sync"    1 (default): siPlanQueries reads the key-digit histograms back once to
+ *   "plan_sync"    1 (default): siPlanQueries reads back once which key bits vary to
  *                  skip constant digits (one stream synchronisation); 0: it sorts every
  *                  digit without a read-back, so the planned calls can be graph-captured
  *   "heavy_ends32" 1 (default): the wave-cooperative walk of an int64 index whose ends

@@ -205,40 +205,50 @@ __global__ void k_pad(S* __restrict__ st, S* __restrict__ en, int32_t* __restric
 
 // Sort keys and payload (the input position).  int32: (start asc, end desc) in one 64-bit
 // unsigned order, so the sorted keys hold both coordinates; int64: the start.
-__global__ void k_keys_i32(const int32_t* __restrict__ s, const int32_t* __restrict__ e, uint64_t* __restrict__ key,
-                           uint32_t* __restrict__ val, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        uint32_t hs = (uint32_t)s[i] ^ 0x80000000u;
-        uint32_t le = ~((uint32_t)e[i] ^ 0x80000000u);
-        key[i] = ((uint64_t)hs << 32) | le;
+__global__ __launch_bounds__(RS_THREADS) void k_keys_i32(const int32_t* __restrict__ s, const int32_t* __restrict__ e,
+                                                         uint64_t* __restrict__ key, uint32_t* __restrict__ val, size_t n,
+                                                         uint64_t* __restrict__ bits) {
+    rs_each_key(n, bits, [&](size_t i) {
+        const uint32_t hs = (uint32_t)s[i] ^ 0x80000000u;
+        const uint32_t le = ~((uint32_t)e[i] ^ 0x80000000u);
+        const uint64_t k = ((uint64_t)hs << 32) | le;
+        key[i] = k;
         val[i] = (uint32_t)i;
-    }
+        return k;
+    });
 }
-__global__ void k_keys_i64(const int64_t* __restrict__ s, uint64_t* __restrict__ key, uint32_t* __restrict__ val,
-                           size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        key[i] = (uint64_t)s[i] ^ 0x8000000000000000ull;
+__global__ __launch_bounds__(RS_THREADS) void k_keys_i64(const int64_t* __restrict__ s, uint64_t* __restrict__ key,
+                                                         uint32_t* __restrict__ val, size_t n, uint64_t* __restrict__ bits) {
+    rs_each_key(n, bits, [&](size_t i) {
+        const uint64_t k = (uint64_t)s[i] ^ 0x8000000000000000ull;
+        key[i] = k;
         val[i] = (uint32_t)i;
-    }
+        return k;
+    });
 }
 
 // int64 by end descending, the first of two stable sorts when runs of equal starts are long.
-__global__ void k_key_end_desc_i64(const int64_t* __restrict__ e, uint64_t* __restrict__ key, uint32_t* __restrict__ val,
-                                   size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        key[i] = ~((uint64_t)e[i] ^ 0x8000000000000000ull);
+__global__ __launch_bounds__(RS_THREADS) void k_key_end_desc_i64(const int64_t* __restrict__ e, uint64_t* __restrict__ key,
+                                                                 uint32_t* __restrict__ val, size_t n,
+                                                                 uint64_t* __restrict__ bits) {
+    rs_each_key(n, bits, [&](size_t i) {
+        const uint64_t k = ~((uint64_t)e[i] ^ 0x8000000000000000ull);
+        key[i] = k;
         val[i] = (uint32_t)i;
-    }
+        return k;
+    });
 }
 
 // int64 second pass key: start ascending, gathered through the first pass's order.
-__global__ void k_key_start_i64(const int64_t* __restrict__ s, const uint32_t* __restrict__ order,
-                                uint64_t* __restrict__ key, size_t n) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) key[i] = (uint64_t)s[order[i]] ^ 0x8000000000000000ull;
+__global__ __launch_bounds__(RS_THREADS) void k_key_start_i64(const int64_t* __restrict__ s,
+                                                              const uint32_t* __restrict__ order,
+                                                              uint64_t* __restrict__ key, size_t n,
+                                                              uint64_t* __restrict__ bits) {
+    rs_each_key(n, bits, [&](size_t i) {
+        const uint64_t k = (uint64_t)s[order[i]] ^ 0x8000000000000000ull;
+        key[i] = k;
+        return k;
+    });
 }
 
 // The sort's last pass writes the index's arrays: the coordinates from the key where it holds
@@ -713,43 +723,43 @@ struct BuildScratch {
 // runs of equal starts by end (k_fix_ties); full = true sorts by (start, end) instead.
 template <typename S>
 int sort_intervals(siIndex* ix, const S* in_s, const S* in_e, const int32_t* in_v, size_t n, bool full, uint64_t* k0,
-                   uint64_t* k1, uint32_t* v0, uint32_t* v1, const RsTemp& rt, BuildInfo* info, bool* end_const,
+                   uint64_t* k1, uint32_t* v0, uint32_t* v1, const RsTemp& rt, BuildInfo* info, uint64_t* varying,
                    hipStream_t st) {
-    const unsigned g = grid_for(n, 256);
+    const unsigned g = grid_for(n, 256), gk = rs_bits_grid(n);
     uint64_t* ks;
     uint32_t* vs;
     bool written = false;
     int rc;
     if constexpr (sizeof(S) == 4) {
         const BuildOutI32 out{(int32_t*)ix->d_starts, (int32_t*)ix->d_ends, ix->d_perm, ix->d_values, in_v};
-        k_keys_i32<<<g, 256, 0, st>>>(in_s, in_e, k0, v0, n);
+        k_keys_i32<<<gk, RS_THREADS, 0, st>>>(in_s, in_e, k0, v0, n, rt.bits);
         LAUNCH_CHECK();
-        // one histogram of all eight digits: the starts' for this sort, the ends' for theirs
-        std::vector<uint32_t> h8(8 * RS_BINS, 0u);
-        if ((rc = rs_digit_hist(k0, n, 0, 8, rt, h8.data(), st)) != SI_OK) return rc;
-        for (int d = 0; d < 4; ++d) end_const[d] = rs_digit_constant(h8.data(), d, n);
-        rc = radix_sort_pairs(k0, v0, k1, v1, n, full ? 0 : 4, 8, rt, &ks, &vs, st, true, &out, &written, h8.data());
+        if ((rc = rs_varying_bits(n, rt, varying, st)) != SI_OK) return rc;
+        rc = radix_sort_pairs(k0, v0, k1, v1, n, full ? 0 : 4, 8, rt, &ks, &vs, st, *varying, &out, &written);
         if (rc != SI_OK) return rc;
+        *varying &= 0xFFFFFFFFull;   // the ends', for their sort
         if (!written) k_write_items<BuildOutI32><<<g, 256, 0, st>>>(ks, vs, n, out);
     } else {
         const BuildOutI64 out{(int64_t*)ix->d_starts, (int64_t*)ix->d_ends, ix->d_perm, ix->d_values, in_v,
                               (const int64_t*)in_e};
-        uint64_t *ka = k0, *kb = k1;
+        uint64_t *ka = k0, *kb = k1, vary = 0;
         uint32_t *va = v0, *vb = v1;
         if (full) {   // two stable sorts: end descending, then start ascending
-            k_key_end_desc_i64<<<g, 256, 0, st>>>((const int64_t*)in_e, k0, v0, n);
+            k_key_end_desc_i64<<<gk, RS_THREADS, 0, st>>>((const int64_t*)in_e, k0, v0, n, rt.bits);
             LAUNCH_CHECK();
-            if ((rc = radix_sort_pairs(k0, v0, k1, v1, n, 0, 8, rt, &ks, &vs, st)) != SI_OK) return rc;
+            if ((rc = rs_varying_bits(n, rt, &vary, st)) != SI_OK) return rc;
+            if ((rc = radix_sort_pairs(k0, v0, k1, v1, n, 0, 8, rt, &ks, &vs, st, vary)) != SI_OK) return rc;
             ka = (ks == k0) ? k1 : k0;   // the free key buffer
             kb = ks;
             va = vs;
             vb = (vs == v0) ? v1 : v0;
-            k_key_start_i64<<<g, 256, 0, st>>>((const int64_t*)in_s, va, ka, n);
+            k_key_start_i64<<<gk, RS_THREADS, 0, st>>>((const int64_t*)in_s, va, ka, n, rt.bits);
         } else {
-            k_keys_i64<<<g, 256, 0, st>>>((const int64_t*)in_s, ka, va, n);
+            k_keys_i64<<<gk, RS_THREADS, 0, st>>>((const int64_t*)in_s, ka, va, n, rt.bits);
         }
         LAUNCH_CHECK();
-        rc = radix_sort_pairs(ka, va, kb, vb, n, 0, 8, rt, &ks, &vs, st, true, &out, &written);
+        if ((rc = rs_varying_bits(n, rt, &vary, st)) != SI_OK) return rc;
+        rc = radix_sort_pairs(ka, va, kb, vb, n, 0, 8, rt, &ks, &vs, st, vary, &out, &written);
         if (rc != SI_OK) return rc;
         if (!written) k_write_items<BuildOutI64><<<g, 256, 0, st>>>(ks, vs, n, out);
     }
@@ -861,7 +871,7 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     struct { BuildInfo info; char gap[align256(sizeof(BuildInfo)) - sizeof(BuildInfo)]; int64_t lens[LEN_SAMPLE]; } back;
     for (bool full = false;; full = true) {
         // ---- the sorted arrays
-        bool end_const[8] = {false};   // digits of the ends that are equal for all of them
+        uint64_t varying = 0;   // the ends' bits that vary
         bool known = false;
         if (presorted) {
             k_iota<<<grid_for(n, 256), 256, 0, st>>>(ix->d_perm, n);
@@ -870,7 +880,7 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
             HIP_TRY(hipMemcpyAsync(ix->d_ends, in_e, nb, hipMemcpyDeviceToDevice, st));
             if (values) HIP_TRY(hipMemcpyAsync(ix->d_values, in_v, n * 4, hipMemcpyDeviceToDevice, st));
         } else {
-            const int rc = sort_intervals<S>(ix, in_s, in_e, in_v, n, full, k0, k1, v0, v1, rt, info, end_const, st);
+            const int rc = sort_intervals<S>(ix, in_s, in_e, in_v, n, full, k0, k1, v0, v1, rt, info, &varying, st);
             if (rc != SI_OK) return rc;
             known = sizeof(S) == 4;
         }
@@ -879,15 +889,13 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
             using K = typename std::conditional<sizeof(S) == 4, uint32_t, uint64_t>::type;
             const K* raw = (const K*)ix->d_ends;
             if (!known) {
-                std::vector<uint32_t> h8(8 * RS_BINS, 0u);
-                const int rc = rs_digit_hist(raw, n, 0, (int)sizeof(S), rt, h8.data(), st);
+                k_rs_bits<K><<<rs_bits_grid(n), RS_THREADS, 0, st>>>(raw, n, rt.bits);
+                LAUNCH_CHECK();
+                const int rc = rs_varying_bits(n, rt, &varying, st);
                 if (rc != SI_OK) return rc;
-                for (int d = 0; d < (int)sizeof(S); ++d) end_const[d] = rs_digit_constant(h8.data(), d, n);
             }
-            bool run[8] = {false}, any = false;
-            for (int d = 0; d < (int)sizeof(S); ++d) any |= (run[d] = !end_const[d]);
-            if (any) {
-                const int rc = radix_sort_signed<K>(raw, (K*)k0, (K*)k1, (K*)ix->d_ends_sorted, n, run, rt, st);
+            if (varying) {
+                const int rc = radix_sort_signed<K>(raw, (K*)k0, (K*)k1, (K*)ix->d_ends_sorted, n, varying, rt, st);
                 if (rc != SI_OK) return rc;
             } else {   // all ends equal
                 HIP_TRY(hipMemcpyAsync(ix->d_ends_sorted, ix->d_ends, nb, hipMemcpyDeviceToDevice, st));

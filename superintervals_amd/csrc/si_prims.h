@@ -230,47 +230,62 @@ constexpr int RS_ROUNDS = SI_RS_ROUNDS;   // rounds of 256 items per tile
 constexpr int RS_TILE = RS_THREADS * RS_ROUNDS;   // items per tile
 constexpr int RS_BINS = 256;
 
-// Histograms of digits [dlo, dhi) at once (to skip constant-digit passes), tile by tile:
-// each thread loads its RS_ROUNDS keys of a tile before counting them.  A digit equal in
-// every lane of a wave (the case this pass looks for) is added once by one lane; others
-// by one LDS atomic per lane.
-template <typename K>
-__global__ __launch_bounds__(RS_THREADS) void k_rs_hist8(const K* __restrict__ keys, size_t n, int dlo,
-                                                          int dhi, uint32_t* __restrict__ hist8 /*[8][256]*/) {
-    __shared__ uint32_t h[8][RS_BINS];
-    for (int k = threadIdx.x; k < 8 * RS_BINS; k += RS_THREADS) (&h[0][0])[k] = 0;
+// Which bits of a sort's keys vary: the kernel that writes (or reads) the keys leaves the AND and
+// the OR of its block's in slots[2 * block], [2 * block + 1], and the host joins them.  A digit
+// whose bits are all alike needs no pass.  (Histograms of every digit, in a pass of their own,
+// said the same for 63 us of a 10M-key sort.)
+constexpr unsigned RS_BITS_BLOCKS = 1024;   // most blocks of a kernel that leaves them
+constexpr unsigned RS_BITS_ITEMS = 4;       // items a thread takes at a time in such a kernel
+inline unsigned rs_bits_grid(size_t n) {
+    return (unsigned)std::min<size_t>((n + RS_THREADS * RS_BITS_ITEMS - 1) / (RS_THREADS * RS_BITS_ITEMS), RS_BITS_BLOCKS);
+}
+
+__device__ __forceinline__ void rs_block_bits(uint64_t all_and, uint64_t all_or, uint64_t* __restrict__ slots) {
+    __shared__ uint64_t s_and[RS_THREADS / WAVE], s_or[RS_THREADS / WAVE];
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        all_and &= __shfl_xor(all_and, d, WAVE);
+        all_or |= __shfl_xor(all_or, d, WAVE);
+    }
+    if (lane_id() == 0) {
+        s_and[threadIdx.x >> 6] = all_and;
+        s_or[threadIdx.x >> 6] = all_or;
+    }
     __syncthreads();
-    const size_t ntiles = (n + RS_TILE - 1) / RS_TILE;
-    for (size_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        const size_t base = t * RS_TILE;
-        const uint32_t tile_n = (uint32_t)min((size_t)RS_TILE, n - base);
-        K key[RS_ROUNDS];
-#pragma unroll
-        for (int r = 0; r < RS_ROUNDS; ++r) {
-            const uint32_t li = (uint32_t)r * RS_THREADS + threadIdx.x;
-            key[r] = li < tile_n ? keys[base + li] : (K)0;
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < RS_THREADS / WAVE; ++w) {
+            all_and &= s_and[w];
+            all_or |= s_or[w];
         }
+        slots[2 * blockIdx.x] = all_and;
+        slots[2 * blockIdx.x + 1] = all_or;
+    }
+}
+
+// Runs f(i) for the items i < n of this thread (a grid of rs_bits_grid(n) blocks), f returning
+// item i's key, and leaves the block's bits in slots.
+template <class F>
+__device__ __forceinline__ void rs_each_key(size_t n, uint64_t* __restrict__ slots, F f) {
+    uint64_t all_and = ~0ull, all_or = 0ull;
+    const size_t step = (size_t)gridDim.x * (RS_THREADS * RS_BITS_ITEMS);
+    for (size_t base = (size_t)blockIdx.x * (RS_THREADS * RS_BITS_ITEMS); base < n; base += step) {
 #pragma unroll
-        for (int r = 0; r < RS_ROUNDS; ++r) {
-            const bool valid = (uint32_t)r * RS_THREADS + threadIdx.x < tile_n;
-            const uint64_t vm = __builtin_amdgcn_ballot_w64(valid);
-            if (vm == 0ull) continue;   // wave-uniform
-            for (int d = dlo; d < dhi; ++d) {
-                const uint32_t digit = (uint32_t)(key[r] >> (8 * d)) & 255u;
-                const uint32_t d0 = __builtin_amdgcn_readfirstlane(digit);   // lane 0's: valid whenever any is
-                if (__builtin_amdgcn_ballot_w64(valid && digit == d0) == vm) {
-                    if (lane_id() == 0) atomicAdd(&h[d][d0], (uint32_t)__popcll(vm));
-                } else if (valid) {
-                    atomicAdd(&h[d][digit], 1u);
-                }
+        for (unsigned k = 0; k < RS_BITS_ITEMS; ++k) {
+            const size_t i = base + k * RS_THREADS + threadIdx.x;
+            if (i < n) {
+                const uint64_t key = f(i);
+                all_and &= key;
+                all_or |= key;
             }
         }
     }
-    __syncthreads();
-    for (int k = threadIdx.x; k < 8 * RS_BINS; k += RS_THREADS) {
-        const uint32_t c = (&h[0][0])[k];
-        if (c) atomicAdd(&hist8[k], c);
-    }
+    rs_block_bits(all_and, all_or, slots);
+}
+
+// The bits of keys that are there already.
+template <typename K>
+__global__ __launch_bounds__(RS_THREADS) void k_rs_bits(const K* __restrict__ keys, size_t n, uint64_t* __restrict__ slots) {
+    rs_each_key(n, slots, [&](size_t i) { return (uint64_t)keys[i]; });
 }
 
 // A pass's digit of a key.  flip = 0x80 on the top digit sorts the raw bits of signed numbers.
@@ -279,9 +294,15 @@ __device__ __forceinline__ uint32_t rs_digit(K key, int shift, uint32_t flip) {
     return ((uint32_t)(key >> shift) & 255u) ^ flip;
 }
 
-// Per-tile digit counts, digit-major: th[d * ntiles + tile].  A digit equal across a wave
-// is added once, from one lane.
-template <typename K>
+// Sorts of at most this many tiles need no scan kernels: every scatter block adds up the tiles'
+// counts itself (SELF), 256 coalesced counts a tile.  Plan of 60K queries 154 -> 99 us (three
+// launches of about 3.5 us less a pass), of 250K (123 tiles) 160 -> 127; at 245 tiles what the
+// blocks read again takes the gain away (172 -> 164).
+constexpr uint32_t RS_SELF_TILES = 128;
+
+// Per-tile digit counts, digit-major (th[d * ntiles + tile], for the scan), or tile-major (SELF:
+// th[tile * 256 + d]).  A digit equal across a wave is added once, from one lane.
+template <typename K, bool SELF>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_tile_hist(const K* __restrict__ keys,
                                                              size_t n, int shift, uint32_t flip,
                                                              uint32_t* __restrict__ th,
@@ -305,7 +326,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_tile_hist(const K* __restrict
         }
     }
     __syncthreads();
-    th[(size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
+    th[SELF ? (size_t)blockIdx.x * RS_BINS + threadIdx.x : (size_t)threadIdx.x * ntiles + blockIdx.x] = h[threadIdx.x];
 }
 
 // Ranking of one tile of up to RS_TILE items held in registers (item r * 256 + tid in
@@ -371,10 +392,10 @@ struct KeyOut {
     __device__ __forceinline__ void put(size_t dst, K key, uint32_t) const { k[dst] = key; }
 };
 
-// Stable scatter of one tile (tile-major digit offsets from the scan of the per-tile digit
-// counts): the tile is ranked in registers, staged in LDS in digit order and written out so
+// Stable scatter of one tile (digit offsets from the scan of the per-tile digit counts, or, with
+// SELF, from the counts themselves): the tile is ranked in registers, staged in LDS in digit order and written out so
 // equal digits land contiguously.
-template <class Out, typename K = uint64_t, bool VALS = true>
+template <class Out, typename K, bool VALS, bool SELF>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     const K* __restrict__ kin, const uint32_t* __restrict__ vin, Out out, size_t n, int shift, uint32_t flip,
     const uint32_t* __restrict__ th_base, uint32_t ntiles) {
@@ -384,6 +405,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     } s_u;
     __shared__ uint32_t s_val[VALS ? RS_TILE : 1];
     __shared__ uint32_t s_dstart[RS_BINS];
+    __shared__ uint32_t s_gbase[SELF ? RS_BINS : 1];   // the tile's first output slot of each digit
     __shared__ uint32_t s_w[4];
 
     const int tid = threadIdx.x;
@@ -398,8 +420,22 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
         key[r] = li < tile_n ? kin[base + li] : (K)0;
         val[r] = VALS && li < tile_n ? vin[base + li] : 0u;
     }
-    const uint32_t cnt = rs_rank_tile(key, tile_n, shift, flip, s_u.c, off);
     uint32_t tot;
+    if (SELF) {   // this thread's digit: its items in the tiles before this one, and in all
+        uint32_t before = 0, all = 0;
+        for (uint32_t t = 0; t < ntiles; t += 8) {
+            uint32_t c[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) c[k] = t + k < ntiles ? th_base[(size_t)(t + k) * RS_BINS + tid] : 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) {
+                all += c[k];
+                before += t + k < tile ? c[k] : 0u;
+            }
+        }
+        s_gbase[tid] = block_excl_scan256<uint32_t>(all, s_w, &tot) + before;
+    }
+    const uint32_t cnt = rs_rank_tile(key, tile_n, shift, flip, s_u.c, off);
     s_dstart[tid] = block_excl_scan256<uint32_t>(cnt, s_w, &tot);   // its barriers free s_u.c
     __syncthreads();
 #pragma unroll
@@ -417,15 +453,16 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
         if (slot < tile_n) {
             const K k = s_u.key[slot];
             const uint32_t digit = rs_digit(k, shift, flip);
-            const size_t dst = (size_t)th_base[(size_t)digit * ntiles + tile] + (slot - s_dstart[digit]);
+            const size_t dst = (size_t)(SELF ? s_gbase[digit] : th_base[(size_t)digit * ntiles + tile]) +
+                               (slot - s_dstart[digit]);
             out.put(dst, k, VALS ? s_val[slot] : 0u);
         }
     }
 }
 
-// Temporary device memory of a radix sort of n items (see rs_temp_bytes).
+// Temporary device memory of a radix sort of n items (rs_temp_bytes).
 struct RsTemp {
-    uint32_t* hist8;   // [8][256] digit histograms
+    uint64_t* bits;    // AND and OR of the keys, per block (rs_each_key)
     uint32_t* th;      // per-tile digit counts, digit-major
     uint32_t* tb;      // their exclusive scan
     uint32_t* ws;      // scan workspace
@@ -437,14 +474,14 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 constexpr size_t rs_temp_bytes(size_t n) {
     const size_t nth = rs_ntiles(n) * RS_BINS;
-    return align256(8 * RS_BINS * 4) + 2 * align256(nth * 4) + align256(scan_ws_items(nth) * 4);
+    return RS_BITS_BLOCKS * 16 + 2 * align256(nth * 4) + align256(scan_ws_items(nth) * 4);
 }
 
 inline RsTemp rs_temp_carve(void* base, size_t n) {
     const size_t nth = rs_ntiles(n) * RS_BINS;
     char* p = (char*)base;
     RsTemp t;
-    t.hist8 = (uint32_t*)p; p += align256(8 * RS_BINS * 4);
+    t.bits = (uint64_t*)p; p += RS_BITS_BLOCKS * 16;
     t.th = (uint32_t*)p; p += align256(nth * 4);
     t.tb = (uint32_t*)p; p += align256(nth * 4);
     t.ws = (uint32_t*)p;
@@ -461,107 +498,100 @@ __global__ void k_zero_u64(uint64_t* __restrict__ p, size_t n) {
     if (i < n) p[i] = 0;
 }
 
-// Histograms of key digits [dlo, dhi) of n > 0 keys, read back into h8 ([8][256], zeroed by
-// the caller; synchronises the stream).
-template <typename K>
-int rs_digit_hist(const K* keys, size_t n, int dlo, int dhi, const RsTemp& tmp, uint32_t* h8, hipStream_t st) {
-    k_zero_u32<<<grid_for(8 * RS_BINS, 256), 256, 0, st>>>(tmp.hist8, 8 * RS_BINS);
-    LAUNCH_CHECK();
-    const unsigned hb = (unsigned)std::min<size_t>(rs_ntiles(n), 1024);
-    k_rs_hist8<K><<<hb, RS_THREADS, 0, st>>>(keys, n, dlo, dhi, tmp.hist8);
-    LAUNCH_CHECK();
-    HIP_TRY(hipMemcpyAsync(h8, tmp.hist8, 8 * RS_BINS * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+// The bits that vary over n > 0 keys, from what a grid of rs_bits_grid(n) blocks has left in
+// tmp.bits (one read-back; synchronises the stream).
+inline int rs_varying_bits(size_t n, const RsTemp& tmp, uint64_t* varying, hipStream_t st) {
+    uint64_t slots[2 * RS_BITS_BLOCKS];
+    const unsigned nb = rs_bits_grid(n);
+    HIP_TRY(hipMemcpyAsync(slots, tmp.bits, (size_t)nb * 16, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    uint64_t all_and = ~0ull, all_or = 0ull;
+    for (unsigned b = 0; b < nb; ++b) {
+        all_and &= slots[2 * b];
+        all_or |= slots[2 * b + 1];
+    }
+    *varying = all_and ^ all_or;
     return SI_OK;
 }
 
-// True when digit d is equal for all n keys.
-inline bool rs_digit_constant(const uint32_t* h8, int d, size_t n) {
-    for (int b = 0; b < RS_BINS; ++b)
-        if (h8[d * RS_BINS + b] == n) return true;
-    return false;
+// True when digit d holds a bit that varies.
+inline bool rs_digit_varies(uint64_t varying, int d) { return ((varying >> (8 * d)) & 255u) != 0; }
+
+// One pass by the digit at `shift`: counts per tile, their scan, the scatter through out.
+template <typename K, bool VALS, class Out>
+int rs_pass(const K* kin, const uint32_t* vin, const Out& out, size_t n, int shift, uint32_t flip, const RsTemp& tmp,
+            hipStream_t st) {
+    const uint32_t ntiles = (uint32_t)rs_ntiles(n);
+    if (ntiles <= RS_SELF_TILES) {
+        k_rs_tile_hist<K, true><<<ntiles, RS_THREADS, 0, st>>>(kin, n, shift, flip, tmp.th, ntiles);
+        LAUNCH_CHECK();
+        k_rs_scatter<Out, K, VALS, true><<<ntiles, RS_THREADS, 0, st>>>(kin, vin, out, n, shift, flip, tmp.th, ntiles);
+        LAUNCH_CHECK();
+        return SI_OK;
+    }
+    k_rs_tile_hist<K, false><<<ntiles, RS_THREADS, 0, st>>>(kin, n, shift, flip, tmp.th, ntiles);
+    LAUNCH_CHECK();
+    const int rc = device_excl_scan<uint32_t, uint32_t>(tmp.th, (size_t)ntiles * RS_BINS, tmp.tb, nullptr, tmp.ws, st);
+    if (rc != SI_OK) return rc;
+    k_rs_scatter<Out, K, VALS, false><<<ntiles, RS_THREADS, 0, st>>>(kin, vin, out, n, shift, flip, tmp.tb, ntiles);
+    LAUNCH_CHECK();
+    return SI_OK;
 }
 
-// Ascending sort of n signed numbers given by their raw bits, by the digits d with run[d] (the
-// others are equal for all of them; at least one must be set): in -> out, through the buffers
-// k0 and k1.  in is not written; out may not be in, k0 or k1.
+// Ascending sort of n signed numbers given by their raw bits, by the digits with a bit of
+// `varying` (at least one): in -> out, through the buffers k0 and k1.  in is not written; out may
+// not be in, k0 or k1.
 template <typename K>
-int radix_sort_signed(const K* in, K* k0, K* k1, K* out, size_t n, const bool (&run)[8], const RsTemp& tmp,
+int radix_sort_signed(const K* in, K* k0, K* k1, K* out, size_t n, uint64_t varying, const RsTemp& tmp,
                       hipStream_t st) {
-    const uint32_t ntiles = (uint32_t)rs_ntiles(n);
     int last_d = -1;
     for (int d = 0; d < (int)sizeof(K); ++d)
-        if (run[d]) last_d = d;
+        if (rs_digit_varies(varying, d)) last_d = d;
     const K* src = in;
     for (int d = 0; d <= last_d; ++d) {
-        if (!run[d]) continue;
+        if (!rs_digit_varies(varying, d)) continue;
         const uint32_t flip = (d == (int)sizeof(K) - 1) ? 0x80u : 0u;
         K* const dst = (d == last_d) ? out : k0;
-        k_rs_tile_hist<K><<<ntiles, RS_THREADS, 0, st>>>(src, n, 8 * d, flip, tmp.th, ntiles);
-        LAUNCH_CHECK();
-        const int rc = device_excl_scan<uint32_t, uint32_t>(tmp.th, (size_t)ntiles * RS_BINS, tmp.tb, nullptr, tmp.ws, st);
+        const int rc = rs_pass<K, false>(src, (const uint32_t*)nullptr, KeyOut<K>{dst}, n, 8 * d, flip, tmp, st);
         if (rc != SI_OK) return rc;
-        k_rs_scatter<KeyOut<K>, K, false><<<ntiles, RS_THREADS, 0, st>>>(src, nullptr, KeyOut<K>{dst}, n, 8 * d, flip,
-                                                                         tmp.tb, ntiles);
-        LAUNCH_CHECK();
         src = dst;
         std::swap(k0, k1);
     }
     return SI_OK;
 }
 
-// Stable sort of (keys, vals) by key digits [digit_lo, digit_hi) (8-bit digits,
-// least significant first).  Digits that are equal for every key are skipped, which
-// needs one host read-back of the digit histograms; skip_constant = false sorts every
-// digit in [digit_lo, digit_hi) with no read-back, so the sort can be captured in a graph.
-// tmp comes from rs_temp_carve.  On return *keys_sorted / *vals_sorted point at whichever
-// buffer holds the result.
-// known_hist (optional, [8][256]): the keys' digit histograms, when the caller has read them back.
+// Stable sort of (keys, vals) by key digits [digit_lo, digit_hi) (8-bit digits, least significant
+// first) that hold a bit of `varying` (rs_varying_bits, or all of them, which needs no read-back,
+// so that the sort can be captured in a graph).  tmp comes from rs_temp_carve.  On return
+// *keys_sorted / *vals_sorted point at whichever buffer holds the result.
 // With last (optional), the last pass run writes the sorted items through it instead of
 // into the buffers, and *last_written says whether one ran; only if none ran are the
 // items in *keys_sorted / *vals_sorted.
 template <class LastOut = ArrayOut>
 int radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, size_t n,
                      int digit_lo, int digit_hi, const RsTemp& tmp, uint64_t** keys_sorted,
-                     uint32_t** vals_sorted, hipStream_t st, bool skip_constant = true,
-                     const LastOut* last = nullptr, bool* last_written = nullptr,
-                     const uint32_t* known_hist = nullptr) {
+                     uint32_t** vals_sorted, hipStream_t st, uint64_t varying = ~0ull,
+                     const LastOut* last = nullptr, bool* last_written = nullptr) {
     if (last_written) *last_written = false;
     *keys_sorted = k0;
     *vals_sorted = v0;
     if (n < 2) return SI_OK;
-    uint32_t h[8 * RS_BINS] = {0};
-    if (skip_constant && !known_hist) {
-        const int rc = rs_digit_hist(k0, n, digit_lo, digit_hi, tmp, h, st);
-        if (rc != SI_OK) return rc;
-    }
-    const uint32_t* const h8 = known_hist ? known_hist : h;
 
-    const uint32_t ntiles = (uint32_t)rs_ntiles(n);
-    const size_t nth = (size_t)ntiles * RS_BINS;
     uint64_t *ka = k0, *kb = k1;
     uint32_t *va = v0, *vb = v1;
-    bool sort_digit[8] = {false};   // the digits sorted: all but those constant over the keys
     int last_d = -1;
+    for (int d = digit_lo; d < digit_hi; ++d)
+        if (rs_digit_varies(varying, d)) last_d = d;
     for (int d = digit_lo; d < digit_hi; ++d) {
-        sort_digit[d] = !(skip_constant && rs_digit_constant(h8, d, n));
-        if (sort_digit[d]) last_d = d;
-    }
-    for (int d = digit_lo; d < digit_hi; ++d) {
-        if (!sort_digit[d]) continue;
-        const int shift = 8 * d;
-        k_rs_tile_hist<uint64_t><<<ntiles, RS_THREADS, 0, st>>>(ka, n, shift, 0u, tmp.th, ntiles);
-        LAUNCH_CHECK();
-        int rc = device_excl_scan<uint32_t, uint32_t>(tmp.th, nth, tmp.tb, nullptr, tmp.ws, st);
-        if (rc != SI_OK) return rc;
+        if (!rs_digit_varies(varying, d)) continue;
+        int rc;
         if (last && d == last_d) {
-            k_rs_scatter<LastOut><<<ntiles, RS_THREADS, 0, st>>>(ka, va, *last, n, shift, 0u, tmp.tb, ntiles);
+            rc = rs_pass<uint64_t, true>(ka, va, *last, n, 8 * d, 0u, tmp, st);
             if (last_written) *last_written = true;
         } else {
-            k_rs_scatter<ArrayOut><<<ntiles, RS_THREADS, 0, st>>>(ka, va, ArrayOut{kb, vb}, n, shift, 0u, tmp.tb,
-                                                                    ntiles);
+            rc = rs_pass<uint64_t, true>(ka, va, ArrayOut{kb, vb}, n, 8 * d, 0u, tmp, st);
         }
-        LAUNCH_CHECK();
+        if (rc != SI_OK) return rc;
         std::swap(ka, kb);
         std::swap(va, vb);
     }

@@ -164,13 +164,15 @@ PlanView<S> plan_view(void* base, size_t nq) {
 
 // int32: key = (biased end << 32) | query number, payload = start bits.  Only the high
 // four digits are sorted, so the key's low half carries the query number.
-__global__ void k_plan_keys_i32(const int32_t* __restrict__ qs, const int32_t* __restrict__ qe,
-                                size_t nq, uint64_t* __restrict__ key, uint32_t* __restrict__ val) {
-    size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nq) {
-        key[k] = ((uint64_t)((uint32_t)qe[k] ^ 0x80000000u) << 32) | (uint32_t)k;
+__global__ __launch_bounds__(RS_THREADS) void k_plan_keys_i32(const int32_t* __restrict__ qs, const int32_t* __restrict__ qe,
+                                                              size_t nq, uint64_t* __restrict__ key,
+                                                              uint32_t* __restrict__ val, uint64_t* __restrict__ bits) {
+    rs_each_key(nq, bits, [&](size_t k) {
+        const uint64_t x = ((uint64_t)((uint32_t)qe[k] ^ 0x80000000u) << 32) | (uint32_t)k;
+        key[k] = x;
         val[k] = (uint32_t)qs[k];
-    }
+        return x;
+    });
 }
 
 // The plan's sort written straight into the plan's arrays by its last pass (the unpacking
@@ -208,13 +210,15 @@ __global__ void k_plan_counters(PlanView<S> pv, bool with_lb, bool with_rank) {
 }
 
 // int64: key = biased end, payload = query number.
-__global__ void k_plan_keys_i64(const int64_t* __restrict__ qe, size_t nq, uint64_t* __restrict__ key,
-                                uint32_t* __restrict__ val) {
-    size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nq) {
-        key[k] = (uint64_t)qe[k] ^ 0x8000000000000000ull;
+__global__ __launch_bounds__(RS_THREADS) void k_plan_keys_i64(const int64_t* __restrict__ qe, size_t nq,
+                                                              uint64_t* __restrict__ key, uint32_t* __restrict__ val,
+                                                              uint64_t* __restrict__ bits) {
+    rs_each_key(nq, bits, [&](size_t k) {
+        const uint64_t x = (uint64_t)qe[k] ^ 0x8000000000000000ull;
+        key[k] = x;
         val[k] = (uint32_t)k;
-    }
+        return x;
+    });
 }
 
 // lower_bound from upper_bound: the first position whose start is >= s is upper_bound(s - 1)
@@ -316,7 +320,7 @@ __global__ __launch_bounds__(Q_THREADS) void k_count_rank(IndexView<S> ix, const
 //                wave-cooperative kernel
 //   ub_tree      1: siUpperBound descends a 64-ary tree of first keys (its top level in
 //                Eytzinger order in LDS); 0: plain halving over all starts
-//   plan_sync    1: the plan's radix sort reads the digit histograms back to skip constant
+//   plan_sync    1: the plan's radix sort reads back which key bits vary to skip constant
 //                digits (one stream synchronisation); 0: it sorts every key digit without
 //                a host read-back, so plan -> offsets -> fill can be captured in a graph
 //   heavy_ends32 1: the wave-cooperative walk of an int64 index reads the 32-bit copy of
@@ -390,18 +394,22 @@ int plan_impl(const siIndex* ix, const S* qs, const S* qe, size_t nq, void* plan
     uint64_t* ks;
     uint32_t* vs;
     int rc;
+    uint64_t varying = ~0ull;   // key bits that vary, as far as is known
     bool unpacked = false;   // the sort's last pass wrote q, s, e (when the bounds come from a search below)
     if (sizeof(S) == 4) {
-        k_plan_keys_i32<<<g, Q_THREADS, 0, st>>>((const int32_t*)qs, (const int32_t*)qe, nq, k0, v0);
+        k_plan_keys_i32<<<rs_bits_grid(nq), RS_THREADS, 0, st>>>((const int32_t*)qs, (const int32_t*)qe, nq, k0, v0,
+                                                                 rt.bits);
         LAUNCH_CHECK();
+        if (read_back && nq > 1 && (rc = rs_varying_bits(nq, rt, &varying, st)) != SI_OK) return rc;
         const PlanOutI32 out{pv.q, (int32_t*)pv.s, (int32_t*)pv.e};
-        rc = radix_sort_pairs(k0, v0, k1, v1, nq, 4 + g_tune.plan_skip_low, 8, rt, &ks, &vs, st, read_back,
+        rc = radix_sort_pairs(k0, v0, k1, v1, nq, 4 + g_tune.plan_skip_low, 8, rt, &ks, &vs, st, varying,
                               (tree || learned) ? &out : nullptr, &unpacked);
     } else {
-        k_plan_keys_i64<<<g, Q_THREADS, 0, st>>>((const int64_t*)qe, nq, k0, v0);
+        k_plan_keys_i64<<<rs_bits_grid(nq), RS_THREADS, 0, st>>>((const int64_t*)qe, nq, k0, v0, rt.bits);
         LAUNCH_CHECK();
+        if (read_back && nq > 1 && (rc = rs_varying_bits(nq, rt, &varying, st)) != SI_OK) return rc;
         const PlanOutI64 out{pv.q, (int64_t*)pv.s, (int64_t*)pv.e, (const int64_t*)qs};
-        rc = radix_sort_pairs(k0, v0, k1, v1, nq, g_tune.plan_skip_low, 8, rt, &ks, &vs, st, read_back,
+        rc = radix_sort_pairs(k0, v0, k1, v1, nq, g_tune.plan_skip_low, 8, rt, &ks, &vs, st, varying,
                               (tree || learned) ? &out : nullptr, &unpacked);
     }
     if (rc != SI_OK) return rc;
@@ -2684,7 +2692,7 @@ SI_EXPORT int siSetTableSearchOffsets(const siSetTable* t, const uint32_t* set_i
     const int slot_digits = (t->nslots <= 256) ? 1 : 2;
     uint64_t* ks;
     uint32_t* vs;
-    rc = radix_sort_pairs(k0, v0, k1, v1, nq, g_tune.plan_skip_low, 4 + slot_digits, rt, &ks, &vs, st, false);
+    rc = radix_sort_pairs(k0, v0, k1, v1, nq, g_tune.plan_skip_low, 4 + slot_digits, rt, &ks, &vs, st);
     if (rc) return rc;
     PlanView<int32_t> pv = multi_view(plan, nq, t->nslots);
     uint32_t* c32 = counts ? counts : (uint32_t*)(p + L.base.off_heavy);

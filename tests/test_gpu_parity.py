@@ -1336,3 +1336,25 @@ def test_builds_from_threads_keep_their_blocks(sia, orc):
     for t in threads:
         t.join()
     assert not errors, errors[0]
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("nq", [2048 * 127 + 1, 2048 * 128, 2048 * 128 + 1])
+def test_plan_sort_around_the_scan_free_size(sia, dtype, nq):
+    """The plan's sort at the batch size from which its passes scan the tiles' digit counts with
+    kernels of their own (above 128 tiles of 2048): numpy's stable argsort of the ends, for ends
+    over the whole range, with one digit that varies, and none."""
+    import torch
+    print(f"[gpu] plan sort dtype={np.dtype(dtype).name} nq={nq}", flush=True)
+    rng = np.random.default_rng(nq)
+    info = np.iinfo(dtype)
+    ix = _dev_index(sia, np.arange(1000, dtype=dtype), np.arange(1000, dtype=dtype) + 5)
+    for qe in (rng.integers(info.min, info.max, nq), 7 + 256 * rng.integers(0, 256, nq), np.full(nq, -1)):
+        qe = qe.astype(dtype)
+        t = torch.from_numpy(qe).cuda()
+        plan = torch.empty(ix.plan_bytes(nq), dtype=torch.uint8, device="cuda")
+        ix.plan_device(t, t, plan)
+        torch.cuda.synchronize()
+        q = plan[256:256 + 4 * nq].view(torch.int32).cpu().numpy()
+        assert np.array_equal(q, np.argsort(qe, kind="stable"))
+    ix.close()
