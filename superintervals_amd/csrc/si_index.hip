@@ -295,7 +295,10 @@ struct BuildInfo {
     unsigned long long inverted;   // intervals with start > end
     long long end_lo, end_hi;      // smallest and largest end
     uint32_t long_run;             // 1: a run of equal starts longer than TIE_RUN was left as it was
+    uint32_t crowded[2];           // sampled keys in crowded buckets of the starts' and the sorted ends' tables
+    uint32_t gaps[2];              // long gaps of the two tables (BucketGap)
     uint32_t pad;
+    long long start_lo, start_hi;  // smallest and largest start
 };
 
 // Intervals sorted by start only, in input order within equal starts: puts every run of equal
@@ -309,8 +312,23 @@ __global__ __launch_bounds__(256) void k_fix_ties(const S* __restrict__ st, S* _
                                                   int32_t* __restrict__ vals, size_t n, BuildInfo* __restrict__ info) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i + 1 >= n) return;
-    const S s = st[i];
-    if (st[i + 1] != s || (i > 0 && st[i - 1] == s)) return;   // not the head of a run
+    // (everything a run of two needs to be judged is loaded at once)
+    const S s = st[i], s1 = st[i + 1], s0 = i > 0 ? st[i - 1] : s, s2 = i + 2 < n ? st[i + 2] : s, e0 = en[i], e1 = en[i + 1];
+    if (s1 != s || (i > 0 && s0 == s)) return;   // not the head of a run
+    if (i + 2 >= n || s2 != s) {
+        if (e0 >= e1) return;
+        const uint32_t p0 = perm[i], p1 = perm[i + 1];
+        const int32_t v0 = vals ? vals[i] : 0, v1 = vals ? vals[i + 1] : 0;
+        en[i] = e1;
+        en[i + 1] = e0;
+        perm[i] = p1;
+        perm[i + 1] = p0;
+        if (vals) {
+            vals[i] = v1;
+            vals[i + 1] = v0;
+        }
+        return;
+    }
     uint32_t len = 2;
     while (len <= TIE_RUN && i + len < n && st[i + len] == s) ++len;
     if (len > TIE_RUN) {
@@ -470,11 +488,81 @@ __global__ __launch_bounds__(256) void k_branch_exit(Max16<S> t, const S* __rest
     if (inv) atomicAdd(&info->inverted, (unsigned long long)inv);
 }
 
+// Sums of 16 consecutive entries of a and of b (lines of n / 16 + 1 each, the last one partial;
+// a is padded to whole lines, b is not), modulo 2^32, into out and out + lines.
+__global__ __launch_bounds__(256) void k_line_sums(const int32_t* __restrict__ a, const int32_t* __restrict__ b, uint32_t n,
+                                                   uint32_t lines, uint32_t* __restrict__ out) {
+    const uint32_t k = blockIdx.x * 256u + threadIdx.x;
+    if (k >= 2u * lines) return;
+    const uint32_t l = k < lines ? k : k - lines;
+    const int32_t* const p = (k < lines ? a : b) + (size_t)l * 16;
+    uint32_t sum = 0;
+    if (l + 1 < lines) {
+        int32_t v[16];
+        load16(p, v);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) sum += (uint32_t)v[j];
+    } else {
+        for (uint32_t j = 0; j < (n & 15u); ++j) sum += (uint32_t)p[j];
+    }
+    out[k] = sum;
+}
+
 template <typename S>
-__global__ void k_end_range(const S* __restrict__ sorted, size_t n, BuildInfo* __restrict__ info) {
+__global__ void k_ranges(const S* __restrict__ starts, const S* __restrict__ sorted, size_t n,
+                         BuildInfo* __restrict__ info) {
     if (threadIdx.x == 0) {
+        info->start_lo = (long long)starts[0];
+        info->start_hi = (long long)starts[n - 1];
         info->end_lo = (long long)sorted[0];
         info->end_hi = (long long)sorted[n - 1];
+    }
+}
+
+// ---- bucket tables (BucketView) ----------------------------------------------------------
+// Entries of a table between the buckets of two neighbouring keys that are too many for one
+// wave; filled by k_bucket_gaps.
+struct BucketGap {
+    uint32_t from, to, value;   // tab[from .. to) = value
+};
+constexpr uint32_t GAP_WAVE = 4096;       // most entries a wave fills by itself
+constexpr uint32_t CROWD = 4096;          // keys of a crowded bucket
+constexpr uint32_t CROWD_STEP = 64;       // every 64th key is sampled
+
+// tab[b] = i for the buckets b above key i - 1's up to key i's, and n above the last key's.
+template <typename S>
+__global__ __launch_bounds__(256) void k_bucket_table(const S* __restrict__ v, uint32_t n, BucketView<S> t, uint32_t nb,
+                                                      uint32_t* __restrict__ tab, BucketGap* __restrict__ gaps,
+                                                      uint32_t* __restrict__ ngaps, uint32_t* __restrict__ crowded) {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;   // n included: the entries past the last key
+    const int lane = lane_id();
+    uint32_t lo = 0, hi = 0;   // entries [lo, hi) are i
+    if (i < n) {
+        hi = (uint32_t)bucket_of(t, v[i]) + 1u;
+        lo = i ? (uint32_t)bucket_of(t, v[i - 1]) + 1u : 0u;
+        // (a bucket of more than CROWD keys holds key i + CROWD too, for most of its keys)
+        if (i % CROWD_STEP == 0 && n - i > CROWD && bucket_of(t, v[i + CROWD]) + 1u == hi) atomicAdd(crowded, 1u);
+    } else if (i == n) {
+        lo = (uint32_t)bucket_of(t, v[n - 1]) + 1u;
+        hi = nb + 1u;
+    }
+    const uint32_t len = hi - lo;
+    if (len == 1u) tab[lo] = i;
+    if (len > GAP_WAVE) gaps[atomicAdd(ngaps, 1u)] = BucketGap{lo, hi, i};
+    for (uint64_t m = __ballot(len > 1u && len <= GAP_WAVE); m; m &= m - 1ull) {
+        const int L = __builtin_ctzll(m);
+        const uint32_t a = __shfl(lo, L, WAVE), b = __shfl(hi, L, WAVE), x = __shfl(i, L, WAVE);
+        for (uint32_t k = a + (uint32_t)lane; k < b; k += WAVE) tab[k] = x;
+    }
+}
+
+__global__ __launch_bounds__(256) void k_bucket_gaps(const BucketGap* __restrict__ gaps, const uint32_t* __restrict__ ngaps,
+                                                     uint32_t* __restrict__ tab) {
+    const uint32_t m = *ngaps;
+    for (uint32_t g = 0; g < m; ++g) {
+        const BucketGap p = gaps[g];
+        for (uint64_t k = (uint64_t)p.from + blockIdx.x * 256u + threadIdx.x; k < p.to; k += (uint64_t)gridDim.x * 256u)
+            tab[k] = p.value;
     }
 }
 
@@ -619,6 +707,35 @@ int build_key_tree(const S* keys, const KeyTreeShape& h, KeyTree& t, hipStream_t
     return SI_OK;
 }
 
+// Entries a bucket table over n keys may take, and its longest list of gaps.
+constexpr size_t bucket_entries(size_t n) { return n / 4 + 2; }
+constexpr size_t bucket_gaps(size_t n) { return bucket_entries(n) / GAP_WAVE + 2; }
+
+// Bucket table over n sorted keys in [lo, hi]: at most n / 4 buckets of a power of two of values.
+// scratch holds bucket_gaps(n) entries.  Whether the table is used (t.ok) is left to the caller,
+// who reads the crowded sample back.
+template <typename S>
+int build_bucket_table(const S* keys, size_t n, int64_t lo, int64_t hi, BucketTable& t, BuildInfo* info, int which,
+                       Carver scratch, hipStream_t st) {
+    t.lo = lo;
+    t.hi = hi;
+    const uint64_t span = (uint64_t)hi - (uint64_t)lo;
+    const uint64_t most = std::max<uint64_t>(n / 4, 1);
+    t.shift = 0;
+    while ((span >> t.shift) >= most && t.shift < 63) ++t.shift;
+    const uint32_t nb = (uint32_t)(span >> t.shift) + 1u;
+    BucketGap* const gaps = scratch.take<BucketGap>(bucket_gaps(n));
+    const BucketView<S> v{t.d_tab, (S)lo, (S)hi, t.shift};
+    k_bucket_table<S><<<grid_for(n + 1, 256), 256, 0, st>>>(keys, (uint32_t)n, v, nb, t.d_tab, gaps, &info->gaps[which],
+                                                            &info->crowded[which]);
+    LAUNCH_CHECK();
+    if (nb > GAP_WAVE) {
+        k_bucket_gaps<<<64, 256, 0, st>>>(gaps, &info->gaps[which], t.d_tab);
+        LAUNCH_CHECK();
+    }
+    return SI_OK;
+}
+
 // Level sizes and offsets of a 64-ary max tree over n entries (level 0); returns the entries of
 // the levels above.
 size_t tree_shape(uint32_t n, int* nlev, size_t* off, uint32_t* size) {
@@ -658,7 +775,7 @@ int build_long_list(siIndex* ix, std::vector<int64_t>& lens, Carver scratch, hip
     const uint32_t n = (uint32_t)ix->n;
     int64_t len = si_tune_long_len();
     const bool automatic = len == 0;
-    if (len < 0 || (automatic && n < LONG_FROM)) return SI_OK;
+    if (len < 0 || (automatic && n < LONG_FROM)) return SI_OK;   // (scratch untouched)
     const S* d_st = (const S*)ix->d_starts;
     const S* d_en = (const S*)ix->d_ends;
     if (automatic) {
@@ -670,15 +787,19 @@ int build_long_list(siIndex* ix, std::vector<int64_t>& lens, Carver scratch, hip
     LongList& L = ix->lng;
     uint32_t* const flags = scratch.take<uint32_t>(n);
     uint32_t* const ws = scratch.take<uint32_t>(scan_ws_items(n));
-    uint32_t* const lrank = scratch.take<uint32_t>((size_t)n + 1);
+    if (!(L.d_lrank = (uint32_t*)si_block_take(((size_t)n + 1) * 4, &L.lrank_bytes)))
+        return si_set_error(SI_ERR_NOMEM, "long list: %zu bytes", ((size_t)n + 1) * 4);
     k_long_flags<S><<<grid_for(n, 256), 256, 0, st>>>(d_st, d_en, n, len, flags);
     LAUNCH_CHECK();
-    const int rc = device_excl_scan<uint32_t, uint32_t>(flags, n, lrank, lrank + n, ws, st);
+    const int rc = device_excl_scan<uint32_t, uint32_t>(flags, n, L.d_lrank, L.d_lrank + n, ws, st);
     if (rc != SI_OK) return rc;
     uint32_t nlong = 0;
-    HIP_TRY(hipMemcpyAsync(&nlong, lrank + n, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(&nlong, L.d_lrank + n, 4, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    if (nlong == 0 || (automatic && nlong > n / 2)) return SI_OK;
+    if (nlong == 0 || (automatic && nlong > n / 2)) {
+        L.release(ix->device, true);
+        return SI_OK;
+    }
     const uint32_t npad = (nlong + 63u) & ~63u;
     const size_t tot = tree_shape(nlong, &L.nlev, L.lvl_off, L.lvl_size);
     Carver c;
@@ -687,7 +808,6 @@ int build_long_list(siIndex* ix, std::vector<int64_t>& lens, Carver scratch, hip
         L.d_pos = c.take<uint32_t>(npad);
         L.d_ends = c.take<S>(npad);
         L.d_ends32 = ix->d_ends32 ? c.take<uint32_t>(npad) : nullptr;
-        L.d_lrank = c.take<uint32_t>((size_t)n + 1);
         L.d_tree = c.take<S>(tot);
         if (pass == 0) {
             if (!(L.d_block = si_block_take(c.used, &L.block_bytes)))
@@ -695,7 +815,6 @@ int build_long_list(siIndex* ix, std::vector<int64_t>& lens, Carver scratch, hip
             c.base = (char*)L.d_block;
         }
     }
-    HIP_TRY(hipMemcpyAsync(L.d_lrank, lrank, ((size_t)n + 1) * 4, hipMemcpyDeviceToDevice, st));
     k_long_fill<S><<<grid_for(std::max(n, npad), 256), 256, 0, st>>>(d_en, ix->d_ends32, flags, L.d_lrank, n, nlong,
                                                                      npad, L.d_pos, (S*)L.d_ends, L.d_ends32);
     LAUNCH_CHECK();
@@ -792,14 +911,17 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     Carver c;
     for (int pass = 0; pass < 2; ++pass) {
         c.used = 0;
-        ix->d_starts = c.take<S>(npad);
+        ix->d_starts = c.take<S>(npad + 64);   // (bucket searches read a little past the last key)
         ix->d_ends = c.take<S>(npad);
         ix->d_branch = c.take<uint32_t>(npad);
         ix->d_exit = c.take<uint32_t>(npad);
         ix->d_perm = c.take<uint32_t>(n);
         ix->d_values = values ? c.take<int32_t>(npad) : nullptr;
-        ix->d_ends_sorted = c.take<S>(n);
+        ix->d_ends_sorted = c.take<S>(npad + 64);   // (bucket searches read a little past the last key)
+        ix->ubt.d_tab = c.take<uint32_t>(bucket_entries(n));
+        ix->ebt.d_tab = c.take<uint32_t>(bucket_entries(n));
         ix->d_tree = c.take<S>(tree_n);
+        ix->d_line_sums = sizeof(S) == 4 ? c.take<uint32_t>(2 * (n / 16 + 1)) : nullptr;
         carve_key_tree<S>(shape, ix->ub, c);
         carve_key_tree<S>(shape, ix->eb, c);
         if (pass == 0) {
@@ -900,7 +1022,7 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
             } else {   // all ends equal
                 HIP_TRY(hipMemcpyAsync(ix->d_ends_sorted, ix->d_ends, nb, hipMemcpyDeviceToDevice, st));
             }
-            k_end_range<S><<<1, 64, 0, st>>>((const S*)ix->d_ends_sorted, n, info);
+            k_ranges<S><<<1, 64, 0, st>>>((const S*)ix->d_starts, (const S*)ix->d_ends_sorted, n, info);
             LAUNCH_CHECK();
         }
         // ---- branch and exits, through the 16-ary max tree
@@ -946,6 +1068,31 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     if (rc == SI_OK) rc = build_key_tree<S>((const S*)ix->d_starts, shape, ix->ub, st);        // upper_bound
     if (rc == SI_OK) rc = build_key_tree<S>((const S*)ix->d_ends_sorted, shape, ix->eb, st);   // rank count
     if (rc != SI_OK) return rc;
+    {
+        Carver m;
+        m.base = (char*)scratch.p;
+        m.used = shared_from;
+        rc = build_bucket_table<S>((const S*)ix->d_starts, n, back.info.start_lo, back.info.start_hi, ix->ubt, info, 0, m, st);
+        m.take<BucketGap>(bucket_gaps(n));
+        if (rc == SI_OK)
+            rc = build_bucket_table<S>((const S*)ix->d_ends_sorted, n, back.info.end_lo, back.info.end_hi, ix->ebt, info, 1,
+                                       m, st);
+        if (rc != SI_OK) return rc;
+    }
+    if constexpr (sizeof(S) == 4) {
+        const size_t lines = ix->sum_lines();
+        Carver m;
+        m.base = (char*)scratch.p;
+        m.used = shared_from;
+        m.take<BucketGap>(2 * bucket_gaps(n) + 64);   // (behind the tables' gaps)
+        uint32_t* const sums = m.take<uint32_t>(2 * lines);
+        uint32_t* const ws = m.take<uint32_t>(scan_ws_items(2 * lines));
+        k_line_sums<<<grid_for(2 * lines, 256), 256, 0, st>>>((const int32_t*)ix->d_starts, (const int32_t*)ix->d_ends_sorted,
+                                                              (uint32_t)n, (uint32_t)lines, sums);
+        LAUNCH_CHECK();
+        rc = device_excl_scan<uint32_t, uint32_t>(sums, 2 * lines, ix->d_line_sums, nullptr, ws, st);
+        if (rc != SI_OK) return rc;
+    }
     // 32-bit ends for the wave-cooperative walk of int64 indexes whose ends span < 2^32:
     // a third fewer bytes per position than ends + exitp at 8 + 4
     if constexpr (sizeof(S) == 8) {
@@ -966,7 +1113,13 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
         rc = build_long_list<S>(ix, lens, m, st);
         if (rc != SI_OK) return rc;
     }
+    HIP_TRY(hipMemcpyAsync(&back.info, info, sizeof(BuildInfo), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    // A search in a bucket of m keys takes about log2(m) - 2 reads after the table's, one through the
+    // 64-ary tree 14 (n > 4095 x 64): the tables are used unless half of the keys share a bucket
+    // with more than 4096 others.
+    const uint32_t half = (uint32_t)(n / CROWD_STEP / 2);
+    ix->ubt.ok = ix->ebt.ok = back.info.crowded[0] <= half && back.info.crowded[1] <= half;
     ix->built = true;
     ix->last_build_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

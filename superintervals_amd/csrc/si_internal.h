@@ -50,6 +50,20 @@ struct KeyTree {
     }
 };
 
+// Bucket table over a sorted key array (BucketView), in the index's block.
+struct BucketTable {
+    uint32_t* d_tab = nullptr;
+    bool ok = false;          // false: too many keys share a bucket, the search trees are used
+    int64_t lo = 0, hi = 0;
+    uint32_t shift = 0;
+    void release() {
+        d_tab = nullptr;
+        ok = false;
+    }
+    template <typename S>
+    BucketView<S> view() const { return BucketView<S>{ok ? d_tab : nullptr, (S)lo, (S)hi, shift}; }
+};
+
 // Scratch of the single-query calls (the host-buffer forms with one query): a pinned host
 // buffer mapped into the device, which the one-wave kernel writes directly (header + up to
 // cap results), and a stream.  Made on the first such call, kept until the index is
@@ -75,11 +89,12 @@ struct OneQuery {
     }
 };
 
-// The long list of an index (LongView): device arrays and the max tree over its ends, in one
-// allocation.
+// The long list of an index (LongView): device arrays and the max tree over its ends, in two
+// blocks.
 struct LongList {
     void* d_block = nullptr;
     size_t block_bytes = 0;
+    size_t lrank_bytes = 0;       // d_lrank is a block of its own (it is there before the list's size is known)
     int64_t len = 0;              // threshold; 0 = no list
     uint32_t n = 0;
     uint32_t* d_pos = nullptr;    // n, padded to 64 entries
@@ -92,6 +107,7 @@ struct LongList {
     uint32_t lvl_size[MAX_LEVELS] = {0};
     void release(int device, bool quiet) {
         if (d_block) si_block_give(d_block, block_bytes, device, quiet);
+        if (d_lrank) si_block_give(d_lrank, lrank_bytes, device, quiet);
         d_block = nullptr;
         d_pos = d_ends32 = d_lrank = nullptr;
         d_ends = d_tree = nullptr;
@@ -122,6 +138,10 @@ struct siIndex {
     void* d_ends_sorted = nullptr;   // ends in ascending order (rank count)
     uint32_t* d_ends32 = nullptr;    // int64 only, ends - ends32_base when they span < 2^32
     int64_t ends32_base = 0;
+    // int32 only (coverage): d_line_sums[k] = sum of starts[0 .. 16 k), and from entry
+    // sum_lines() on the same over the sorted ends plus a constant, modulo 2^32
+    uint32_t* d_line_sums = nullptr;
+    size_t sum_lines() const { return n / 16 + 1; }
     // intervals with start > end: the rank form of count and the guaranteed-hit run
     // [first start >= s, upper_bound] both assume start <= end, so queries on an index
     // holding any such interval take the walk
@@ -135,6 +155,7 @@ struct siIndex {
     LongList lng;                     // intervals longer than a threshold (LongView)
     KeyTree ub;   // search tree over the starts (upper_bound)
     KeyTree eb;   // search tree over the sorted ends (rank count)
+    BucketTable ubt, ebt;   // bucket tables over the same
     int nlev = 0;
     size_t lvl_off[MAX_LEVELS] = {0};   // element offsets into d_tree (level >= 1)
     uint32_t lvl_size[MAX_LEVELS] = {0};
@@ -155,7 +176,9 @@ struct siIndex {
         ++generation;
         ub.release();
         eb.release();
-        d_branch = d_exit = d_perm = nullptr;
+        ubt.release();
+        ebt.release();
+        d_branch = d_exit = d_perm = d_line_sums = nullptr;
         d_values = nullptr;
         n = 0;
         nlev = 0;

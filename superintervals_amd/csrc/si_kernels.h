@@ -64,6 +64,76 @@ struct LongView {
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
 
+// Bucket table over n sorted keys: the range [lo, hi] cut into nb equal buckets of 2^shift values,
+// tab[b] = the number of keys below bucket b (nb + 1 entries, about one for every four keys).  A
+// search reads the two entries around its bucket and looks through the keys between them.
+// tab == null: none (see build_bucket_table).
+template <typename S>
+struct BucketView {
+    const uint32_t* __restrict__ tab;
+    S lo, hi;
+    uint32_t shift;
+};
+
+template <typename S>
+__device__ __forceinline__ uint64_t bucket_of(const BucketView<S>& t, S x) {   // lo <= x
+    return (sizeof(S) == 4 ? (uint64_t)((uint32_t)x - (uint32_t)t.lo) : (uint64_t)x - (uint64_t)t.lo) >> t.shift;
+}
+
+// Numbers of keys <= x[i] in the N arrays v[i] of n keys, through their tables, together: the
+// loads of a step are issued at once.  Buckets of up to 16 keys are counted through 16 bytes at
+// a time (whatever their alignment), larger ones halved down to that first.  Reads up to 15 bytes
+// past a bucket's keys: the arrays are padded by that much.
+template <typename S, int N>
+__device__ __forceinline__ void bucket_ranks(const BucketView<S> (&t)[N], const S* const (&v)[N], uint32_t n,
+                                             const S (&x)[N], uint32_t (&rank)[N]) {
+    constexpr uint32_t W = 16 / sizeof(S);   // keys of a 16-byte load
+    uint32_t from[N], len[N], most = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        from[i] = x[i] < t[i].lo ? 0u : n;
+        len[i] = 0;
+        if (x[i] >= t[i].lo && x[i] < t[i].hi) {
+            const uint64_t b = bucket_of(t[i], x[i]);
+            uint32_t r[2];
+            __builtin_memcpy(r, t[i].tab + b, 8);
+            from[i] = r[0];
+            len[i] = r[1] - r[0];
+        }
+        most = len[i] > most ? len[i] : most;
+    }
+    while (most > 16u) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (len[i] > 16u) {
+                const uint32_t half = len[i] >> 1;
+                if (v[i][from[i] + half] <= x[i]) {
+                    from[i] += half + 1u;
+                    len[i] -= half + 1u;
+                } else {
+                    len[i] = half;
+                }
+            }
+        }
+        most = 0;
+#pragma unroll
+        for (int i = 0; i < N; ++i) most = len[i] > most ? len[i] : most;
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) rank[i] = from[i];
+    for (uint32_t k = 0; k < most; k += W) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (k < len[i]) {
+                S w[W];
+                __builtin_memcpy(w, v[i] + from[i] + k, 16);
+#pragma unroll
+                for (uint32_t c = 0; c < W; ++c) rank[i] += (k + c < len[i] && w[c] <= x[i]) ? 1u : 0u;
+            }
+        }
+    }
+}
+
 // ---- upper_bound ------------------------------------------------------------
 // Last position with starts[pos] <= x, or NONE (superintervals.hpp:501-516
 // semantics; written as the branchless "base/len" halving).

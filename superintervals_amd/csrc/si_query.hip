@@ -134,6 +134,8 @@ struct SetView {
     uint32_t eb_h;
     TreeDesc<S> td;               // max tree over the ends
     uint32_t rank_exact;          // 1 when no interval has start > end
+    const S* ends_sorted;
+    BucketView<S> ubt, ebt;       // bucket tables (tab null: the trees are used)
 };
 
 // Tiles of a plan over several sets: the sorted queries of set g are [sbeg[g], sbeg[g] +
@@ -269,6 +271,10 @@ int launch_ub_tree(const siIndex* ix, const S* xs, size_t n, uint32_t* out, hipS
 // search trees (below).
 template <typename S>
 int launch_plan_bounds(const siIndex* ix, PlanView<S> pv, size_t nq, bool with_lb, bool with_rank, hipStream_t st);
+
+// The same through the bucket tables.
+template <typename S>
+int launch_plan_table(const siIndex* ix, PlanView<S> pv, size_t nq, bool with_lb, bool with_rank, hipStream_t st);
 
 // The rank form needs no interval with start > end (defined with the launch helpers below).
 inline bool rank_exact(const siIndex* ix);
@@ -413,10 +419,12 @@ int plan_impl(const siIndex* ix, const S* qs, const S* qe, size_t nq, void* plan
                               (tree || learned) ? &out : nullptr, &unpacked);
     }
     if (rc != SI_OK) return rc;
-    if (unpacked) k_plan_counters<S><<<1, 64, 0, st>>>(pv, with_lb, with_rank);
-    else k_plan_finish<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), ks, vs, qs, nq, pv, !tree && !learned, with_lb, with_rank);
+    const bool table = tree && ix->ubt.ok;   // (k_plan_bounds_table sets the flags itself)
+    if (unpacked && !table) k_plan_counters<S><<<1, 64, 0, st>>>(pv, with_lb, with_rank);
+    else if (!unpacked) k_plan_finish<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), ks, vs, qs, nq, pv, !tree && !learned, with_lb, with_rank);
     LAUNCH_CHECK();
     if (learned) return si_learned_plan_bounds(ix, pv.e, pv.s, nq, pv.idx, with_lb ? pv.lb : nullptr, st);
+    if (table) return launch_plan_table<S>(ix, pv, nq, with_lb, with_rank, st);
     if (tree) return launch_plan_bounds<S>(ix, pv, nq, with_lb, with_rank, st);
     return SI_OK;
 }
@@ -1727,6 +1735,87 @@ int launch_plan_bounds(const siIndex* ix, PlanView<S> pv, size_t nq, bool with_l
     return SI_OK;
 }
 
+// The plan's bounds and counts through the bucket tables: what k_plan_bounds_tree finds, in two
+// or three rounds of reads (a table entry, then the few keys of its bucket, 16 bytes at a time) in
+// place of twelve LDS steps and seven reads a tree level.  Sets the plan's flags.
+template <typename S, bool LB, bool RANK>
+__global__ __launch_bounds__(Q_THREADS) void k_plan_bounds_table(IndexView<S> ix, const S* __restrict__ ends_sorted,
+                                                                 BucketView<S> ts, BucketView<S> te, PlanView<S> pv,
+                                                                 size_t nq) {
+    constexpr int N = 1 + (LB ? 1 : 0) + (RANK ? 1 : 0);
+    constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
+    const size_t k = (size_t)blockIdx.x * Q_THREADS + threadIdx.x;
+    if (k == 0) {
+        pv.counter[0] = 0;
+        pv.counter[4] = LB ? 1u : 0u;
+        pv.counter[5] = RANK ? 1u : 0u;
+    }
+    if (k >= nq) return;
+    const S e = pv.e[k], s = pv.s[k];
+    const bool s1 = s != SMIN;   // s - 1 exists
+    const S x1 = s1 ? (S)(s - 1) : s;
+    // searches: upper_bound(e), then lower bound (starts at s - 1), then #{ends < s}
+    BucketView<S> t[N];
+    const S* v[N];
+    S x[N];
+    uint32_t r[N];
+    t[0] = ts; v[0] = ix.starts; x[0] = e;
+    if (LB) { t[LB ? 1 : 0] = ts; v[LB ? 1 : 0] = ix.starts; x[LB ? 1 : 0] = x1; }
+    if (RANK) { t[N - 1] = te; v[N - 1] = ends_sorted; x[N - 1] = x1; }
+    bucket_ranks<S, N>(t, v, ix.n, x, r);
+    pv.idx[k] = r[0] - 1u;   // 0 wraps to NONE
+    if (LB) pv.lb[k] = s1 ? r[LB ? 1 : 0] : 0u;
+    if (RANK) {
+        uint32_t c = 0;
+        if (r[0] != 0u) c = s <= e ? r[0] - (s1 ? r[N - 1] : 0u) : walk_count(ix, r[0] - 1u, s);
+        pv.cnt[k] = c;
+    }
+}
+
+template <typename S>
+int launch_plan_table(const siIndex* ix, PlanView<S> pv, size_t nq, bool with_lb, bool with_rank, hipStream_t st) {
+    const BucketView<S> ts = ix->ubt.view<S>(), te = ix->ebt.view<S>();
+    const S* es = (const S*)ix->d_ends_sorted;
+    const unsigned g = grid_for(nq, Q_THREADS);
+    if (with_lb && with_rank) k_plan_bounds_table<S, true, true><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, pv, nq);
+    else if (with_lb) k_plan_bounds_table<S, true, false><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, pv, nq);
+    else if (with_rank) k_plan_bounds_table<S, false, true><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, pv, nq);
+    else k_plan_bounds_table<S, false, false><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, pv, nq);
+    LAUNCH_CHECK();
+    return SI_OK;
+}
+
+// upper_bound through the starts' bucket table.
+template <typename S>
+__global__ __launch_bounds__(Q_THREADS) void k_upper_bound_table(const S* __restrict__ starts, uint32_t n, BucketView<S> t,
+                                                                 const S* __restrict__ xs, size_t nx,
+                                                                 uint32_t* __restrict__ out) {
+    const size_t q = (size_t)blockIdx.x * Q_THREADS + threadIdx.x;
+    if (q >= nx) return;
+    const BucketView<S> tt[1] = {t};
+    const S* const v[1] = {starts};
+    const S x[1] = {xs[q]};
+    uint32_t r[1];
+    bucket_ranks<S, 1>(tt, v, n, x, r);
+    out[q] = r[0] - 1u;   // 0 wraps to NONE
+}
+
+// has_overlaps through the starts' bucket table (4M unsorted queries on 10M int32 intervals:
+// plain halving read 24 positions in turn).
+template <typename S>
+__global__ __launch_bounds__(Q_THREADS) void k_has_overlaps_table(IndexView<S> ix, BucketView<S> t,
+                                                                  const S* __restrict__ qs, const S* __restrict__ qe,
+                                                                  size_t nq, uint8_t* __restrict__ out) {
+    const size_t q = (size_t)blockIdx.x * Q_THREADS + threadIdx.x;
+    if (q >= nq) return;
+    const BucketView<S> tt[1] = {t};
+    const S* const v[1] = {ix.starts};
+    const S x[1] = {qe[q]};
+    uint32_t r[1];
+    bucket_ranks<S, 1>(tt, v, ix.n, x, r);
+    out[q] = (r[0] != 0u && qs[q] <= ix.ends[r[0] - 1u]) ? 1 : 0;
+}
+
 template <typename S>
 __global__ __launch_bounds__(Q_THREADS) void k_has_overlaps(IndexView<S> ix, const S* __restrict__ qs,
                                                             const S* __restrict__ qe, size_t nq,
@@ -1781,14 +1870,10 @@ __global__ __launch_bounds__(Q_THREADS) void k_gather_keys(IndexView<S> ix, cons
     if (out_v) out_v[k] = vals[i];
 }
 
-__global__ __launch_bounds__(Q_THREADS) void k_coverage_i32(IndexView<int32_t> ix,
-                                                            const int32_t* __restrict__ qs,
-                                                            const int32_t* __restrict__ qe, size_t nq,
-                                                            uint32_t* __restrict__ cnt,
-                                                            int32_t* __restrict__ cov) {
-    size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= nq) return;
-    const int32_t s = qs[q], e = qe[q];
+// One query's count and covered length by the reference walk, element by element
+// (c_superintervals.h:758-792).
+__device__ __forceinline__ void coverage_walk(const IndexView<int32_t>& ix, int32_t s, int32_t e, uint32_t* cnt,
+                                              uint32_t* cov) {
     uint32_t i = upper_bound_pos(ix.starts, ix.n, e);
     uint32_t c = 0, acc = 0;   // unsigned accumulation = int32 wraparound
     while (i != NONE) {
@@ -1803,6 +1888,75 @@ __global__ __launch_bounds__(Q_THREADS) void k_coverage_i32(IndexView<int32_t> i
         } else {
             i = ix.branch[i];
         }
+    }
+    *cnt = c;
+    *cov = acc;
+}
+
+__global__ __launch_bounds__(Q_THREADS) void k_coverage_i32(IndexView<int32_t> ix,
+                                                            const int32_t* __restrict__ qs,
+                                                            const int32_t* __restrict__ qe, size_t nq,
+                                                            uint32_t* __restrict__ cnt,
+                                                            int32_t* __restrict__ cov) {
+    size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= nq) return;
+    uint32_t c, acc;
+    coverage_walk(ix, qs[q], qe[q], &c, &acc);
+    if (cnt) cnt[q] = c;
+    if (cov) cov[q] = (int32_t)acc;
+}
+
+// Sum of the first r entries of sorted values v (an array of n, line k's sum below it in
+// sums[k]), modulo 2^32.
+__device__ __forceinline__ uint32_t sum_below(const int32_t* __restrict__ v, const uint32_t* __restrict__ sums, uint32_t r) {
+    const uint32_t l = r >> 4, k = r & 15u;
+    uint32_t sum = sums[l];
+    const int32_t* const p = v + (size_t)l * 16;
+#pragma unroll
+    for (uint32_t j = 0; j < 16u; j += 4u) {
+        if (j < k) {   // (16 bytes of the line: the arrays are padded past n)
+            int32_t w[4];
+            memcpy(w, p + j, 16);
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i) sum += j + i < k ? (uint32_t)w[i] : 0u;
+        }
+    }
+    return sum;
+}
+
+// coverage from ranks, for indexes without start > end.  With A = #{starts <= e}, B =
+// #{starts <= s}, C = #{ends < s}, D = #{ends < e} and s <= e, the hits are the A - C intervals
+// that start by e and do not end before s; the A - B of them that start in (s, e] add their own
+// start, the others s, to the sum of max(start, s), and the D - C that end in [s, e) their own
+// end, the others e, to the sum of min(end, e): four table searches and four line sums in place of
+// a walk over the hits (1M queries on 1M intervals, 12 hits each: 0.47 ms before).  All sums are
+// modulo 2^32, as the walk's int32 arithmetic.  Queries with s > e take the walk.
+__global__ __launch_bounds__(Q_THREADS) void k_coverage_rank(IndexView<int32_t> ix, const int32_t* __restrict__ ends_sorted,
+                                                             BucketView<int32_t> ts, BucketView<int32_t> te,
+                                                             const uint32_t* __restrict__ line_sums, uint32_t lines,
+                                                             const int32_t* __restrict__ qs,
+                                                             const int32_t* __restrict__ qe, size_t nq,
+                                                             uint32_t* __restrict__ cnt, int32_t* __restrict__ cov) {
+    const size_t q = (size_t)blockIdx.x * Q_THREADS + threadIdx.x;
+    if (q >= nq) return;
+    const int32_t s = qs[q], e = qe[q];
+    uint32_t c, acc;
+    if (s <= e) {
+        const bool s1 = s != INT32_MIN, e1 = e != INT32_MIN;   // s - 1, e - 1 exist
+        const BucketView<int32_t> t[4] = {ts, ts, te, te};
+        const int32_t* const v[4] = {ix.starts, ix.starts, ends_sorted, ends_sorted};
+        const int32_t x[4] = {e, s, s1 ? s - 1 : s, e1 ? e - 1 : e};
+        uint32_t r[4];
+        bucket_ranks<int32_t, 4>(t, v, ix.n, x, r);
+        const uint32_t A = r[0], B = r[1], C = s1 ? r[2] : 0u, D = e1 ? r[3] : 0u;
+        c = A - C;
+        const uint32_t* const es = line_sums + lines;
+        const uint32_t smax = sum_below(ix.starts, line_sums, A) - sum_below(ix.starts, line_sums, B) +
+                              (uint32_t)s * (c - (A - B));
+        const uint32_t smin = sum_below(ends_sorted, es, D) - sum_below(ends_sorted, es, C) + (uint32_t)e * (c - (D - C));
+        acc = smin - smax;
+    } else {
+        coverage_walk(ix, s, e, &c, &acc);
     }
     if (cnt) cnt[q] = c;
     if (cov) cov[q] = (int32_t)acc;
@@ -2196,6 +2350,13 @@ SI_EXPORT int siUpperBound(const siIndex* ix, const void* xs, size_t n, uint32_t
     if (n == 0) return SI_OK;
     if (!xs || !out) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
+    if (g_tune.ub_tree && ix->ubt.ok)
+        return DISPATCH_S(ix, ([&]() -> int {
+            k_upper_bound_table<S><<<grid_for(n, Q_THREADS), Q_THREADS, 0, st>>>((const S*)ix->d_starts, (uint32_t)ix->n,
+                                                                                 ix->ubt.view<S>(), (const S*)xs, n, out);
+            LAUNCH_CHECK();
+            return SI_OK;
+        }()));
     if (g_tune.ub_tree && ix->ub.d_top && ix->n > 0)
         return DISPATCH_S(ix, (launch_ub_tree<S>(ix, (const S*)xs, n, out, st)));
     return DISPATCH_S(ix, ([&]() -> int {
@@ -2213,6 +2374,12 @@ SI_EXPORT int siHasOverlaps(const siIndex* ix, const void* qs, const void* qe, s
     if (!qs || !qe || !out) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
     return DISPATCH_S(ix, ([&]() -> int {
+        if (g_tune.ub_tree && ix->ubt.ok) {
+            k_has_overlaps_table<S><<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(ix->view<S>(), ix->ubt.view<S>(),
+                                                                                  (const S*)qs, (const S*)qe, nq, out);
+            LAUNCH_CHECK();
+            return SI_OK;
+        }
         k_has_overlaps<S><<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(ix->view<S>(), (const S*)qs,
                                                                         (const S*)qe, nq, out);
         LAUNCH_CHECK();
@@ -2386,6 +2553,13 @@ SI_EXPORT int siCoverage(const siIndex* ix, const void* qs, const void* qe, size
     if (nq == 0) return SI_OK;
     if (!qs || !qe) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
+    if (rank_exact(ix) && ix->ubt.ok) {
+        k_coverage_rank<<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(
+            ix->view<int32_t>(), (const int32_t*)ix->d_ends_sorted, ix->ubt.view<int32_t>(), ix->ebt.view<int32_t>(),
+            ix->d_line_sums, (uint32_t)ix->sum_lines(), (const int32_t*)qs, (const int32_t*)qe, nq, count_out, cov_out);
+        LAUNCH_CHECK();
+        return SI_OK;
+    }
     k_coverage_i32<<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(ix->view<int32_t>(), (const int32_t*)qs,
                                                                  (const int32_t*)qe, nq, count_out, cov_out);
     LAUNCH_CHECK();
@@ -2441,6 +2615,9 @@ SetView<int32_t> set_view_of(const siIndex* ix) {
     v.eb_h = ix->eb.top_h;
     v.td = ix->tree<int32_t>();
     v.rank_exact = ix->n_inverted == 0 ? 1u : 0u;
+    v.ends_sorted = (const int32_t*)ix->d_ends_sorted;
+    v.ubt = ix->ubt.view<int32_t>();
+    v.ebt = ix->ebt.view<int32_t>();
     return v;
 }
 
@@ -2513,16 +2690,25 @@ __global__ __launch_bounds__(Q_THREADS) void k_multi_finish(const SetView<int32_
     const SetView<int32_t>& sv = sets[g];
     uint32_t ub = NONE, lb = NONE, c = 0;
     if (sv.v.n) {
-        ub = ub_tree_pos(sv.ub, sv.ub_top, sv.ub_h, e);
-        if (sv.rank_exact) lb = (s == INT32_MIN) ? 0u : ub_tree_pos(sv.ub, sv.ub_top, sv.ub_h, s - 1) + 1u;
-        if (ub != NONE) {
-            if (sv.rank_exact && s <= e) {
-                const uint32_t below = (s == INT32_MIN) ? 0u : ub_tree_pos(sv.eb, sv.eb_top, sv.eb_h, s - 1) + 1u;
-                c = ub + 1u - below;
-            } else {
-                c = walk_count(sv.v, ub, s);
+        const bool s1 = s != INT32_MIN;
+        uint32_t below = 0;   // #{ends < s}
+        if (sv.ubt.tab) {
+            const BucketView<int32_t> t[3] = {sv.ubt, sv.ubt, sv.ebt};
+            const int32_t* const v[3] = {sv.v.starts, sv.v.starts, sv.ends_sorted};
+            const int32_t x[3] = {e, s1 ? s - 1 : s, s1 ? s - 1 : s};
+            uint32_t r[3];
+            bucket_ranks<int32_t, 3>(t, v, sv.v.n, x, r);
+            ub = r[0] - 1u;
+            if (sv.rank_exact) lb = s1 ? r[1] : 0u;
+            below = s1 ? r[2] : 0u;
+        } else {
+            ub = ub_tree_pos(sv.ub, sv.ub_top, sv.ub_h, e);
+            if (sv.rank_exact) {
+                lb = s1 ? ub_tree_pos(sv.ub, sv.ub_top, sv.ub_h, s - 1) + 1u : 0u;
+                below = s1 ? ub_tree_pos(sv.eb, sv.eb_top, sv.eb_h, s - 1) + 1u : 0u;
             }
         }
+        if (ub != NONE) c = (sv.rank_exact && s <= e) ? ub + 1u - below : walk_count(sv.v, ub, s);
     }
     pv.idx[k] = ub;
     pv.lb[k] = lb;

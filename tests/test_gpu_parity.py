@@ -1358,3 +1358,35 @@ def test_plan_sort_around_the_scan_free_size(sia, dtype, nq):
         q = plan[256:256 + 4 * nq].view(torch.int32).cpu().numpy()
         assert np.array_equal(q, np.argsort(qe, kind="stable"))
     ix.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 64, 4095, 4096, 4097, 70_003])
+@pytest.mark.parametrize("inverted", [False, True])
+def test_coverage(sia, orc, n, inverted):
+    """Count and covered length against the oracle around the sizes of lines and tree nodes, with
+    coordinates over the whole int32 range (the sums wrap), equal starts and ends, queries with
+    s > e, s = e, at both ends of the range and beyond all intervals, and with intervals of
+    start > end in the index (the walk)."""
+    print(f"[gpu] coverage n={n} inverted={inverted}", flush=True)
+    rng = np.random.default_rng(n)
+    info = np.iinfo(np.int32)
+    for wide in (False, True):
+        lo, hi = (info.min, info.max) if wide else (-1000, 10 * n)
+        s = rng.integers(lo, hi, n)
+        length = rng.integers(0, (hi - lo) // 8 if wide else 300, n)
+        e = np.minimum(s + length, info.max)
+        s[: n // 4], e[: n // 4] = s[0], e[0]
+        if inverted:
+            s[-1], e[-1] = e[-1], s[-1] - 1 if s[-1] > info.min else s[-1]
+        s, e = s.astype(np.int32), e.astype(np.int32)
+        qs = np.concatenate([rng.integers(lo, hi, 400), s[:100], e[:100], [info.min, info.min, info.max, 0]])
+        qe = np.concatenate([qs[:400] + rng.integers(-50, 3000, 400), s[:100], e[:100] + 0, [info.min, info.max, info.max, -1]])
+        qe = np.clip(qe, info.min, info.max)
+        qs, qe = qs.astype(np.int32), qe.astype(np.int32)
+        ix = _dev_index(sia, s, e)
+        oix = orc.build_index(s, e)
+        c, v = ix.coverage(qs, qe)
+        want = [orc.coverage(oix, a, b) for a, b in zip(qs, qe)]
+        assert np.array_equal(c.astype(np.int64), [w[0] for w in want])
+        assert np.array_equal(v.astype(np.int64), [w[1] for w in want])
+        ix.close()
