@@ -392,10 +392,13 @@ struct KeyOut {
     __device__ __forceinline__ void put(size_t dst, K key, uint32_t) const { k[dst] = key; }
 };
 
+// What a scatter moves beside the keys: a payload array, nothing, or the item's input position.
+enum RsVals { RS_NONE = 0, RS_ARRAY = 1, RS_INDEX = 2 };
+
 // Stable scatter of one tile (digit offsets from the scan of the per-tile digit counts, or, with
 // SELF, from the counts themselves): the tile is ranked in registers, staged in LDS in digit order and written out so
 // equal digits land contiguously.
-template <class Out, typename K, bool VALS, bool SELF>
+template <class Out, typename K, RsVals VALS, bool SELF>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     const K* __restrict__ kin, const uint32_t* __restrict__ vin, Out out, size_t n, int shift, uint32_t flip,
     const uint32_t* __restrict__ th_base, uint32_t ntiles) {
@@ -418,7 +421,7 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     for (int r = 0; r < RS_ROUNDS; ++r) {
         const uint32_t li = (uint32_t)r * RS_THREADS + tid;
         key[r] = li < tile_n ? kin[base + li] : (K)0;
-        val[r] = VALS && li < tile_n ? vin[base + li] : 0u;
+        val[r] = VALS == RS_INDEX ? (uint32_t)(base + li) : VALS == RS_ARRAY && li < tile_n ? vin[base + li] : 0u;
     }
     uint32_t tot;
     if (SELF) {   // this thread's digit: its items in the tiles before this one, and in all
@@ -518,7 +521,7 @@ inline int rs_varying_bits(size_t n, const RsTemp& tmp, uint64_t* varying, hipSt
 inline bool rs_digit_varies(uint64_t varying, int d) { return ((varying >> (8 * d)) & 255u) != 0; }
 
 // One pass by the digit at `shift`: counts per tile, their scan, the scatter through out.
-template <typename K, bool VALS, class Out>
+template <typename K, RsVals VALS, class Out>
 int rs_pass(const K* kin, const uint32_t* vin, const Out& out, size_t n, int shift, uint32_t flip, const RsTemp& tmp,
             hipStream_t st) {
     const uint32_t ntiles = (uint32_t)rs_ntiles(n);
@@ -552,7 +555,7 @@ int radix_sort_signed(const K* in, K* k0, K* k1, K* out, size_t n, uint64_t vary
         if (!rs_digit_varies(varying, d)) continue;
         const uint32_t flip = (d == (int)sizeof(K) - 1) ? 0x80u : 0u;
         K* const dst = (d == last_d) ? out : k0;
-        const int rc = rs_pass<K, false>(src, (const uint32_t*)nullptr, KeyOut<K>{dst}, n, 8 * d, flip, tmp, st);
+        const int rc = rs_pass<K, RS_NONE>(src, (const uint32_t*)nullptr, KeyOut<K>{dst}, n, 8 * d, flip, tmp, st);
         if (rc != SI_OK) return rc;
         src = dst;
         std::swap(k0, k1);
@@ -586,10 +589,10 @@ int radix_sort_pairs(uint64_t* k0, uint32_t* v0, uint64_t* k1, uint32_t* v1, siz
         if (!rs_digit_varies(varying, d)) continue;
         int rc;
         if (last && d == last_d) {
-            rc = rs_pass<uint64_t, true>(ka, va, *last, n, 8 * d, 0u, tmp, st);
+            rc = rs_pass<uint64_t, RS_ARRAY>(ka, va, *last, n, 8 * d, 0u, tmp, st);
             if (last_written) *last_written = true;
         } else {
-            rc = rs_pass<uint64_t, true>(ka, va, ArrayOut{kb, vb}, n, 8 * d, 0u, tmp, st);
+            rc = rs_pass<uint64_t, RS_ARRAY>(ka, va, ArrayOut{kb, vb}, n, 8 * d, 0u, tmp, st);
         }
         if (rc != SI_OK) return rc;
         std::swap(ka, kb);

@@ -37,6 +37,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "si_internal.h"
@@ -1570,17 +1571,19 @@ __global__ __launch_bounds__(Q_THREADS) void k_count_rank_tree(IndexView<S> ix, 
     for (size_t k0 = (size_t)blockIdx.x * Q_THREADS; k0 < nq; k0 += (size_t)gridDim.x * Q_THREADS) {
         const size_t k = k0 + threadIdx.x;
         if (k >= nq) continue;
-        const uint32_t i = pv.idx[k];
-        const S s = pv.s[k], e = pv.e[k];
         uint32_t c = 0;
-        if (planned) {
+        if (planned) {   // (nothing else of the plan is read)
             c = pv.cnt[k];
-        } else if (i != NONE) {
-            if (s <= e) {
-                const uint32_t below = (s == SMIN) ? 0u : ub_tree_pos(t, s_top, h, (S)(s - 1)) + 1u;
-                c = i + 1u - below;
-            } else {
-                c = walk_count(ix, i, s);
+        } else {
+            const uint32_t i = pv.idx[k];
+            const S s = pv.s[k], e = pv.e[k];
+            if (i != NONE) {
+                if (s <= e) {
+                    const uint32_t below = (s == SMIN) ? 0u : ub_tree_pos(t, s_top, h, (S)(s - 1)) + 1u;
+                    c = i + 1u - below;
+                } else {
+                    c = walk_count(ix, i, s);
+                }
             }
         }
         const uint32_t q = pv.q[k];
@@ -1772,6 +1775,19 @@ __global__ __launch_bounds__(Q_THREADS) void k_plan_bounds_table(IndexView<S> ix
     }
 }
 
+// Device memory of a call, stream-ordered.
+struct ScopedPlan {
+    void* p = nullptr;
+    hipStream_t st;
+    explicit ScopedPlan(hipStream_t s) : st(s) {}
+    int alloc(size_t bytes) {
+        hipError_t e = hipMallocAsync(&p, bytes, st);
+        if (e != hipSuccess) { p = nullptr; return si_set_error(SI_ERR_NOMEM, "hipMallocAsync(%zu): %s", bytes, hipGetErrorString(e)); }
+        return SI_OK;
+    }
+    ~ScopedPlan() { if (p) (void)hipFreeAsync(p, st); }
+};
+
 template <typename S>
 int launch_plan_table(const siIndex* ix, PlanView<S> pv, size_t nq, bool with_lb, bool with_rank, hipStream_t st) {
     const BucketView<S> ts = ix->ubt.view<S>(), te = ix->ebt.view<S>();
@@ -1781,6 +1797,88 @@ int launch_plan_table(const siIndex* ix, PlanView<S> pv, size_t nq, bool with_lb
     else if (with_lb) k_plan_bounds_table<S, true, false><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, pv, nq);
     else if (with_rank) k_plan_bounds_table<S, false, true><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, pv, nq);
     else k_plan_bounds_table<S, false, false><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, pv, nq);
+    LAUNCH_CHECK();
+    return SI_OK;
+}
+
+// Block b's place in the order in which the 8 XCDs take contiguous eighths of the grid (blocks are
+// dealt to them round robin), so that each XCD's L2 serves one stretch of the index.
+__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb) {
+    const uint32_t per = nb / 8u;
+    return b < per * 8u ? (b % 8u) * per + b / 8u : b;
+}
+
+// Counts in the rank form without a plan: #{starts <= e} - #{ends < s} through the bucket tables
+// (inverted queries take the reference walk).  order: null, or the query at each position of qs
+// and qe.
+template <typename S>
+__global__ __launch_bounds__(Q_THREADS) void k_count_table(IndexView<S> ix, const S* __restrict__ ends_sorted,
+                                                           BucketView<S> ts, BucketView<S> te, const S* __restrict__ qs,
+                                                           const S* __restrict__ qe, const uint32_t* __restrict__ order,
+                                                           size_t nq, uint32_t* __restrict__ counts) {
+    constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
+    const size_t k = (size_t)(order ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * Q_THREADS + threadIdx.x;
+    if (k >= nq) return;
+    const S s = qs[k], e = qe[k];
+    const bool s1 = s != SMIN;   // s - 1 exists
+    const BucketView<S> t[2] = {ts, te};
+    const S* const v[2] = {ix.starts, ends_sorted};
+    const S x[2] = {e, s1 ? (S)(s - 1) : s};
+    uint32_t r[2];
+    bucket_ranks<S, 2>(t, v, ix.n, x, r);
+    counts[order ? order[k] : k] =
+        s <= e ? r[0] - (s1 ? r[1] : 0u) : (r[0] ? walk_count(ix, r[0] - 1u, s) : 0u);
+}
+
+// The queries grouped by their ends, one pass of the radix sort: the scatter's output.
+template <typename S>
+struct GroupOut {
+    uint32_t* __restrict__ q;
+    S* __restrict__ s;
+    S* __restrict__ e;
+    const S* __restrict__ qs;
+    template <typename K>
+    __device__ __forceinline__ void put(size_t dst, K key, uint32_t val) const {
+        q[dst] = val;
+        s[dst] = qs[val];
+        e[dst] = (S)key;
+    }
+};
+
+// count() through the tables.  The searches of unsorted queries read their table entries and keys
+// from all over the index: once that outgrows an XCD's 4 MB of L2, large batches are first grouped
+// into 256 stretches of the coordinates (one radix pass by eight bits of the end).
+// int32, 10M intervals: 10M queries 0.97 ms ungrouped, 0.56 grouped (through the sorted plan 0.87),
+// 2M 189 and 104 us, 1M 93 and 73, 500K 46 and 57; int64: 1M 135 and 98, 500K 66 and 77.  1M int32
+// intervals (4 MB): 2M queries 88 and 85, 800K 35 and 54.  100K: 10M queries 236 and 270.
+constexpr size_t GROUP_FROM = 3u << 18;
+template <typename S>
+int launch_count_table(const siIndex* ix, const S* qs, const S* qe, size_t nq, uint32_t* counts, hipStream_t st) {
+    const S* es = (const S*)ix->d_ends_sorted;
+    const BucketView<S> ts = ix->ubt.view<S>(), te = ix->ebt.view<S>();
+    const unsigned g = grid_for(nq, Q_THREADS);
+    if (nq < GROUP_FROM || ix->n * sizeof(S) < ((size_t)4 << 20)) {
+        k_count_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, qs, qe, nullptr, nq, counts);
+        LAUNCH_CHECK();
+        return SI_OK;
+    }
+    using K = typename std::conditional<sizeof(S) == 4, uint32_t, uint64_t>::type;
+    // the eight highest bits in which the index's starts differ (ends outside wrap around: the
+    // order only has to keep neighbours together)
+    const uint64_t differ = (uint64_t)ts.lo ^ (uint64_t)ts.hi;
+    int top = 0;
+    while (top < (int)sizeof(S) * 8 && (differ >> top) != 0) ++top;
+    const int shift = std::max(0, top - 8);
+    const size_t off_s = align256(4 * nq), off_e = off_s + align256(sizeof(S) * nq), off_rs = off_e + align256(sizeof(S) * nq);
+    ScopedPlan P(st);
+    int rc = P.alloc(off_rs + rs_temp_bytes(nq));
+    if (rc) return rc;
+    char* const p = (char*)P.p;
+    const GroupOut<S> out{(uint32_t*)p, (S*)(p + off_s), (S*)(p + off_e), qs};
+    const RsTemp rt = rs_temp_carve(p + off_rs, nq);
+    rc = rs_pass<K, RS_INDEX>((const K*)qe, nullptr, out, nq, shift, 0u, rt, st);
+    if (rc) return rc;
+    k_count_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, out.s, out.e, out.q, nq, counts);
     LAUNCH_CHECK();
     return SI_OK;
 }
@@ -2081,19 +2179,6 @@ int check_plan(const siIndex* ix, const void* plan, size_t plan_bytes, size_t nq
     return SI_OK;
 }
 
-// Stream-ordered scratch plan for the unplanned entry points.
-struct ScopedPlan {
-    void* p = nullptr;
-    hipStream_t st;
-    explicit ScopedPlan(hipStream_t s) : st(s) {}
-    int alloc(size_t bytes) {
-        hipError_t e = hipMallocAsync(&p, bytes, st);
-        if (e != hipSuccess) { p = nullptr; return si_set_error(SI_ERR_NOMEM, "hipMallocAsync(%zu): %s", bytes, hipGetErrorString(e)); }
-        return SI_OK;
-    }
-    ~ScopedPlan() { if (p) (void)hipFreeAsync(p, st); }
-};
-
 }  // namespace
 
 // ============================================================================
@@ -2283,6 +2368,8 @@ SI_EXPORT int siCount(const siIndex* ix, const void* qs, const void* qe, size_t 
     if (nq == 0) return SI_OK;
     if (!qs || !qe || !counts) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
+    if (g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF)
+        return DISPATCH_S(ix, (launch_count_table<S>(ix, (const S*)qs, (const S*)qe, nq, counts, st)));
     ScopedPlan P(st);
     const size_t pb = siPlanBytes(ix, nq);
     if ((rc = P.alloc(pb))) return rc;

@@ -1390,3 +1390,68 @@ def test_coverage(sia, orc, n, inverted):
         assert np.array_equal(c.astype(np.int64), [w[0] for w in want])
         assert np.array_equal(v.astype(np.int64), [w[1] for w in want])
         ix.close()
+
+
+@pytest.mark.parametrize("shape", ["even", "gap", "crowd", "one point", "wide"])
+@pytest.mark.parametrize("n", [1, 4, 15, 17, 4096, 20_011])
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_bucket_tables(sia, orc, dtype, n, shape):
+    """upper_bound, count and has_overlaps through the bucket tables: buckets of one key, of up to
+    16 and of more, empty buckets in runs longer than a wave fills (a far interval), tables given
+    up because most keys share a bucket, all keys equal, and coordinates over the whole range of
+    the type."""
+    print(f"[gpu] bucket tables {np.dtype(dtype).name} n={n} {shape}", flush=True)
+    rng = np.random.default_rng(n)
+    info = np.iinfo(dtype)
+    if shape == "wide":
+        s = rng.integers(info.min, info.max, n, dtype=dtype)
+        e = np.maximum(s, rng.integers(info.min, info.max, n, dtype=dtype))
+        s[0], e[-1] = info.min, info.max
+    else:
+        s = rng.integers(0, 1 if shape == "one point" else 9 * n, n).astype(dtype)
+        e = (s + (0 if shape == "one point" else rng.integers(0, 200, n))).astype(dtype)
+        if shape == "gap":
+            s[-1], e[-1] = 900 * n, 900 * n + 10
+        elif shape == "crowd":
+            s[-1], e[-1] = 2**30, 2**30 + 1
+    ix = _dev_index(sia, s, e)
+    oix = orc.build_index(s, e)
+    near = rng.integers(-3, 4, 200)
+    at = np.concatenate([s[rng.integers(0, n, 100)], e[rng.integers(0, n, 100)]]).astype(object) + near
+    any_ = rng.integers(info.min, info.max, 100, dtype=dtype).astype(object)
+    qs = np.concatenate([at, any_, [info.min, info.min, info.max, info.max, 0]])
+    qe = np.concatenate([at + rng.integers(-5, 300, 200), any_[::-1], [info.min, info.max, info.max, info.min, 0]])
+    qs = np.clip(qs, info.min, info.max).astype(dtype)
+    qe = np.clip(qe, info.min, info.max).astype(dtype)
+    ub = ix.upper_bound(qs).astype(np.uint32).view(np.int32)
+    assert np.array_equal(ub, np.searchsorted(np.sort(s), qs, side="right").astype(np.int64) - 1)
+    assert np.array_equal(ix.count(qs, qe), orc.count_batch(oix, qs, qe))
+    want = [bool(orc.has_overlaps(oix, a, b)) for a, b in zip(qs, qe)]
+    assert np.array_equal(np.asarray(ix.has_overlaps(qs, qe)).astype(bool), want)
+    ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("nq", [786_431, 786_432, 1_000_003])
+def test_count_grouped(sia, orc, dtype, nq):
+    """count() on both sides of the batch size from which its queries are grouped by their ends,
+    on an index of more than 4 MB, with queries around, beyond and far outside the intervals and
+    inverted ones."""
+    torch = pytest.importorskip("torch")
+    print(f"[gpu] count grouped {np.dtype(dtype).name} nq={nq}", flush=True)
+    rng = np.random.default_rng(nq)
+    info = np.iinfo(dtype)
+    n = 1_100_000
+    s = rng.integers(-5_000_000, 60_000_000, n).astype(dtype)
+    e = (s + rng.integers(0, 400, n)).astype(dtype)
+    qs = rng.integers(-6_000_000, 70_000_000, nq).astype(dtype)
+    qe = (qs + rng.integers(-2, 3000, nq)).astype(dtype)
+    qs[:4], qe[:4] = [info.min, info.min, info.max, 7], [info.min, info.max, info.max, info.min]
+    ix = _dev_index(sia, s, e)
+    want = orc.count_batch(orc.build_index(s, e), qs, qe)
+    c = torch.full((nq + 64,), -7, dtype=torch.int32, device="cuda")
+    ix.count_device(torch.from_numpy(qs).cuda(), torch.from_numpy(qe).cuda(), c)
+    torch.cuda.synchronize()
+    c = c.cpu().numpy()
+    assert np.array_equal(c[:nq], want) and np.all(c[nq:] == -7)
+    ix.close()
