@@ -512,6 +512,8 @@ __device__ __forceinline__ uint32_t kbit_entry(uint32_t b) {
 // A 32-bit word in global memory: output addresses rebuilt from integers keep their address
 // space, so their stores stay global stores (a generic pointer would make them flat ones).
 typedef __attribute__((address_space(1))) uint32_t global_u32;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));   // 16 bytes at any element
+typedef __attribute__((address_space(1))) u32x4 global_u32x4;
 
 // One output segment of a lane: c values at output offset o, either the ascending range
 // base .. base + c - 1 (asc), the descending range base .. base - c + 1 (desc), or the set
@@ -1235,19 +1237,13 @@ __device__ __forceinline__ void guided_walk(const S* __restrict__ ends, const ui
     }
 }
 
-// Walks the hits at and below cur (see above).  acc: the count so far (count mode) or the
-// next output offset (fill modes, writes below oend only); left: in fill modes the hits
-// still expected, counted down.  With a long list (lv.len > 0) the positions below P0 = the
-// first position starting at or after s - lv.len hold no hit but a long interval, so the
-// walk reads the index's arrays down to P0 only and takes the rest from the long list,
-// whose entries all lie below P0: the output order is unchanged.
-template <typename S, int MODE>
-__device__ __forceinline__ void wave_walk(const IndexView<S>& ix, const TreeDesc<S>& td, const UbTree<S>& ub,
-                                          const LongView<S>& lv, int lane, S s, uint32_t cur, uint32_t top, bool lead,
-                                          uint64_t& acc, uint64_t oend, uint32_t& left, uint32_t* __restrict__ out_idx,
-                                          const int32_t* __restrict__ vals, int32_t* __restrict__ out_val) {
-    // leading run (vector order): consecutive lines while every position down from cur is a hit
-    while (MODE == W_VECTOR && lead && cur != NONE) {
+// The leading run of the vector order: consecutive lines while every position down from cur is a
+// hit.  cur is left at the first miss (NONE: there is none).
+template <typename S>
+__device__ __forceinline__ void wave_lead(const IndexView<S>& ix, int lane, S s, uint32_t& cur, uint32_t top, uint64_t& acc,
+                                          uint64_t oend, uint32_t& left, uint32_t* __restrict__ out_idx) {
+    bool lead = true;
+    while (lead && cur != NONE) {
         const uint32_t b0 = cur & ~63u;
         const uint32_t kc = cur - b0;
         const bool hit = ((uint32_t)lane <= kc) && (wave_end(ix, b0 + lane) >= s);
@@ -1269,6 +1265,34 @@ __device__ __forceinline__ void wave_walk(const IndexView<S>& ix, const TreeDesc
             lead = false;
         }
     }
+}
+
+// The hits among the positions [P0, cur] of the index.
+template <typename S, int MODE>
+__device__ __forceinline__ void wave_near(const IndexView<S>& ix, const TreeDesc<S>& td, int lane, S s, uint32_t cur,
+                                          uint32_t P0, uint64_t& acc, uint64_t oend, uint32_t& left,
+                                          uint32_t* __restrict__ out_idx, const int32_t* __restrict__ vals,
+                                          int32_t* __restrict__ out_val) {
+    if (sizeof(S) == 8 && ix.ends32)
+        guided_walk<S, MODE, false, true, WAVE_LINES>(ix.ends, ix.ends32, ix.ends32_base, nullptr, td, lane, s, cur, P0,
+                                                      acc, oend, left, out_idx, vals, out_val);
+    else
+        guided_walk<S, MODE, false, false, WAVE_LINES>(ix.ends, nullptr, 0, nullptr, td, lane, s, cur, P0, acc, oend,
+                                                       left, out_idx, vals, out_val);
+}
+
+// Walks the hits at and below cur (see above).  acc: the count so far (count mode) or the
+// next output offset (fill modes, writes below oend only); left: in fill modes the hits
+// still expected, counted down.  With a long list (lv.len > 0) the positions below P0 = the
+// first position starting at or after s - lv.len hold no hit but a long interval, so the
+// walk reads the index's arrays down to P0 only and takes the rest from the long list,
+// whose entries all lie below P0: the output order is unchanged.
+template <typename S, int MODE>
+__device__ __forceinline__ void wave_walk(const IndexView<S>& ix, const TreeDesc<S>& td, const UbTree<S>& ub,
+                                          const LongView<S>& lv, int lane, S s, uint32_t cur, uint32_t top, bool lead,
+                                          uint64_t& acc, uint64_t oend, uint32_t& left, uint32_t* __restrict__ out_idx,
+                                          const int32_t* __restrict__ vals, int32_t* __restrict__ out_val) {
+    if (MODE == W_VECTOR && lead) wave_lead(ix, lane, s, cur, top, acc, oend, left, out_idx);
     if (cur == NONE) return;
     uint32_t P0 = 0;
     if (lv.len > 0) {
@@ -1276,12 +1300,7 @@ __device__ __forceinline__ void wave_walk(const IndexView<S>& ix, const TreeDesc
         // x = s - len - 1 (upper_bound(x) + 1 = the first position starting at >= s - len)
         if ((int64_t)s > (int64_t)SMIN + lv.len) P0 = wave_tree_ub(ub, (S)((int64_t)s - lv.len - 1), lane) + 1u;
     }
-    if (sizeof(S) == 8 && ix.ends32)
-        guided_walk<S, MODE, false, true, WAVE_LINES>(ix.ends, ix.ends32, ix.ends32_base, nullptr, td, lane, s, cur, P0,
-                                                      acc, oend, left, out_idx, vals, out_val);
-    else
-        guided_walk<S, MODE, false, false, WAVE_LINES>(ix.ends, nullptr, 0, nullptr, td, lane, s, cur, P0, acc, oend,
-                                                       left, out_idx, vals, out_val);
+    wave_near<S, MODE>(ix, td, lane, s, cur, P0, acc, oend, left, out_idx, vals, out_val);
     if (P0 > 0) {
         const uint32_t J = lv.lrank[min(P0, cur + 1u)];   // long entries below that position
         if (J > 0 && sizeof(S) == 8 && lv.ends32)
@@ -1305,6 +1324,52 @@ __device__ __forceinline__ void wave_walk(const IndexView<S>& ix, const TreeDesc
 constexpr uint32_t HEAVY_CHUNKS = SI_HEAVY_CHUNKS;
 static_assert(HEAVY_CHUNKS >= 1 && HEAVY_CHUNKS <= 8, "the plan holds 8 chunk counters");
 
+// The entries [0, n) dealt to the waves (or workgroups) of a grid, in HEAVY_CHUNKS chunks: worker w
+// of `workers` (a multiple of HEAVY_CHUNKS) starts on chunk w % HEAVY_CHUNKS with that chunk's entry
+// w / HEAVY_CHUNKS, takes what is left of it by the counter ctr[chunk], and once it is used up looks
+// at all counters with one load and goes on with a chunk that has entries left.  (With an atomic for
+// every entry and every chunk found empty, up to 9 a worker on one cache line, 8192 waves took 0.8 ms
+// whatever the batch.)  Called by whole waves.
+struct EntryDeal {
+    uint32_t* __restrict__ ctr;
+    uint32_t n, per, fixed;   // entries, of a chunk, and of these dealt without the counter
+    uint32_t c, next;         // chunk in hand; the entry dealt first (NONE: taken)
+
+    __device__ __forceinline__ EntryDeal(uint32_t* counters, uint32_t entries, uint32_t w, uint32_t workers)
+        : ctr(counters), n(entries), per((entries + HEAVY_CHUNKS - 1u) / HEAVY_CHUNKS), fixed(workers / HEAVY_CHUNKS),
+          c(w % HEAVY_CHUNKS), next(w / HEAVY_CHUNKS) {}
+
+    __device__ __forceinline__ uint32_t size(uint32_t chunk) const {
+        const uint64_t beg = (uint64_t)chunk * per;
+        return beg < n ? min(per, n - (uint32_t)beg) : 0u;
+    }
+
+    __device__ __forceinline__ uint32_t take(int lane) {
+        if (next != NONE) {
+            const uint32_t h = next;
+            next = NONE;
+            if (h < size(c)) return c * per + h;
+        }
+        if (per <= fixed) return NONE;   // all dealt
+        while (true) {
+            bool open = false;
+            if ((uint32_t)lane < HEAVY_CHUNKS)
+                open = fixed + __hip_atomic_load(&ctr[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
+                       size((uint32_t)lane);
+            const uint64_t m = __builtin_amdgcn_ballot_w64(open);
+            if (m == 0) return NONE;
+            if (!((m >> c) & 1ull)) {
+                const uint64_t after = m & ~mask_upto(c);
+                c = (uint32_t)__builtin_ctzll(after ? after : m);
+            }
+            uint32_t h = 0;
+            if (lane == 0) h = atomicAdd(&ctr[c], 1u);
+            h = fixed + (uint32_t)__builtin_amdgcn_readfirstlane((int)h);
+            if (h < size(c)) return c * per + h;
+        }
+    }
+};
+
 // Clears the counters a walk launch uses (tiles, heavy list, mismatch flag, chunk counters).
 __global__ void k_walk_counters_reset(uint32_t* __restrict__ c) {
     const uint32_t i = threadIdx.x;
@@ -1312,43 +1377,26 @@ __global__ void k_walk_counters_reset(uint32_t* __restrict__ c) {
 }
 
 template <typename S, int MODE, bool MULTI = false>
-__global__ __launch_bounds__(Q_THREADS) void k_walk_heavy(IndexView<S> ix_arg, TreeDesc<S> td_arg, UbTree<S> ub_arg,
+__global__ __launch_bounds__(Q_THREADS) void k_walk_heavy(IndexView<S> ix, TreeDesc<S> td, UbTree<S> ub,
                                                           LongView<S> lv, PlanView<S> pv,
                                                           uint32_t* __restrict__ counts,
                                                           uint64_t* __restrict__ counts64,
                                                           const uint64_t* __restrict__ offsets,
                                                           uint32_t* __restrict__ out_idx,
-                                                          const int32_t* __restrict__ vals_arg,
+                                                          const int32_t* __restrict__ vals,
                                                           int32_t* __restrict__ out_val, uint64_t cap,
                                                           const SetView<S>* __restrict__ sets) {
-    IndexView<S> ix = ix_arg;
-    TreeDesc<S> td = td_arg;
-    UbTree<S> ub = ub_arg;
-    const int32_t* __restrict__ vals = vals_arg;
     const int lane = lane_id();
     const uint32_t nheavy = __builtin_amdgcn_readfirstlane(pv.counter[1]);
     if (nheavy == 0) return;   // nothing parked: no wave touches the shared counters
-    const uint32_t chunk = (nheavy + HEAVY_CHUNKS - 1u) / HEAVY_CHUNKS;
-    uint32_t c = blockIdx.x % HEAVY_CHUNKS, tried = 0;
+    constexpr uint32_t WAVES = Q_THREADS / WAVE;
+    EntryDeal deal(pv.counter + 8, nheavy, (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE * gridDim.x + blockIdx.x)),
+                   gridDim.x * WAVES);
     while (true) {
-        uint32_t h = 0;
-        if (lane == 0) h = atomicAdd(&pv.counter[8 + c], 1u);
-        h = __builtin_amdgcn_readfirstlane(__shfl(h, 0, WAVE));
-        const uint32_t beg = c * chunk, len = (beg < nheavy) ? min(chunk, nheavy - beg) : 0u;
-        if (h >= len) {   // chunk c is exhausted: the next one
-            if (++tried == HEAVY_CHUNKS) break;
-            c = (c + 1u) % HEAVY_CHUNKS;
-            continue;
-        }
-        const HeavyEntry he = pv.heavy[beg + h];
+        const uint32_t h = deal.take(lane);
+        if (h == NONE) break;
+        const HeavyEntry he = pv.heavy[h];
         const uint32_t k = __builtin_amdgcn_readfirstlane(he.k);
-        if (MULTI) {   // the parked query's set
-            const uint32_t g = __builtin_amdgcn_readfirstlane(pv.set[k]);
-            ix = sets[g].v;
-            td = sets[g].td;
-            ub = sets[g].ub;
-            vals = sets[g].values;
-        }
         const uint32_t q = __builtin_amdgcn_readfirstlane(pv.q[k]);
         const S s = pv.s[k];
         const uint32_t cur = __builtin_amdgcn_readfirstlane(he.cur);
@@ -1358,7 +1406,12 @@ __global__ __launch_bounds__(Q_THREADS) void k_walk_heavy(IndexView<S> ix_arg, T
         uint64_t acc = he.acc;
         // (never below acc: offsets that decrease give an empty room, not a wrapped one)
         const uint64_t oend = (MODE != W_COUNT) ? max(min(offsets[q + 1], cap), acc) : 0;
-        wave_walk<S, MODE>(ix, td, ub, lv, lane, s, cur, top, lead, acc, oend, left, out_idx, vals, out_val);
+        if (MULTI) {   // the parked query's set
+            const SetView<S>& sv = sets[__builtin_amdgcn_readfirstlane(pv.set[k])];
+            wave_walk<S, MODE>(sv.v, sv.td, sv.ub, lv, lane, s, cur, top, lead, acc, oend, left, out_idx, sv.values, out_val);
+        } else {
+            wave_walk<S, MODE>(ix, td, ub, lv, lane, s, cur, top, lead, acc, oend, left, out_idx, vals, out_val);
+        }
         if (MODE == W_COUNT) {
             // every lane stores the same value (no lane-dependent branch in the loop)
             if (counts) counts[q] = (uint32_t)acc;
@@ -2120,6 +2173,24 @@ inline uint32_t sweep_chunk(size_t nq, int cus) {
     return (uint32_t)std::min<size_t>(SW_CHUNK, (nq + waves - 1) / waves);
 }
 
+// The queries that the sweep left, through the long list: spans of up to 32 queries (or one
+// chunk), fewer where that would leave workgroups without one.
+template <typename S, int MODE>
+int launch_sweep_shared(const siIndex* ix, const PlanView<S>& pv, size_t nq, uint32_t chunk, int cus,
+                        const uint64_t* offsets, uint32_t* out_idx, int32_t* out_val, uint64_t cap, hipStream_t st) {
+    IndexView<S> hv = ix->view<S>();
+    LongView<S> lv = long_view_of<S>(ix);
+    if (!g_tune.heavy_ends32) { hv.ends32 = nullptr; lv.ends32 = nullptr; }
+    const size_t grid = (size_t)cus * sh_wgs(MODE);
+    const uint32_t want = (uint32_t)std::min<size_t>(32, nq / grid);
+    const uint32_t span = chunk * std::max(1u, want / chunk);
+    k_sweep_shared<S, MODE><<<(unsigned)std::min<size_t>(grid, ((nq + span - 1) / span + HEAVY_CHUNKS - 1) / HEAVY_CHUNKS * HEAVY_CHUNKS), SH_THREADS, 0, st>>>(
+        hv, ix->tree<S>(), ub_tree_of<S>(ix->ub, (const S*)ix->d_starts, ix->n), ix->ubt.view<S>(), lv, pv, (uint32_t)nq,
+        chunk, span, offsets, out_idx, ix->d_values, out_val, cap);
+    LAUNCH_CHECK();
+    return SI_OK;
+}
+
 template <typename S, int MODE>
 int launch_walk(const siIndex* ix, void* plan, size_t nq, uint32_t* counts, uint64_t* counts64,
                 const uint64_t* offsets, uint32_t* out_idx, int32_t* out_val, hipStream_t st,
@@ -2142,9 +2213,15 @@ int launch_walk(const siIndex* ix, void* plan, size_t nq, uint32_t* counts, uint
         swept = range_skip_on(ix);
         if (swept) {
             const uint32_t chunk = sweep_chunk(nq, cus);
+            const LongView<S> lv = long_view_of<S>(ix);
+            const bool by_place = lv.len > 0;   // (k_sweep_shared)
             k_sweep<S, MODE><<<grid_for(nq, chunk * SW_WAVES), SW_THREADS, 0, st>>>(
-                ix->view<S>(), ix->tree<S>(), pv, (uint32_t)nq, chunk, offsets,
+                ix->view<S>(), ix->tree<S>(), nullptr, pv, (uint32_t)nq, chunk, by_place, offsets,
                 MODE == W_VALUES ? (uint32_t*)out_val : out_idx, ix->d_values, cap);
+            if (by_place) {
+                LAUNCH_CHECK();
+                return launch_sweep_shared<S, MODE>(ix, pv, nq, chunk, cus, offsets, out_idx, out_val, cap, st);
+            }
         }
     }
     if (!swept) {

@@ -219,14 +219,33 @@ __device__ __forceinline__ void sweep_emit(SweepGroup<S>& g, uint64_t todo, int 
         // the (leading) run
         uint32_t p = (MODE == W_VECTOR) ? ub + 1u - lead + (uint32_t)lane : ub - (uint32_t)lane;
         uint32_t w = min(lead, room);
-        if (w >= 8u * WAVE) {
+        if (w >= 8u * WAVE) {   // to a 256-byte boundary, then four values a lane and store
             global_u32* o = reinterpret_cast<global_u32*>((uintptr_t)at);
-            for (; w >= (uint32_t)WAVE; w -= WAVE) {
-                o[(uint32_t)lane] = VALUES ? (uint32_t)vals[p] : p;
-                o += WAVE;
-                p += (MODE == W_VECTOR) ? (uint32_t)WAVE : 0u - (uint32_t)WAVE;
+            constexpr uint32_t STEP = 4u * WAVE, UP = (MODE == W_VECTOR) ? 1u : 0u - 1u;   // (positions a slot)
+            uint32_t done = (0u - (uint32_t)(at >> 2)) & 63u;
+            if ((uint32_t)lane < done) o[(uint32_t)lane] = VALUES ? (uint32_t)vals[p] : p;
+            p += UP * (done + 3u * (uint32_t)lane);
+            o += done + 4u * (uint32_t)lane;
+            if (VALUES) {
+                for (; w - done >= 4u * STEP; done += 4u * STEP) {   // four loads before their stores
+                    u32x4 v[4];
+#pragma unroll
+                    for (uint32_t x = 0; x < 4u; ++x) v[x] = *reinterpret_cast<const u32x4*>(vals + (p - x * STEP - 3u));
+#pragma unroll
+                    for (uint32_t x = 0; x < 4u; ++x) *reinterpret_cast<global_u32x4*>(o + x * STEP) = v[x].wzyx;
+                    o += 4u * STEP;
+                    p -= 4u * STEP;
+                }
             }
-            const uint32_t done = (min(lead, room)) - w;
+            for (; w - done >= STEP; done += STEP) {
+                const u32x4 v = VALUES ? (*reinterpret_cast<const u32x4*>(vals + (p - 3u))).wzyx
+                                       : u32x4{p, p + UP, p + 2u * UP, p + 3u * UP};
+                *reinterpret_cast<global_u32x4*>(o) = v;
+                o += STEP;
+                p += UP * STEP;
+            }
+            p -= UP * 3u * (uint32_t)lane;
+            w -= done;
             at += (uint64_t)done * 4u;
             lead -= done;
             room -= done;
@@ -314,30 +333,20 @@ __device__ __forceinline__ void sweep_lanes(SweepGroup<S>& g, uint64_t todo, int
     g.found = mine ? k : g.found;
 }
 
-// One wave per chunk of `chunk` consecutive sorted queries (see above).  MODE: W_DESC,
-// W_VECTOR or W_VALUES; out: the positions or values as 32-bit words; only slots below cap
-// and inside a query's segment [offsets[q], offsets[q + 1]) are written.  Queries left to the
-// wave-cooperative kernel go to the plan's heavy list, their run already written (not in
-// vector order, where the run is part of the leading run).
+// The plan's queries t0 .. t0 + m - 1 (of one index), by one wave with its part of the LDS (see above).
+// out: the positions or values as 32-bit words; only slots below cap and inside a query's segment
+// [offsets[q], offsets[q + 1]) are written.  Queries left to the wave-cooperative kernels go to the
+// plan's heavy list, their run already written (not in vector order, where the run is part of
+// the leading run); returns their number.  bad: a query's hits differ from its offsets.
 template <typename S, int MODE>
-__global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<S> td, PlanView<S> pv, uint32_t nq,
-                                                      uint32_t chunk, const uint64_t* __restrict__ offsets,
-                                                      uint32_t* __restrict__ out, const int32_t* __restrict__ vals,
-                                                      uint64_t cap) {
+__device__ __forceinline__ uint32_t sweep_queries(const IndexView<S>& ix, const TreeDesc<S>& td, const PlanView<S>& pv,
+                                                  uint32_t t0, uint32_t m, bool by_place, int lane,
+                                                  S* __restrict__ l_end, uint32_t* __restrict__ l_pay,
+                                                  uint32_t* __restrict__ l_key, const uint64_t* __restrict__ offsets,
+                                                  uint32_t* __restrict__ out, const int32_t* __restrict__ vals,
+                                                  uint64_t cap, bool& bad) {
     constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
     constexpr bool VALUES = MODE == W_VALUES;
-    __shared__ S s_end[SW_WAVES][SW_CAP];
-    __shared__ uint32_t s_pay[SW_WAVES][SW_CAP];
-    __shared__ uint32_t s_key[SW_WAVES][SW_CHUNK];
-    const int lane = lane_id();
-    const uint32_t wv = uniform(threadIdx.x / WAVE);
-    S* const l_end = s_end[wv];
-    uint32_t* const l_pay = s_pay[wv];
-    uint32_t* const l_key = s_key[wv];
-    const uint64_t t0w = (uint64_t)(blockIdx.x * (uint32_t)SW_WAVES + wv) * chunk;
-    if (t0w >= nq) return;
-    const uint32_t t0 = (uint32_t)t0w;
-    const uint32_t m = min(chunk, nq - t0);   // this wave's queries
 
     // ---- the chunk's queries in the order of their starts: keys (start - smallest) >> sh in
     // 24 bits, query in 8
@@ -396,7 +405,7 @@ __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<
     uint32_t A = 0, wbase = NONE;               // wbase NONE: no list yet
     S we = SMIN;                                // window: ends and payloads
     uint32_t wp = 0, full = 0;                  // full: a list outgrew SW_CAP, the chunk's other queries are left too
-    bool bad = false;
+    uint32_t parked = 0;                        // queries left so far
 
     // the packed entries l_end / l_pay[0 .. n) as the list
     auto take_list = [&](uint32_t n) {
@@ -434,10 +443,13 @@ __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<
         g.found = 0;
         const uint32_t gline = (g.lb - 1u) & ~63u;
         const bool ordered = g.lb <= g.ub + 1u;   // else start > end, with starts between the two
-        // queries whose hits all lie in their run, then those the list serves
-        const uint64_t runs = __builtin_amdgcn_ballot_w64(mine && ordered && g.lb == 0u);
-        uint64_t todo = __builtin_amdgcn_ballot_w64(mine && ordered && g.lb != 0u);
-        uint64_t left = __builtin_amdgcn_ballot_w64(mine && !ordered && g.ub != NONE);
+        // queries whose hits all lie in their run, those held by more intervals than a list takes (by
+        // their counts), then those the list serves
+        const uint64_t many =
+            __builtin_amdgcn_ballot_w64(mine && ordered && g.lb != 0u && gcnt > SW_CAP && gcnt - (g.ub + 1u - g.lb) > SW_CAP);
+        uint64_t todo = __builtin_amdgcn_ballot_w64(mine && ordered && g.lb != 0u) & ~many;
+        uint64_t left = __builtin_amdgcn_ballot_w64(mine && !ordered && g.ub != NONE) | many;
+        const uint64_t runs = __builtin_amdgcn_ballot_w64(mine && ordered && g.lb == 0u) | (MODE == W_VECTOR ? 0ull : many);
         const uint64_t few = __builtin_amdgcn_ballot_w64(mine && ordered && gcnt <= SW_FEW && g.ub + 1u - g.lb <= SW_FEW);
         if (runs) {
             const uint64_t rf = (uint32_t)__popcll(runs & few) >= 8u ? runs & few : 0ull;
@@ -518,16 +530,332 @@ __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<
         if (leave) {
             // (per lane, outside every wave-wide step; the run [lb, ub] is written, but for the vector order)
             const uint32_t c = ordered && MODE != W_VECTOR ? g.ub + 1u - g.lb : 0u;
-            HeavyEntry he;
+            // (field by field: the first entry's pad is the chunk's number of them)
+            HeavyEntry& he = pv.heavy[by_place ? t0 + parked + lanes_below(left) : atomicAdd(&pv.counter[1], 1u)];
             he.k = gk;
             he.cur = ordered ? g.lb - 1u : g.ub;
             he.top = g.ub;
             he.lead = MODE == W_VECTOR ? 1u : 0u;
             he.acc = go + min(c, g.room);
             he.left = gcnt - c;
-            he.pad = 0u;
-            pv.heavy[atomicAdd(&pv.counter[1], 1u)] = he;
+        }
+        parked += (uint32_t)__popcll(left);
+    }
+    return parked;
+}
+
+// One wave per chunk of `chunk` consecutive sorted queries.  MODE: W_DESC, W_VECTOR or W_VALUES.
+// by_place: a chunk's heavy entries lie at its first query's place, their number in the first one's
+// pad; else they follow each other in any order.  MULTI: the plan's queries are sorted by their set
+// (pv.set), a chunk's are answered set by set.
+template <typename S, int MODE, bool MULTI = false>
+__global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<S> td, const SetView<S>* __restrict__ sets,
+                                                      PlanView<S> pv, uint32_t nq, uint32_t chunk, bool by_place,
+                                                      const uint64_t* __restrict__ offsets,
+                                                      uint32_t* __restrict__ out, const int32_t* __restrict__ vals,
+                                                      uint64_t cap) {
+    __shared__ S s_end[SW_WAVES][SW_CAP];
+    __shared__ uint32_t s_pay[SW_WAVES][SW_CAP];
+    __shared__ uint32_t s_key[SW_WAVES][SW_CHUNK];
+    const int lane = lane_id();
+    const uint32_t wv = uniform(threadIdx.x / WAVE);
+    const uint64_t t0w = (uint64_t)(blockIdx.x * (uint32_t)SW_WAVES + wv) * chunk;
+    if (t0w >= nq) return;
+    uint32_t t0 = (uint32_t)t0w;
+    const uint32_t m = min(chunk, nq - t0);   // this wave's queries
+    bool bad = false;
+    if (MULTI) {
+        for (uint32_t n; t0 < (uint32_t)t0w + m; t0 += n) {
+            const uint32_t g = uniform(pv.set[t0]);
+            n = 0;
+            for (uint64_t other = 0; other == 0 && t0 + n < (uint32_t)t0w + m;) {
+                const uint32_t i = t0 + n + (uint32_t)lane;
+                other = __builtin_amdgcn_ballot_w64(i >= (uint32_t)t0w + m || pv.set[i] != g);
+                n += other ? (uint32_t)__builtin_ctzll(other) : (uint32_t)WAVE;
+            }
+            sweep_queries<S, MODE>(sets[g].v, sets[g].td, pv, t0, n, false, lane, s_end[wv], s_pay[wv], s_key[wv], offsets,
+                                   out, nullptr, cap, bad);
+        }
+    } else {
+        const uint32_t parked = sweep_queries<S, MODE>(ix, td, pv, t0, m, by_place, lane, s_end[wv], s_pay[wv], s_key[wv],
+                                                       offsets, out, vals, cap, bad);
+        if (by_place && lane == 0) {
+            pv.heavy[t0].pad = parked;
+            if (parked) atomicAdd(&pv.counter[1], parked);
         }
     }
     if (bad) atomicOr(&pv.counter[3], 1u);   // a query's hits differ from its offsets
+}
+
+// ---- the queries that the sweep left, several answered from one candidate list
+//
+// Where more than SW_CAP intervals hold a query's start, most of them are long: they lie far below
+// it, thinly spread over the entries of the long list (300 lines of 64 for 4100 hits, one in five
+// a hit, in 20M int64 intervals with 20 % of 10^5 .. 10^7 long), and neighbouring queries share
+// nearly all of them.  A workgroup takes a span of the plan's queries, orders those left by their
+// starts and cuts them into groups (SH_SPREAD).  For a group its waves collect the long entries
+// that reach the first start into LDS, highest first, CAP at a time; then each wave answers
+// its queries from the list, two compares, a ballot and a store for 64 entries.  The positions
+// at and above s - len are read from the index for each query.  A group of fewer than SH_LEAST
+// queries would leave the other waves idle: each walks on its own (wave_walk).
+//
+// What bounds it: waits for memory, at 16 waves a CU (the lists' LDS).  100K queries on 20M such
+// intervals: 0.75 ms (2.0 with a walk of the long list for each query), of which without the
+// lists' stores 0.64, without the scan 0.48, without lists 0.33, without the index's positions
+// too 0.21.  2000 queries on 20M: 0.15 ms (0.80), 30K on 5M: 0.17 (1.15).  CAP 6144 (12 waves a CU)
+// and 8 waves a workgroup were slower by 20 and 10 %, CAP 2048 by 10 %, but with payloads, which
+// take another word of LDS an entry, faster by 15 %.  SH_SPREAD 512: 1.30 ms for that fill,
+// 1024: 1.10, 2048 and 4096: 1.00.
+constexpr int SH_THREADS = 256;
+constexpr int SH_WAVES = SH_THREADS / WAVE;
+constexpr uint32_t SH_SPREAD = 2048;     // long entries that start within a group's range
+constexpr uint32_t SH_LEAST = 3;         // smallest group that shares a list
+constexpr uint32_t sh_cap(int mode) { return mode == W_VALUES ? 2048u : 4096u; }
+constexpr unsigned sh_wgs(int mode) { return mode == W_VALUES ? 6u : 4u; }   // workgroups a CU (160 KB of LDS)
+
+template <typename S, int MODE>
+__global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, TreeDesc<S> td, UbTree<S> ub, BucketView<S> tab,
+                                                             LongView<S> lv, PlanView<S> pv, uint32_t nq, uint32_t chunk,
+                                                             uint32_t span, const uint64_t* __restrict__ offsets,
+                                                             uint32_t* __restrict__ out_idx,
+                                                             const int32_t* __restrict__ vals,
+                                                             int32_t* __restrict__ out_val, uint64_t cap) {
+    constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
+    constexpr bool VALUES = MODE == W_VALUES;
+    constexpr uint32_t CAP = sh_cap(MODE);            // candidates held at a time
+    constexpr uint32_t LINES = VALUES ? 4 : 8;        // lines a wave collects at a time
+    constexpr uint32_t ROUND = SH_WAVES * LINES * 64u;   // most that one round of lines adds
+    constexpr uint32_t UNROLL = 4;
+    __shared__ uint32_t c_rel[CAP + UNROLL * WAVE], c_pos[CAP + UNROLL * WAVE], c_val[VALUES ? CAP + UNROLL * WAVE : 1];
+    __shared__ S q_s[WAVE];
+    __shared__ uint64_t q_acc[WAVE];
+    __shared__ uint32_t q_slot[WAVE], q_p0[WAVE], q_j[WAVE], q_left[WAVE], q_room[WAVE], q_bound[WAVE];
+    __shared__ uint32_t w_tot[2][SH_WAVES], s_n, s_work;
+    if (uniform(pv.counter[1]) == 0u) return;   // nothing was left
+    const int lane = lane_id();
+    const uint32_t wv = uniform(threadIdx.x / WAVE);
+    EntryDeal deal(pv.counter + 8, (nq + span - 1u) / span, blockIdx.x, gridDim.x);
+    while (true) {
+        // the next span of the plan's queries
+        __syncthreads();   // (the span before is done with the lists)
+        if (wv == 0) {
+            const uint32_t h = deal.take(lane);
+            if (lane == 0) s_work = h;
+        }
+        __syncthreads();
+        const uint32_t h = uniform(s_work);
+        if (h == NONE) break;
+        const uint32_t k0 = h * span, kn = min(span, nq - k0);
+        if (span == chunk && uniform(pv.heavy[k0].pad) == 0u) continue;
+        for (uint32_t b0 = 0; b0 < kn; b0 += WAVE) {
+            if (b0) __syncthreads();   // (the batch before is done with the lists)
+            if (wv == 0) {
+                // up to 64 entries, in the order of their starts, with the part of the long list each needs
+                const uint32_t t = b0 + (uint32_t)lane, i = t % chunk;
+                const bool mine = t < kn && i < pv.heavy[k0 + t - i].pad;
+                const uint64_t all = __builtin_amdgcn_ballot_w64(mine);
+                const HeavyEntry* const he = pv.heavy + k0 + (mine ? t : 0u);
+                S s = SMIN;
+                uint32_t cur = 0;
+                if (mine) {
+                    s = pv.s[he->k];
+                    cur = he->cur;
+                }
+                uint32_t rank = 0;
+                for (uint64_t m = all; m; m &= m - 1ull) {
+                    const uint32_t j = (uint32_t)__builtin_ctzll(m);
+                    const S o = read_lane(s, j);
+                    rank += (o < s || (o == s && j < (uint32_t)lane)) ? 1u : 0u;
+                }
+                uint32_t p0 = 0;   // the first position starting at or after s - len
+                if (mine && (int64_t)s > (int64_t)SMIN + lv.len) {
+                    const S x = (S)((int64_t)s - lv.len - 1);
+                    if (tab.tab) {
+                        const BucketView<S> tt[1] = {tab};
+                        const S* const v[1] = {ix.starts};
+                        const S xs[1] = {x};
+                        uint32_t r[1];
+                        bucket_ranks<S, 1>(tt, v, ix.n, xs, r);
+                        p0 = r[0];
+                    } else {
+                        for (uint32_t m = ix.n; m; ) {
+                            const uint32_t half = m >> 1;
+                            if (ix.starts[p0 + half] <= x) {
+                                p0 += half + 1u;
+                                m -= half + 1u;
+                            } else {
+                                m = half;
+                            }
+                        }
+                    }
+                }
+                if (mine) {
+                    q_s[rank] = s;
+                    q_slot[rank] = k0 + t;
+                    q_p0[rank] = p0;
+                    q_j[rank] = lv.lrank[min(p0, cur + 1u)];
+                }
+                if (lane == 0) s_n = (uint32_t)__popcll(all);
+            }
+            __syncthreads();
+            const uint32_t n = uniform(s_n);
+            const bool in = (uint32_t)lane < n;
+            const uint32_t J = in ? q_j[lane] : 0u;
+            const S sl = in ? q_s[lane] : SMIN;
+            for (uint32_t g = 0, cnt = 0; g < n; g += cnt) {
+                // the next queries that share a list
+                const uint32_t Jg = read_lane(J, g);
+                const S smin = read_lane(sl, g);
+                const uint64_t fit = __builtin_amdgcn_ballot_w64(in && J - Jg + SH_SPREAD <= 2u * SH_SPREAD &&
+                                                                 (uint64_t)sl - (uint64_t)smin < 0xFFFFFFFFull);
+                const uint64_t out_of = ~(fit >> g);
+                cnt = out_of ? (uint32_t)__builtin_ctzll(out_of) : (uint32_t)WAVE;
+                const bool share = cnt >= SH_LEAST;
+                // their hits at and above s - len, from the index
+                for (uint32_t i = g; i < g + cnt; ++i) {
+                    if (i % SH_WAVES != wv) continue;
+                    const HeavyEntry he = pv.heavy[uniform(q_slot[i])];
+                    const uint32_t q = uniform(pv.q[uniform(he.k)]);
+                    const S s = read_lane(sl, i);
+                    uint32_t cur = uniform(he.cur), left = uniform(he.left);
+                    const uint32_t top = uniform(he.top);
+                    uint64_t acc = read_lane(he.acc, 0);
+                    const uint64_t oend = max(min(offsets[q + 1], cap), acc);
+                    if (!share) {
+                        wave_walk<S, MODE>(ix, td, ub, lv, lane, s, cur, top, MODE == W_VECTOR, acc, oend, left, out_idx,
+                                           vals, out_val);
+                        if (left != 0u) atomicOr(&pv.counter[3], 1u);
+                        continue;
+                    }
+                    const uint32_t p0 = uniform(q_p0[i]);
+                    uint32_t bound = 0;
+                    if (MODE == W_VECTOR) wave_lead(ix, lane, s, cur, top, acc, oend, left, out_idx);
+                    if (cur != NONE) {
+                        wave_near<S, MODE>(ix, td, lane, s, cur, p0, acc, oend, left, out_idx, vals, out_val);
+                        bound = min(p0, cur + 1u);
+                    }
+                    q_acc[i] = acc;
+                    q_left[i] = left;
+                    q_room[i] = (uint32_t)min(oend - acc, (uint64_t)1 << 28);
+                    q_bound[i] = bound;   // (every lane stores the same values)
+                }
+                if (!share) continue;
+                // ---- the long entries below the group's bounds that reach its first start, highest first
+                const uint32_t jmax = uniform(wave_max((uint32_t)lane >= g && (uint32_t)lane < g + cnt ? J : 0u));
+                bool more = jmax != 0u;
+                uint32_t g1 = 0, par = 0;
+                uint64_t rem = 0;
+                if (more) {
+                    const uint32_t hi_line = (jmax - 1u) >> 6;
+                    g1 = hi_line & ~63u;
+                    rem = lv.td.nlev >= 2 ? group_mask(lv.td, g1, smin, lane) & mask_upto(hi_line - g1) : 1ull;
+                }
+                while (more) {
+                    uint32_t C = 0;
+                    while (C + ROUND <= CAP) {
+                        if (rem == 0) {
+                            const uint32_t l = g1 ? prev_line(lv.td, g1, 0u, smin, lane) : NONE;
+                            if (l == NONE) {
+                                more = false;
+                                break;
+                            }
+                            g1 = l & ~63u;
+                            rem = group_mask(lv.td, g1, smin, lane) & mask_upto(l - g1);
+                            continue;
+                        }
+                        uint32_t e32[LINES], pos[LINES], line[LINES];
+                        S ev[LINES];
+                        // the next SH_WAVES * LINES lines, a contiguous part for each wave
+                        auto drop = [](uint64_t m, uint32_t n) {
+                            for (; n && m; --n) m &= ~(1ull << (63u - (uint32_t)__builtin_clzll(m)));
+                            return m;
+                        };
+                        uint64_t own = drop(rem, wv * LINES);
+                        rem = drop(rem, SH_WAVES * LINES);
+                        const uint32_t nl = min((uint32_t)__popcll(own), LINES);
+#pragma unroll
+                        for (uint32_t j = 0; j < LINES; ++j) {
+                            const uint32_t b = own ? 63u - (uint32_t)__builtin_clzll(own) : 0u;
+                            if (own) own &= ~(1ull << b);
+                            line[j] = g1 + b;
+                        }
+#pragma unroll
+                        for (uint32_t j = 0; j < LINES; ++j) {
+                            const uint32_t p = line[j] * 64u + 63u - (uint32_t)lane;
+                            if (sizeof(S) == 8 && lv.ends32) e32[j] = lv.ends32[p];
+                            else ev[j] = lv.ends[p];
+                            pos[j] = lv.pos[p];
+                        }
+                        uint32_t rel[LINES], tot = 0;
+                        uint64_t m[LINES];
+#pragma unroll
+                        for (uint32_t j = 0; j < LINES; ++j) {
+                            const uint32_t p = line[j] * 64u + 63u - (uint32_t)lane;
+                            const int64_t e = (sizeof(S) == 8 && lv.ends32) ? (int64_t)((uint64_t)lv.ends32_base + e32[j])
+                                                                            : (int64_t)ev[j];
+                            const bool hit = j < nl && p < jmax && e >= (int64_t)smin;
+                            rel[j] = (uint32_t)min((uint64_t)e - (uint64_t)(int64_t)smin, (uint64_t)0xFFFFFFFFu);
+                            m[j] = __builtin_amdgcn_ballot_w64(hit);
+                            tot += (uint32_t)__popcll(m[j]);
+                        }
+                        if (lane == 0) w_tot[par][wv] = tot;
+                        __syncthreads();
+                        uint32_t at = C;
+#pragma unroll
+                        for (uint32_t w = 0; w < SH_WAVES; ++w) {
+                            const uint32_t x = uniform(w_tot[par][w]);
+                            at += w < wv ? x : 0u;
+                            C += x;
+                        }
+                        par ^= 1u;
+#pragma unroll
+                        for (uint32_t j = 0; j < LINES; ++j) {
+                            if (__builtin_amdgcn_inverse_ballot_w64(m[j])) {
+                                const uint32_t slot = at + lanes_below(m[j]);
+                                c_rel[slot] = rel[j];
+                                c_pos[slot] = pos[j];
+                                if (VALUES) c_val[slot] = (uint32_t)vals[pos[j]];
+                            }
+                            at += (uint32_t)__popcll(m[j]);
+                        }
+                    }
+                    if (threadIdx.x < UNROLL * WAVE) c_pos[C + threadIdx.x] = NONE;   // (below no bound)
+                    __syncthreads();
+                    // ---- each query's hits among them
+                    for (uint32_t i = g; i < g + cnt; ++i) {
+                        if (i % SH_WAVES != wv) continue;
+                        const uint32_t from = (uint32_t)((uint64_t)read_lane(sl, i) - (uint64_t)smin), bound = uniform(q_bound[i]);
+                        const uint32_t room = uniform(q_room[i]);
+                        const uint64_t acc = read_lane(q_acc[i], 0);
+                        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                            (VALUES ? (uint32_t*)out_val : out_idx) + acc, (short)0, (int)(room * 4u), 0x00020000);
+                        uint32_t k = 0;
+                        for (uint32_t x = (uint32_t)lane; x < C + (uint32_t)lane; x += UNROLL * WAVE) {
+                            uint32_t r[UNROLL], p[UNROLL], v[UNROLL];
+#pragma unroll
+                            for (uint32_t u = 0; u < UNROLL; ++u) {
+                                r[u] = c_rel[x + u * WAVE];
+                                p[u] = c_pos[x + u * WAVE];
+                                v[u] = VALUES ? c_val[x + u * WAVE] : p[u];
+                            }
+#pragma unroll
+                            for (uint32_t u = 0; u < UNROLL; ++u) {
+                                const uint64_t m = __builtin_amdgcn_ballot_w64(r[u] >= from && p[u] < bound);
+                                const uint32_t off = (lanes_below(m) + k) << 2;
+                                __builtin_amdgcn_raw_buffer_store_b32(
+                                    v[u], rs, __builtin_amdgcn_inverse_ballot_w64(m) ? off : 0xFFFFFFFFu, 0, SI_OUT_AUX);
+                                k += (uint32_t)__popcll(m);
+                            }
+                        }
+                        q_acc[i] = acc + min(k, room);
+                        q_room[i] = room - min(k, room);
+                        q_left[i] = uniform(q_left[i]) - k;
+                    }
+                    __syncthreads();
+                }
+                for (uint32_t i = g; i < g + cnt; ++i)
+                    if (i % SH_WAVES == wv && uniform(q_left[i]) != 0u) atomicOr(&pv.counter[3], 1u);
+            }
+        }
+    }
 }

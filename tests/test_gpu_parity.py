@@ -1455,3 +1455,50 @@ def test_count_grouped(sia, orc, dtype, nq):
     c = c.cpu().numpy()
     assert np.array_equal(c[:nq], want) and np.all(c[nq:] == -7)
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n,nq,depth", [(70_000, 1, 300), (70_000, 9, 5000), (200_000, 3000, 9000),
+                                        (200_000, 40_000, 600), (100_000, 300_001, 300), (100_000, 600_001, 270)])
+def test_sweep_shared_lists(sia, orc, dtype, n, nq, depth):
+    """Queries whose start about `depth` intervals hold, most of them long: answered from candidate
+    lists that neighbouring queries share (one list, several in turn, more candidates than one
+    holds), batches that give a workgroup one query, several chunks of them, one chunk, and one
+    of more than 64; queries that share with nobody, inverted ones and ones at the ends of the
+    range; both orders, the values, and a capacity below the total."""
+    import torch
+    print(f"[gpu] sweep shared dtype={np.dtype(dtype).name} n={n} nq={nq} depth={depth}", flush=True)
+    rng = np.random.default_rng(n + nq + depth)
+    info = np.iinfo(dtype)
+    hot = 7 * n // 5   # long intervals start below this
+    s = rng.integers(0, 7 * n, n)
+    long_ = rng.random(n) < 0.3
+    s = np.where(long_, rng.integers(0, hot, n), s)
+    e = s + np.where(long_, rng.integers(1, 2 * depth * hot // (3 * n // 10), n), rng.integers(1, 6, n))
+    qs = np.where(rng.random(nq) < min(1.0, 20_000 / nq), rng.integers(0, hot, nq), rng.integers(hot, 9 * n, nq))
+    qe = qs + np.where(rng.random(nq) < 0.97, rng.integers(0, 40, nq), rng.integers(-300, 60_000, nq))
+    if nq > 3:
+        qs[:3], qe[:3] = [info.min, info.max, info.max], [info.max, info.max, info.min]
+    s, e, qs, qe = (x.astype(dtype) for x in (s, e, qs, qe))
+    vals = (np.arange(n, dtype=np.int64) * 7 % 1_000_003).astype(np.int32)
+    ix = _dev_index(sia, s, e, vals)
+    oix = orc.build_index(s, e, vals)
+    for order, mode in (("vector", 1), ("desc", 0)):
+        off, idx = ix.search(qs, qe, order=order)
+        ooff, oidx = orc.search_batch(oix, qs, qe, mode=mode)
+        assert np.array_equal(off, ooff) and np.array_equal(idx.astype(np.int64), oidx), order
+    off, v = ix.search(qs, qe, values=True)
+    assert np.array_equal(v, oix["data"][oidx])
+    tqs, tqe = torch.from_numpy(qs).cuda(), torch.from_numpy(qe).cuda()
+    plan = torch.empty(ix.plan_bytes(nq), dtype=torch.uint8, device="cuda")
+    ix.plan_device(tqs, tqe, plan)
+    toff = torch.empty(nq + 1, dtype=torch.int64, device="cuda")
+    ix.offsets_planned(plan, nq, toff)
+    total = int(ooff[-1])
+    out = torch.full((total + 64,), -7, dtype=torch.int32, device="cuda")
+    for capacity in (total - total // 3, total):
+        ix.fill_planned(plan, nq, toff, out, capacity=capacity)
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        assert np.array_equal(got[:capacity], oidx[:capacity]) and np.all(got[capacity:] == -7)
+    ix.close()
