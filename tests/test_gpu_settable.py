@@ -164,3 +164,42 @@ def test_set_table_graph_replays(sia, orc):
     table.close()
     for ix in idxs:
         ix.close()
+
+
+@pytest.mark.parametrize("nsets,nq", [(1, 1), (2, 9000), (300, 1000), (300, 9000), (1500, 70_000), (3, 600_001)])
+def test_set_table_sweep(sia, orc, nsets, nq):
+    """Sets without start > end take the sweep: a wave's queries of one set, of several and of
+    many (one query each), up to 256 in a chunk, sets of one interval to thousands, with queries
+    that hundreds of intervals hold, an empty slot among them, both orders; then, with a set
+    that holds start > end put into the table, the lane walk gives the same lists."""
+    print(f"[gpu] set table sweep nsets={nsets} nq={nq}", flush=True)
+    rng = np.random.default_rng(nsets + nq)
+    table = sia.SetTable(nsets + 2)
+    idxs, oixs = [], [None] * (nsets + 2)
+    for g in range(nsets):
+        n = int(rng.integers(1, 200)) if nsets > 10 else 4000
+        s = rng.integers(0, 50_000, n).astype(np.int32)
+        e = (s + np.where(rng.random(n) < 0.1, rng.integers(1, 20_000, n), rng.integers(0, 100, n))).astype(np.int32)
+        if nsets > 2 and g == 1:
+            continue
+        idxs.append(sia.DeviceIndex(np.int32).build(s, e))
+        table.put(g, idxs[-1])
+        oixs[g] = orc.build_index(s, e)
+    sid = rng.integers(0, nsets + 1, nq).astype(np.uint32)
+    qs = rng.integers(-100, 52_000 if nq < 100_000 else 3_000_000, nq)
+    qe = qs + rng.integers(0, 300, nq)
+    qe[5::97] = qs[5::97] - 50
+    qs, qe = qs.astype(np.int32), qe.astype(np.int32)
+    for walk in (False, True):
+        if walk:
+            bad = sia.DeviceIndex(np.int32).build(np.array([5, 9], np.int32), np.array([50, 2], np.int32))
+            idxs.append(bad)
+            table.put(nsets + 1, bad)
+        for order, mode in (("desc", 0), ("vector", 1)):
+            off, idx = table.search(sid, qs, qe, order=order)
+            woff, widx = _expect(orc, oixs, sid, qs, qe, mode)
+            assert np.array_equal(off, woff), (walk, order)
+            assert np.array_equal(idx.astype(np.int64), widx), (walk, order)
+    table.close()
+    for ix in idxs:
+        ix.close()
