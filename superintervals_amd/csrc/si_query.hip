@@ -2573,7 +2573,15 @@ SI_EXPORT int siGatherKeys(const siIndex* ix, const uint32_t* idx, size_t n, voi
 
 // Intersection pieces (superintervals.hpp:1158-1174): hit j of query k (search_idxs
 // vector order) gives [max(a_s, b_s), min(a_e, b_e)] with A's data (the default combine)
-// and B's, one thread per query.
+// and B's.  The grid's waves share the hits evenly, whatever query they belong to: a wave finds
+// the query of its first hit, then holds 64 queries at a time (a lane each, and in LDS for the hits
+// to look up) and goes through the hits PC_HITS at a time, which mark where a query's hits
+// begin; ballots of the marks number the others.  200K queries with 12 hits each on 1M int32
+// intervals: 30 us, 1.6 TB/s of hits and pieces, bound by the launch and a few dependent reads a
+// wave (one thread per query, every store to lines of its own: 421 us).  2 and 8 hits: the same.
+constexpr int PC_WAVES = Q_THREADS / WAVE;
+constexpr int PC_ITEMS = 4;                          // hits per lane and step
+constexpr uint32_t PC_HITS = PC_ITEMS * WAVE;
 template <typename S>
 __global__ __launch_bounds__(Q_THREADS) void k_intersect_pieces(IndexView<S> ix, const int32_t* __restrict__ bvals,
                                                                 const S* __restrict__ as, const S* __restrict__ ae,
@@ -2582,17 +2590,78 @@ __global__ __launch_bounds__(Q_THREADS) void k_intersect_pieces(IndexView<S> ix,
                                                                 const uint32_t* __restrict__ idx,
                                                                 S* __restrict__ os, S* __restrict__ oe,
                                                                 int32_t* __restrict__ oad, int32_t* __restrict__ obd) {
-    const size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= na) return;
-    const S s = as[k], e = ae[k];
-    const int32_t d = ad ? ad[k] : 0;
-    for (uint64_t j = off[k]; j < off[k + 1]; ++j) {
-        const uint32_t h = idx[j];
-        const S bs = ix.starts[h], be = ix.ends[h];
-        if (os) os[j] = s > bs ? s : bs;
-        if (oe) oe[j] = e < be ? e : be;
-        if (oad) oad[j] = d;
-        if (obd) obd[j] = bvals ? bvals[h] : 0;
+    __shared__ S l_s[PC_WAVES][WAVE], l_e[PC_WAVES][WAVE];
+    __shared__ int32_t l_d[PC_WAVES][WAVE];
+    __shared__ uint8_t l_lane[PC_WAVES][WAVE];       // the lanes of queries with hits, in order
+    __shared__ uint32_t l_mark[PC_WAVES][WAVE];      // a byte per hit: a query's first
+    const int lane = lane_id();
+    const uint32_t wv = uniform(threadIdx.x / WAVE);
+    uint8_t* const mark = reinterpret_cast<uint8_t*>(l_mark[wv]);
+    const uint64_t first = off[0], total = off[na] - first;
+    const uint64_t waves = (uint64_t)gridDim.x * PC_WAVES, w = (uint64_t)blockIdx.x * PC_WAVES + wv;
+    const uint64_t per = ((total + waves - 1u) / waves + PC_HITS - 1u) / PC_HITS * PC_HITS;
+    if (w * per >= total) return;
+    uint64_t j = first + w * per;
+    const uint64_t stop = first + min(w * per + per, total);
+    // the last query with off <= j, 64 samples a step
+    size_t k0 = 0;
+    for (size_t n = na; n > 1;) {
+        const size_t step = (n + WAVE - 1) / WAVE, i = (size_t)lane * step;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(i < n && off[k0 + i] <= j);   // (a prefix of the lanes, not empty)
+        const size_t at = (size_t)(63 - __builtin_clzll(m)) * step;
+        k0 += at;
+        n = min(step, n - at);
+    }
+    while (j < stop) {
+        // queries k0 .. k0 + 63
+        const size_t k = min(k0 + (size_t)lane, na);
+        const uint64_t o0 = off[k], o1 = off[min(k + 1, na)];
+        const uint64_t end = off[min(k0 + (size_t)WAVE, na)], to = min(end, stop);
+        const uint64_t some = __builtin_amdgcn_ballot_w64(o1 > o0);
+        wave_lds_sync();
+        if (k < na) {
+            l_s[wv][lane] = as[k];
+            l_e[wv][lane] = ae[k];
+            l_d[wv][lane] = ad ? ad[k] : 0;
+        }
+        if (o1 > o0) l_lane[wv][lanes_below(some)] = (uint8_t)lane;
+        while (j < to) {
+            const uint32_t n = (uint32_t)min((uint64_t)PC_HITS, to - j);
+            uint32_t rank = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(o1 > o0 && o0 <= j)) - 1u;   // of j's query
+            l_mark[wv][lane] = 0u;
+            wave_lds_sync();
+            if (o1 > o0 && o0 > j && o0 - j < n) mark[(uint32_t)(o0 - j)] = 1u;
+            wave_lds_sync();
+            uint32_t h[PC_ITEMS], a[PC_ITEMS];
+#pragma unroll
+            for (int u = 0; u < PC_ITEMS; ++u) {
+                const uint32_t x = (uint32_t)(u * WAVE + lane);
+                const uint64_t m = __builtin_amdgcn_ballot_w64(mark[x] != 0);
+                a[u] = l_lane[wv][(rank + lanes_below(m) + (uint32_t)((m >> lane) & 1u)) & 63u];
+                rank += (uint32_t)__popcll(m);
+                h[u] = x < n ? idx[j + x] : 0u;
+            }
+            S bs[PC_ITEMS], be[PC_ITEMS];
+            int32_t bd[PC_ITEMS];
+#pragma unroll
+            for (int u = 0; u < PC_ITEMS; ++u) {
+                bs[u] = os ? ix.starts[h[u]] : 0;
+                be[u] = oe ? ix.ends[h[u]] : 0;
+                bd[u] = (obd && bvals) ? bvals[h[u]] : 0;
+            }
+#pragma unroll
+            for (int u = 0; u < PC_ITEMS; ++u) {
+                const uint32_t x = (uint32_t)(u * WAVE + lane);
+                if (x >= n) continue;
+                const S s = l_s[wv][a[u]], e = l_e[wv][a[u]];
+                if (os) os[j + x] = s > bs[u] ? s : bs[u];
+                if (oe) oe[j + x] = e < be[u] ? e : be[u];
+                if (oad) oad[j + x] = l_d[wv][a[u]];
+                if (obd) obd[j + x] = bd[u];
+            }
+            j += n;
+        }
+        k0 += WAVE;
     }
 }
 
@@ -2649,6 +2718,19 @@ __global__ __launch_bounds__(Q_THREADS) void k_difference_pieces(IndexView<S> ix
     if (!FILL) pieces[k] = w;
 }
 
+// Workgroups of k_intersect_pieces (the number of hits is on the device): a full chip, fewer for
+// few queries.
+static unsigned pieces_grid(size_t na) {
+    static int cus = 0;
+    if (cus == 0) {
+        int dev = 0;
+        hipGetDevice(&dev);
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+        cus = std::max(cus, 1);
+    }
+    return (unsigned)std::min<size_t>((size_t)cus * 8u, 64 + na / 4);
+}
+
 SI_EXPORT int siIntersectPieces(const siIndex* ix, const void* as, const void* ae, const int32_t* ad, size_t na,
                                 const uint64_t* offsets, const uint32_t* idx, void* out_starts, void* out_ends,
                                 int32_t* out_adata, int32_t* out_bdata, void* stream) {
@@ -2659,7 +2741,7 @@ SI_EXPORT int siIntersectPieces(const siIndex* ix, const void* as, const void* a
     if (out_bdata && !ix->d_values) return si_set_error(SI_ERR_ARG, "index was built without values");
     hipStream_t st = (hipStream_t)stream;
     return DISPATCH_S(ix, ([&]() -> int {
-        k_intersect_pieces<S><<<grid_for(na, Q_THREADS), Q_THREADS, 0, st>>>(
+        k_intersect_pieces<S><<<pieces_grid(na), Q_THREADS, 0, st>>>(
             ix->view<S>(), ix->d_values, (const S*)as, (const S*)ae, ad, na, offsets, idx, (S*)out_starts,
             (S*)out_ends, out_adata, out_bdata);
         LAUNCH_CHECK();

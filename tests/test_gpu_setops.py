@@ -255,3 +255,48 @@ def test_python_and_cpp_set_ops_golden(sia):
         # the C++ header drops empty intersection pieces on the host
         assert np.array_equal(inter, x[f"set_{sfx}_cpp_intersection"]), sfx
         assert np.array_equal(diff, x[f"set_{sfx}_cpp_difference"]), sfx
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("na", [1, 63, 64, 65, 5000, 200_003])
+def test_intersection_pieces_balanced(sia, dtype, na):
+    """siIntersectPieces shares the hits, not the queries, among its waves: queries with no hit in
+    runs longer than a wave, with one hit, and with tens of thousands; one query, and numbers
+    around 64; payloads, outputs left out, offsets that do not begin at 0."""
+    import torch
+    print(f"[gpu] intersection pieces dtype={np.dtype(dtype).name} na={na}", flush=True)
+    rng = np.random.default_rng(na)
+    n = 70_000
+    s = np.sort(rng.integers(0, 10 * n, n)).astype(dtype)
+    e = (s + rng.integers(0, 30, n)).astype(dtype)
+    vals = rng.integers(-1000, 1000, n).astype(np.int32)
+    a_s = np.where(rng.random(na) < 0.5, rng.integers(0, 10 * n, na), 20 * n)
+    a_s[na // 4: na // 2] = 20 * n
+    a_e = a_s + rng.integers(0, 40, na)
+    a_s[:: max(1, na // 5)], a_e[:: max(1, na // 5)] = 5, 9 * n
+    a_s, a_e = a_s.astype(dtype), a_e.astype(dtype)
+    ad = rng.integers(-9, 9, na).astype(np.int32)
+    ix = sia.DeviceIndex(dtype).build(s, e, vals)
+    off, idx = ix.search(a_s, a_e, order="vector")
+    k = np.repeat(np.arange(na), np.diff(off.astype(np.int64)))
+    d = ix.download(values=True)
+    hs, he, hv = d["starts"], d["ends"], d["values"]
+    want = [np.maximum(a_s[k], hs[idx]), np.minimum(a_e[k], he[idx]), ad[k], hv[idx]]
+    t = lambda x: torch.from_numpy(np.ascontiguousarray(x)).cuda()
+    ts, te, td, tidx = t(a_s), t(a_e), t(ad), t(idx.view(np.int32))
+    total = idx.size
+    for skip, k0 in ((None, 0), (0, 0), (1, 0), (3, 0), (None, na // 3)):
+        o0 = int(off[k0])
+        tdt = {4: torch.int32, 8: torch.int64}[np.dtype(dtype).itemsize]
+        outs = [torch.full((total + 8,), -77, dtype=dt, device="cuda") for dt in (tdt, tdt, torch.int32, torch.int32)]
+        ptr = [None if i == skip else o.data_ptr() for i, o in enumerate(outs)]
+        toff = t(off.view(np.int64)[k0:])
+        sia._native.check(sia._native.lib.siIntersectPieces(
+            ix.handle, ts[k0:].data_ptr(), te[k0:].data_ptr(), td[k0:].data_ptr(), na - k0, toff.data_ptr(),
+            tidx.data_ptr(), *ptr, None), "siIntersectPieces")
+        torch.cuda.synchronize()
+        for i, o in enumerate(outs):
+            got = o.cpu().numpy()
+            assert np.all(got[total:] == -77) and np.all(got[:o0] == -77)
+            assert np.array_equal(got[o0:total], want[i][o0:]) if i != skip else np.all(got == -77), (i, skip, k0)
+    ix.close()
