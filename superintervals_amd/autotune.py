@@ -89,7 +89,7 @@ def tune(ix, plan_t, nq, offsets_t, idx_t, stream=None, reps=3, tiles=CANDIDATE_
     ix is a DeviceIndex, plan_t a planned batch (plan_device), offsets_t the batch's
     offsets (offsets_planned already run) and idx_t an output buffer of offsets[nq]
     entries.  With the batch's query tensors (qs_t, qe_t) the plan's constant-digit check
-    (plan_sync: a digit histogram and one host read-back, which pay off when key digits
+    (plan_sync: one host read-back of the key bits that vary, which pays off when key digits
     are constant, as in int64 coordinates) is timed both ways too; the plan is then redone
     into plan_t.  Returns (best params, table of measured ms)."""
     import torch

@@ -157,10 +157,14 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(TO* __restrict__ ts, size_t
 // SCAN_ITEMS consecutive items; the tile passes through LDS (one pad entry per 32 items)
 // so that global loads and stores are coalesced across the wave.  A block reads and
 // writes only its own tile, all reads before any write, so in and out may alias.
-template <typename TI, typename TO>
+//
+// SELF: tile_pre holds the tiles' sums, and every block adds up those before its own (a launch and
+// 2.5 us less; one tile is scanned by this kernel alone).
+constexpr size_t SCAN_SELF_TILES = 256;
+template <typename TI, typename TO, bool SELF>
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_down(const TI* in, size_t n,
                                                             const TO* __restrict__ tile_pre,
-                                                            TO* out) {
+                                                            TO* out, TO* grand) {
     __shared__ TO s_w[4];
     __shared__ TO s_v[SCAN_TILE + SCAN_TILE / 32];
     const size_t tbase = (size_t)blockIdx.x * SCAN_TILE;
@@ -180,7 +184,16 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_down(const TI* in, size_t
         sum += v[k];
     }
     TO tot;
-    TO run = block_excl_scan256<TO>(sum, s_w, &tot) + tile_pre[blockIdx.x];
+    TO run = block_excl_scan256<TO>(sum, s_w, &tot);
+    if (SELF) {
+        const TO mine = threadIdx.x < blockIdx.x ? tile_pre[threadIdx.x] : (TO)0;   // (blockIdx.x < SCAN_SELF_TILES)
+        TO before;
+        block_excl_scan256<TO>(mine, s_w, &before);
+        run += before;
+        if (grand && threadIdx.x == 0 && blockIdx.x == gridDim.x - 1) *grand = before + tot;
+    } else {
+        run += tile_pre[blockIdx.x];
+    }
 #pragma unroll
     for (int k = 0; k < SCAN_ITEMS; ++k) {
         const uint32_t li = threadIdx.x * SCAN_ITEMS + k;
@@ -207,12 +220,19 @@ int device_excl_scan(const TI* in, size_t n, TO* out, TO* total, TO* ws, hipStre
         if (total) HIP_TRY(hipMemsetAsync(total, 0, sizeof(TO), st));
         return SI_OK;
     }
-    size_t nt = (n + SCAN_TILE - 1) / SCAN_TILE;
-    k_scan_reduce<TI, TO><<<(unsigned)nt, SCAN_THREADS, 0, st>>>(in, n, ws);
-    LAUNCH_CHECK();
+    const size_t nt = (n + SCAN_TILE - 1) / SCAN_TILE;
+    if (nt > 1) {
+        k_scan_reduce<TI, TO><<<(unsigned)nt, SCAN_THREADS, 0, st>>>(in, n, ws);
+        LAUNCH_CHECK();
+    }
+    if (nt <= SCAN_SELF_TILES) {
+        k_scan_down<TI, TO, true><<<(unsigned)nt, SCAN_THREADS, 0, st>>>(in, n, ws, out, total);
+        LAUNCH_CHECK();
+        return SI_OK;
+    }
     k_scan_tiles<TO><<<1, 1024, 0, st>>>(ws, nt, total);
     LAUNCH_CHECK();
-    k_scan_down<TI, TO><<<(unsigned)nt, SCAN_THREADS, 0, st>>>(in, n, ws, out);
+    k_scan_down<TI, TO, false><<<(unsigned)nt, SCAN_THREADS, 0, st>>>(in, n, ws, out, nullptr);
     LAUNCH_CHECK();
     return SI_OK;
 }
@@ -294,11 +314,10 @@ __device__ __forceinline__ uint32_t rs_digit(K key, int shift, uint32_t flip) {
     return ((uint32_t)(key >> shift) & 255u) ^ flip;
 }
 
-// Sorts of at most this many tiles need no scan kernels: every scatter block adds up the tiles'
-// counts itself (SELF), 256 coalesced counts a tile.  Plan of 60K queries 154 -> 99 us (three
-// launches of about 3.5 us less a pass), of 250K (123 tiles) 160 -> 127; at 245 tiles what the
-// blocks read again takes the gain away (172 -> 164).
-constexpr uint32_t RS_SELF_TILES = 128;
+// Sorts of at most this many tiles need no scan kernel: every scatter block adds up the tiles'
+// counts itself (SELF), 256 coalesced counts a tile.  int32 plans, four passes: 30K queries (15 tiles)
+// 53 us, with the scan kernel 62; 100K 62.6 and 64.1; 150K (73 tiles) 69 and 66; 250K 82 and 70.
+constexpr uint32_t RS_SELF_TILES = 56;
 
 // Per-tile digit counts, digit-major (th[d * ntiles + tile], for the scan), or tile-major (SELF:
 // th[tile * 256 + d]).  A digit equal across a wave is added once, from one lane.
@@ -401,14 +420,14 @@ enum RsVals { RS_NONE = 0, RS_ARRAY = 1, RS_INDEX = 2 };
 template <class Out, typename K, RsVals VALS, bool SELF>
 __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
     const K* __restrict__ kin, const uint32_t* __restrict__ vin, Out out, size_t n, int shift, uint32_t flip,
-    const uint32_t* __restrict__ th_base, uint32_t ntiles) {
+    const uint32_t* __restrict__ th_base, const uint32_t* __restrict__ totals, uint32_t ntiles) {
     __shared__ union {
         uint16_t c[RS_ROUNDS * 4][RS_BINS];
         K key[RS_TILE];
     } s_u;
     __shared__ uint32_t s_val[VALS ? RS_TILE : 1];
     __shared__ uint32_t s_dstart[RS_BINS];
-    __shared__ uint32_t s_gbase[SELF ? RS_BINS : 1];   // the tile's first output slot of each digit
+    __shared__ uint32_t s_gbase[RS_BINS];   // the tile's first output slot of each digit
     __shared__ uint32_t s_w[4];
 
     const int tid = threadIdx.x;
@@ -437,6 +456,8 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
             }
         }
         s_gbase[tid] = block_excl_scan256<uint32_t>(all, s_w, &tot) + before;
+    } else {
+        s_gbase[tid] = block_excl_scan256<uint32_t>(totals[tid], s_w, &tot) + th_base[(size_t)tid * ntiles + tile];
     }
     const uint32_t cnt = rs_rank_tile(key, tile_n, shift, flip, s_u.c, off);
     s_dstart[tid] = block_excl_scan256<uint32_t>(cnt, s_w, &tot);   // its barriers free s_u.c
@@ -456,19 +477,56 @@ __global__ __launch_bounds__(RS_THREADS) void k_rs_scatter(
         if (slot < tile_n) {
             const K k = s_u.key[slot];
             const uint32_t digit = rs_digit(k, shift, flip);
-            const size_t dst = (size_t)(SELF ? s_gbase[digit] : th_base[(size_t)digit * ntiles + tile]) +
-                               (slot - s_dstart[digit]);
+            const size_t dst = (size_t)s_gbase[digit] + (slot - s_dstart[digit]);
             out.put(dst, k, VALS ? s_val[slot] : 0u);
         }
     }
 }
 
+// Exclusive scan of each digit's tile counts (digit-major, a block a digit) in place, and the digits'
+// totals, which the scatter's blocks add up themselves.  (A scan over all the counts in three kernels:
+// two launches and 35 us more for the passes of a 300K sort, 50 of 850 us for a 10M one.)
+constexpr int DS_THREADS = 1024;
+constexpr int DS_ITEMS = 4;
+__global__ __launch_bounds__(DS_THREADS) void k_rs_digit_scan(uint32_t* __restrict__ th, uint32_t ntiles,
+                                                              uint32_t* __restrict__ totals) {
+    __shared__ uint32_t s_w[2][DS_THREADS / WAVE];
+    uint32_t* const row = th + (size_t)blockIdx.x * ntiles;
+    const uint32_t lane = (uint32_t)lane_id(), w = threadIdx.x >> 6;
+    uint32_t carry = 0, par = 0;
+    for (uint32_t base = 0; base < ntiles; base += DS_THREADS * DS_ITEMS, par ^= 1u) {
+        uint32_t c[DS_ITEMS], sum = 0;
+#pragma unroll
+        for (int k = 0; k < DS_ITEMS; ++k) {
+            const uint32_t i = base + threadIdx.x * DS_ITEMS + k;
+            c[k] = i < ntiles ? row[i] : 0u;
+            sum += c[k];
+        }
+        const uint32_t inc = wave_incl_scan(sum);
+        if (lane == WAVE - 1) s_w[par][w] = inc;
+        __syncthreads();
+        uint32_t run = carry + inc - sum;
+#pragma unroll
+        for (uint32_t k = 0; k < DS_THREADS / WAVE; ++k) {
+            const uint32_t x = s_w[par][k];
+            run += k < w ? x : 0u;
+            carry += x;
+        }
+#pragma unroll
+        for (int k = 0; k < DS_ITEMS; ++k) {
+            const uint32_t i = base + threadIdx.x * DS_ITEMS + k;
+            if (i < ntiles) row[i] = run;
+            run += c[k];
+        }
+    }
+    if (threadIdx.x == 0) totals[blockIdx.x] = carry;
+}
+
 // Temporary device memory of a radix sort of n items (rs_temp_bytes).
 struct RsTemp {
     uint64_t* bits;    // AND and OR of the keys, per block (rs_each_key)
-    uint32_t* th;      // per-tile digit counts, digit-major
-    uint32_t* tb;      // their exclusive scan
-    uint32_t* ws;      // scan workspace
+    uint32_t* th;      // per-tile digit counts
+    uint32_t* totals;  // of the digits
 };
 
 constexpr size_t rs_ntiles(size_t n) { return (n + RS_TILE - 1) / RS_TILE; }
@@ -477,7 +535,7 @@ constexpr size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 constexpr size_t rs_temp_bytes(size_t n) {
     const size_t nth = rs_ntiles(n) * RS_BINS;
-    return RS_BITS_BLOCKS * 16 + 2 * align256(nth * 4) + align256(scan_ws_items(nth) * 4);
+    return RS_BITS_BLOCKS * 16 + align256(nth * 4) + RS_BINS * 4;
 }
 
 inline RsTemp rs_temp_carve(void* base, size_t n) {
@@ -486,8 +544,7 @@ inline RsTemp rs_temp_carve(void* base, size_t n) {
     RsTemp t;
     t.bits = (uint64_t*)p; p += RS_BITS_BLOCKS * 16;
     t.th = (uint32_t*)p; p += align256(nth * 4);
-    t.tb = (uint32_t*)p; p += align256(nth * 4);
-    t.ws = (uint32_t*)p;
+    t.totals = (uint32_t*)p;
     return t;
 }
 
@@ -517,6 +574,151 @@ inline int rs_varying_bits(size_t n, const RsTemp& tmp, uint64_t* varying, hipSt
     return SI_OK;
 }
 
+// ---- sorts of one workgroup
+// Batches of a few thousand keys are sorted by one workgroup in LDS, with the digits to sort by
+// found on the way: the passes of the kernels above are two launches each, and a read-back of the
+// varying bits stands before them.  A wave holds ITEMS consecutive lines of 64 items in registers;
+// a pass ranks them by ballots, a line at a time, against its own counts of each digit, a column
+// scan over the waves' counts and a scan over the digits make the positions, and the items move
+// through LDS.  Bound by one CU's chain of passes, four for int32 (4 us each at 4096 items): plan of 500
+// int32 queries 12 us (78 before), 4096 23 (78), 8192 36 (82; by the passes above without a
+// read-back 49); of 16384 by this sort 67, by the passes 50.  int64: 4096 26 us, 8192 42.
+constexpr int RS1_THREADS = 1024;
+constexpr int RS1_WAVES = RS1_THREADS / WAVE;
+constexpr size_t RS1_MAX = 8 * RS1_THREADS;
+
+// in.key(i): the key of input item i (ordered as an unsigned number); out.put(position, key, i).
+template <typename K, int ITEMS, class In, class Out>
+__global__ __launch_bounds__(RS1_THREADS) void k_rs_one(In in, Out out, uint32_t n, int digit_lo, int digit_hi) {
+    __shared__ K s_key[RS1_THREADS * ITEMS];
+    __shared__ uint16_t s_item[RS1_THREADS * ITEMS];
+    __shared__ uint16_t s_h[RS1_WAVES][RS_BINS];   // a wave's items of each digit, then those of the waves before
+    __shared__ uint32_t s_base[RS_BINS];           // items of the smaller digits
+    __shared__ K s_and[RS1_WAVES], s_or[RS1_WAVES];
+    const uint32_t lane = (uint32_t)lane_id(), w = threadIdx.x >> 6, x0 = w * (WAVE * ITEMS) + lane;
+    K key[ITEMS];
+    uint32_t item[ITEMS], rank[ITEMS];
+    K all_and = (K)~(K)0, all_or = 0;
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t x = x0 + (uint32_t)r * WAVE;
+        item[r] = x;
+        key[r] = x < n ? in.key(x) : (K)0;
+        all_and &= x < n ? key[r] : (K)~(K)0;
+        all_or |= key[r];
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        all_and &= __shfl_xor(all_and, d, WAVE);
+        all_or |= __shfl_xor(all_or, d, WAVE);
+    }
+    if (lane == 0) {
+        s_and[w] = all_and;
+        s_or[w] = all_or;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < RS1_WAVES; ++k) {
+        all_and &= s_and[k];
+        all_or |= s_or[k];
+    }
+    const K varying = all_and ^ all_or;   // the same in every thread
+    for (int d = digit_lo; d < digit_hi; ++d) {
+        if (((uint32_t)(varying >> (8 * d)) & 255u) == 0u) continue;
+        // ranks within the wave
+        uint32_t* const h32 = reinterpret_cast<uint32_t*>(s_h[w]);
+        h32[lane] = 0u;
+        h32[lane + WAVE] = 0u;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const bool valid = x0 + (uint32_t)r * WAVE < n;
+            const uint32_t digit = (uint32_t)(key[r] >> (8 * d)) & 255u;
+            uint64_t peers = __builtin_amdgcn_ballot_w64(valid);
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                const uint64_t bal = __builtin_amdgcn_ballot_w64((digit >> b) & 1u);
+                peers &= ((digit >> b) & 1u) ? bal : ~bal;
+            }
+            const uint32_t below = __builtin_amdgcn_mbcnt_hi((uint32_t)(peers >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)peers, 0u));
+            const uint32_t before = s_h[w][digit];
+            rank[r] = before + below;
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+            if (valid && below == 0u) s_h[w][digit] = (uint16_t)(before + (uint32_t)__popcll(peers));
+            __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        }
+        __syncthreads();
+        if (threadIdx.x < RS_BINS) {   // over the waves, a digit a thread
+            uint32_t c[RS1_WAVES], run = 0;
+#pragma unroll
+            for (int k = 0; k < RS1_WAVES; ++k) c[k] = s_h[k][threadIdx.x];
+#pragma unroll
+            for (int k = 0; k < RS1_WAVES; ++k) {
+                s_h[k][threadIdx.x] = (uint16_t)run;
+                run += c[k];
+            }
+            s_base[threadIdx.x] = run;
+        }
+        __syncthreads();
+        if (w == 0) {   // over the digits, four a lane
+            uint32_t c[4], sum = 0;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                c[k] = s_base[4u * lane + k];
+                sum += c[k];
+            }
+            uint32_t run = sum;
+#pragma unroll
+            for (int o = 1; o < WAVE; o <<= 1) {
+                const uint32_t y = __shfl_up(run, o, WAVE);
+                run += lane >= (uint32_t)o ? y : 0u;
+            }
+            run -= sum;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                s_base[4u * lane + k] = run;
+                run += c[k];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const uint32_t digit = (uint32_t)(key[r] >> (8 * d)) & 255u;
+            const uint32_t to = s_base[digit] + s_h[w][digit] + rank[r];
+            if (x0 + (uint32_t)r * WAVE < n) {
+                s_key[to] = key[r];
+                s_item[to] = (uint16_t)item[r];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < ITEMS; ++r) {
+            const uint32_t x = x0 + (uint32_t)r * WAVE;
+            if (x < n) {
+                key[r] = s_key[x];
+                item[r] = s_item[x];
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t x = x0 + (uint32_t)r * WAVE;
+        if (x < n) out.put(x, key[r], item[r]);
+    }
+}
+
+// Stable sort of n <= RS1_MAX items by the key digits [digit_lo, digit_hi), through out.
+template <typename K, class In, class Out>
+int rs_sort_one(const In& in, const Out& out, size_t n, int digit_lo, int digit_hi, hipStream_t st) {
+    const uint32_t m = (uint32_t)n;
+    if (n <= 1 * RS1_THREADS) k_rs_one<K, 1><<<1, RS1_THREADS, 0, st>>>(in, out, m, digit_lo, digit_hi);
+    else if (n <= 2 * RS1_THREADS) k_rs_one<K, 2><<<1, RS1_THREADS, 0, st>>>(in, out, m, digit_lo, digit_hi);
+    else if (n <= 4 * RS1_THREADS) k_rs_one<K, 4><<<1, RS1_THREADS, 0, st>>>(in, out, m, digit_lo, digit_hi);
+    else k_rs_one<K, 8><<<1, RS1_THREADS, 0, st>>>(in, out, m, digit_lo, digit_hi);
+    LAUNCH_CHECK();
+    return SI_OK;
+}
+
 // True when digit d holds a bit that varies.
 inline bool rs_digit_varies(uint64_t varying, int d) { return ((varying >> (8 * d)) & 255u) != 0; }
 
@@ -528,15 +730,16 @@ int rs_pass(const K* kin, const uint32_t* vin, const Out& out, size_t n, int shi
     if (ntiles <= RS_SELF_TILES) {
         k_rs_tile_hist<K, true><<<ntiles, RS_THREADS, 0, st>>>(kin, n, shift, flip, tmp.th, ntiles);
         LAUNCH_CHECK();
-        k_rs_scatter<Out, K, VALS, true><<<ntiles, RS_THREADS, 0, st>>>(kin, vin, out, n, shift, flip, tmp.th, ntiles);
+        k_rs_scatter<Out, K, VALS, true><<<ntiles, RS_THREADS, 0, st>>>(kin, vin, out, n, shift, flip, tmp.th, tmp.totals, ntiles);
         LAUNCH_CHECK();
         return SI_OK;
     }
     k_rs_tile_hist<K, false><<<ntiles, RS_THREADS, 0, st>>>(kin, n, shift, flip, tmp.th, ntiles);
     LAUNCH_CHECK();
-    const int rc = device_excl_scan<uint32_t, uint32_t>(tmp.th, (size_t)ntiles * RS_BINS, tmp.tb, nullptr, tmp.ws, st);
-    if (rc != SI_OK) return rc;
-    k_rs_scatter<Out, K, VALS, false><<<ntiles, RS_THREADS, 0, st>>>(kin, vin, out, n, shift, flip, tmp.tb, ntiles);
+    k_rs_digit_scan<<<RS_BINS, DS_THREADS, 0, st>>>(tmp.th, ntiles, tmp.totals);
+    LAUNCH_CHECK();
+    k_rs_scatter<Out, K, VALS, false><<<ntiles, RS_THREADS, 0, st>>>(kin, vin, out, n, shift, flip, tmp.th, tmp.totals,
+                                                                    ntiles);
     LAUNCH_CHECK();
     return SI_OK;
 }

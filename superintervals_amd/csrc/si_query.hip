@@ -202,6 +202,28 @@ struct PlanOutI64 {
     }
 };
 
+// A small batch's sort: keys straight from the queries' ends, the plan's arrays written at its end.
+template <typename S>
+struct PlanInOne {
+    using K = typename std::conditional<sizeof(S) == 4, uint32_t, uint64_t>::type;
+    static constexpr K BIAS = (K)1 << (8 * sizeof(S) - 1);
+    const S* __restrict__ qe;
+    __device__ __forceinline__ K key(uint32_t i) const { return (K)qe[i] ^ BIAS; }
+};
+template <typename S>
+struct PlanOutOne {
+    using K = typename PlanInOne<S>::K;
+    uint32_t* __restrict__ q;
+    S* __restrict__ s;
+    S* __restrict__ e;
+    const S* __restrict__ qs;
+    __device__ __forceinline__ void put(uint32_t dst, K key, uint32_t item) const {
+        q[dst] = item;
+        e[dst] = (S)(key ^ PlanInOne<S>::BIAS);
+        s[dst] = qs[item];
+    }
+};
+
 // The plan's flags, when its last sort pass wrote the arrays (k_plan_finish sets them otherwise).
 template <typename S>
 __global__ void k_plan_counters(PlanView<S> pv, bool with_lb, bool with_rank) {
@@ -327,8 +349,8 @@ __global__ __launch_bounds__(Q_THREADS) void k_count_rank(IndexView<S> ix, const
 //                wave-cooperative kernel
 //   ub_tree      1: siUpperBound descends a 64-ary tree of first keys (its top level in
 //                Eytzinger order in LDS); 0: plain halving over all starts
-//   plan_sync    1: the plan's radix sort reads back which key bits vary to skip constant
-//                digits (one stream synchronisation); 0: it sorts every key digit without
+//   plan_sync    1: the plan's radix sort of a large batch reads back which key bits vary to skip
+//                constant digits (one stream synchronisation); 0: it sorts every key digit without
 //                a host read-back, so plan -> offsets -> fill can be captured in a graph
 //   heavy_ends32 1: the wave-cooperative walk of an int64 index reads the 32-bit copy of
 //                the ends when the build made one (ends spanning < 2^32); 0: the ends
@@ -378,6 +400,11 @@ LongView<S> long_view_of(const siIndex* ix) {
 // start <= end (each starts at or after s, so ends at or after s).
 inline bool range_skip_on(const siIndex* ix) { return g_tune.range_skip && ix->n_inverted == 0; }
 
+// The read-back of the varying bits costs a plan about 40 us.  Of int64 ends it saves four passes of
+// eight as a rule; of int32 ends none, or one where they span less than 2^24: from this batch size
+// on a pass costs more than the read-back (23 us at 2M queries, 37 at 4M, 90 at 10M).
+constexpr size_t PLAN32_READ_BACK = 4000000;
+
 template <typename S>
 int plan_impl(const siIndex* ix, const S* qs, const S* qe, size_t nq, void* plan, hipStream_t st, bool read_back) {
     PlanLayout L(sizeof(S), nq);
@@ -403,11 +430,18 @@ int plan_impl(const siIndex* ix, const S* qs, const S* qe, size_t nq, void* plan
     int rc;
     uint64_t varying = ~0ull;   // key bits that vary, as far as is known
     bool unpacked = false;   // the sort's last pass wrote q, s, e (when the bounds come from a search below)
-    if (sizeof(S) == 4) {
+    using K = typename PlanInOne<S>::K;
+    if (nq <= RS1_MAX && (tree || learned)) {
+        ks = nullptr;
+        vs = nullptr;
+        unpacked = true;
+        rc = rs_sort_one<K>(PlanInOne<S>{qe}, PlanOutOne<S>{pv.q, pv.s, pv.e, qs}, nq,
+                            std::min<int>(g_tune.plan_skip_low, sizeof(S)), sizeof(S), st);
+    } else if (sizeof(S) == 4) {
         k_plan_keys_i32<<<rs_bits_grid(nq), RS_THREADS, 0, st>>>((const int32_t*)qs, (const int32_t*)qe, nq, k0, v0,
                                                                  rt.bits);
         LAUNCH_CHECK();
-        if (read_back && nq > 1 && (rc = rs_varying_bits(nq, rt, &varying, st)) != SI_OK) return rc;
+        if (read_back && nq >= PLAN32_READ_BACK && (rc = rs_varying_bits(nq, rt, &varying, st)) != SI_OK) return rc;
         const PlanOutI32 out{pv.q, (int32_t*)pv.s, (int32_t*)pv.e};
         rc = radix_sort_pairs(k0, v0, k1, v1, nq, 4 + g_tune.plan_skip_low, 8, rt, &ks, &vs, st, varying,
                               (tree || learned) ? &out : nullptr, &unpacked);
@@ -1645,6 +1679,58 @@ __global__ __launch_bounds__(Q_THREADS) void k_count_rank_tree(IndexView<S> ix, 
     }
 }
 
+// Offsets (and counts) of a batch of up to RS1_MAX planned queries by one workgroup: the counts go to
+// their queries' places in LDS and are added up there: 4096 queries 5.2 us, as a scatter and a scan of
+// their own, four launches, 14.6; 8192 7.8 and 14.8.
+template <typename S>
+__global__ __launch_bounds__(RS1_THREADS) void k_offsets_one(IndexView<S> ix, UbTree<S> t, const S* __restrict__ top,
+                                                             uint32_t h, PlanView<S> pv, uint32_t nq,
+                                                             uint32_t* __restrict__ counts,
+                                                             uint64_t* __restrict__ offsets) {
+    constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
+    constexpr uint32_t ITEMS = RS1_MAX / RS1_THREADS;
+    __shared__ __align__(16) uint32_t s_c[RS1_MAX];
+    __shared__ uint64_t s_w[RS1_WAVES];
+    const bool planned = __builtin_amdgcn_readfirstlane(pv.counter[5]) != 0u;   // the plan holds the counts
+    for (uint32_t k = threadIdx.x; k < nq; k += RS1_THREADS) {
+        uint32_t c = 0;
+        if (planned) {
+            c = pv.cnt[k];
+        } else {
+            const uint32_t i = pv.idx[k];
+            const S s = pv.s[k], e = pv.e[k];
+            if (i != NONE) {
+                if (s <= e) c = i + 1u - ((s == SMIN) ? 0u : ub_tree_pos(t, top, h, (S)(s - 1)) + 1u);
+                else c = walk_count(ix, i, s);
+            }
+        }
+        s_c[pv.q[k]] = c;
+    }
+    __syncthreads();
+    const uint32_t q0 = threadIdx.x * ITEMS, w = threadIdx.x / WAVE;
+    uint32_t c[ITEMS];
+    uint64_t sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < ITEMS; ++k) {
+        c[k] = q0 + k < nq ? s_c[q0 + k] : 0u;
+        sum += c[k];
+    }
+    const uint64_t inc = wave_incl_scan(sum);
+    if (lane_id() == WAVE - 1) s_w[w] = inc;
+    __syncthreads();
+    uint64_t run = inc - sum;
+    for (uint32_t k = 0; k < w; ++k) run += s_w[k];
+#pragma unroll
+    for (uint32_t k = 0; k < ITEMS; ++k) {
+        if (q0 + k < nq) {
+            offsets[q0 + k] = run;
+            if (counts) counts[q0 + k] = c[k];
+        }
+        run += c[k];
+        if (q0 + k + 1u == nq) offsets[nq] = run;
+    }
+}
+
 template <typename S>
 UbTree<S> ub_tree_of(const KeyTree& kt, const S* keys, size_t n) {
     UbTree<S> t;
@@ -2373,6 +2459,14 @@ SI_EXPORT int siSearchOffsetsPlanned(const siIndex* ix, void* plan, size_t nq, u
     const PlanLayout L(ix->cb, nq);
     uint64_t* ws = (uint64_t*)((char*)plan + L.off_scratch);
     if (g_tune.offsets_rank && rank_exact(ix)) {
+        if (nq > 0 && nq <= RS1_MAX && g_tune.ub_tree && ix->eb.d_top && ix->n > 0)
+            return DISPATCH_S(ix, ([&]() -> int {
+                k_offsets_one<S><<<1, RS1_THREADS, 0, st>>>(
+                    ix->view<S>(), ub_tree_of<S>(ix->eb, (const S*)ix->d_ends_sorted, ix->n), (const S*)ix->eb.d_top,
+                    ix->eb.top_h, plan_view<S>(plan, nq), (uint32_t)nq, counts, offsets);
+                LAUNCH_CHECK();
+                return SI_OK;
+            }()));
         // 32-bit counts (the caller's, or the heavy-list area of the plan, which the rank
         // form does not use), then one scan to 64-bit offsets: half the scattered bytes
         uint32_t* c32 = counts ? counts : (uint32_t*)((char*)plan + L.off_heavy);

@@ -1502,3 +1502,58 @@ def test_sweep_shared_lists(sia, orc, dtype, n, nq, depth):
         got = out.cpu().numpy()
         assert np.array_equal(got[:capacity], oidx[:capacity]) and np.all(got[capacity:] == -7)
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("nq", [1, 63, 1023, 1024, 1025, 2049, 4097, 8191, 8192, 8193, 114_687, 114_689])
+def test_small_batches(sia, orc, dtype, nq):
+    """Batches sorted by one workgroup, with one to eight items a thread, and the next larger forms:
+    the plan is numpy's stable argsort of the ends (over the whole range, with one digit that
+    varies, few distinct, all equal, and with low digits left unsorted); offsets, counts and
+    lists equal the oracle's, with the counts from the plan and, planned by the learned model or
+    on an index of one interval, found by the offsets pass."""
+    import torch
+    from superintervals_amd import autotune
+    print(f"[gpu] small batches dtype={np.dtype(dtype).name} nq={nq}", flush=True)
+    rng = np.random.default_rng(nq)
+    info = np.iinfo(dtype)
+    n = 30_000
+    s = rng.integers(0, 400_000, n).astype(dtype)
+    e = (s + rng.integers(0, 500, n)).astype(dtype)
+    ix, one = _dev_index(sia, s, e), _dev_index(sia, s[:1], e[:1])
+    model = sia.LearnedIndex(ix, 64)
+    model.train(steps=20, batch=4096, lr=3e-3)
+    oix, oone = orc.build_index(s, e), orc.build_index(s[:1], e[:1])
+    some = rng.integers(-100, 500_000, nq)
+    saved = autotune.current()
+    try:
+        for qe in (rng.integers(info.min, info.max, nq), 300_007 + 256 * rng.integers(0, 256, nq), rng.choice([-1, 0, 300], nq),
+                   np.full(nq, 70_000), some):
+            qe = qe.astype(dtype)
+            qs = (qe - np.minimum(rng.integers(-20, 3000, nq), qe.astype(object) - int(info.min))).astype(dtype)
+            tqs, tqe = torch.from_numpy(qs).cuda(), torch.from_numpy(qe).cuda()
+            for index, o, knobs in ((ix, oix, {}), (ix, oix, {"ub_learned": 1}), (one, oone, {}),
+                                    (ix, oix, {"plan_skip_low": 2, "plan_sync": 0})):
+                autotune.apply(dict(saved, **knobs))
+                plan = torch.full((index.plan_bytes(nq),), 0xA5, dtype=torch.uint8, device="cuda")
+                index.plan_device(tqs, tqe, plan)
+                off = torch.full((nq + 9,), -7, dtype=torch.int64, device="cuda")
+                cnt = torch.full((nq + 8,), -7, dtype=torch.int32, device="cuda")
+                index.offsets_planned(plan, nq, off, cnt)
+                torch.cuda.synchronize()
+                q = plan[256:256 + 4 * nq].view(torch.int32).cpu().numpy()
+                low = 0xFFFF if "plan_skip_low" in knobs else 0
+                assert np.array_equal(q, np.argsort(qe.astype(np.int64) & ~low, kind="stable")), knobs
+                want = orc.count_batch(o, qs, qe)
+                off, cnt = off.cpu().numpy(), cnt.cpu().numpy()
+                assert np.array_equal(cnt[:nq], want) and np.all(cnt[nq:] == -7)
+                assert np.array_equal(off[:nq + 1], np.concatenate([[0], np.cumsum(want)])) and np.all(off[nq + 1:] == -7)
+            autotune.apply(saved)
+        woff, widx = orc.search_batch(oix, qs, qe, mode=0)
+        off, idx = ix.search(qs, qe)
+        assert np.array_equal(off, woff) and np.array_equal(idx.astype(np.int64), widx)
+    finally:
+        autotune.apply(saved)
+    model.close()
+    ix.close()
+    one.close()
