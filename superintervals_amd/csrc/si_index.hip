@@ -19,6 +19,7 @@
 #include <chrono>
 #include <cstring>
 #include <mutex>
+#include <new>
 #include <type_traits>
 #include <vector>
 
@@ -54,6 +55,7 @@ struct Kept {
     std::vector<KeptBlock> blocks;   // oldest first
     size_t bytes = 0;
     int users = 0;
+    HostStage* stages[STAGE_KEEP] = {};
 };
 // (never destroyed: an index may outlive the library's own static objects)
 Kept& kept() {
@@ -140,11 +142,69 @@ bool si_device_quiet(int device) {
     return e == hipSuccess;
 }
 
+namespace {
+void drop_stage(HostStage* s) {
+    for (hipEvent_t e : s->ev)
+        if (e) (void)hipEventDestroy(e);
+    if (s->p) (void)hipHostFree(s->p);
+    delete s;
+}
+}  // namespace
+
 void si_block_users(int change) {
     Kept& k = kept();
     std::lock_guard<std::mutex> lock(k.mu);
     k.users += change;
-    if (k.users == 0) drop_kept(k, -1);
+    if (k.users == 0) {
+        drop_kept(k, -1);
+        for (HostStage*& s : k.stages) {
+            if (s) drop_stage(s);
+            s = nullptr;
+        }
+    }
+}
+
+HostStage* si_stage_take() {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    Kept& k = kept();
+    {
+        std::lock_guard<std::mutex> lock(k.mu);
+        for (HostStage*& s : k.stages) {
+            if (s && s->device == dev) {   // (its events are the device's)
+                HostStage* const got = s;
+                s = nullptr;
+                return got;
+            }
+        }
+    }
+    HostStage* const s = new (std::nothrow) HostStage;
+    if (!s) return nullptr;
+    s->device = dev;
+    bool ok = hipHostMalloc((void**)&s->p, STAGE_SLOTS * STAGE_CHUNK + 256, hipHostMallocDefault) == hipSuccess;
+    for (hipEvent_t& e : s->ev) ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        drop_stage(s);
+        return nullptr;
+    }
+    return s;
+}
+
+void si_stage_give(HostStage* s) {
+    Kept& k = kept();
+    {
+        std::lock_guard<std::mutex> lock(k.mu);
+        if (k.users > 0) {
+            for (HostStage*& slot : k.stages) {
+                if (!slot) {
+                    slot = s;
+                    return;
+                }
+            }
+        }
+    }
+    drop_stage(s);
 }
 
 SI_EXPORT const char* siGetLastError(void) { return g_err; }

@@ -64,6 +64,23 @@ struct BucketTable {
     BucketView<S> view() const { return BucketView<S>{ok ? d_tab : nullptr, (S)lo, (S)hi, shift}; }
 };
 
+// Pinned host memory that the host-buffer calls copy through, STAGE_SLOTS chunks in turn with an
+// event each.  4.9 MB of results (100K queries on 1M intervals) came to pageable memory in 265 us,
+// now in about 170, bound by one core's copy out of the chunks (with streaming stores; 200 without).
+// The whole call 700 us -> 415, for 195 MB of results 14.4 ms -> 6.9.  Chunks of 1 and 4 MB: within
+// 10 %.  Taken by a call and given back, at most STAGE_KEEP kept until the last index is destroyed.
+constexpr size_t STAGE_CHUNK = (size_t)2 << 20;
+constexpr int STAGE_SLOTS = 4;
+constexpr size_t STAGE_KEEP = 4;
+struct HostStage {
+    char* p = nullptr;                       // STAGE_SLOTS chunks, then 256 bytes for a flag
+    hipEvent_t ev[STAGE_SLOTS] = {};
+    bool busy[STAGE_SLOTS] = {};             // the slot's event is recorded and not waited for
+    int device = 0;
+};
+HostStage* si_stage_take();                  // null: none to be had
+void si_stage_give(HostStage* s);            // (no copy through it is under way)
+
 // Scratch of the single-query calls (the host-buffer forms with one query): a pinned host
 // buffer mapped into the device, which the one-wave kernel writes directly (header + up to
 // cap results), and a stream.  Made on the first such call, kept until the index is

@@ -2494,6 +2494,10 @@ SI_EXPORT int siSearchFillPlannedBounded(const siIndex* ix, void* plan, size_t n
                                                     capacity)));
 }
 
+static int plan_mismatch() {
+    return si_set_error(SI_ERR_MISMATCH, "a fill pass found a different number of hits than its offsets give");
+}
+
 SI_EXPORT int siPlanCheck(const siIndex* ix, const void* plan, void* stream) {
     int rc = check_ix(ix);
     if (rc) return rc;
@@ -2502,8 +2506,7 @@ SI_EXPORT int siPlanCheck(const siIndex* ix, const void* plan, void* stream) {
     uint32_t flag = 0;
     HIP_TRY(hipMemcpyAsync(&flag, (const uint32_t*)plan + 3, sizeof(flag), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    if (flag) return si_set_error(SI_ERR_MISMATCH, "a fill pass found a different number of hits than its offsets give");
-    return SI_OK;
+    return flag ? plan_mismatch() : SI_OK;
 }
 
 SI_EXPORT int siSearchFillPlanned(const siIndex* ix, void* plan, size_t nq, int order,
@@ -3347,14 +3350,136 @@ SI_EXPORT int siSearchNoAlloc(const siIndex* ix, const void* qs, const void* qe,
 // Host-buffer forms
 // ============================================================================
 namespace {
+// Copies results out of the stage with streaming stores (the destination is not read first).
+void copy_results(void* dst, const void* src, size_t n) {
+    typedef float f4 __attribute__((vector_size(16)));
+    char* d = (char*)dst;
+    const char* s = (const char*)src;
+    const size_t head = std::min(n, (size_t)((0 - (uintptr_t)d) & 63u));
+    std::memcpy(d, s, head);
+    d += head;
+    s += head;
+    n -= head;
+    for (; n >= 64; n -= 64, d += 64, s += 64) {
+        f4 v[4];
+        std::memcpy(v, s, 64);
+        for (int k = 0; k < 4; ++k) __builtin_nontemporal_store(v[k], (f4*)d + k);
+    }
+    __builtin_ia32_sfence();   // other threads may read them after any store of this one
+    std::memcpy(d, s, n);
+}
+
+// The memory of one host-buffer call on the null stream: device blocks from the kept ones and a
+// pinned stage that its copies go through (plain copies when there is none).  `out` waits for
+// all that the call has put on the stream before it.
+struct HostCall {
+    static constexpr int BLOCKS = 12;
+    void* blocks[BLOCKS] = {};
+    size_t bytes[BLOCKS] = {};
+    int n = 0, device = 0;
+    HostStage* stage = nullptr;
+
+    HostCall() {
+        (void)hipGetDevice(&device);
+        stage = si_stage_take();
+    }
+    HostCall(const HostCall&) = delete;
+    HostCall& operator=(const HostCall&) = delete;
+    ~HostCall() {
+        const bool quiet = hipStreamSynchronize(nullptr) == hipSuccess;   // (3 us when it is idle)
+        for (int i = 0; i < n; ++i) si_block_give(blocks[i], bytes[i], device, quiet);
+        if (!stage) return;
+        for (bool& b : stage->busy) b = false;
+        si_stage_give(stage);
+    }
+    void* alloc(size_t want) {
+        if (n == BLOCKS) return nullptr;
+        void* const p = si_block_take(want, &bytes[n]);
+        if (p) blocks[n++] = p;
+        return p;
+    }
+    int slot_free(int s) {
+        if (stage->busy[s]) HIP_TRY(hipEventSynchronize(stage->ev[s]));
+        stage->busy[s] = false;
+        return SI_OK;
+    }
+    int slot_mark(int s) {
+        HIP_TRY(hipEventRecord(stage->ev[s], nullptr));
+        stage->busy[s] = true;
+        return SI_OK;
+    }
+    // host -> device; h may be reused at once
+    int in(void* d, const void* h, size_t len) {
+        if (!stage) {
+            HIP_TRY(hipMemcpy(d, h, len, hipMemcpyHostToDevice));
+            return SI_OK;
+        }
+        for (size_t at = 0; at < len; at += STAGE_CHUNK) {
+            const int s = next++ % STAGE_SLOTS;
+            const size_t m = std::min(STAGE_CHUNK, len - at);
+            char* const c = stage->p + (size_t)s * STAGE_CHUNK;
+            int rc = slot_free(s);
+            if (rc) return rc;
+            std::memcpy(c, (const char*)h + at, m);
+            HIP_TRY(hipMemcpyAsync((char*)d + at, c, m, hipMemcpyHostToDevice, nullptr));
+            if ((rc = slot_mark(s))) return rc;
+        }
+        return SI_OK;
+    }
+    // up to a chunk of device memory, in the stage on return (until the slot is used again)
+    int peek(const void* d, size_t len, const void** h) {
+        const int s = next++ % STAGE_SLOTS;
+        char* const c = stage->p + (size_t)s * STAGE_CHUNK;
+        int rc = slot_free(s);
+        if (rc) return rc;
+        HIP_TRY(hipMemcpyAsync(c, d, len, hipMemcpyDeviceToHost, nullptr));
+        HIP_TRY(hipStreamSynchronize(nullptr));
+        *h = c;
+        return SI_OK;
+    }
+    // device -> host, complete on return; plan: a plan whose fill pass is checked first
+    int out(void* h, const void* d, size_t len, const void* plan = nullptr) {
+        if (!stage) {
+            uint32_t flag = 0;
+            if (plan) HIP_TRY(hipMemcpy(&flag, (const uint32_t*)plan + 3, 4, hipMemcpyDeviceToHost));
+            if (flag) return plan_mismatch();
+            HIP_TRY(hipMemcpy(h, d, len, hipMemcpyDeviceToHost));
+            return SI_OK;
+        }
+        uint32_t* const flag = (uint32_t*)(stage->p + STAGE_SLOTS * STAGE_CHUNK);
+        if (plan) HIP_TRY(hipMemcpyAsync(flag, (const uint32_t*)plan + 3, 4, hipMemcpyDeviceToHost, nullptr));
+        const size_t chunks = (len + STAGE_CHUNK - 1) / STAGE_CHUNK;
+        const unsigned first = next;
+        next += (unsigned)chunks;
+        for (size_t i = 0; i < chunks + STAGE_SLOTS - 1; ++i) {
+            if (i < chunks) {   // ask for chunk i
+                const int s = (int)((first + i) % STAGE_SLOTS);
+                int rc = slot_free(s);
+                if (rc) return rc;
+                HIP_TRY(hipMemcpyAsync(stage->p + (size_t)s * STAGE_CHUNK, (const char*)d + i * STAGE_CHUNK,
+                                       std::min(STAGE_CHUNK, len - i * STAGE_CHUNK), hipMemcpyDeviceToHost, nullptr));
+                if ((rc = slot_mark(s))) return rc;
+            }
+            if (i + 1 >= STAGE_SLOTS) {   // take the chunk asked for STAGE_SLOTS - 1 turns before
+                const size_t k = i + 1 - STAGE_SLOTS;
+                const int s = (int)((first + k) % STAGE_SLOTS), rc = slot_free(s);
+                if (rc) return rc;
+                if (plan && *(volatile uint32_t*)flag) return plan_mismatch();
+                copy_results((char*)h + k * STAGE_CHUNK, stage->p + (size_t)s * STAGE_CHUNK,
+                            std::min(STAGE_CHUNK, len - k * STAGE_CHUNK));
+            }
+        }
+        return SI_OK;
+    }
+    unsigned next = 0;   // the slot of the next chunk
+};
+
+// A device buffer of a host-buffer call.
 struct DevBuf {
     void* p = nullptr;
-    ~DevBuf() { if (p) (void)hipFree(p); }
-    int alloc(size_t bytes) {
-        if (bytes == 0) bytes = 8;
-        hipError_t e = hipMalloc(&p, bytes);
-        if (e != hipSuccess) { p = nullptr; return si_set_error(SI_ERR_NOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e)); }
-        return SI_OK;
+    int alloc(HostCall& call, size_t bytes) {
+        p = call.alloc(bytes);
+        return p ? SI_OK : si_set_error(SI_ERR_NOMEM, "%zu bytes of device memory", bytes);
     }
 };
 
@@ -3413,13 +3538,12 @@ int one_query(const siIndex* cix, int mode, const void* qs, const void* qe, uint
     return one_query_run<int64_t>(ix, mode, qs ? *(const int64_t*)qs : 0, *(const int64_t*)qe, total);
 }
 
-int upload_queries(const siIndex* ix, const void* qs, const void* qe, size_t nq, DevBuf& dq) {
+int upload_queries(HostCall& call, const siIndex* ix, const void* qs, const void* qe, size_t nq, DevBuf& dq) {
     const size_t qb = nq * ix->cb;
-    int rc = dq.alloc(2 * qb);
-    if (rc) return rc;
-    HIP_TRY(hipMemcpy(dq.p, qs, qb, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy((char*)dq.p + qb, qe, qb, hipMemcpyHostToDevice));
-    return SI_OK;
+    int rc = dq.alloc(call, 2 * qb);
+    if (rc == SI_OK) rc = call.in(dq.p, qs, qb);
+    if (rc == SI_OK) rc = call.in((char*)dq.p + qb, qe, qb);
+    return rc;
 }
 }  // namespace
 
@@ -3435,11 +3559,12 @@ SI_EXPORT int siCountHost(const siIndex* ix, const void* qs, const void* qe, siz
         counts[0] = (uint32_t)c;
         return SI_OK;
     }
+    HostCall call;
     DevBuf dq, dc;
-    if ((rc = upload_queries(ix, qs, qe, nq, dq)) || (rc = dc.alloc(nq * 4))) return rc;
+    if ((rc = upload_queries(call, ix, qs, qe, nq, dq)) || (rc = dc.alloc(call, nq * 4))) return rc;
     rc = siCount(ix, dq.p, (char*)dq.p + nq * ix->cb, nq, (uint32_t*)dc.p, nullptr);
     if (rc) return rc;
-    HIP_TRY(hipMemcpy(counts, dc.p, nq * 4, hipMemcpyDeviceToHost));
+    if ((rc = call.out(counts, dc.p, nq * 4))) return rc;
     return SI_OK;
 }
 
@@ -3455,12 +3580,13 @@ SI_EXPORT int siUpperBoundHost(const siIndex* ix, const void* xs, size_t n, uint
         out[0] = (uint32_t)u;
         return SI_OK;
     }
+    HostCall call;
     DevBuf dx, dout;
-    if ((rc = dx.alloc(n * ix->cb)) || (rc = dout.alloc(n * 4))) return rc;
-    HIP_TRY(hipMemcpy(dx.p, xs, n * ix->cb, hipMemcpyHostToDevice));
+    if ((rc = dx.alloc(call, n * ix->cb)) || (rc = dout.alloc(call, n * 4))) return rc;
+    if ((rc = call.in(dx.p, xs, n * ix->cb))) return rc;
     rc = siUpperBound(ix, dx.p, n, (uint32_t*)dout.p, nullptr);
     if (rc) return rc;
-    HIP_TRY(hipMemcpy(out, dout.p, n * 4, hipMemcpyDeviceToHost));
+    if ((rc = call.out(out, dout.p, n * 4))) return rc;
     return SI_OK;
 }
 
@@ -3476,11 +3602,12 @@ SI_EXPORT int siHasOverlapsHost(const siIndex* ix, const void* qs, const void* q
         out[0] = a ? 1 : 0;
         return SI_OK;
     }
+    HostCall call;
     DevBuf dq, dout;
-    if ((rc = upload_queries(ix, qs, qe, nq, dq)) || (rc = dout.alloc(nq))) return rc;
+    if ((rc = upload_queries(call, ix, qs, qe, nq, dq)) || (rc = dout.alloc(call, nq))) return rc;
     rc = siHasOverlaps(ix, dq.p, (char*)dq.p + nq * ix->cb, nq, (uint8_t*)dout.p, nullptr);
     if (rc) return rc;
-    HIP_TRY(hipMemcpy(out, dout.p, nq, hipMemcpyDeviceToHost));
+    if ((rc = call.out(out, dout.p, nq))) return rc;
     return SI_OK;
 }
 
@@ -3490,12 +3617,13 @@ SI_EXPORT int siCoverageHost(const siIndex* ix, const void* qs, const void* qe, 
     if (rc) return rc;
     if (nq == 0) return SI_OK;
     if (!qs || !qe || !count_out || !cov_out) return si_set_error(SI_ERR_ARG, "null buffer");
+    HostCall call;
     DevBuf dq, dc, dv;
-    if ((rc = upload_queries(ix, qs, qe, nq, dq)) || (rc = dc.alloc(nq * 4)) || (rc = dv.alloc(nq * 4))) return rc;
+    if ((rc = upload_queries(call, ix, qs, qe, nq, dq)) || (rc = dc.alloc(call, nq * 4)) || (rc = dv.alloc(call, nq * 4))) return rc;
     rc = siCoverage(ix, dq.p, (char*)dq.p + nq * ix->cb, nq, (uint32_t*)dc.p, (int32_t*)dv.p, nullptr);
     if (rc) return rc;
-    HIP_TRY(hipMemcpy(count_out, dc.p, nq * 4, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(cov_out, dv.p, nq * 4, hipMemcpyDeviceToHost));
+    if ((rc = call.out(count_out, dc.p, nq * 4))) return rc;
+    if ((rc = call.out(cov_out, dv.p, nq * 4))) return rc;
     return SI_OK;
 }
 
@@ -3527,42 +3655,48 @@ SI_EXPORT int siSearchHost(const siIndex* ix, const void* qs, const void* qe, si
         }
     }
     const size_t pb = siPlanBytes(ix, nq);
+    HostCall call;
     DevBuf dq, doff, dplan;
-    if ((rc = upload_queries(ix, qs, qe, nq, dq)) || (rc = doff.alloc((nq + 1) * 8)) || (rc = dplan.alloc(pb)))
+    if ((rc = upload_queries(call, ix, qs, qe, nq, dq)) || (rc = doff.alloc(call, (nq + 1) * 8)) || (rc = dplan.alloc(call, pb)))
         return rc;
     if ((rc = siPlanQueries(ix, dq.p, (char*)dq.p + nq * ix->cb, nq, dplan.p, pb, nullptr))) return rc;
     if ((rc = siSearchOffsetsPlanned(ix, dplan.p, nq, nullptr, (uint64_t*)doff.p, nullptr))) return rc;
-    HIP_TRY(hipMemcpy(offsets, doff.p, (nq + 1) * 8, hipMemcpyDeviceToHost));
-    const uint64_t tot = offsets[nq];
-    if (total) *total = tot;
-    if (tot > cap) return si_set_error(SI_ERR_CAPACITY, "%llu results exceed capacity %zu", (unsigned long long)tot, cap);
-    if (tot == 0) return SI_OK;
-    if (!values && !idx) return si_set_error(SI_ERR_ARG, "null idx");
-    DevBuf dout;
-    if ((rc = dout.alloc(tot * 4))) return rc;
-    if (values) rc = siSearchValuesFillPlanned(ix, dplan.p, nq, (const uint64_t*)doff.p, (int32_t*)dout.p, nullptr);
-    else rc = siSearchFillPlanned(ix, dplan.p, nq, order, (const uint64_t*)doff.p, (uint32_t*)dout.p, nullptr);
+    // the caller's offsets are copied out of the stage while the fill runs
+    const size_t ob = (nq + 1) * 8;
+    const void* staged = nullptr;
+    if (call.stage && ob <= STAGE_CHUNK) rc = call.peek(doff.p, ob, &staged);
+    else rc = call.out(offsets, doff.p, ob);
     if (rc) return rc;
-    if ((rc = siPlanCheck(ix, dplan.p, nullptr))) return rc;
-    HIP_TRY(hipMemcpy(values ? (void*)values : (void*)idx, dout.p, tot * 4, hipMemcpyDeviceToHost));
-    return SI_OK;
+    const uint64_t tot = (staged ? (const uint64_t*)staged : offsets)[nq];
+    if (total) *total = tot;
+    DevBuf dout;
+    if (tot > cap) rc = si_set_error(SI_ERR_CAPACITY, "%llu results exceed capacity %zu", (unsigned long long)tot, cap);
+    else if (tot && !values && !idx) rc = si_set_error(SI_ERR_ARG, "null idx");
+    else if (tot) rc = dout.alloc(call, tot * 4);
+    if (rc == SI_OK && tot) {
+        if (values) rc = siSearchValuesFillPlanned(ix, dplan.p, nq, (const uint64_t*)doff.p, (int32_t*)dout.p, nullptr);
+        else rc = siSearchFillPlanned(ix, dplan.p, nq, order, (const uint64_t*)doff.p, (uint32_t*)dout.p, nullptr);
+    }
+    if (staged) std::memcpy(offsets, staged, ob);
+    if (rc || tot == 0) return rc;
+    return call.out(values ? (void*)values : (void*)idx, dout.p, tot * 4, dplan.p);
 }
 
 // ---- Set operations on host buffers (the C-ABI's intersection / difference) ----------
 namespace {
 // Uploads A's int32 intervals as queries and runs plan -> offsets -> descending fill on
 // the device; off receives the CSR offsets (host), didx the positions (device).
-int search_desc_host(const siIndex* ix, const int32_t* as, const int32_t* ae, size_t na, DevBuf& dq,
+int search_desc_host(HostCall& call, const siIndex* ix, const int32_t* as, const int32_t* ae, size_t na, DevBuf& dq,
                      DevBuf& dplan, DevBuf& doff, DevBuf& didx, std::vector<uint64_t>& off) {
     const size_t pb = siPlanBytes(ix, na);
     int rc;
-    if ((rc = upload_queries(ix, as, ae, na, dq)) || (rc = doff.alloc((na + 1) * 8)) || (rc = dplan.alloc(pb)))
+    if ((rc = upload_queries(call, ix, as, ae, na, dq)) || (rc = doff.alloc(call, (na + 1) * 8)) || (rc = dplan.alloc(call, pb)))
         return rc;
     if ((rc = siPlanQueries(ix, dq.p, (char*)dq.p + na * 4, na, dplan.p, pb, nullptr))) return rc;
     if ((rc = siSearchOffsetsPlanned(ix, dplan.p, na, nullptr, (uint64_t*)doff.p, nullptr))) return rc;
     off.resize(na + 1);
-    HIP_TRY(hipMemcpy(off.data(), doff.p, (na + 1) * 8, hipMemcpyDeviceToHost));
-    if ((rc = didx.alloc(off[na] * 4))) return rc;
+    if ((rc = call.out(off.data(), doff.p, (na + 1) * 8))) return rc;
+    if ((rc = didx.alloc(call, off[na] * 4))) return rc;
     if (off[na] == 0) return SI_OK;
     if ((rc = siSearchFillPlanned(ix, dplan.p, na, SI_ORDER_DESC, (const uint64_t*)doff.p, (uint32_t*)didx.p,
                                   nullptr)))
@@ -3580,18 +3714,19 @@ int si_intersect_host(const siIndex* ix, const int32_t* as, const int32_t* ae, s
     off.assign(na + 1, 0);
     pos.clear(); ps.clear(); pe.clear();
     if (na == 0) return SI_OK;
+    HostCall call;
     DevBuf dq, dplan, doff, didx, dps, dpe;
-    if ((rc = search_desc_host(ix, as, ae, na, dq, dplan, doff, didx, off))) return rc;
+    if ((rc = search_desc_host(call, ix, as, ae, na, dq, dplan, doff, didx, off))) return rc;
     const uint64_t total = off[na];
     if (total == 0) return SI_OK;
-    if ((rc = dps.alloc(total * 4)) || (rc = dpe.alloc(total * 4))) return rc;
+    if ((rc = dps.alloc(call, total * 4)) || (rc = dpe.alloc(call, total * 4))) return rc;
     if ((rc = siIntersectPieces(ix, dq.p, (char*)dq.p + na * 4, nullptr, na, (const uint64_t*)doff.p,
                                 (const uint32_t*)didx.p, dps.p, dpe.p, nullptr, nullptr, nullptr)))
         return rc;
     pos.resize(total); ps.resize(total); pe.resize(total);
-    HIP_TRY(hipMemcpy(pos.data(), didx.p, total * 4, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(ps.data(), dps.p, total * 4, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(pe.data(), dpe.p, total * 4, hipMemcpyDeviceToHost));
+    if ((rc = call.out(pos.data(), didx.p, total * 4))) return rc;
+    if ((rc = call.out(ps.data(), dps.p, total * 4))) return rc;
+    if ((rc = call.out(pe.data(), dpe.p, total * 4))) return rc;
     return SI_OK;
 }
 
@@ -3603,27 +3738,28 @@ int si_difference_host(const siIndex* ix, const int32_t* as, const int32_t* ae, 
     ps.clear(); pe.clear(); pd.clear();
     if (na == 0) return SI_OK;
     std::vector<uint64_t> off;
+    HostCall call;
     DevBuf dq, dplan, doff, didx, dpoff, dws, dad, dps, dpe, dpd;
-    if ((rc = search_desc_host(ix, as, ae, na, dq, dplan, doff, didx, off))) return rc;
+    if ((rc = search_desc_host(call, ix, as, ae, na, dq, dplan, doff, didx, off))) return rc;
     const size_t wsb = siSearchWorkspaceBytes(na);
-    if ((rc = dpoff.alloc((na + 1) * 8)) || (rc = dws.alloc(wsb)) || (rc = dad.alloc(na * 4))) return rc;
-    HIP_TRY(hipMemcpy(dad.p, ad, na * 4, hipMemcpyHostToDevice));
+    if ((rc = dpoff.alloc(call, (na + 1) * 8)) || (rc = dws.alloc(call, wsb)) || (rc = dad.alloc(call, na * 4))) return rc;
+    if ((rc = call.in(dad.p, ad, na * 4))) return rc;
     const void* dqs = dq.p;
     const void* dqe = (const char*)dq.p + na * 4;
     if ((rc = siDifferenceOffsets(ix, dqs, dqe, na, (const uint64_t*)doff.p, (const uint32_t*)didx.p,
                                   (uint64_t*)dpoff.p, dws.p, wsb, nullptr)))
         return rc;
     uint64_t np_ = 0;
-    HIP_TRY(hipMemcpy(&np_, (const uint64_t*)dpoff.p + na, 8, hipMemcpyDeviceToHost));
+    if ((rc = call.out(&np_, (const uint64_t*)dpoff.p + na, 8))) return rc;
     if (np_ == 0) return SI_OK;
-    if ((rc = dps.alloc(np_ * 4)) || (rc = dpe.alloc(np_ * 4)) || (rc = dpd.alloc(np_ * 4))) return rc;
+    if ((rc = dps.alloc(call, np_ * 4)) || (rc = dpe.alloc(call, np_ * 4)) || (rc = dpd.alloc(call, np_ * 4))) return rc;
     if ((rc = siDifferenceFill(ix, dqs, dqe, (const int32_t*)dad.p, na, (const uint64_t*)doff.p,
                                (const uint32_t*)didx.p, (const uint64_t*)dpoff.p, dps.p, dpe.p, (int32_t*)dpd.p,
                                nullptr)))
         return rc;
     ps.resize(np_); pe.resize(np_); pd.resize(np_);
-    HIP_TRY(hipMemcpy(ps.data(), dps.p, np_ * 4, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(pe.data(), dpe.p, np_ * 4, hipMemcpyDeviceToHost));
-    HIP_TRY(hipMemcpy(pd.data(), dpd.p, np_ * 4, hipMemcpyDeviceToHost));
+    if ((rc = call.out(ps.data(), dps.p, np_ * 4))) return rc;
+    if ((rc = call.out(pe.data(), dpe.p, np_ * 4))) return rc;
+    if ((rc = call.out(pd.data(), dpd.p, np_ * 4))) return rc;
     return SI_OK;
 }

@@ -1557,3 +1557,44 @@ def test_small_batches(sia, orc, dtype, nq):
     model.close()
     ix.close()
     one.close()
+
+
+@pytest.mark.parametrize("nq", [2, 1000, 524_287, 524_288, 524_289, 2_097_152, 2_097_153, 3_500_000])
+def test_host_calls_in_chunks(sia, nq):
+    """The host-buffer calls copy through pinned chunks of 2 MB, four in turn: results of one chunk,
+    exactly so, one more, more than all four, from four threads at once, into buffers at odd
+    places; a capacity that is too small leaves the offsets and the total."""
+    import ctypes
+    import threading
+    print(f"[gpu] host calls in chunks nq={nq}", flush=True)
+    ix = _dev_index(sia, np.array([0, 1000], np.int32), np.array([999, 2_000_000_000], np.int32), np.array([7, 9], np.int32))
+    lib, bad = sia._native.lib, []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        qs = rng.integers(0, 4000, nq).astype(np.int32)
+        off, total = np.zeros(nq + 1, np.uint64), ctypes.c_uint64(0)
+        want = (qs >= 1000).astype(np.uint32)
+        for cap in (nq - 1, nq):
+            buf = np.full(nq + 3, 77, np.uint32)
+            out = buf[1:]
+            rc = lib.siSearchHost(ix.handle, qs.ctypes.data, qs.ctypes.data, nq, sia.SI_ORDER_DESC, off.ctypes.data,
+                                  out.ctypes.data, None, cap, ctypes.byref(total))
+            ok = rc == (0 if cap == nq else sia._native.SI_ERR_CAPACITY) and total.value == nq
+            ok = ok and np.array_equal(off, np.arange(nq + 1)) and buf[0] == 77 and np.all(buf[nq + 1:] == 77)
+            ok = ok and (np.array_equal(out[:nq], want) if cap == nq else np.all(buf == 77))
+            if not ok:
+                bad.append((seed, cap, rc))
+        v = np.zeros(nq, np.int32)
+        rc = lib.siSearchHost(ix.handle, qs.ctypes.data, qs.ctypes.data, nq, sia.SI_ORDER_DESC, off.ctypes.data, None,
+                              v.ctypes.data, nq, ctypes.byref(total))
+        if rc or not np.array_equal(v, np.where(want, 9, 7)) or not np.array_equal(ix.count(qs, qs), np.ones(nq)):
+            bad.append((seed, "values", rc))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4 if nq < 1_000_000 else 2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    ix.close()
