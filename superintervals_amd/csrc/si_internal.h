@@ -88,7 +88,8 @@ void si_stage_give(HostStage* s);            // (no copy through it is under way
 // that sized its buffer from the first) is answered without a launch.
 struct OneQuery {
     std::mutex mu;
-    void* h = nullptr;          // pinned host memory: [0] total, [1] spare, then cap uint32 results
+    void* h = nullptr;          // pinned host memory: [0] total, [1] the last finished call's seq, then cap uint32 results
+    uint64_t seq = 0;           // calls launched
     void* d = nullptr;          // its device address
     hipStream_t st = nullptr;
     uint64_t cap = 0;
@@ -97,6 +98,7 @@ struct OneQuery {
     int64_t last_s = 0, last_e = 0;
     uint64_t last_total = 0;
     void release() {
+        if (st) (void)hipStreamSynchronize(st);   // (a call ends before its kernel does)
         if (h) (void)hipHostFree(h);
         if (st) (void)hipStreamDestroy(st);
         h = d = nullptr;

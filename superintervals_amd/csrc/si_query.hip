@@ -34,6 +34,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstring>
 #include <mutex>
 #include <string>
@@ -1463,34 +1464,57 @@ __global__ __launch_bounds__(Q_THREADS) void k_walk_heavy(IndexView<S> ix, TreeD
 // ============================================================================
 enum OneMode { ONE_UB = 4, ONE_ANY = 5 };
 
-// out (pinned host memory mapped into the device): out[0] = the count (or upper_bound /
-// has_overlaps), then up to cap results as uint32 (positions) or int32 (payload) from
-// out + 2.  The count is exact whatever cap is.
+// What one wave finds for one query: the count (or upper_bound / has_overlaps), and up to cap
+// results as uint32 (positions) or int32 (payload) from out + 2.  The count is exact whatever cap is.
 template <typename S, int MODE>
-__global__ __launch_bounds__(WAVE) void k_one_query(IndexView<S> ix, UbTree<S> ub, UbTree<S> eb, TreeDesc<S> td,
-                                                    LongView<S> lv,
-                                                    const int32_t* __restrict__ vals, uint32_t rank_exact, S s, S e,
-                                                    uint64_t* __restrict__ out, uint64_t cap) {
-    const int lane = lane_id();
-    const uint32_t idx = ix.n ? wave_tree_ub(ub, e, lane) : NONE;
-    if (MODE == ONE_UB) {
-        if (lane == 0) out[0] = idx;
-        return;
-    }
-    if (MODE == ONE_ANY) {   // superintervals.hpp:865-871: the last interval starting at or before e
-        if (lane == 0) out[0] = (idx != NONE && s <= ix.ends[idx]) ? 1u : 0u;
-        return;
-    }
-    if (idx == NONE) {
-        if (lane == 0) out[0] = 0;
-        return;
-    }
+__device__ __forceinline__ uint64_t one_query_wave(const IndexView<S>& ix, const UbTree<S>& ub, const UbTree<S>& eb,
+                                                   const BucketView<S>& ubt, const BucketView<S>& ebt,
+                                                   const S* __restrict__ ends_sorted, const TreeDesc<S>& td,
+                                                   const LongView<S>& lv, const int32_t* __restrict__ vals,
+                                                   uint32_t rank_exact, S s, S e, uint64_t* __restrict__ out,
+                                                   uint64_t cap, int lane) {
     constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
-    if (MODE == W_COUNT && rank_exact && s <= e) {   // the rank form
-        const uint32_t below = (s == SMIN) ? 0u : wave_tree_ub(eb, (S)(s - 1), lane) + 1u;
-        if (lane == 0) out[0] = idx + 1u - below;
-        return;
+    const bool s1 = s != SMIN;   // s - 1 exists
+    const S x1 = s1 ? (S)(s - 1) : s;
+    uint32_t idx = NONE, lb = 0, below = 0;   // upper_bound(e), #{starts < s}, #{ends < s}
+    if (ix.n) {
+        if (MODE == ONE_UB || MODE == ONE_ANY) {
+            if (ubt.tab) {
+                const BucketView<S> t[1] = {ubt};
+                const S* const v[1] = {ix.starts};
+                const S x[1] = {e};
+                uint32_t r[1];
+                bucket_ranks<S, 1>(t, v, ix.n, x, r);
+                idx = r[0] - 1u;
+            } else {
+                idx = wave_tree_ub(ub, e, lane);
+            }
+        } else if (ubt.tab) {   // the three searches together: two dependent reads as a rule
+            const BucketView<S> t[3] = {ubt, ubt, ebt};
+            const S* const v[3] = {ix.starts, ix.starts, ends_sorted};
+            const S x[3] = {e, x1, x1};
+            uint32_t r[3];
+            bucket_ranks<S, 3>(t, v, ix.n, x, r);
+            idx = r[0] - 1u;
+            lb = s1 ? r[1] : 0u;
+            below = s1 ? r[2] : 0u;
+        } else {
+            idx = wave_tree_ub(ub, e, lane);
+            if (rank_exact && s1) {
+                if (MODE != W_COUNT || s > e) lb = wave_tree_ub(ub, x1, lane) + 1u;
+                if (s <= e) below = wave_tree_ub(eb, x1, lane) + 1u;
+            }
+        }
     }
+    idx = uniform(idx);
+    lb = uniform(lb);
+    if (MODE == ONE_UB) return idx;
+    if (MODE == ONE_ANY)   // superintervals.hpp:865-871: the last interval starting at or before e
+        return (idx != NONE && s <= ix.ends[idx]) ? 1u : 0u;
+    if (idx == NONE) return 0;
+    const uint32_t hits = uniform(idx + 1u - below);   // the rank form
+    const bool exact = rank_exact && s <= e;
+    if (MODE == W_COUNT && exact) return hits;
     uint32_t* res = reinterpret_cast<uint32_t*>(out + 2);
     int32_t* resv = reinterpret_cast<int32_t*>(out + 2);
     uint64_t acc = 0, found = 0;
@@ -1498,7 +1522,6 @@ __global__ __launch_bounds__(WAVE) void k_one_query(IndexView<S> ix, UbTree<S> u
     bool lead = (MODE == W_VECTOR);
     if (rank_exact) {
         // [lower_bound(s), idx]: every position there starts inside the query, all hits
-        const uint32_t lb = (s == SMIN) ? 0u : wave_tree_ub(ub, (S)(s - 1), lane) + 1u;
         if (lb <= cur) {
             const uint32_t c = cur - lb + 1u;
             if (MODE == W_COUNT) {
@@ -1525,10 +1548,26 @@ __global__ __launch_bounds__(WAVE) void k_one_query(IndexView<S> ix, UbTree<S> u
             }
         }
     }
+    if (exact && (MODE == W_DESC || MODE == W_VALUES) && found == hits) return found;   // nothing below the run
     // the rest by the wave walk; left counts down from 0, so -left is what it found
     wave_walk<S, MODE>(ix, td, ub, lv, lane, s, cur, idx, lead, acc, (MODE == W_COUNT) ? 0 : cap, left, res, vals, resv);
-    const uint64_t total = (MODE == W_COUNT) ? acc : found + (uint64_t)(uint32_t)(0u - left);
-    if (lane == 0) out[0] = total;
+    return (MODE == W_COUNT) ? acc : found + (uint64_t)(uint32_t)(0u - left);
+}
+
+// out (pinned host memory mapped into the device): out[0] = what was found, then, once everything
+// else is there to be read, out[1] = seq, for which the host waits: the end of a stream is seen
+// some 8 us later.
+template <typename S, int MODE>
+__global__ __launch_bounds__(WAVE) void k_one_query(IndexView<S> ix, UbTree<S> ub, UbTree<S> eb, BucketView<S> ubt,
+                                                    BucketView<S> ebt, const S* __restrict__ ends_sorted, TreeDesc<S> td,
+                                                    LongView<S> lv, const int32_t* __restrict__ vals, uint32_t rank_exact,
+                                                    S s, S e, uint64_t* __restrict__ out, uint64_t cap, uint64_t seq) {
+    const int lane = lane_id();
+    const uint64_t found = one_query_wave<S, MODE>(ix, ub, eb, ubt, ebt, ends_sorted, td, lv, vals, rank_exact, s, e, out, cap,
+                                                   lane);
+    if (lane == 0) out[0] = found;
+    __threadfence_system();   // every lane's results
+    if (lane == 0) __hip_atomic_store(&out[1], seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ============================================================================
@@ -3495,6 +3534,8 @@ int one_query_run(siIndex* ix, int mode, S s, S e, uint64_t* total) {
     OneQuery& o = ix->one;
     if (!o.h) {
         HIP_TRY(hipHostMalloc(&o.h, 16 + ONE_CAP * 4, hipHostMallocMapped));
+        ((uint64_t*)o.h)[1] = 0;   // (may hold what an earlier index left there)
+        o.seq = 0;
         HIP_TRY(hipHostGetDevicePointer(&o.d, o.h, 0));
         HIP_TRY(hipStreamCreateWithFlags(&o.st, hipStreamNonBlocking));
         o.cap = ONE_CAP;
@@ -3511,17 +3552,34 @@ int one_query_run(siIndex* ix, int mode, S s, S e, uint64_t* total) {
     const TreeDesc<S> td = ix->tree<S>();
     const LongView<S> lv = long_view_of<S>(ix);
     const uint32_t rx = ix->n_inverted == 0 ? 1u : 0u;
+    const BucketView<S> ubt = ix->ubt.view<S>(), ebt = ix->ebt.view<S>();
+    const S* const es = (const S*)ix->d_ends_sorted;
     uint64_t* out = (uint64_t*)o.d;
+    const uint64_t seq = ++o.seq;
+    const auto run = [&](auto m) {
+        k_one_query<S, decltype(m)::value><<<1, WAVE, 0, o.st>>>(v, ub, eb, ubt, ebt, es, td, lv, ix->d_values, rx, s, e, out,
+                                                                 o.cap, seq);
+    };
     switch (mode) {
-        case W_COUNT: k_one_query<S, W_COUNT><<<1, WAVE, 0, o.st>>>(v, ub, eb, td, lv, ix->d_values, rx, s, e, out, o.cap); break;
-        case W_DESC: k_one_query<S, W_DESC><<<1, WAVE, 0, o.st>>>(v, ub, eb, td, lv, ix->d_values, rx, s, e, out, o.cap); break;
-        case W_VECTOR: k_one_query<S, W_VECTOR><<<1, WAVE, 0, o.st>>>(v, ub, eb, td, lv, ix->d_values, rx, s, e, out, o.cap); break;
-        case W_VALUES: k_one_query<S, W_VALUES><<<1, WAVE, 0, o.st>>>(v, ub, eb, td, lv, ix->d_values, rx, s, e, out, o.cap); break;
-        case ONE_UB: k_one_query<S, ONE_UB><<<1, WAVE, 0, o.st>>>(v, ub, eb, td, lv, ix->d_values, rx, s, e, out, o.cap); break;
-        default: k_one_query<S, ONE_ANY><<<1, WAVE, 0, o.st>>>(v, ub, eb, td, lv, ix->d_values, rx, s, e, out, o.cap); break;
+        case W_COUNT: run(std::integral_constant<int, W_COUNT>()); break;
+        case W_DESC: run(std::integral_constant<int, W_DESC>()); break;
+        case W_VECTOR: run(std::integral_constant<int, W_VECTOR>()); break;
+        case W_VALUES: run(std::integral_constant<int, W_VALUES>()); break;
+        case ONE_UB: run(std::integral_constant<int, ONE_UB>()); break;
+        default: run(std::integral_constant<int, ONE_ANY>()); break;
     }
     LAUNCH_CHECK();
-    HIP_TRY(hipStreamSynchronize(o.st));
+    // (the stream is asked now and then, so that a kernel that never gets there ends the wait)
+    const volatile uint64_t* const done = (const volatile uint64_t*)o.h + 1;
+    for (uint32_t turn = 1; *done != seq; ++turn) {
+        __builtin_ia32_pause();
+        if (turn % 8192u) continue;
+        const hipError_t q = hipStreamQuery(o.st);
+        if (q == hipErrorNotReady) continue;
+        HIP_TRY(q);
+        if (*done != seq) HIP_TRY(hipErrorUnknown);
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
     *total = ((volatile uint64_t*)o.h)[0];
     o.last_valid = true;
     o.last_mode = mode;

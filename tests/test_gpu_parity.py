@@ -1598,3 +1598,51 @@ def test_host_calls_in_chunks(sia, nq):
         t.join()
     assert not bad
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("shape", ["even", "crowd", "inverted", "long", "one"])
+def test_one_query_forms(sia, orc, dtype, shape):
+    """Single queries, whose kernel says itself when its results are there: through the bucket tables,
+    the trees (most intervals in one bucket), on an index with start > end, with a long list, of
+    one interval; every mode against the oracle, ends of the range, inverted queries, no hit below
+    the run and none at all, results past the scratch, and from four threads at once."""
+    import threading
+    print(f"[gpu] one query {np.dtype(dtype).name} {shape}", flush=True)
+    rng = np.random.default_rng(5)
+    info = np.iinfo(dtype)
+    n = 1 if shape == "one" else 120_000
+    s = rng.integers(0, 10 if shape == "crowd" else 800_000, n)
+    e = s + np.where(rng.random(n) < (0.2 if shape == "long" else 0.0), rng.integers(1, 90_000, n), rng.integers(0, 9, n))
+    if shape == "crowd":
+        s[-1], e[-1] = 2**30, 2**30
+    if shape == "inverted":
+        e[::50] = s[::50] - 7
+    s, e = s.astype(dtype), e.astype(dtype)
+    vals = rng.integers(-5, 5, n).astype(np.int32)
+    ix, oix = _dev_index(sia, s, e, vals), orc.build_index(s, e, vals)
+    qs = rng.integers(-5, 800_100, 60).astype(object)
+    qe = qs + rng.integers(-3, 2000, 60)
+    qs = np.array(list(qs) + [info.min, info.min, info.max, 0, 2**30]).astype(dtype)
+    qe = np.array(list(qe) + [info.max, info.min, info.max, 700_000, 2**30]).astype(dtype)
+    bad = []
+
+    def work(order):
+        for k in order:
+            a, b = qs[k:k + 1], qe[k:k + 1]
+            want = orc.search(oix, qs[k], qe[k], 0)
+            ok = [ix.count(a, b)[0] == want.size, bool(ix.has_overlaps(a, b)[0]) == bool(orc.has_overlaps(oix, qs[k], qe[k])),
+                  np.int32(ix.upper_bound(b).view(np.int32)[0]) == np.searchsorted(np.sort(s), qe[k], side="right") - 1,
+                  np.array_equal(ix.search(a, b)[1].astype(np.int64), want),
+                  np.array_equal(ix.search(a, b, order="vector")[1].astype(np.int64), orc.search(oix, qs[k], qe[k], 1)),
+                  np.array_equal(ix.search(a, b, values=True)[1], oix["data"][want])]
+            if not all(ok):
+                bad.append((int(qs[k]), int(qe[k]), ok))
+
+    threads = [threading.Thread(target=work, args=(rng.permutation(len(qs)),)) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad, bad[:3]
+    ix.close()
