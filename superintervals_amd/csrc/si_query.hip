@@ -2023,42 +2023,66 @@ struct GroupOut {
     }
 };
 
-// count() through the tables.  The searches of unsorted queries read their table entries and keys
-// from all over the index: once that outgrows an XCD's 4 MB of L2, large batches are first grouped
-// into 256 stretches of the coordinates (one radix pass by eight bits of the end).
-// int32, 10M intervals: 10M queries 0.97 ms ungrouped, 0.56 grouped (through the sorted plan 0.87),
-// 2M 189 and 104 us, 1M 93 and 73, 500K 46 and 57; int64: 1M 135 and 98, 500K 66 and 77.  1M int32
-// intervals (4 MB): 2M queries 88 and 85, 800K 35 and 54.  100K: 10M queries 236 and 270.
-constexpr size_t GROUP_FROM = 3u << 18;
-template <typename S>
-int launch_count_table(const siIndex* ix, const S* qs, const S* qe, size_t nq, uint32_t* counts, hipStream_t st) {
-    const S* es = (const S*)ix->d_ends_sorted;
-    const BucketView<S> ts = ix->ubt.view<S>(), te = ix->ebt.view<S>();
+// Runs launch(starts, ends, order, blocks) over unsorted queries (order null), or, when `group` says
+// so, over copies of them grouped into 256 stretches of the coordinates (one radix pass by eight
+// bits of the end), order[k] the input query at place k.  The searches of unsorted queries read
+// their table entries and keys from all over the index; once that outgrows an XCD's 4 MB of
+// L2, large batches gain more from the order than it costs.
+template <typename S, class F>
+int launch_grouped(const siIndex* ix, const S* qs, const S* qe, size_t nq, bool group, hipStream_t st, F launch) {
     const unsigned g = grid_for(nq, Q_THREADS);
-    if (nq < GROUP_FROM || ix->n * sizeof(S) < ((size_t)4 << 20)) {
-        k_count_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, qs, qe, nullptr, nq, counts);
+    const size_t off_s = align256(4 * nq), off_e = off_s + align256(sizeof(S) * nq), off_rs = off_e + align256(sizeof(S) * nq);
+    ScopedPlan P(st);
+    // (in a captured stream, or without memory for the copies, the queries go as they are)
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    group = group && nq < (size_t)0x7FFFFFFF && hipStreamIsCapturing(st, &capture) == hipSuccess &&
+            capture == hipStreamCaptureStatusNone && P.alloc(off_rs + rs_temp_bytes(nq)) == SI_OK;
+    if (!group) {
+        (void)hipGetLastError();
+        launch(qs, qe, (const uint32_t*)nullptr, g);
         LAUNCH_CHECK();
         return SI_OK;
     }
     using K = typename std::conditional<sizeof(S) == 4, uint32_t, uint64_t>::type;
     // the eight highest bits in which the index's starts differ (ends outside wrap around: the
     // order only has to keep neighbours together)
+    const BucketView<S> ts = ix->ubt.view<S>();
     const uint64_t differ = (uint64_t)ts.lo ^ (uint64_t)ts.hi;
     int top = 0;
     while (top < (int)sizeof(S) * 8 && (differ >> top) != 0) ++top;
     const int shift = std::max(0, top - 8);
-    const size_t off_s = align256(4 * nq), off_e = off_s + align256(sizeof(S) * nq), off_rs = off_e + align256(sizeof(S) * nq);
-    ScopedPlan P(st);
-    int rc = P.alloc(off_rs + rs_temp_bytes(nq));
-    if (rc) return rc;
     char* const p = (char*)P.p;
     const GroupOut<S> out{(uint32_t*)p, (S*)(p + off_s), (S*)(p + off_e), qs};
     const RsTemp rt = rs_temp_carve(p + off_rs, nq);
-    rc = rs_pass<K, RS_INDEX>((const K*)qe, nullptr, out, nq, shift, 0u, rt, st);
+    const int rc = rs_pass<K, RS_INDEX>((const K*)qe, nullptr, out, nq, shift, 0u, rt, st);
     if (rc) return rc;
-    k_count_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), es, ts, te, out.s, out.e, out.q, nq, counts);
+    launch((const S*)out.s, (const S*)out.e, (const uint32_t*)out.q, g);
     LAUNCH_CHECK();
     return SI_OK;
+}
+
+// count() through the tables.  Grouped, from GROUP_FROM queries and 4 MB of starts on:
+// int32, 10M intervals: 10M queries 0.97 ms ungrouped, 0.56 grouped (through the sorted plan 0.87),
+// 2M 189 and 104 us, 1M 93 and 73, 500K 46 and 57; int64: 1M 135 and 98, 500K 66 and 77.  1M int32
+// intervals (4 MB): 2M queries 88 and 85, 800K 35 and 54.  100K: 10M queries 236 and 270.
+constexpr size_t GROUP_FROM = 3u << 18;
+constexpr size_t GROUP_BYTES = (size_t)4 << 20;
+// has_overlaps reads the ends at one place where count searches them: int32, 10M intervals: 4M queries
+// 230 us ungrouped, 134 grouped, 1.5M 87 and 66, 800K 47 and 47; 1.1M intervals: 2M 57 and 63.
+constexpr size_t ANY_GROUP_FROM = (size_t)1 << 20;
+constexpr size_t ANY_GROUP_BYTES = (size_t)8 << 20;
+// coverage reads up to 24 lines a query, which neighbours in a group share in the L1: 1M intervals:
+// 1M queries 132 us ungrouped, 86 grouped, 400K 54 and 50, 200K 31 and 36; 10M intervals: 1M 325
+// and 137; 100K intervals: 1M 95 and 73.
+constexpr size_t COVERAGE_GROUP_FROM = 3u << 17;
+constexpr size_t COVERAGE_GROUP_BYTES = (size_t)256 << 10;
+template <typename S>
+int launch_count_table(const siIndex* ix, const S* qs, const S* qe, size_t nq, uint32_t* counts, hipStream_t st) {
+    const bool group = nq >= GROUP_FROM && ix->n * sizeof(S) >= GROUP_BYTES;
+    return launch_grouped<S>(ix, qs, qe, nq, group, st, [&](const S* s, const S* e, const uint32_t* order, unsigned g) {
+        k_count_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), (const S*)ix->d_ends_sorted, ix->ubt.view<S>(),
+                                                  ix->ebt.view<S>(), s, e, order, nq, counts);
+    });
 }
 
 // upper_bound through the starts' bucket table.
@@ -2077,19 +2101,20 @@ __global__ __launch_bounds__(Q_THREADS) void k_upper_bound_table(const S* __rest
 }
 
 // has_overlaps through the starts' bucket table (4M unsorted queries on 10M int32 intervals:
-// plain halving read 24 positions in turn).
+// plain halving read 24 positions in turn).  order: see launch_grouped.
 template <typename S>
 __global__ __launch_bounds__(Q_THREADS) void k_has_overlaps_table(IndexView<S> ix, BucketView<S> t,
                                                                   const S* __restrict__ qs, const S* __restrict__ qe,
-                                                                  size_t nq, uint8_t* __restrict__ out) {
-    const size_t q = (size_t)blockIdx.x * Q_THREADS + threadIdx.x;
+                                                                  const uint32_t* __restrict__ order, size_t nq,
+                                                                  uint8_t* __restrict__ out) {
+    const size_t q = (size_t)(order ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * Q_THREADS + threadIdx.x;
     if (q >= nq) return;
     const BucketView<S> tt[1] = {t};
     const S* const v[1] = {ix.starts};
     const S x[1] = {qe[q]};
     uint32_t r[1];
     bucket_ranks<S, 1>(tt, v, ix.n, x, r);
-    out[q] = (r[0] != 0u && qs[q] <= ix.ends[r[0] - 1u]) ? 1 : 0;
+    out[order ? order[q] : q] = (r[0] != 0u && qs[q] <= ix.ends[r[0] - 1u]) ? 1 : 0;
 }
 
 template <typename S>
@@ -2211,11 +2236,13 @@ __global__ __launch_bounds__(Q_THREADS) void k_coverage_rank(IndexView<int32_t> 
                                                              BucketView<int32_t> ts, BucketView<int32_t> te,
                                                              const uint32_t* __restrict__ line_sums, uint32_t lines,
                                                              const int32_t* __restrict__ qs,
-                                                             const int32_t* __restrict__ qe, size_t nq,
+                                                             const int32_t* __restrict__ qe,
+                                                             const uint32_t* __restrict__ order, size_t nq,
                                                              uint32_t* __restrict__ cnt, int32_t* __restrict__ cov) {
-    const size_t q = (size_t)blockIdx.x * Q_THREADS + threadIdx.x;
-    if (q >= nq) return;
-    const int32_t s = qs[q], e = qe[q];
+    const size_t k = (size_t)(order ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * Q_THREADS + threadIdx.x;
+    if (k >= nq) return;
+    const int32_t s = qs[k], e = qe[k];
+    const size_t q = order ? order[k] : k;
     uint32_t c, acc;
     if (s <= e) {
         const bool s1 = s != INT32_MIN, e1 = e != INT32_MIN;   // s - 1, e - 1 exist
@@ -2675,10 +2702,11 @@ SI_EXPORT int siHasOverlaps(const siIndex* ix, const void* qs, const void* qe, s
     hipStream_t st = (hipStream_t)stream;
     return DISPATCH_S(ix, ([&]() -> int {
         if (g_tune.ub_tree && ix->ubt.ok) {
-            k_has_overlaps_table<S><<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(ix->view<S>(), ix->ubt.view<S>(),
-                                                                                  (const S*)qs, (const S*)qe, nq, out);
-            LAUNCH_CHECK();
-            return SI_OK;
+            const bool group = nq >= ANY_GROUP_FROM && ix->n * sizeof(S) >= ANY_GROUP_BYTES;
+            return launch_grouped<S>(ix, (const S*)qs, (const S*)qe, nq, group, st,
+                                     [&](const S* s, const S* e, const uint32_t* order, unsigned g) {
+                k_has_overlaps_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), ix->ubt.view<S>(), s, e, order, nq, out);
+            });
         }
         k_has_overlaps<S><<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(ix->view<S>(), (const S*)qs,
                                                                         (const S*)qe, nq, out);
@@ -2936,11 +2964,13 @@ SI_EXPORT int siCoverage(const siIndex* ix, const void* qs, const void* qe, size
     if (!qs || !qe) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
     if (rank_exact(ix) && ix->ubt.ok) {
-        k_coverage_rank<<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(
-            ix->view<int32_t>(), (const int32_t*)ix->d_ends_sorted, ix->ubt.view<int32_t>(), ix->ebt.view<int32_t>(),
-            ix->d_line_sums, (uint32_t)ix->sum_lines(), (const int32_t*)qs, (const int32_t*)qe, nq, count_out, cov_out);
-        LAUNCH_CHECK();
-        return SI_OK;
+        const bool group = nq >= COVERAGE_GROUP_FROM && ix->n * 4 >= COVERAGE_GROUP_BYTES;
+        return launch_grouped<int32_t>(ix, (const int32_t*)qs, (const int32_t*)qe, nq, group, st,
+                                       [&](const int32_t* s, const int32_t* e, const uint32_t* order, unsigned g) {
+            k_coverage_rank<<<g, Q_THREADS, 0, st>>>(
+                ix->view<int32_t>(), (const int32_t*)ix->d_ends_sorted, ix->ubt.view<int32_t>(), ix->ebt.view<int32_t>(),
+                ix->d_line_sums, (uint32_t)ix->sum_lines(), s, e, order, nq, count_out, cov_out);
+        });
     }
     k_coverage_i32<<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(ix->view<int32_t>(), (const int32_t*)qs,
                                                                  (const int32_t*)qe, nq, count_out, cov_out);

@@ -1646,3 +1646,56 @@ def test_one_query_forms(sia, orc, dtype, shape):
         t.join()
     assert not bad, bad[:3]
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("nq", [393_215, 393_216, 1_048_575, 1_048_576, 1_100_003])
+def test_grouped_forms(sia, orc, dtype, nq):
+    """has_overlaps and coverage on both sides of the batch sizes from which their queries are
+    grouped, on indexes that are and are not large enough for it, with queries outside the
+    intervals, inverted ones, and captured in a graph (where they go ungrouped)."""
+    import torch
+    print(f"[gpu] grouped forms {np.dtype(dtype).name} nq={nq}", flush=True)
+    rng = np.random.default_rng(nq)
+    info = np.iinfo(dtype)
+    for n in (65_535, 65_537, 2_100_000):
+        span = 40 * n
+        s = rng.integers(-1000, span, n)
+        e = s + rng.integers(0, 30, n)
+        qs = rng.integers(-span // 4, span + span // 4, nq)
+        qe = qs + rng.integers(-2, 20, nq)
+        s, e, qs, qe = (x.astype(dtype) for x in (s, e, qs, qe))
+        qs[:4], qe[:4] = [info.min, info.min, info.max, 7], [info.min, info.max, info.max, info.min]
+        ix, oix = _dev_index(sia, s, e), orc.build_index(s, e)
+        starts = np.sort(s)
+        ends = ix.download()["ends"]
+        ub = np.searchsorted(starts, qe, side="right") - 1
+        want = (ub >= 0) & (ends[np.maximum(ub, 0)] >= qs)
+        tqs, tqe = torch.from_numpy(qs).cuda(), torch.from_numpy(qe).cuda()
+        lib, check = sia._native.lib, sia._native.check
+        out = torch.full((nq + 9,), 5, dtype=torch.uint8, device="cuda")
+        check(lib.siHasOverlaps(ix.handle, tqs.data_ptr(), tqe.data_ptr(), nq, out.data_ptr(), None), "siHasOverlaps")
+        torch.cuda.synchronize()
+        got = out.cpu().numpy()
+        assert np.array_equal(got[:nq], want.astype(np.uint8)) and np.all(got[nq:] == 5)
+        out.fill_(5)
+        g, st = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+        st.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.graph(g, stream=st):
+            check(lib.siHasOverlaps(ix.handle, tqs.data_ptr(), tqe.data_ptr(), nq, out.data_ptr(),
+                                    torch.cuda.current_stream().cuda_stream), "siHasOverlaps")
+        for _ in range(2):
+            g.replay()
+            torch.cuda.synchronize()
+            got = out.cpu().numpy()
+            assert np.array_equal(got[:nq], want.astype(np.uint8)) and np.all(got[nq:] == 5)
+            out.fill_(5)
+        if dtype == np.int32:
+            cnt, cov = (torch.full((nq + 9,), -5, dtype=torch.int32, device="cuda") for _ in range(2))
+            check(lib.siCoverage(ix.handle, tqs.data_ptr(), tqe.data_ptr(), nq, cnt.data_ptr(), cov.data_ptr(), None), "siCoverage")
+            torch.cuda.synchronize()
+            cnt, cov = cnt.cpu().numpy(), cov.cpu().numpy()
+            assert np.array_equal(cnt[:nq], orc.count_batch(oix, qs, qe)) and np.all(cnt[nq:] == -5) and np.all(cov[nq:] == -5)
+            some = np.concatenate([np.arange(200), rng.integers(0, nq, 3000), [nq - 1]])
+            assert [int(cov[k]) for k in some] == [int(orc.coverage(oix, qs[k], qe[k])[1]) for k in some]
+        ix.close()
