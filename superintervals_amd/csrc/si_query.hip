@@ -2033,12 +2033,13 @@ int launch_grouped(const siIndex* ix, const S* qs, const S* qe, size_t nq, bool 
     const unsigned g = grid_for(nq, Q_THREADS);
     const size_t off_s = align256(4 * nq), off_e = off_s + align256(sizeof(S) * nq), off_rs = off_e + align256(sizeof(S) * nq);
     ScopedPlan P(st);
-    // (in a captured stream, or without memory for the copies, the queries go as they are)
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    group = group && nq < (size_t)0x7FFFFFFF && hipStreamIsCapturing(st, &capture) == hipSuccess &&
-            capture == hipStreamCaptureStatusNone && P.alloc(off_rs + rs_temp_bytes(nq)) == SI_OK;
+    if (group) {   // (not in a captured stream, nor without memory for the copies)
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        group = nq < (size_t)0x7FFFFFFF && hipStreamIsCapturing(st, &capture) == hipSuccess &&
+                capture == hipStreamCaptureStatusNone && P.alloc(off_rs + rs_temp_bytes(nq)) == SI_OK;
+        if (!group) (void)hipGetLastError();
+    }
     if (!group) {
-        (void)hipGetLastError();
         launch(qs, qe, (const uint32_t*)nullptr, g);
         LAUNCH_CHECK();
         return SI_OK;
@@ -3047,32 +3048,22 @@ struct MultiLayout {
     }
 };
 
-constexpr int MK_THREADS = 256;
-constexpr int MK_ITEMS = 8;   // queries per thread in the key kernel
-
-// Sort keys (slot << 32 | biased end), payload = input number; per-slot query counts through
-// an LDS histogram.  Slots past the table map to the empty slot.
-__global__ __launch_bounds__(MK_THREADS) void k_multi_keys(const uint32_t* __restrict__ set_ids,
-                                                           const int32_t* __restrict__ qe, size_t nq,
-                                                           uint32_t nslots, uint64_t* __restrict__ key,
-                                                           uint32_t* __restrict__ val, uint32_t* __restrict__ scnt) {
-    extern __shared__ uint32_t s_hist[];
-    for (uint32_t b = threadIdx.x; b < nslots; b += MK_THREADS) s_hist[b] = 0;
-    __syncthreads();
-    const size_t base = (size_t)blockIdx.x * MK_THREADS * MK_ITEMS;
-    for (int j = 0; j < MK_ITEMS; ++j) {
-        const size_t k = base + (size_t)j * MK_THREADS + threadIdx.x;
-        if (k < nq) {
-            uint32_t g = set_ids[k];
-            if (g >= nslots - 1) g = nslots - 1;
-            key[k] = ((uint64_t)g << 32) | (uint32_t)((uint32_t)qe[k] ^ 0x80000000u);
-            val[k] = (uint32_t)k;
-            atomicAdd(&s_hist[g], 1u);
-        }
+// Sort key of a query: slot << 32 | biased end.  Slots past the table map to the empty slot.
+struct MultiIn {
+    const uint32_t* __restrict__ set_ids;
+    const int32_t* __restrict__ qe;
+    uint32_t nslots;
+    __device__ __forceinline__ uint64_t key(size_t k) const {
+        return (uint64_t)min(set_ids[k], nslots - 1u) << 32 | ((uint32_t)qe[k] ^ 0x80000000u);
     }
-    __syncthreads();
-    for (uint32_t b = threadIdx.x; b < nslots; b += MK_THREADS)
-        if (s_hist[b]) atomicAdd(&scnt[b], s_hist[b]);
+};
+
+__global__ __launch_bounds__(Q_THREADS) void k_multi_keys(MultiIn in, size_t nq, uint64_t* __restrict__ key,
+                                                          uint32_t* __restrict__ val) {
+    const size_t k = (size_t)blockIdx.x * Q_THREADS + threadIdx.x;
+    if (k >= nq) return;
+    key[k] = in.key(k);
+    val[k] = (uint32_t)k;
 }
 
 // Per sorted query: its slot, start, end; upper_bound and lower_bound through its set's
@@ -3127,18 +3118,35 @@ __global__ __launch_bounds__(Q_THREADS) void k_multi_finish(const SetView<int32_
     counts[q] = c;
 }
 
-// First sorted query and first tile of every slot (one workgroup, a run of slots per thread: 3000
-// slots 5 us, by one thread 280).
+// Number, first sorted query and first tile of every slot, from the sorted queries' slots (one
+// workgroup, a run of slots per thread).
 constexpr int MT_THREADS = 1024;
-__global__ __launch_bounds__(MT_THREADS) void k_multi_tiles(const uint32_t* __restrict__ scnt, uint32_t nslots, uint32_t tile,
+__global__ __launch_bounds__(MT_THREADS) void k_multi_tiles(const uint32_t* __restrict__ set, uint32_t nq, uint32_t nslots,
+                                                            uint32_t tile, uint32_t* __restrict__ scnt,
                                                             uint32_t* __restrict__ sbeg, uint32_t* __restrict__ tbeg) {
     __shared__ uint32_t s_q[MT_THREADS], s_t[MT_THREADS];
     const uint32_t i = threadIdx.x, run = (nslots + MT_THREADS - 1u) / MT_THREADS;
     const uint32_t g0 = min(i * run, nslots), g1 = min(g0 + run, nslots);
+    auto first_of = [&](uint32_t g) {   // sorted queries of the slots below g
+        uint32_t at = 0;
+        for (uint32_t m = nq; m;) {
+            const uint32_t half = m >> 1;
+            if (set[at + half] < g) {
+                at += half + 1u;
+                m -= half + 1u;
+            } else {
+                m = half;
+            }
+        }
+        return at;
+    };
     uint32_t a = 0, b = 0;
-    for (uint32_t g = g0; g < g1; ++g) {
-        a += scnt[g];
-        b += (scnt[g] + tile - 1u) / tile;
+    for (uint32_t g = g0, at = g0 < g1 ? first_of(g0) : 0u; g < g1; ++g) {
+        const uint32_t next = first_of(g + 1u);
+        scnt[g] = next - at;
+        a += next - at;
+        b += (next - at + tile - 1u) / tile;
+        at = next;
     }
     s_q[i] = a;
     s_t[i] = b;
@@ -3220,8 +3228,8 @@ int launch_walk_multi(const siSetTable* tb, void* plan, size_t nq, const uint64_
         const uint32_t tile = multi_tile();
         const size_t tiles_max = (nq + tile - 1) / tile + tb->nslots;
         const unsigned grid = (unsigned)std::max<size_t>(1, std::min<size_t>((size_t)cus * wgs, tiles_max));
-        k_multi_tiles<<<1, MT_THREADS, 0, st>>>(mt.scnt, tb->nslots, tile, const_cast<uint32_t*>(mt.sbeg),
-                                                const_cast<uint32_t*>(mt.tbeg));
+        k_multi_tiles<<<1, MT_THREADS, 0, st>>>(pv.set, (uint32_t)nq, tb->nslots, tile, const_cast<uint32_t*>(mt.scnt),
+                                                const_cast<uint32_t*>(mt.sbeg), const_cast<uint32_t*>(mt.tbeg));
         LAUNCH_CHECK();
         k_walk<int32_t, MODE, true><<<grid, T_THREADS, 0, st>>>(
             IndexView<int32_t>{}, pv, (uint32_t)nq, tile, NONE - 1u, g_tune.lane_steps, true, pv.counter, nullptr,
@@ -3316,19 +3324,20 @@ SI_EXPORT int siSetTableSearchOffsets(const siSetTable* t, const uint32_t* set_i
     uint32_t* v0 = (uint32_t*)(p + L.base.off_v0);
     uint32_t* v1 = (uint32_t*)(p + L.base.off_v1);
     RsTemp rt = rs_temp_carve(p + L.base.off_rs, nq);
-    uint32_t* scnt = (uint32_t*)(p + L.off_scnt);
-    k_zero_u32<<<grid_for(t->nslots, 256), 256, 0, st>>>(scnt, t->nslots);
-    LAUNCH_CHECK();
-    const unsigned gk = grid_for(nq, MK_THREADS * MK_ITEMS);
-    k_multi_keys<<<gk, MK_THREADS, t->nslots * sizeof(uint32_t), st>>>(set_ids, (const int32_t*)qe, nq, t->nslots, k0,
-                                                                       v0, scnt);
-    LAUNCH_CHECK();
-    // sort by (slot, end): the end's digits (the lowest plan_skip_low left unsorted) and the
-    // slot's one or two; no host read-back, so the batch can be captured in a graph
-    const int slot_digits = (t->nslots <= 256) ? 1 : 2;
-    uint64_t* ks;
-    uint32_t* vs;
-    rc = radix_sort_pairs(k0, v0, k1, v1, nq, g_tune.plan_skip_low, 4 + slot_digits, rt, &ks, &vs, st);
+    // sort by (slot, end): the end's digits, the lowest (plan_skip_low of them, at least one) left
+    // unsorted, as the sweep orders a chunk's queries by start anyway, and the slot's one or
+    // two; no host read-back, so the batch can be captured in a graph
+    const int low = std::max(1, g_tune.plan_skip_low), high = 4 + ((t->nslots <= 256) ? 1 : 2);
+    const MultiIn in{set_ids, (const int32_t*)qe, t->nslots};
+    uint64_t* ks = k1;
+    uint32_t* vs = v1;
+    if (nq <= RS1_MAX) {
+        rc = rs_sort_one<uint64_t>(in, ArrayOut{k1, v1}, nq, low, high, st);
+    } else {
+        k_multi_keys<<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>(in, nq, k0, v0);
+        LAUNCH_CHECK();
+        rc = radix_sort_pairs(k0, v0, k1, v1, nq, low, high, rt, &ks, &vs, st);
+    }
     if (rc) return rc;
     PlanView<int32_t> pv = multi_view(plan, nq, t->nslots);
     uint32_t* c32 = counts ? counts : (uint32_t*)(p + L.base.off_heavy);

@@ -736,7 +736,7 @@ __global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, Tr
                     }
                     q_acc[i] = acc;
                     q_left[i] = left;
-                    q_room[i] = (uint32_t)min(oend - acc, (uint64_t)1 << 28);
+                    q_room[i] = (uint32_t)min(oend - acc, (uint64_t)0xFFFFFFFFu);
                     q_bound[i] = bound;   // (every lane stores the same values)
                 }
                 if (!share) continue;
@@ -828,7 +828,7 @@ __global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, Tr
                         const uint32_t room = uniform(q_room[i]);
                         const uint64_t acc = read_lane(q_acc[i], 0);
                         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                            (VALUES ? (uint32_t*)out_val : out_idx) + acc, (short)0, (int)(room * 4u), 0x00020000);
+                            (VALUES ? (uint32_t*)out_val : out_idx) + acc, (short)0, (int)(min(room, 1u << 28) * 4u), 0x00020000);
                         uint32_t k = 0;
                         for (uint32_t x = (uint32_t)lane; x < C + (uint32_t)lane; x += UNROLL * WAVE) {
                             uint32_t r[UNROLL], p[UNROLL], v[UNROLL];
