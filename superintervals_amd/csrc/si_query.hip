@@ -2326,20 +2326,27 @@ inline uint32_t sweep_chunk(size_t nq, int cus) {
     return (uint32_t)std::min<size_t>(SW_CHUNK, (nq + waves - 1) / waves);
 }
 
-// The queries that the sweep left, through the long list: spans of up to 32 queries (or one
-// chunk), fewer where that would leave workgroups without one.
+// Spans of the queries that the sweep left: up to 32 of the plan's queries (or one chunk), fewer
+// where that would leave workgroups without one.
+inline uint32_t shared_span(size_t nq, uint32_t chunk, int cus, int mode) {
+    const uint32_t want = (uint32_t)std::min<size_t>(32, nq / ((size_t)cus * sh_wgs(mode)));
+    return chunk * std::max(1u, want / chunk);
+}
+inline unsigned shared_grid(size_t nq, uint32_t span, int cus, int mode) {
+    const size_t spans = (nq + span - 1) / span, full = (spans + HEAVY_CHUNKS - 1) / HEAVY_CHUNKS * HEAVY_CHUNKS;
+    return (unsigned)std::min<size_t>((size_t)cus * sh_wgs(mode), full);
+}
+
 template <typename S, int MODE>
 int launch_sweep_shared(const siIndex* ix, const PlanView<S>& pv, size_t nq, uint32_t chunk, int cus,
                         const uint64_t* offsets, uint32_t* out_idx, int32_t* out_val, uint64_t cap, hipStream_t st) {
     IndexView<S> hv = ix->view<S>();
     LongView<S> lv = long_view_of<S>(ix);
     if (!g_tune.heavy_ends32) { hv.ends32 = nullptr; lv.ends32 = nullptr; }
-    const size_t grid = (size_t)cus * sh_wgs(MODE);
-    const uint32_t want = (uint32_t)std::min<size_t>(32, nq / grid);
-    const uint32_t span = chunk * std::max(1u, want / chunk);
-    k_sweep_shared<S, MODE><<<(unsigned)std::min<size_t>(grid, ((nq + span - 1) / span + HEAVY_CHUNKS - 1) / HEAVY_CHUNKS * HEAVY_CHUNKS), SH_THREADS, 0, st>>>(
-        hv, ix->tree<S>(), ub_tree_of<S>(ix->ub, (const S*)ix->d_starts, ix->n), ix->ubt.view<S>(), lv, pv, (uint32_t)nq,
-        chunk, span, offsets, out_idx, ix->d_values, out_val, cap);
+    const uint32_t span = shared_span(nq, chunk, cus, MODE);
+    k_sweep_shared<S, MODE><<<shared_grid(nq, span, cus, MODE), SH_THREADS, 0, st>>>(
+        hv, ix->tree<S>(), ub_tree_of<S>(ix->ub, (const S*)ix->d_starts, ix->n), ix->ubt.view<S>(), lv, nullptr, pv,
+        (uint32_t)nq, chunk, span, offsets, out_idx, ix->d_values, out_val, cap);
     LAUNCH_CHECK();
     return SI_OK;
 }
@@ -2366,15 +2373,11 @@ int launch_walk(const siIndex* ix, void* plan, size_t nq, uint32_t* counts, uint
         swept = range_skip_on(ix);
         if (swept) {
             const uint32_t chunk = sweep_chunk(nq, cus);
-            const LongView<S> lv = long_view_of<S>(ix);
-            const bool by_place = lv.len > 0;   // (k_sweep_shared)
             k_sweep<S, MODE><<<grid_for(nq, chunk * SW_WAVES), SW_THREADS, 0, st>>>(
-                ix->view<S>(), ix->tree<S>(), nullptr, pv, (uint32_t)nq, chunk, by_place, offsets,
+                ix->view<S>(), ix->tree<S>(), nullptr, pv, (uint32_t)nq, chunk, offsets,
                 MODE == W_VALUES ? (uint32_t*)out_val : out_idx, ix->d_values, cap);
-            if (by_place) {
-                LAUNCH_CHECK();
-                return launch_sweep_shared<S, MODE>(ix, pv, nq, chunk, cus, offsets, out_idx, out_val, cap, st);
-            }
+            LAUNCH_CHECK();
+            return launch_sweep_shared<S, MODE>(ix, pv, nq, chunk, cus, offsets, out_idx, out_val, cap, st);
         }
     }
     if (!swept) {
@@ -3235,10 +3238,15 @@ int launch_walk_multi(const siSetTable* tb, void* plan, size_t nq, const uint64_
             IndexView<int32_t>{}, pv, (uint32_t)nq, tile, NONE - 1u, g_tune.lane_steps, true, pv.counter, nullptr,
             nullptr, offsets, out_idx, nullptr, nullptr, cap, sets, mt);
     } else {
-        const uint32_t chunk = sweep_chunk(nq, cus);
+        const uint32_t chunk = sweep_chunk(nq, cus), span = shared_span(nq, chunk, cus, MODE);
         k_sweep<int32_t, MODE, true><<<grid_for(nq, chunk * SW_WAVES), SW_THREADS, 0, st>>>(
-            IndexView<int32_t>{}, TreeDesc<int32_t>{}, sets, pv, (uint32_t)nq, chunk, false, offsets, out_idx, nullptr,
-            cap);
+            IndexView<int32_t>{}, TreeDesc<int32_t>{}, sets, pv, (uint32_t)nq, chunk, offsets, out_idx, nullptr, cap);
+        LAUNCH_CHECK();
+        k_sweep_shared<int32_t, MODE, true><<<shared_grid(nq, span, cus, MODE), SH_THREADS, 0, st>>>(
+            IndexView<int32_t>{}, TreeDesc<int32_t>{}, UbTree<int32_t>{}, BucketView<int32_t>{}, LongView<int32_t>{}, sets, pv,
+            (uint32_t)nq, chunk, span, offsets, out_idx, nullptr, nullptr, cap);
+        LAUNCH_CHECK();
+        return SI_OK;
     }
     LAUNCH_CHECK();
     LongView<int32_t> none{};   // the sets' walks read their own arrays only

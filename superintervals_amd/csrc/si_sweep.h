@@ -28,9 +28,8 @@
 // unaligned in 1.8 ms).  100K queries on 10M: 66 us (143), 1M: 276 us (656), 4096: 14 us (111);
 // 3M queries with 1.2 hits each on 100K intervals: 108 us (116).
 //
-// A query is left to the wave-cooperative kernel (k_walk_heavy), which continues below the
-// run, when more than SW_CAP intervals hold its start, and when it ends below its own start's
-// lower bound (start > end).
+// A query is left to k_sweep_shared, which continues below the run, when more than SW_CAP intervals
+// hold its start, and when it ends below its own start's lower bound (start > end).
 #pragma once
 
 constexpr int SW_THREADS = 256;
@@ -335,12 +334,12 @@ __device__ __forceinline__ void sweep_lanes(SweepGroup<S>& g, uint64_t todo, int
 
 // The plan's queries t0 .. t0 + m - 1 (of one index), by one wave with its part of the LDS (see above).
 // out: the positions or values as 32-bit words; only slots below cap and inside a query's segment
-// [offsets[q], offsets[q + 1]) are written.  Queries left to the wave-cooperative kernels go to the
-// plan's heavy list, their run already written (not in vector order, where the run is part of
-// the leading run); returns their number.  bad: a query's hits differ from its offsets.
+// [offsets[q], offsets[q + 1]) are written.  Queries left to k_sweep_shared go to the plan's heavy
+// list from place + parked on, their run already written (not in vector order, where the run is
+// part of the leading run); parked counts them.  bad: a query's hits differ from its offsets.
 template <typename S, int MODE>
-__device__ __forceinline__ uint32_t sweep_queries(const IndexView<S>& ix, const TreeDesc<S>& td, const PlanView<S>& pv,
-                                                  uint32_t t0, uint32_t m, bool by_place, int lane,
+__device__ __forceinline__ void sweep_queries(const IndexView<S>& ix, const TreeDesc<S>& td, const PlanView<S>& pv,
+                                                  uint32_t t0, uint32_t m, uint32_t place, uint32_t& parked, int lane,
                                                   S* __restrict__ l_end, uint32_t* __restrict__ l_pay,
                                                   uint32_t* __restrict__ l_key, const uint64_t* __restrict__ offsets,
                                                   uint32_t* __restrict__ out, const int32_t* __restrict__ vals,
@@ -405,7 +404,6 @@ __device__ __forceinline__ uint32_t sweep_queries(const IndexView<S>& ix, const 
     uint32_t A = 0, wbase = NONE;               // wbase NONE: no list yet
     S we = SMIN;                                // window: ends and payloads
     uint32_t wp = 0, full = 0;                  // full: a list outgrew SW_CAP, the chunk's other queries are left too
-    uint32_t parked = 0;                        // queries left so far
 
     // the packed entries l_end / l_pay[0 .. n) as the list
     auto take_list = [&](uint32_t n) {
@@ -531,7 +529,7 @@ __device__ __forceinline__ uint32_t sweep_queries(const IndexView<S>& ix, const 
             // (per lane, outside every wave-wide step; the run [lb, ub] is written, but for the vector order)
             const uint32_t c = ordered && MODE != W_VECTOR ? g.ub + 1u - g.lb : 0u;
             // (field by field: the first entry's pad is the chunk's number of them)
-            HeavyEntry& he = pv.heavy[by_place ? t0 + parked + lanes_below(left) : atomicAdd(&pv.counter[1], 1u)];
+            HeavyEntry& he = pv.heavy[place + parked + lanes_below(left)];
             he.k = gk;
             he.cur = ordered ? g.lb - 1u : g.ub;
             he.top = g.ub;
@@ -541,16 +539,14 @@ __device__ __forceinline__ uint32_t sweep_queries(const IndexView<S>& ix, const 
         }
         parked += (uint32_t)__popcll(left);
     }
-    return parked;
 }
 
 // One wave per chunk of `chunk` consecutive sorted queries.  MODE: W_DESC, W_VECTOR or W_VALUES.
-// by_place: a chunk's heavy entries lie at its first query's place, their number in the first one's
-// pad; else they follow each other in any order.  MULTI: the plan's queries are sorted by their set
-// (pv.set), a chunk's are answered set by set.
+// A chunk's heavy entries lie at its first query's place, their number in the first one's pad.
+// MULTI: the plan's queries are sorted by their set (pv.set), a chunk's are answered set by set.
 template <typename S, int MODE, bool MULTI = false>
 __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<S> td, const SetView<S>* __restrict__ sets,
-                                                      PlanView<S> pv, uint32_t nq, uint32_t chunk, bool by_place,
+                                                      PlanView<S> pv, uint32_t nq, uint32_t chunk,
                                                       const uint64_t* __restrict__ offsets,
                                                       uint32_t* __restrict__ out, const int32_t* __restrict__ vals,
                                                       uint64_t cap) {
@@ -564,6 +560,7 @@ __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<
     uint32_t t0 = (uint32_t)t0w;
     const uint32_t m = min(chunk, nq - t0);   // this wave's queries
     bool bad = false;
+    uint32_t parked = 0;
     if (MULTI) {
         for (uint32_t n; t0 < (uint32_t)t0w + m; t0 += n) {
             const uint32_t g = uniform(pv.set[t0]);
@@ -573,49 +570,59 @@ __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<
                 other = __builtin_amdgcn_ballot_w64(i >= (uint32_t)t0w + m || pv.set[i] != g);
                 n += other ? (uint32_t)__builtin_ctzll(other) : (uint32_t)WAVE;
             }
-            sweep_queries<S, MODE>(sets[g].v, sets[g].td, pv, t0, n, false, lane, s_end[wv], s_pay[wv], s_key[wv], offsets,
-                                   out, nullptr, cap, bad);
+            sweep_queries<S, MODE>(sets[g].v, sets[g].td, pv, t0, n, (uint32_t)t0w, parked, lane, s_end[wv], s_pay[wv],
+                                   s_key[wv], offsets, out, nullptr, cap, bad);
         }
     } else {
-        const uint32_t parked = sweep_queries<S, MODE>(ix, td, pv, t0, m, by_place, lane, s_end[wv], s_pay[wv], s_key[wv],
-                                                       offsets, out, vals, cap, bad);
-        if (by_place && lane == 0) {
-            pv.heavy[t0].pad = parked;
-            if (parked) atomicAdd(&pv.counter[1], parked);
-        }
+        sweep_queries<S, MODE>(ix, td, pv, t0, m, t0, parked, lane, s_end[wv], s_pay[wv], s_key[wv], offsets, out, vals, cap,
+                               bad);
+    }
+    if (lane == 0) {
+        pv.heavy[(uint32_t)t0w].pad = parked;
+        if (parked) pv.counter[1] = 1u;   // (a flag: an atomic a wave on one line took 70 us of 100K queries)
     }
     if (bad) atomicOr(&pv.counter[3], 1u);   // a query's hits differ from its offsets
 }
 
 // ---- the queries that the sweep left, several answered from one candidate list
 //
-// Where more than SW_CAP intervals hold a query's start, most of them are long: they lie far below
-// it, thinly spread over the entries of the long list (300 lines of 64 for 4100 hits, one in five
-// a hit, in 20M int64 intervals with 20 % of 10^5 .. 10^7 long), and neighbouring queries share
-// nearly all of them.  A workgroup takes a span of the plan's queries, orders those left by their
-// starts and cuts them into groups (SH_SPREAD).  For a group its waves collect the long entries
-// that reach the first start into LDS, highest first, CAP at a time; then each wave answers
-// its queries from the list, two compares, a ballot and a store for 64 entries.  The positions
-// at and above s - len are read from the index for each query.  A group of fewer than SH_LEAST
-// queries would leave the other waves idle: each walks on its own (wave_walk).
+// Where more than SW_CAP intervals hold a query's start, neighbouring queries share nearly all of
+// them.  A workgroup takes a span of the plan's queries, orders those left by their starts
+// (and sets) and cuts them into groups.  For a group its waves collect the candidates into LDS,
+// highest first, CAP at a time; then each wave answers its queries from the list, two compares, a
+// ballot and a store for 64 entries.  Two kinds of list:
+//   all of it   the positions below the group's runs whose end reaches its first start: from
+//               the index, through the max tree, down to the first start - len, from the long
+//               list below that.  For starts close together (SH_NEAR);
+//   far         only the long entries below each query's start - len (SH_SPREAD), the positions
+//               above it read from the index for each query: long intervals lie thinly spread far
+//               below (300 lines of 64 for 4100 hits, one in five a hit, in 20M int64 intervals
+//               with 20 % of 10^5 .. 10^7 long) and are shared by starts further apart.
+// The kind that takes in more queries is used.  A group of fewer than SH_LEAST queries would leave
+// the other waves idle: each walks on its own (wave_walk).
 //
 // What bounds it: waits for memory, at 16 waves a CU (the lists' LDS).  100K queries on 20M such
-// intervals: 0.75 ms (2.0 with a walk of the long list for each query), of which without the
-// lists' stores 0.64, without the scan 0.48, without lists 0.33, without the index's positions
-// too 0.21.  2000 queries on 20M: 0.15 ms (0.80), 30K on 5M: 0.17 (1.15).  CAP 6144 (12 waves a CU)
-// and 8 waves a workgroup were slower by 20 and 10 %, CAP 2048 by 10 %, but with payloads, which
-// take another word of LDS an entry, faster by 15 %.  SH_SPREAD 512: 1.30 ms for that fill,
-// 1024: 1.10, 2048 and 4096: 1.00.
+// intervals: 0.77 ms (2.0 with a walk of the long list for each query), of which, far lists only,
+// without the lists' stores 0.64, without the scan 0.48, without lists 0.33, without the index's
+// positions too 0.21.  2000 queries on 20M: 0.13 ms (0.80).  1M queries that 320 of 10M intervals
+// hold, none long: fill 0.83 ms (lane walk 1.06, a walk for each query 2.0); 50M on 200M intervals,
+// two fifths of them held by 330: 32 ms (52; 76).  CAP 6144 (12 waves a CU) and 8 waves a workgroup
+// were slower by 20 and 10 %, CAP 2048 by 10 %, but with payloads, which take another word of LDS
+// an entry, faster by 15 %.  SH_SPREAD 512: 1.30 ms for the first fill, 1024: 1.10, 2048 and 4096:
+// 1.00.  SH_NEAR 1024 and 4096: the same.  Spans of 64: 0.95 for the first, 0.12 against 0.21 for
+// 100K queries that 400 of 1M hold.
 constexpr int SH_THREADS = 256;
 constexpr int SH_WAVES = SH_THREADS / WAVE;
 constexpr uint32_t SH_SPREAD = 2048;     // long entries that start within a group's range
+constexpr uint32_t SH_NEAR = 2048;       // positions between the starts of a group that shares all of its list
 constexpr uint32_t SH_LEAST = 3;         // smallest group that shares a list
 constexpr uint32_t sh_cap(int mode) { return mode == W_VALUES ? 2048u : 4096u; }
 constexpr unsigned sh_wgs(int mode) { return mode == W_VALUES ? 6u : 4u; }   // workgroups a CU (160 KB of LDS)
 
-template <typename S, int MODE>
-__global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, TreeDesc<S> td, UbTree<S> ub, BucketView<S> tab,
-                                                             LongView<S> lv, PlanView<S> pv, uint32_t nq, uint32_t chunk,
+template <typename S, int MODE, bool MULTI = false>
+__global__ __launch_bounds__(SH_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_sweep_shared(IndexView<S> ix_one, TreeDesc<S> td_one, UbTree<S> ub_one,
+                                                             BucketView<S> tab, LongView<S> lv,
+                                                             const SetView<S>* __restrict__ sets, PlanView<S> pv, uint32_t nq, uint32_t chunk,
                                                              uint32_t span, const uint64_t* __restrict__ offsets,
                                                              uint32_t* __restrict__ out_idx,
                                                              const int32_t* __restrict__ vals,
@@ -629,24 +636,32 @@ __global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, Tr
     __shared__ uint32_t c_rel[CAP + UNROLL * WAVE], c_pos[CAP + UNROLL * WAVE], c_val[VALUES ? CAP + UNROLL * WAVE : 1];
     __shared__ S q_s[WAVE];
     __shared__ uint64_t q_acc[WAVE];
-    __shared__ uint32_t q_slot[WAVE], q_p0[WAVE], q_j[WAVE], q_left[WAVE], q_room[WAVE], q_bound[WAVE];
+    __shared__ uint32_t q_top[WAVE], q_p0[WAVE], q_j[WAVE], q_left[WAVE], q_room[WAVE], q_bound[WAVE];
+    __shared__ uint32_t q_cur[WAVE], q_set[MULTI ? WAVE : 1];
     __shared__ uint32_t w_tot[2][SH_WAVES], s_n, s_work;
     if (uniform(pv.counter[1]) == 0u) return;   // nothing was left
     const int lane = lane_id();
     const uint32_t wv = uniform(threadIdx.x / WAVE);
     EntryDeal deal(pv.counter + 8, (nq + span - 1u) / span, blockIdx.x, gridDim.x);
-    while (true) {
-        // the next span of the plan's queries
-        __syncthreads();   // (the span before is done with the lists)
-        if (wv == 0) {
-            const uint32_t h = deal.take(lane);
-            if (lane == 0) s_work = h;
-        }
-        __syncthreads();
-        const uint32_t h = uniform(s_work);
-        if (h == NONE) break;
+    // the next span of the plan's queries is taken by the last wave while the first prepares this one's
+    if (wv == SH_WAVES - 1u) {
+        const uint32_t first = deal.take(lane);
+        if (lane == 0) s_work = first;
+    }
+    __syncthreads();
+    uint32_t h = uniform(s_work);
+    while (h != NONE) {
         const uint32_t k0 = h * span, kn = min(span, nq - k0);
-        if (span == chunk && uniform(pv.heavy[k0].pad) == 0u) continue;
+        __syncthreads();   // (the span before is done with the lists, and s_work is read)
+        if (wv == SH_WAVES - 1u) {
+            const uint32_t then = deal.take(lane);
+            if (lane == 0) s_work = then;
+        }
+        if (span == chunk && uniform(pv.heavy[k0].pad) == 0u) {
+            __syncthreads();
+            h = uniform(s_work);
+            continue;
+        }
         for (uint32_t b0 = 0; b0 < kn; b0 += WAVE) {
             if (b0) __syncthreads();   // (the batch before is done with the lists)
             if (wv == 0) {
@@ -656,31 +671,45 @@ __global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, Tr
                 const uint64_t all = __builtin_amdgcn_ballot_w64(mine);
                 const HeavyEntry* const he = pv.heavy + k0 + (mine ? t : 0u);
                 S s = SMIN;
-                uint32_t cur = 0;
+                uint32_t cur = 0, set = 0, top = 0, left = 0, room = 0;
+                uint64_t acc = 0;
                 if (mine) {
-                    s = pv.s[he->k];
+                    const uint32_t k = he->k;
                     cur = he->cur;
+                    top = he->top;
+                    left = he->left;
+                    acc = he->acc;
+                    s = pv.s[k];
+                    if (MULTI) set = pv.set[k];
+                    // (never below acc: offsets that decrease give an empty room, not a wrapped one)
+                    room = (uint32_t)min(max(min(offsets[pv.q[k] + 1u], cap), acc) - acc, (uint64_t)0xFFFFFFFFu);
                 }
                 uint32_t rank = 0;
                 for (uint64_t m = all; m; m &= m - 1ull) {
                     const uint32_t j = (uint32_t)__builtin_ctzll(m);
                     const S o = read_lane(s, j);
-                    rank += (o < s || (o == s && j < (uint32_t)lane)) ? 1u : 0u;
+                    const bool below = o < s || (o == s && j < (uint32_t)lane);
+                    if (MULTI) {
+                        const uint32_t so = read_lane(set, j);
+                        rank += (so < set || (so == set && below)) ? 1u : 0u;
+                    } else {
+                        rank += below ? 1u : 0u;
+                    }
                 }
-                uint32_t p0 = 0;   // the first position starting at or after s - len
-                if (mine && (int64_t)s > (int64_t)SMIN + lv.len) {
+                uint32_t p0 = 0;   // the first position starting at or after s - len (0: no long list)
+                if (!MULTI && mine && lv.len > 0 && (int64_t)s > (int64_t)SMIN + lv.len) {
                     const S x = (S)((int64_t)s - lv.len - 1);
                     if (tab.tab) {
                         const BucketView<S> tt[1] = {tab};
-                        const S* const v[1] = {ix.starts};
+                        const S* const v[1] = {ix_one.starts};
                         const S xs[1] = {x};
                         uint32_t r[1];
-                        bucket_ranks<S, 1>(tt, v, ix.n, xs, r);
+                        bucket_ranks<S, 1>(tt, v, ix_one.n, xs, r);
                         p0 = r[0];
                     } else {
-                        for (uint32_t m = ix.n; m; ) {
+                        for (uint32_t m = ix_one.n; m;) {
                             const uint32_t half = m >> 1;
-                            if (ix.starts[p0 + half] <= x) {
+                            if (ix_one.starts[p0 + half] <= x) {
                                 p0 += half + 1u;
                                 m -= half + 1u;
                             } else {
@@ -691,76 +720,120 @@ __global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, Tr
                 }
                 if (mine) {
                     q_s[rank] = s;
-                    q_slot[rank] = k0 + t;
+                    q_top[rank] = top;
+                    q_left[rank] = left;
+                    q_acc[rank] = acc;
+                    q_room[rank] = room;
+                    q_bound[rank] = cur + 1u;
                     q_p0[rank] = p0;
-                    q_j[rank] = lv.lrank[min(p0, cur + 1u)];
+                    q_j[rank] = (!MULTI && lv.len > 0) ? lv.lrank[min(p0, cur + 1u)] : 0u;
+                    q_cur[rank] = cur;
+                    if (MULTI) q_set[rank] = set;
                 }
                 if (lane == 0) s_n = (uint32_t)__popcll(all);
             }
             __syncthreads();
             const uint32_t n = uniform(s_n);
+            h = uniform(s_work);
             const bool in = (uint32_t)lane < n;
-            const uint32_t J = in ? q_j[lane] : 0u;
+            const uint32_t J = in ? q_j[lane] : 0u, C1 = in ? q_cur[lane] + 1u : 0u, G = (MULTI && in) ? q_set[lane] : 0u;
             const S sl = in ? q_s[lane] : SMIN;
             for (uint32_t g = 0, cnt = 0; g < n; g += cnt) {
-                // the next queries that share a list
-                const uint32_t Jg = read_lane(J, g);
+                // the next queries that share a list: of all positions below them, or of the long entries
+                const uint32_t Jg = read_lane(J, g), Cg = read_lane(C1, g), set = read_lane(G, g);
                 const S smin = read_lane(sl, g);
-                const uint64_t fit = __builtin_amdgcn_ballot_w64(in && J - Jg + SH_SPREAD <= 2u * SH_SPREAD &&
-                                                                 (uint64_t)sl - (uint64_t)smin < 0xFFFFFFFFull);
-                const uint64_t out_of = ~(fit >> g);
-                cnt = out_of ? (uint32_t)__builtin_ctzll(out_of) : (uint32_t)WAVE;
+                const bool same = in && G == set && (uint64_t)sl - (uint64_t)smin < 0xFFFFFFFFull;
+                auto prefix = [&](bool fit) {
+                    const uint64_t out_of = ~(__builtin_amdgcn_ballot_w64(fit) >> g);
+                    return out_of ? (uint32_t)__builtin_ctzll(out_of) : (uint32_t)WAVE;
+                };
+                const uint32_t all = prefix(same && C1 - Cg + SH_NEAR <= 2u * SH_NEAR);
+                const uint32_t far = (!MULTI && lv.len > 0) ? prefix(same && J - Jg + SH_SPREAD <= 2u * SH_SPREAD) : 0u;
+                const bool near = all >= far;
+                cnt = near ? all : far;
                 const bool share = cnt >= SH_LEAST;
-                // their hits at and above s - len, from the index
-                for (uint32_t i = g; i < g + cnt; ++i) {
+                const IndexView<S>& ix = [&]() -> const IndexView<S>& { if constexpr (MULTI) return sets[set].v; else return ix_one; }();
+                const TreeDesc<S>& td = [&]() -> const TreeDesc<S>& { if constexpr (MULTI) return sets[set].td; else return td_one; }();
+                const UbTree<S>& ub = [&]() -> const UbTree<S>& { if constexpr (MULTI) return sets[set].ub; else return ub_one; }();
+                // without a list of all positions, their hits at and above s - len from the index; in vector
+                // order the leading run; alone, everything
+                for (uint32_t i = g; (!share || !near || MODE == W_VECTOR) && i < g + cnt; ++i) {
                     if (i % SH_WAVES != wv) continue;
-                    const HeavyEntry he = pv.heavy[uniform(q_slot[i])];
-                    const uint32_t q = uniform(pv.q[uniform(he.k)]);
                     const S s = read_lane(sl, i);
-                    uint32_t cur = uniform(he.cur), left = uniform(he.left);
-                    const uint32_t top = uniform(he.top);
-                    uint64_t acc = read_lane(he.acc, 0);
-                    const uint64_t oend = max(min(offsets[q + 1], cap), acc);
+                    uint32_t cur = uniform(q_cur[i]), left = uniform(q_left[i]), bound = 0;
+                    const uint32_t top = uniform(q_top[i]);
+                    uint64_t acc = read_lane(q_acc[i], 0);
+                    const uint64_t oend = acc + uniform(q_room[i]);
                     if (!share) {
                         wave_walk<S, MODE>(ix, td, ub, lv, lane, s, cur, top, MODE == W_VECTOR, acc, oend, left, out_idx,
                                            vals, out_val);
                         if (left != 0u) atomicOr(&pv.counter[3], 1u);
                         continue;
                     }
-                    const uint32_t p0 = uniform(q_p0[i]);
-                    uint32_t bound = 0;
                     if (MODE == W_VECTOR) wave_lead(ix, lane, s, cur, top, acc, oend, left, out_idx);
                     if (cur != NONE) {
-                        wave_near<S, MODE>(ix, td, lane, s, cur, p0, acc, oend, left, out_idx, vals, out_val);
-                        bound = min(p0, cur + 1u);
+                        bound = cur + 1u;
+                        if (!near) {
+                            const uint32_t p0 = uniform(q_p0[i]);
+                            wave_near<S, MODE>(ix, td, lane, s, cur, p0, acc, oend, left, out_idx, vals, out_val);
+                            bound = min(p0, bound);
+                        }
                     }
                     q_acc[i] = acc;
                     q_left[i] = left;
-                    q_room[i] = (uint32_t)min(oend - acc, (uint64_t)0xFFFFFFFFu);
+                    q_room[i] = (uint32_t)(oend - acc);
                     q_bound[i] = bound;   // (every lane stores the same values)
                 }
                 if (!share) continue;
-                // ---- the long entries below the group's bounds that reach its first start, highest first
-                const uint32_t jmax = uniform(wave_max((uint32_t)lane >= g && (uint32_t)lane < g + cnt ? J : 0u));
-                bool more = jmax != 0u;
-                uint32_t g1 = 0, par = 0;
+                // ---- the positions from p0 on (near), then the long entries below the group's bounds, that
+                // reach its first start, highest first
+                const bool mine = (uint32_t)lane >= g && (uint32_t)lane < g + cnt;
+                const uint32_t p0 = near ? uniform(q_p0[g]) : 0u;
+                const uint32_t phi = near ? uniform(wave_max(mine ? C1 : 0u)) : 0u;
+                uint32_t jmax = 0;
+                if (!MULTI && lv.len > 0) jmax = near ? uniform(lv.lrank[p0]) : uniform(wave_max(mine ? J : 0u));
+                uint32_t g1 = 0, par = 0, lo = 0, hi = 0;   // the source's entries [lo, hi) are looked at
                 uint64_t rem = 0;
-                if (more) {
-                    const uint32_t hi_line = (jmax - 1u) >> 6;
+                int source = near ? 0 : 1;                  // 0: the index, 1: the long list
+                auto lines_of = [&](uint32_t group) -> uint64_t {
+                    if (source == 0) return td.nlev >= 2 ? group_mask(td, group, smin, lane) : 1ull;
+                    return lv.td.nlev >= 2 ? group_mask(lv.td, group, smin, lane) : 1ull;
+                };
+                auto in_range = [&](uint64_t m, uint32_t group) {   // lines from lo's on
+                    const uint32_t l = lo >> 6;
+                    return l > group ? (l - group > 63u ? 0ull : m & (~0ull << (l - group))) : m;
+                };
+                auto open = [&]() {   // the source's last group of lines; false: it holds nothing
+                    lo = source == 0 ? p0 : 0u;
+                    hi = source == 0 ? phi : jmax;
+                    rem = 0;
+                    if (hi <= lo) return false;
+                    const uint32_t hi_line = (hi - 1u) >> 6;
                     g1 = hi_line & ~63u;
-                    rem = lv.td.nlev >= 2 ? group_mask(lv.td, g1, smin, lane) & mask_upto(hi_line - g1) : 1ull;
+                    rem = in_range(lines_of(g1) & mask_upto(hi_line - g1), g1);
+                    return true;
+                };
+                bool more = open();
+                if (!more && source == 0) {
+                    source = 1;
+                    more = open();
                 }
                 while (more) {
                     uint32_t C = 0;
                     while (C + ROUND <= CAP) {
                         if (rem == 0) {
-                            const uint32_t l = g1 ? prev_line(lv.td, g1, 0u, smin, lane) : NONE;
-                            if (l == NONE) {
-                                more = false;
-                                break;
+                            uint32_t l = NONE;
+                            if (g1 > (lo >> 6))
+                                l = source == 0 ? prev_line(td, g1, lo >> 6, smin, lane) : prev_line(lv.td, g1, 0u, smin, lane);
+                            if (l != NONE) {
+                                g1 = l & ~63u;
+                                rem = in_range(lines_of(g1) & mask_upto(l - g1), g1);
+                                continue;
                             }
-                            g1 = l & ~63u;
-                            rem = group_mask(lv.td, g1, smin, lane) & mask_upto(l - g1);
+                            more = source == 0;
+                            source = 1;
+                            if (more) more = open();
+                            if (!more) break;
                             continue;
                         }
                         uint32_t e32[LINES], pos[LINES], line[LINES];
@@ -782,18 +855,25 @@ __global__ __launch_bounds__(SH_THREADS) void k_sweep_shared(IndexView<S> ix, Tr
 #pragma unroll
                         for (uint32_t j = 0; j < LINES; ++j) {
                             const uint32_t p = line[j] * 64u + 63u - (uint32_t)lane;
-                            if (sizeof(S) == 8 && lv.ends32) e32[j] = lv.ends32[p];
-                            else ev[j] = lv.ends[p];
-                            pos[j] = lv.pos[p];
+                            if (source == 0) {
+                                if (sizeof(S) == 8 && ix.ends32) e32[j] = ix.ends32[p];
+                                else ev[j] = ix.ends[p];
+                                pos[j] = p;
+                            } else {
+                                if (sizeof(S) == 8 && lv.ends32) e32[j] = lv.ends32[p];
+                                else ev[j] = lv.ends[p];
+                                pos[j] = lv.pos[p];
+                            }
                         }
+                        const bool by32 = sizeof(S) == 8 && (source == 0 ? ix.ends32 : lv.ends32) != nullptr;
+                        const int64_t base32 = source == 0 ? ix.ends32_base : lv.ends32_base;
                         uint32_t rel[LINES], tot = 0;
                         uint64_t m[LINES];
 #pragma unroll
                         for (uint32_t j = 0; j < LINES; ++j) {
                             const uint32_t p = line[j] * 64u + 63u - (uint32_t)lane;
-                            const int64_t e = (sizeof(S) == 8 && lv.ends32) ? (int64_t)((uint64_t)lv.ends32_base + e32[j])
-                                                                            : (int64_t)ev[j];
-                            const bool hit = j < nl && p < jmax && e >= (int64_t)smin;
+                            const int64_t e = by32 ? (int64_t)((uint64_t)base32 + e32[j]) : (int64_t)ev[j];
+                            const bool hit = j < nl && p >= lo && p < hi && e >= (int64_t)smin;
                             rel[j] = (uint32_t)min((uint64_t)e - (uint64_t)(int64_t)smin, (uint64_t)0xFFFFFFFFu);
                             m[j] = __builtin_amdgcn_ballot_w64(hit);
                             tot += (uint32_t)__popcll(m[j]);

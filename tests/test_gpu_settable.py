@@ -203,3 +203,33 @@ def test_set_table_sweep(sia, orc, nsets, nq):
     table.close()
     for ix in idxs:
         ix.close()
+
+
+@pytest.mark.parametrize("nsets,nq", [(1, 5), (2, 3000), (40, 3000), (7, 60_001)])
+def test_set_table_held_by_many(sia, orc, nsets, nq):
+    """Queries that hundreds of intervals of their set hold share candidate lists, set by set: spans
+    that hold one set's queries and several sets', sets that fit one line and sets that do not,
+    inverted queries among them, both orders."""
+    print(f"[gpu] set table held by many nsets={nsets} nq={nq}", flush=True)
+    rng = np.random.default_rng(nsets * nq)
+    table = sia.SetTable(nsets)
+    idxs, oixs = [], [None] * nsets
+    for g in range(nsets):
+        n = int(rng.integers(1, 60)) if g % 5 == 3 else int(rng.integers(2000, 6000))
+        s = rng.integers(0, n, n).astype(np.int32)
+        e = (s + rng.integers(0, n // 2 + 2, n)).astype(np.int32)
+        idxs.append(sia.DeviceIndex(np.int32).build(s, e))
+        table.put(g, idxs[-1])
+        oixs[g] = orc.build_index(s, e)
+    sid = rng.integers(0, nsets, nq).astype(np.uint32)
+    qs = rng.integers(-5, 7000, nq)
+    qe = qs + rng.integers(-3, 60, nq)
+    qs, qe = qs.astype(np.int32), qe.astype(np.int32)
+    for order, mode in (("desc", 0), ("vector", 1)):
+        off, idx = table.search(sid, qs, qe, order=order)
+        woff, widx = _expect(orc, oixs, sid, qs, qe, mode)
+        assert np.array_equal(off, woff), order
+        assert np.array_equal(idx.astype(np.int64), widx), order
+    table.close()
+    for ix in idxs:
+        ix.close()
