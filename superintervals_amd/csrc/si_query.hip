@@ -1364,7 +1364,8 @@ static_assert(HEAVY_CHUNKS >= 1 && HEAVY_CHUNKS <= 8, "the plan holds 8 chunk co
 // w / HEAVY_CHUNKS, takes what is left of it by the counter ctr[chunk], and once it is used up looks
 // at all counters with one load and goes on with a chunk that has entries left.  (With an atomic for
 // every entry and every chunk found empty, up to 9 a worker on one cache line, 8192 waves took 0.8 ms
-// whatever the batch.)  Called by whole waves.
+// whatever the batch; with the load before every entry 20M entries took 1.46 s in place of 0.28.)
+// Called by whole waves.
 struct EntryDeal {
     uint32_t* __restrict__ ctr;
     uint32_t n, per, fixed;   // entries, of a chunk, and of these dealt without the counter
@@ -1387,20 +1388,18 @@ struct EntryDeal {
         }
         if (per <= fixed) return NONE;   // all dealt
         while (true) {
+            uint32_t h = 0;
+            if (lane == 0) h = atomicAdd(&ctr[c], 1u);
+            h = fixed + (uint32_t)__builtin_amdgcn_readfirstlane((int)h);
+            if (h < size(c)) return c * per + h;
             bool open = false;
             if ((uint32_t)lane < HEAVY_CHUNKS)
                 open = fixed + __hip_atomic_load(&ctr[lane], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) <
                        size((uint32_t)lane);
             const uint64_t m = __builtin_amdgcn_ballot_w64(open);
             if (m == 0) return NONE;
-            if (!((m >> c) & 1ull)) {
-                const uint64_t after = m & ~mask_upto(c);
-                c = (uint32_t)__builtin_ctzll(after ? after : m);
-            }
-            uint32_t h = 0;
-            if (lane == 0) h = atomicAdd(&ctr[c], 1u);
-            h = fixed + (uint32_t)__builtin_amdgcn_readfirstlane((int)h);
-            if (h < size(c)) return c * per + h;
+            const uint64_t after = m & ~mask_upto(c);
+            c = (uint32_t)__builtin_ctzll(after ? after : m);
         }
     }
 };
