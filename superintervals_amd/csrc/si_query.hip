@@ -58,7 +58,8 @@ struct HeavyEntry;
 
 template <typename S>
 struct PlanView {
-    uint32_t* counter;   // [0] tiles taken, [1] heavy entries written, [3] set by a fill pass
+    uint32_t* counter;   // [0] tiles taken, [1] heavy entries written (by the sweep: 1 when there
+                         // are any), [3] set by a fill pass
                          // when a query's hits differ from its offsets, [4] 1 when the plan
                          // holds lower_bound positions (lb), [5] 1 when it holds the counts
                          // (cnt), [8 + c] entries taken from chunk c of the heavy list
@@ -79,7 +80,8 @@ struct PlanView {
 // A query whose walk exceeds the per-lane step budget, parked for the wave-cooperative
 // kernel: sorted position, current position, leading-run top and phase, the count so far
 // (count mode) or the next output offset (fill modes), and in fill modes the hits still
-// expected by the query's offsets.
+// expected by the query's offsets.  The sweep writes a chunk's entries from its first query's
+// place on, and their number into the pad at that place.
 struct HeavyEntry {
     uint32_t k;
     uint32_t cur;
@@ -3347,7 +3349,9 @@ SI_EXPORT int siSetTableSearchOffsets(const siSetTable* t, const uint32_t* set_i
     }
     if (rc) return rc;
     PlanView<int32_t> pv = multi_view(plan, nq, t->nslots);
-    uint32_t* c32 = counts ? counts : (uint32_t*)(p + L.base.off_heavy);
+    // (the plan keeps no counts: their place serves the scan.  Not the heavy list's, which the
+    // sorted keys lie in after an even number of passes.)
+    uint32_t* c32 = counts ? counts : pv.cnt;
     k_multi_finish<<<grid_for(nq, Q_THREADS), Q_THREADS, 0, st>>>((const SetView<int32_t>*)t->d_views, ks, vs,
                                                                  (const int32_t*)qs, nq, pv, c32);
     LAUNCH_CHECK();

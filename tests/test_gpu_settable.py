@@ -233,3 +233,35 @@ def test_set_table_held_by_many(sia, orc, nsets, nq):
     table.close()
     for ix in idxs:
         ix.close()
+
+
+@pytest.mark.parametrize("nsets", [3, 300])
+def test_set_table_counts_beside_sorted_keys(sia, orc, nsets):
+    """Offsets without a counts buffer for a batch of more blocks than the GPU holds at once, with an
+    even and an odd number of sort passes: the counts must not be written over sorted keys that
+    later blocks still read."""
+    import torch
+    print(f"[gpu] set table counts beside keys nsets={nsets}", flush=True)
+    rng = np.random.default_rng(nsets)
+    nq = 3_000_000
+    table = sia.SetTable(nsets)
+    idxs, want = [], np.zeros(nq, np.int64)
+    sid = rng.integers(0, nsets + 1, nq).astype(np.uint32)
+    qs = rng.integers(0, 4000, nq).astype(np.int32)
+    qe = (qs + rng.integers(0, 20, nq)).astype(np.int32)
+    for g in range(nsets):
+        s = rng.integers(0, 4000, 50).astype(np.int32)
+        e = (s + rng.integers(0, 30, 50)).astype(np.int32)
+        idxs.append(sia.DeviceIndex(np.int32).build(s, e))
+        table.put(g, idxs[-1])
+        sel = np.flatnonzero(sid == g)
+        want[sel] = orc.count_batch(orc.build_index(s, e), qs[sel], qe[sel])
+    d = [torch.from_numpy(x).cuda() for x in (sid.view(np.int32), qs, qe)]
+    plan = torch.empty(table.plan_bytes(nq), dtype=torch.uint8, device="cuda")
+    off = torch.empty(nq + 1, dtype=torch.int64, device="cuda")
+    table.offsets_device(*d, plan, off)
+    torch.cuda.synchronize()
+    assert np.array_equal(off.cpu().numpy(), np.concatenate([[0], np.cumsum(want)]))
+    table.close()
+    for ix in idxs:
+        ix.close()
