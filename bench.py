@@ -581,7 +581,7 @@ def bench_skewed(a):
     # launches, when the summary of a PMC run is committed
     alg = 4 * tot + (2 * 8 + 4 + 8 + 8) * nq
     ach = alg / (t_fill / 1e3) / 1e9
-    roof = {"bound": "hbm", "kernel": "k_walk<long, desc fill> + k_walk_heavy<long, desc fill> (streamed fill)",
+    roof = {"bound": "hbm", "kernel": "k_sweep<long, desc fill> + k_sweep_shared<long, desc fill> (streamed fill)",
             "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
             "traffic": None,
             "basis": "achieved = (4 B per position written + 36 B of plan entry, offsets and query per query) / "
@@ -971,13 +971,13 @@ def main():
     dom = max(("plan", t_plan), ("search_offsets", t_off), ("search_fill", t_fill), key=lambda x: x[1])[0]
     ach = b_fill / t_fill / 1e6
     tr = load_traffic()
-    roof = {"bound": "hbm", "kernel": "k_walk<int, desc fill> (search_idxs fill pass, one launch over all queries)",
+    roof = {"bound": "hbm", "kernel": "k_sweep<int, desc fill> (search_idxs fill pass, one launch over all queries)",
             "achieved": round(ach, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(ach / HBM_PEAK_GBS, 4),
             "traffic": tr["fill"]["bytes_per_launch"] if tr else None,
             "basis": "achieved = algorithmic bytes per launch (per query: 12 B plan entry + c*V ends + 4*J "
                      "branch reads of the reference walk + 4*h positions + 8 B offset) / launch time; the "
-                     "walk serves most ends reads from its LDS window, so the counter-measured HBM traffic "
+                     "sweep reads a line of ends once for a wave's queries, so the counter-measured HBM traffic "
                      "(traffic, measured_GBps) is below the algorithmic bytes"}
     if tr:
         roof["measured_GBps"] = round(tr["fill"]["bytes_per_launch"] / t_fill / 1e6, 1)

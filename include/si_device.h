@@ -130,9 +130,10 @@ double siIndexLastBuildMs(const siIndex* ix);
  *                  count descend 64-ary trees of first keys (top level of at most 4096
  *                  keys in Eytzinger order in LDS, then one 64-key node per level) over
  *                  the starts / the sorted ends; 0: plain halving
- *   "plan_sync"    1 (default): siPlanQueries reads back once which key bits vary to
- *                  skip constant digits (one stream synchronisation); 0: it sorts every
- *                  digit without a read-back, so the planned calls can be graph-captured
+ *   "plan_sync"    1 (default): siPlanQueries of a large batch (more than 8192 int64
+ *                  queries, or 4M int32 ones) reads back once which key bits vary to skip
+ *                  constant digits (one stream synchronisation); 0: it sorts every digit
+ *                  without a read-back, so the planned calls can be graph-captured
  *   "heavy_ends32" 1 (default): the wave-cooperative walk of an int64 index whose ends
  *                  span less than 2^32 reads a 32-bit copy of them (8 B per position with
  *                  exitp instead of 12); 0: the int64 ends

@@ -630,7 +630,7 @@ __global__ __launch_bounds__(SH_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     constexpr S SMIN = (sizeof(S) == 4) ? (S)INT32_MIN : (S)INT64_MIN;
     constexpr bool VALUES = MODE == W_VALUES;
     constexpr uint32_t CAP = sh_cap(MODE);            // candidates held at a time
-    constexpr uint32_t LINES = VALUES ? 4 : 8;        // lines a wave collects at a time
+    constexpr uint32_t LINES = (VALUES || sizeof(S) == 8) ? 4 : 8;   // lines a wave collects at a time (registers)
     constexpr uint32_t ROUND = SH_WAVES * LINES * 64u;   // most that one round of lines adds
     constexpr uint32_t UNROLL = 4;
     __shared__ uint32_t c_rel[CAP + UNROLL * WAVE], c_pos[CAP + UNROLL * WAVE], c_val[VALUES ? CAP + UNROLL * WAVE : 1];
