@@ -604,7 +604,7 @@ def bench_skewed(a):
            "plan_ms": t_plan, "count_walk_ms": t_walk, "count_walk_int64_ends_ms": t_walk64,
            "count_rank_ms": t_rank, "count_identical": same, "count_call_ms": t_call,
            "count_note": "plan_ms: sort by end, bounds and rank-form counts of all queries (warm); count_rank_ms: "
-                         "the scatter of the plan's counts; count_call_ms: count() from the queries (plan + scatter); "
+                         "the scatter of the plan's counts; count_call_ms: count() from the queries (grouping + table searches); "
                          "count_walk_ms: the walk form on the planned batch",
            "hits": hits, "queries_over_1e5_hits": wide,
            "lane_steps_sweep_ms": {str(k): v for k, v in sweep.items()}, "lane_steps": best_ls,
@@ -961,7 +961,7 @@ def main():
         "count": {"ms": t_count, "alg_bytes": b_count_walk, "GBps": b_count_walk / t_count / 1e6},
         "count_rank": {"ms": t_count_rank, "queries_per_s": nq / (t_count_rank / 1e3)},
         "count_call": {"ms": t_count_call, "queries_per_s": nq / (t_count_call / 1e3),
-                       "note": "count() from the queries, the whole call: plan (sort, bounds, rank counts) + scatter"},
+                       "note": "count() from the queries, the whole call: the queries grouped by their ends, then two table searches each"},
         "plan": {"ms": t_plan},
         "search_offsets": {"ms": t_off},
         "search_fill": {"ms": t_fill, "alg_bytes": b_fill, "GBps": b_fill / t_fill / 1e6},

@@ -606,7 +606,7 @@ __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<
 // without the lists' stores 0.64, without the scan 0.48, without lists 0.33, without the index's
 // positions too 0.21.  2000 queries on 20M: 0.13 ms (0.80).  1M queries that 320 of 10M intervals
 // hold, none long: fill 0.83 ms (lane walk 1.06, a walk for each query 2.0); 50M on 200M intervals,
-// two fifths of them held by 330: 32 ms (52; 76).  CAP 6144 (12 waves a CU) and 8 waves a workgroup
+// two fifths of them held by 330: 26 ms (52; 76).  CAP 6144 (12 waves a CU) and 8 waves a workgroup
 // were slower by 20 and 10 %, CAP 2048 by 10 %, but with payloads, which take another word of LDS
 // an entry, faster by 15 %.  SH_SPREAD 512: 1.30 ms for the first fill, 1024: 1.10, 2048 and 4096:
 // 1.00.  SH_NEAR 1024 and 4096: the same.  Spans of 64: 0.95 for the first, 0.12 against 0.21 for
