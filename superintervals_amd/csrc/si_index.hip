@@ -229,7 +229,12 @@ template <typename S>
 __global__ __launch_bounds__(256) void k_add_flags(const S* __restrict__ s, const S* __restrict__ e, size_t n,
                                                    unsigned long long* __restrict__ out) {
     const size_t base = (size_t)blockIdx.x * (256 * FLAG_ITEMS);
-    if (__hip_atomic_load(&out[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < base) return;
+    // (one thread reads out[0], which other workgroups lower meanwhile: all waves leave, or none)
+    __shared__ unsigned long long s_m[3];
+    if (threadIdx.x < 2) s_m[threadIdx.x] = ~0ull;
+    else if (threadIdx.x == 2) s_m[2] = __hip_atomic_load(&out[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_m[2] < base) return;
     unsigned long long bad = ~0ull, tie = ~0ull;
 #pragma unroll
     for (int k = FLAG_ITEMS - 1; k >= 0; --k) {
@@ -241,9 +246,6 @@ __global__ __launch_bounds__(256) void k_add_flags(const S* __restrict__ s, cons
         }
     }
     // one pair of atomics a block, and only when it has found something earlier
-    __shared__ unsigned long long s_m[2];
-    if (threadIdx.x < 2) s_m[threadIdx.x] = ~0ull;
-    __syncthreads();
     if (bad != ~0ull) atomicMin(&s_m[0], bad);
     if (tie != ~0ull) atomicMin(&s_m[1], tie);
     __syncthreads();

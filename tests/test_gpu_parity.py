@@ -1245,6 +1245,33 @@ def test_build_finds_add_flags(sia, orc, dtype, n):
     ref.close()
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("first", [0, 2046, 2047, 2048, 100_000])
+def test_build_flags_with_breaks_everywhere(sia, orc, dtype, first):
+    """Flags found while many workgroups report breaks and others leave because of them: sorted up
+    to the first break, then in random order (every workgroup from there on holds breaks and rising
+    ties), with a rising tie before the break or none; arrays as the oracle builds them."""
+    print(f"[gpu] add flags, breaks from {first} dtype={np.dtype(dtype).name}", flush=True)
+    rng = np.random.default_rng(first)
+    n = 1_000_000
+    s = rng.integers(0, n // 4, n)
+    e = s + rng.integers(0, 60, n)
+    o = np.lexsort((-e[:first + 1], s[:first + 1]))
+    s[:first + 1], e[:first + 1] = s[:first + 1][o], e[:first + 1][o]
+    s[first + 1] = s[first] - 1
+    s, e = s.astype(dtype), e.astype(dtype)
+    ix = sia.DeviceIndex(dtype)
+    for tie in (False, True):
+        if tie and first > 1:
+            s[1], e[1] = s[0], e[0] + 1
+        got = ix.build(s, e).download()
+        want = orc.build_index(s, e, np.arange(n, dtype=np.int32))
+        for key in ("starts", "ends", "branch"):
+            assert np.array_equal(got[key], want[key]), (tie, key)
+        assert np.array_equal(got["perm"], want["data"]), tie
+    ix.close()
+
+
 def _end_sorted(s, e):
     """add()'s end flag by comparisons (add_flags subtracts, which wraps at the int64 limits)."""
     for k in range(s.size - 1):
