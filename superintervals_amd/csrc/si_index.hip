@@ -359,7 +359,7 @@ struct BuildInfo {
     uint32_t long_run;             // 1: a run of equal starts longer than TIE_RUN was left as it was
     uint32_t crowded[2];           // sampled keys in crowded buckets of the starts' and the sorted ends' tables
     uint32_t gaps[2];              // long gaps of the two tables (BucketGap)
-    uint32_t pad;
+    uint32_t unsorted;             // 1: a start is below the one before it
     long long start_lo, start_hi;  // smallest and largest start
 };
 
@@ -491,7 +491,8 @@ __device__ __forceinline__ uint32_t last_ge(const Max16<S>& t, uint32_t u, S x) 
 // lie further left the larger they are, so the lane finds them in one sweep leftwards through
 // the max tree, 16 entries a step.  10M int32 intervals: 0.095 ms, where a lane per position
 // scanning its 64-group and climbing entry by entry took 0.36 ms (and exitp another 0.08).
-// Also counts the intervals with start > end.
+// Also counts the intervals with start > end, and says whether the starts are in order (a caller's
+// promise that they are may be wrong).
 template <typename S>
 __global__ __launch_bounds__(256) void k_branch_exit(Max16<S> t, const S* __restrict__ starts, uint32_t n, uint32_t ngroups,
                                                      uint32_t* __restrict__ branch, uint32_t* __restrict__ ex,
@@ -548,6 +549,10 @@ __global__ __launch_bounds__(256) void k_branch_exit(Max16<S> t, const S* __rest
 #pragma unroll
     for (int k = 0; k < 16; ++k) inv += (st[k] > v[k] && i0 + (uint32_t)k < n) ? 1u : 0u;
     if (inv) atomicAdd(&info->inverted, (unsigned long long)inv);
+    bool falls = g + 1u < ngroups && starts[i0 + 16u] < st[15];   // (padded with the maximum)
+#pragma unroll
+    for (int k = 1; k < 16; ++k) falls |= st[k] < st[k - 1];
+    if (falls) info->unsorted = 1u;
 }
 
 // Sums of 16 consecutive entries of a and of b (lines of n / 16 + 1 each, the last one partial;
@@ -1130,7 +1135,7 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     if (rc == SI_OK) rc = build_key_tree<S>((const S*)ix->d_starts, shape, ix->ub, st);        // upper_bound
     if (rc == SI_OK) rc = build_key_tree<S>((const S*)ix->d_ends_sorted, shape, ix->eb, st);   // rank count
     if (rc != SI_OK) return rc;
-    {
+    if (!back.info.unsorted) {   // (else a key may lie in no bucket: the searches go through the trees)
         Carver m;
         m.base = (char*)scratch.p;
         m.used = shared_from;
@@ -1181,7 +1186,7 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     // 64-ary tree 14 (n > 4095 x 64): the tables are used unless half of the keys share a bucket
     // with more than 4096 others.
     const uint32_t half = (uint32_t)(n / CROWD_STEP / 2);
-    ix->ubt.ok = ix->ebt.ok = back.info.crowded[0] <= half && back.info.crowded[1] <= half;
+    ix->ubt.ok = ix->ebt.ok = !back.info.unsorted && back.info.crowded[0] <= half && back.info.crowded[1] <= half;
     ix->built = true;
     ix->last_build_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -1272,6 +1272,48 @@ def test_build_flags_with_breaks_everywhere(sia, orc, dtype, first):
     ix.close()
 
 
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n", [17, 1000, 70_001])
+def test_build_with_a_wrong_promise(sia, dtype, n):
+    """A build told that unsorted starts are sorted stays within its arrays and keeps the order it
+    was given.  One start is out of place (larger than all, at the front, in the middle, or across
+    a group of 16), so that every search bound on one side of it is still well defined; count,
+    upper_bound, has_overlaps, coverage and both orders there equal a scan of the given arrays,
+    for one query and for a batch."""
+    print(f"[gpu] wrong promise dtype={np.dtype(dtype).name} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    for place in (0, 15, 16, n // 2):
+        s = np.sort(rng.integers(1000, 1000 + 8 * n, n))
+        e = s + rng.integers(0, 90, n)
+        high = 1000 + 9 * n
+        s[place], e[place] = high, high + 5
+        # searches by a value x agree on the order where all keys <= x precede the others
+        lo, hi = (high, high + 200) if place == 0 else (900, s[place - 1])
+        qs = rng.integers(lo + 1, hi + 1, 40)
+        qe = np.minimum(qs + rng.integers(0, 60, 40), hi)
+        s, e, qs, qe = (x.astype(dtype) for x in (s, e, qs, qe))
+        ix = sia.DeviceIndex(dtype).build(s, e, None, start_sorted=True, end_sorted=True)
+        got = ix.download()
+        assert np.array_equal(got["starts"], s) and np.array_equal(got["ends"], e)
+        hits = [np.flatnonzero((s <= b) & (e >= a))[::-1] for a, b in zip(qs, qe)]
+        ub = np.array([np.flatnonzero(s <= b).max(initial=-1) for b in qe])
+        one = [(slice(k, k + 1), hits[k:k + 1]) for k in range(5)]
+        for at, want in [(slice(0, 40), hits)] + one:
+            a, b = qs[at], qe[at]
+            assert np.array_equal(ix.count(a, b), [len(h) for h in want])
+            assert np.array_equal(ix.upper_bound(b).view(np.int32), ub[at])
+            any_ = (ub[at] >= 0) & (e[np.maximum(ub[at], 0)] >= a)
+            assert np.array_equal(ix.has_overlaps(a, b), any_)
+            off, idx = ix.search(a, b)
+            assert np.array_equal(off, np.concatenate([[0], np.cumsum([len(h) for h in want])]))
+            assert np.array_equal(idx.astype(np.int64), np.concatenate(want))
+            if dtype == np.int32:
+                c, v = ix.coverage(a, b)
+                cov = [int((np.minimum(e[h], y) - np.maximum(s[h], x)).sum()) for h, x, y in zip(want, a, b)]
+                assert np.array_equal(c, [len(h) for h in want]) and np.array_equal(v, cov)
+        ix.close()
+
+
 def _end_sorted(s, e):
     """add()'s end flag by comparisons (add_flags subtracts, which wraps at the int64 limits)."""
     for k in range(s.size - 1):
