@@ -97,6 +97,25 @@ struct OneQuery {
     int last_mode = -1;
     int64_t last_s = 0, last_e = 0;
     uint64_t last_total = 0;
+    // Makes the scratch for `results` results when it is not there: all of it or, on an error, nothing
+    // (the next call tries again).
+    int make(uint64_t results) {
+        if (cap) return SI_OK;
+        const char* what = "hipHostMalloc";
+        hipError_t e = hipHostMalloc(&h, 16 + results * 4, hipHostMallocMapped);
+        if (e != hipSuccess) h = nullptr;
+        if (e == hipSuccess) e = hipHostGetDevicePointer(&d, h, 0), what = "hipHostGetDevicePointer";
+        if (e == hipSuccess) e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking), what = "hipStreamCreateWithFlags";
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            release();
+            return si_set_error(SI_ERR_HIP, "single-query scratch: %s: %s", what, hipGetErrorString(e));
+        }
+        ((uint64_t*)h)[1] = 0;   // (may hold what an earlier index left there)
+        seq = 0;
+        cap = results;
+        return SI_OK;
+    }
     void release() {
         if (st) (void)hipStreamSynchronize(st);   // (a call ends before its kernel does)
         if (h) (void)hipHostFree(h);

@@ -3582,15 +3582,8 @@ constexpr uint64_t ONE_CAP = 1u << 16;   // results the single-query scratch hol
 template <typename S>
 int one_query_run(siIndex* ix, int mode, S s, S e, uint64_t* total) {
     OneQuery& o = ix->one;
-    if (!o.h) {
-        HIP_TRY(hipHostMalloc(&o.h, 16 + ONE_CAP * 4, hipHostMallocMapped));
-        ((uint64_t*)o.h)[1] = 0;   // (may hold what an earlier index left there)
-        o.seq = 0;
-        HIP_TRY(hipHostGetDevicePointer(&o.d, o.h, 0));
-        HIP_TRY(hipStreamCreateWithFlags(&o.st, hipStreamNonBlocking));
-        o.cap = ONE_CAP;
-        o.last_valid = false;
-    }
+    const int rc = o.make(ONE_CAP);
+    if (rc) return rc;
     if (o.last_valid && o.last_mode == mode && o.last_s == (int64_t)s && o.last_e == (int64_t)e) {
         *total = o.last_total;
         return SI_OK;
