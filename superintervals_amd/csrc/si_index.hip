@@ -50,9 +50,11 @@ struct KeptBlock {
     size_t bytes;
     int device;
 };
+constexpr size_t KEPT_BLOCKS = 64;
 struct Kept {
     std::mutex mu;
-    std::vector<KeptBlock> blocks;   // oldest first
+    std::vector<KeptBlock> blocks;   // oldest first, at most KEPT_BLOCKS (room for all of them from the start)
+    Kept() { blocks.reserve(KEPT_BLOCKS); }
     size_t bytes = 0;
     int users = 0;
     HostStage* stages[STAGE_KEEP] = {};
@@ -65,16 +67,16 @@ Kept& kept() {
 
 // Frees the kept blocks of one device (of all: -1).  The caller holds k.mu.
 void drop_kept(Kept& k, int device) {
-    std::vector<KeptBlock> rest;
+    size_t left = 0;
     for (const KeptBlock& b : k.blocks) {
         if (device >= 0 && b.device != device) {
-            rest.push_back(b);
+            k.blocks[left++] = b;
         } else {
             (void)hipFree(b.p);
             k.bytes -= b.bytes;
         }
     }
-    k.blocks.swap(rest);
+    k.blocks.resize(left);
 }
 }  // namespace
 
@@ -102,18 +104,39 @@ void* si_block_take(size_t bytes, size_t* got) {
         }
     }
     void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        std::lock_guard<std::mutex> lock(k.mu);
-        drop_kept(k, dev);
-        p = nullptr;
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            return nullptr;
-        }
-    }
+    if (si_malloc(&p, bytes) != hipSuccess) return nullptr;
     *got = bytes;
     return p;
+}
+
+namespace {
+template <class Alloc>
+hipError_t malloc_or_drop(void** p, bool may_drop, Alloc alloc) {
+    hipError_t e = alloc();
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    if (may_drop) {
+        Kept& k = kept();
+        std::lock_guard<std::mutex> lock(k.mu);
+        drop_kept(k, dev);
+    }
+    if (may_drop && (e = alloc()) == hipSuccess) return e;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return e;
+}
+}  // namespace
+
+hipError_t si_malloc(void** p, size_t bytes) {
+    return malloc_or_drop(p, true, [&] { return hipMalloc(p, bytes); });
+}
+
+hipError_t si_malloc_async(void** p, size_t bytes, hipStream_t st) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const bool free_stream = hipStreamIsCapturing(st, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+    return malloc_or_drop(p, free_stream, [&] { return hipMallocAsync(p, bytes, st); });
 }
 
 void si_block_give(void* p, size_t bytes, int device, bool quiet) {
@@ -123,7 +146,7 @@ void si_block_give(void* p, size_t bytes, int device, bool quiet) {
         (void)hipFree(p);
         return;
     }
-    while (k.bytes + bytes > BLOCK_KEEP || k.blocks.size() >= 64) {   // the oldest go first
+    while (k.bytes + bytes > BLOCK_KEEP || k.blocks.size() >= KEPT_BLOCKS) {   // the oldest go first
         (void)hipFree(k.blocks.front().p);
         k.bytes -= k.blocks.front().bytes;
         k.blocks.erase(k.blocks.begin());

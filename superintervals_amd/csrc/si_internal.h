@@ -22,6 +22,10 @@ constexpr size_t BLOCK_KEEP = (size_t)2 << 30;
 // A block of at least `bytes` bytes on the current device (null when there is no memory);
 // *got receives its size, to be given back with it.
 void* si_block_take(size_t bytes, size_t* got);
+// hipMalloc and hipMallocAsync; when there is no memory the current device's kept blocks are freed
+// and it is tried again (not while the stream is captured, where freeing would end the capture).
+hipError_t si_malloc(void** p, size_t bytes);
+hipError_t si_malloc_async(void** p, size_t bytes, hipStream_t st);
 // Gives a block back: with quiet, nothing on its device uses it any more; otherwise it is freed
 // (which waits).
 void si_block_give(void* p, size_t bytes, int device, bool quiet);

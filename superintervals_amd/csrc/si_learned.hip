@@ -548,10 +548,10 @@ int train_impl(siLearned* m, const siIndex* ix, int steps, uint32_t batch, float
     if (steps > 0) {
         const int nblocks = std::max(1, std::min<int>(256, (int)((batch + RMI_THREADS - 1) / RMI_THREADS)));
         float *d_part = nullptr, *d_grad = nullptr, *d_m = nullptr, *d_v = nullptr;
-        HIP_TRY(hipMalloc(&d_part, (size_t)nblocks * GRAD_SLOTS * 4));
-        HIP_TRY(hipMalloc(&d_grad, GRAD_SLOTS * 4));
-        HIP_TRY(hipMalloc(&d_m, NPARAM * 4));
-        HIP_TRY(hipMalloc(&d_v, NPARAM * 4));
+        HIP_TRY(si_malloc((void**)&d_part, (size_t)nblocks * GRAD_SLOTS * 4));
+        HIP_TRY(si_malloc((void**)&d_grad, GRAD_SLOTS * 4));
+        HIP_TRY(si_malloc((void**)&d_m, NPARAM * 4));
+        HIP_TRY(si_malloc((void**)&d_v, NPARAM * 4));
         HIP_TRY(hipMemsetAsync(d_m, 0, NPARAM * 4, st));
         HIP_TRY(hipMemsetAsync(d_v, 0, NPARAM * 4, st));
         const float b1 = 0.9f, b2 = 0.999f;
@@ -596,9 +596,9 @@ SI_EXPORT siLearned* siLearnedCreate(const siIndex* ix, uint32_t leaves) {
     const_cast<siIndex*>(ix)->models.push_back(m);
     m->ix_n = ix->n;
     m->generation = ix->generation;
-    if (hipMalloc(&m->d_params, NPARAM * 4) != hipSuccess ||
-        hipMalloc(&m->d_leaves, (size_t)m->L * sizeof(Leaf)) != hipSuccess ||
-        hipMalloc(&m->d_kb, (size_t)m->L * ix->cb) != hipSuccess) {
+    if (si_malloc((void**)&m->d_params, NPARAM * 4) != hipSuccess ||
+        si_malloc((void**)&m->d_leaves, (size_t)m->L * sizeof(Leaf)) != hipSuccess ||
+        si_malloc((void**)&m->d_kb, (size_t)m->L * ix->cb) != hipSuccess) {
         si_set_error(SI_ERR_NOMEM, "learned index allocation");
         siLearnedDestroy(m);
         return nullptr;
@@ -674,10 +674,10 @@ SI_EXPORT int siLearnedGradient(siLearned* m, const float* params, const uint32_
     float *d_p = nullptr, *d_part = nullptr, *d_grad = nullptr;
     uint32_t* d_pos = nullptr;
     const int nblocks = std::max(1, std::min<int>(256, (int)((count + RMI_THREADS - 1) / RMI_THREADS)));
-    HIP_TRY(hipMalloc(&d_p, NPARAM * 4));
-    HIP_TRY(hipMalloc(&d_pos, (size_t)count * 4));
-    HIP_TRY(hipMalloc(&d_part, (size_t)nblocks * GRAD_SLOTS * 4));
-    HIP_TRY(hipMalloc(&d_grad, GRAD_SLOTS * 4));
+    HIP_TRY(si_malloc((void**)&d_p, NPARAM * 4));
+    HIP_TRY(si_malloc((void**)&d_pos, (size_t)count * 4));
+    HIP_TRY(si_malloc((void**)&d_part, (size_t)nblocks * GRAD_SLOTS * 4));
+    HIP_TRY(si_malloc((void**)&d_grad, GRAD_SLOTS * 4));
     if (params) HIP_TRY(hipMemcpy(d_p, params, NPARAM * 4, hipMemcpyHostToDevice));
     else HIP_TRY(hipMemcpy(d_p, m->d_params, NPARAM * 4, hipMemcpyDeviceToDevice));
     HIP_TRY(hipMemcpy(d_pos, pos, (size_t)count * 4, hipMemcpyHostToDevice));

@@ -1959,8 +1959,9 @@ struct ScopedPlan {
     void* p = nullptr;
     hipStream_t st;
     explicit ScopedPlan(hipStream_t s) : st(s) {}
-    int alloc(size_t bytes) {
-        hipError_t e = hipMallocAsync(&p, bytes, st);
+    // needed: what the call cannot do without (the library's kept blocks make room for it)
+    int alloc(size_t bytes, bool needed = true) {
+        const hipError_t e = needed ? si_malloc_async(&p, bytes, st) : hipMallocAsync(&p, bytes, st);
         if (e != hipSuccess) { p = nullptr; return si_set_error(SI_ERR_NOMEM, "hipMallocAsync(%zu): %s", bytes, hipGetErrorString(e)); }
         return SI_OK;
     }
@@ -2037,7 +2038,7 @@ int launch_grouped(const siIndex* ix, const S* qs, const S* qe, size_t nq, bool 
     if (group) {   // (not in a captured stream, nor without memory for the copies)
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         group = nq < (size_t)0x7FFFFFFF && hipStreamIsCapturing(st, &capture) == hipSuccess &&
-                capture == hipStreamCaptureStatusNone && P.alloc(off_rs + rs_temp_bytes(nq)) == SI_OK;
+                capture == hipStreamCaptureStatusNone && P.alloc(off_rs + rs_temp_bytes(nq), false) == SI_OK;
         if (!group) (void)hipGetLastError();
     }
     if (!group) {
@@ -3276,7 +3277,7 @@ SI_EXPORT siSetTable* siSetTableCreate(int coord_bytes, uint32_t max_sets) {
     t->gens.assign(t->nslots, 0);
     const size_t bytes = (size_t)t->nslots * sizeof(SetView<int32_t>);
     std::vector<char> zero(bytes, 0);
-    if (hipMalloc(&t->d_views, bytes) != hipSuccess ||
+    if (si_malloc(&t->d_views, bytes) != hipSuccess ||
         hipMemcpy(t->d_views, zero.data(), bytes, hipMemcpyHostToDevice) != hipSuccess) {
         si_set_error(SI_ERR_NOMEM, "set table allocation");
         (void)hipFree(t->d_views);

@@ -67,15 +67,24 @@ def test_tuning_knobs_round_trip():
     assert autotune.current() == saved
 
 
-def test_single_query_scratch_is_made_whole_or_not_at_all(tmp_path):
-    """Each HIP call that makes the single-query scratch fails in turn: the call reports it, keeps
-    nothing, and a later call makes all of it (tests/cpp/test_one_query_scratch.cpp, which brings
-    its own HIP calls)."""
+def _run_host_program(name, tmp_path):
+    """Builds and runs a program of tests/cpp that brings its own HIP calls (no GPU)."""
     import subprocess
-    exe = str(tmp_path / "scratch")
+    exe = str(tmp_path / name)
     subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "-O1", "-std=c++17", "-Wno-unused-result",
                     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                     "-I", os.path.join(ROOT, "superintervals_amd", "csrc"),
-                    os.path.join(ROOT, "tests", "cpp", "test_one_query_scratch.cpp"), "-o", exe], check=True)
+                    os.path.join(ROOT, "tests", "cpp", name + ".cpp"), "-o", exe], check=True)
     out = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout + out.stderr
+
+
+def test_single_query_scratch_is_made_whole_or_not_at_all(tmp_path):
+    """Each HIP call that makes the single-query scratch fails in turn: the call reports it, keeps
+    nothing, and a later call makes all of it."""
+    _run_host_program("test_one_query_scratch", tmp_path)
+
+
+def test_kept_blocks(tmp_path):
+    """The device blocks kept between uses make room when an allocation finds no memory."""
+    _run_host_program("test_kept_blocks", tmp_path)
