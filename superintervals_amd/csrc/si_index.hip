@@ -80,18 +80,19 @@ void drop_kept(Kept& k, int device) {
 }
 }  // namespace
 
-void* si_block_take(size_t bytes, size_t* got) {
+void* si_block_take(size_t bytes, size_t* got, bool lasting) {
     bytes = (std::max<size_t>(bytes, 256) + 255) & ~(size_t)255;
     int dev = 0;
     (void)hipGetDevice(&dev);
+    const size_t most = lasting ? bytes + bytes / 8 + (64u << 10) : 2 * bytes + (1u << 20);
     Kept& k = kept();
     {
         std::lock_guard<std::mutex> lock(k.mu);
         size_t best = k.blocks.size();
         for (size_t i = 0; i < k.blocks.size(); ++i) {
             const KeptBlock& b = k.blocks[i];
-            // (a block more than twice the size is left for a request that needs it)
-            if (b.device == dev && b.bytes >= bytes && b.bytes <= 2 * bytes + (1u << 20) &&
+            // (a larger block is left for a request that needs it)
+            if (b.device == dev && b.bytes >= bytes && b.bytes <= most &&
                 (best == k.blocks.size() || b.bytes < k.blocks[best].bytes))
                 best = i;
         }
@@ -877,7 +878,7 @@ int build_long_list(siIndex* ix, std::vector<int64_t>& lens, Carver scratch, hip
     LongList& L = ix->lng;
     uint32_t* const flags = scratch.take<uint32_t>(n);
     uint32_t* const ws = scratch.take<uint32_t>(scan_ws_items(n));
-    if (!(L.d_lrank = (uint32_t*)si_block_take(((size_t)n + 1) * 4, &L.lrank_bytes)))
+    if (!(L.d_lrank = (uint32_t*)si_block_take(((size_t)n + 1) * 4, &L.lrank_bytes, true)))
         return si_set_error(SI_ERR_NOMEM, "long list: %zu bytes", ((size_t)n + 1) * 4);
     k_long_flags<S><<<grid_for(n, 256), 256, 0, st>>>(d_st, d_en, n, len, flags);
     LAUNCH_CHECK();
@@ -900,7 +901,7 @@ int build_long_list(siIndex* ix, std::vector<int64_t>& lens, Carver scratch, hip
         L.d_ends32 = ix->d_ends32 ? c.take<uint32_t>(npad) : nullptr;
         L.d_tree = c.take<S>(tot);
         if (pass == 0) {
-            if (!(L.d_block = si_block_take(c.used, &L.block_bytes)))
+            if (!(L.d_block = si_block_take(c.used, &L.block_bytes, true)))
                 return si_set_error(SI_ERR_NOMEM, "long list: %zu bytes", c.used);
             c.base = (char*)L.d_block;
         }
@@ -1015,7 +1016,7 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
         carve_key_tree<S>(shape, ix->ub, c);
         carve_key_tree<S>(shape, ix->eb, c);
         if (pass == 0) {
-            if (!(ix->d_block = si_block_take(c.used, &ix->block_bytes)))
+            if (!(ix->d_block = si_block_take(c.used, &ix->block_bytes, true)))
                 return si_set_error(SI_ERR_NOMEM, "index of %zu intervals: %zu bytes", n, c.used);
             c.base = (char*)ix->d_block;
         }
@@ -1187,7 +1188,7 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     // a third fewer bytes per position than ends + exitp at 8 + 4
     if constexpr (sizeof(S) == 8) {
         if ((uint64_t)back.info.end_hi - (uint64_t)back.info.end_lo < 0xFFFFFFFFull) {
-            if (!(ix->d_ends32 = (uint32_t*)si_block_take(npad * sizeof(uint32_t), &ix->ends32_bytes)))
+            if (!(ix->d_ends32 = (uint32_t*)si_block_take(npad * sizeof(uint32_t), &ix->ends32_bytes, true)))
                 return si_set_error(SI_ERR_NOMEM, "32-bit ends: %zu bytes", npad * sizeof(uint32_t));
             ix->ends32_base = back.info.end_lo;
             k_ends32<<<grid_for(npad, 256), 256, 0, st>>>((const int64_t*)ix->d_ends, n, npad, ix->ends32_base,

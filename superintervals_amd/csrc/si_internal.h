@@ -20,8 +20,9 @@ using namespace sik;
 // and only while an index exists; a block is handed out to one owner at a time, from any thread.
 constexpr size_t BLOCK_KEEP = (size_t)2 << 30;
 // A block of at least `bytes` bytes on the current device (null when there is no memory);
-// *got receives its size, to be given back with it.
-void* si_block_take(size_t bytes, size_t* got);
+// *got receives its size, to be given back with it: at most an eighth more for memory that stays
+// with an index (lasting), at most twice as much for what a call gives back at its end.
+void* si_block_take(size_t bytes, size_t* got, bool lasting = false);
 // hipMalloc and hipMallocAsync; when there is no memory the current device's kept blocks are freed
 // and it is tried again (not while the stream is captured, where freeing would end the capture).
 hipError_t si_malloc(void** p, size_t bytes);

@@ -84,6 +84,17 @@ int main() {
     g_capture = true;
     CHECK(si_malloc_async(&p, 900 * MB, nullptr) != hipSuccess && !p && g_used == 600 * MB);
     g_capture = false;
+    // memory that lasts does not sit in a block much larger than itself; a call's may
+    const size_t was = g_used;
+    size_t lasting = 0, passing = 0;
+    void *l = si_block_take(180 * MB, &lasting, true), *t = si_block_take(105 * MB, &passing);
+    CHECK(l && lasting == 200 * MB && t && passing == 105 * MB);
+    si_block_give(l, lasting, 0, true);
+    si_block_give(t, passing, 0, true);
+    CHECK((l = si_block_take(170 * MB, &lasting, true)) && lasting == 170 * MB && g_used == was + 275 * MB);
+    CHECK((t = si_block_take(110 * MB, &passing)) && passing == 200 * MB && g_used == was + 275 * MB);
+    si_block_give(l, lasting, 0, true);
+    si_block_give(t, passing, 0, true);
     si_block_users(-1);   // the last user takes them along
     CHECK(g_used == 0);
     printf("ok\n");

@@ -86,5 +86,6 @@ def test_single_query_scratch_is_made_whole_or_not_at_all(tmp_path):
 
 
 def test_kept_blocks(tmp_path):
-    """The device blocks kept between uses make room when an allocation finds no memory."""
+    """The device blocks kept between uses make room when an allocation finds no memory,
+    and an index does not sit in one much larger than it needs."""
     _run_host_program("test_kept_blocks", tmp_path)
