@@ -2329,14 +2329,16 @@ inline uint32_t sweep_chunk(size_t nq, int cus) {
 }
 
 // Spans of the queries that the sweep left: up to 32 of the plan's queries (or one chunk), fewer
-// where that would leave workgroups without one.
+// where that would leave workgroups without one: four spans a CU at least, for payloads, whose
+// lists are half as long, six (20K queries that 5000 of 1M int32 intervals hold: five 230 us, six
+// 205, eight 235).
 inline uint32_t shared_span(size_t nq, uint32_t chunk, int cus, int mode) {
-    const uint32_t want = (uint32_t)std::min<size_t>(32, nq / ((size_t)cus * sh_wgs(mode)));
+    const uint32_t want = (uint32_t)std::min<size_t>(32, nq / ((size_t)cus * (mode == W_VALUES ? 6u : 4u)));
     return chunk * std::max(1u, want / chunk);
 }
-inline unsigned shared_grid(size_t nq, uint32_t span, int cus, int mode) {
-    const size_t spans = (nq + span - 1) / span, full = (spans + HEAVY_CHUNKS - 1) / HEAVY_CHUNKS * HEAVY_CHUNKS;
-    return (unsigned)std::min<size_t>((size_t)cus * sh_wgs(mode), full);
+inline unsigned shared_grid(size_t nq, uint32_t span, int cus, unsigned wgs) {   // (whole rounds of EntryDeal's chunks)
+    const size_t spans = (nq + span - 1) / span, rounds = (spans + HEAVY_CHUNKS - 1) / HEAVY_CHUNKS;
+    return (unsigned)(HEAVY_CHUNKS * std::min(std::max<size_t>(1, (size_t)cus * wgs / HEAVY_CHUNKS), rounds));
 }
 
 template <typename S, int MODE>
@@ -2346,7 +2348,7 @@ int launch_sweep_shared(const siIndex* ix, const PlanView<S>& pv, size_t nq, uin
     LongView<S> lv = long_view_of<S>(ix);
     if (!g_tune.heavy_ends32) { hv.ends32 = nullptr; lv.ends32 = nullptr; }
     const uint32_t span = shared_span(nq, chunk, cus, MODE);
-    k_sweep_shared<S, MODE><<<shared_grid(nq, span, cus, MODE), SH_THREADS, 0, st>>>(
+    k_sweep_shared<S, MODE><<<shared_grid(nq, span, cus, sh_wgs<S>(MODE)), SH_THREADS, 0, st>>>(
         hv, ix->tree<S>(), ub_tree_of<S>(ix->ub, (const S*)ix->d_starts, ix->n), ix->ubt.view<S>(), lv, nullptr, pv,
         (uint32_t)nq, chunk, span, offsets, out_idx, ix->d_values, out_val, cap);
     LAUNCH_CHECK();
@@ -3244,7 +3246,7 @@ int launch_walk_multi(const siSetTable* tb, void* plan, size_t nq, const uint64_
         k_sweep<int32_t, MODE, true><<<grid_for(nq, chunk * SW_WAVES), SW_THREADS, 0, st>>>(
             IndexView<int32_t>{}, TreeDesc<int32_t>{}, sets, pv, (uint32_t)nq, chunk, offsets, out_idx, nullptr, cap);
         LAUNCH_CHECK();
-        k_sweep_shared<int32_t, MODE, true><<<shared_grid(nq, span, cus, MODE), SH_THREADS, 0, st>>>(
+        k_sweep_shared<int32_t, MODE, true><<<shared_grid(nq, span, cus, sh_wgs<int32_t>(MODE)), SH_THREADS, 0, st>>>(
             IndexView<int32_t>{}, TreeDesc<int32_t>{}, UbTree<int32_t>{}, BucketView<int32_t>{}, LongView<int32_t>{}, sets, pv,
             (uint32_t)nq, chunk, span, offsets, out_idx, nullptr, nullptr, cap);
         LAUNCH_CHECK();

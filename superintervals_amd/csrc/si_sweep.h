@@ -616,11 +616,22 @@ constexpr int SH_WAVES = SH_THREADS / WAVE;
 constexpr uint32_t SH_SPREAD = 2048;     // long entries that start within a group's range
 constexpr uint32_t SH_NEAR = 2048;       // positions between the starts of a group that shares all of its list
 constexpr uint32_t SH_LEAST = 3;         // smallest group that shares a list
+constexpr uint32_t SH_UNROLL = 4;        // groups of 64 candidates a wave looks at together
 constexpr uint32_t sh_cap(int mode) { return mode == W_VALUES ? 2048u : 4096u; }
-constexpr unsigned sh_wgs(int mode) { return mode == W_VALUES ? 6u : 4u; }   // workgroups a CU (160 KB of LDS)
+// Workgroups a CU, among which the spans are dealt: as many as its LDS holds, but for int64
+// payloads, whose registers leave room for four.  (Six for payloads, more than fit, made the last
+// ones wait with the spans dealt to them: 100K queries that 400 of 1M hold 200 us, now 181.)
+template <typename S>
+constexpr unsigned sh_wgs(int mode) { return mode == W_VALUES && sizeof(S) == 4 ? 5u : 4u; }
+template <typename S>
+constexpr size_t sh_lds(int mode, bool multi) {   // bytes of a workgroup (the arrays of k_sweep_shared)
+    return (sh_cap(mode) + SH_UNROLL * WAVE) * 4u * (mode == W_VALUES ? 3u : 2u) +
+           WAVE * (sizeof(S) + 8u + 7u * 4u + (multi ? 4u : 0u)) + 64u;
+}
+constexpr size_t CU_LDS = 160u << 10;
 
 template <typename S, int MODE, bool MULTI = false>
-__global__ __launch_bounds__(SH_THREADS) __attribute__((amdgpu_waves_per_eu(4))) void k_sweep_shared(IndexView<S> ix_one, TreeDesc<S> td_one, UbTree<S> ub_one,
+__global__ __launch_bounds__(SH_THREADS) __attribute__((amdgpu_waves_per_eu(sh_wgs<S>(MODE)))) void k_sweep_shared(IndexView<S> ix_one, TreeDesc<S> td_one, UbTree<S> ub_one,
                                                              BucketView<S> tab, LongView<S> lv,
                                                              const SetView<S>* __restrict__ sets, PlanView<S> pv, uint32_t nq, uint32_t chunk,
                                                              uint32_t span, const uint64_t* __restrict__ offsets,
@@ -632,7 +643,9 @@ __global__ __launch_bounds__(SH_THREADS) __attribute__((amdgpu_waves_per_eu(4)))
     constexpr uint32_t CAP = sh_cap(MODE);            // candidates held at a time
     constexpr uint32_t LINES = (VALUES || sizeof(S) == 8) ? 4 : 8;   // lines a wave collects at a time (registers)
     constexpr uint32_t ROUND = SH_WAVES * LINES * 64u;   // most that one round of lines adds
-    constexpr uint32_t UNROLL = 4;
+    constexpr uint32_t UNROLL = SH_UNROLL;
+    static_assert(SH_WAVES == 4, "a workgroup is one wave of each SIMD (amdgpu_waves_per_eu)");
+    static_assert(sh_wgs<S>(MODE) * sh_lds<S>(MODE, MULTI) <= CU_LDS, "the workgroups dealt for fit a CU");
     __shared__ uint32_t c_rel[CAP + UNROLL * WAVE], c_pos[CAP + UNROLL * WAVE], c_val[VALUES ? CAP + UNROLL * WAVE : 1];
     __shared__ S q_s[WAVE];
     __shared__ uint64_t q_acc[WAVE];
