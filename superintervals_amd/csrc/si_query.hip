@@ -2616,7 +2616,12 @@ SI_EXPORT int siCount(const siIndex* ix, const void* qs, const void* qe, size_t 
     if (nq == 0) return SI_OK;
     if (!qs || !qe || !counts) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
-    if (g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF)
+    // (counts over the queries' own arrays: the plan reads all of these before it writes one)
+    const auto over = [&](const void* q) {
+        const uintptr_t a = (uintptr_t)counts, b = (uintptr_t)q;
+        return a < b + nq * ix->cb && b < a + nq * 4;
+    };
+    if (g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF && !over(qs) && !over(qe))
         return DISPATCH_S(ix, (launch_count_table<S>(ix, (const S*)qs, (const S*)qe, nq, counts, st)));
     ScopedPlan P(st);
     const size_t pb = siPlanBytes(ix, nq);

@@ -1527,6 +1527,30 @@ def test_count_grouped(sia, orc, dtype, nq):
 
 
 @pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("nq", [2, 8193, 300_001])
+@pytest.mark.parametrize("place", ["starts", "ends", "starts + 1"])
+def test_count_over_its_queries(sia, orc, dtype, nq, place):
+    """Counts written over the arrays the queries came in: a caller that needs them no more."""
+    import torch
+    print(f"[gpu] count over {place} {np.dtype(dtype).name} nq={nq}", flush=True)
+    rng = np.random.default_rng(nq)
+    n = 200_000
+    s = rng.integers(0, 3_000_000, n).astype(dtype)
+    e = (s + rng.integers(0, 400, n)).astype(dtype)
+    qs = rng.integers(0, 3_000_000, nq).astype(dtype)
+    qe = (qs + rng.integers(-2, 3000, nq)).astype(dtype)
+    ix = _dev_index(sia, s, e)
+    want = orc.count_batch(orc.build_index(s, e), qs, qe)
+    for _ in range(3):
+        tqs, tqe = torch.from_numpy(np.append(qs, [0]).astype(dtype)).cuda(), torch.from_numpy(qe).cuda()
+        out = (tqe if place == "ends" else tqs).view(torch.int32)[1 if place == "starts + 1" else 0:][:nq]
+        sia._native.check(sia._native.lib.siCount(ix.handle, tqs.data_ptr(), tqe.data_ptr(), nq, out.data_ptr(), None), "siCount")
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), want)
+    ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
 @pytest.mark.parametrize("n,nq,depth", [(70_000, 1, 300), (70_000, 9, 5000), (200_000, 3000, 9000),
                                         (200_000, 40_000, 600), (100_000, 300_001, 300), (100_000, 600_001, 270)])
 def test_sweep_shared_lists(sia, orc, dtype, n, nq, depth):
