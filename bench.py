@@ -496,8 +496,8 @@ def bench_skewed(a):
     nb = (nq + bq - 1) // bq
     bplan = torch.empty(ix.plan_bytes(bq), dtype=torch.uint8, device=dev)
     off = torch.empty(bq + 1, dtype=torch.int64, device=dev)
-    # the per-lane step budget before a walk is parked for the one-wave kernel, tuned on the
-    # first batch: these walks are long but sparse, which the lane walk serves better
+    # the per-lane step budget before a walk is parked for the one-wave kernel, by the count walk of
+    # the first batch (the fill, a sweep over the query starts, does not read it)
     m0 = min(nq, bq)
     ix.plan_device(tqs[:m0], tqe[:m0], bplan, stream=stream)
     ix.offsets_planned(bplan, m0, off, stream=stream)
@@ -516,7 +516,7 @@ def bench_skewed(a):
                   % (ls, sweep[ls], csweep[ls]), file=sys.stderr, flush=True)
     finally:
         autotune.apply(saved)
-    best_ls = min(sweep, key=sweep.get)
+    best_ls = min(csweep, key=csweep.get)
     autotune.apply({"lane_steps": best_ls})
     # the wave walk's ends: the 32-bit copy or the int64 array, by the fill of one batch
     ends32_ms = {}

@@ -4,10 +4,13 @@ The kernels' results never depend on these choices (tile size, resident workgrou
 CU for the count and the fill pass, the per-lane step budget before a long walk is
 parked for the one-wave-per-query kernel, walk or rank form of the count); only their
 speed does.  tune() times every candidate on the caller's own index and planned batch
-with HIP events: first tile x workgroups for count + fill, then, with those fixed, the
-lane step budget by the fill's time, the count form by the count's and, given the
-queries, the plan's constant-digit check by the plan's and the unsorted low end digit
-by plan + fill.  Results are
+with HIP events, each by the kernels that read it.  The fill of an index without start >
+end intervals is the sweep over the query starts (range_skip = 1), which reads neither the
+tile nor the workgroups nor the step budget: there the tile, the count's workgroups and the
+budget are judged by the walk form of the count alone, and fill_wgs is left as it is.  Where
+fills walk, first tile x workgroups by count + fill, then the budget by the fill's time.
+Then the count form by the count's time and, given the queries, the plan's constant-digit
+check by the plan's and the unsorted low end digit by plan + fill.  Results are
 cached per workload signature (coordinate width, log2 of the index size, log2 of the
 batch size, log2 of the mean hits per query) in a JSON file, so later runs of the same
 shape reuse them.
@@ -21,6 +24,7 @@ import time
 
 from . import _native as N
 
+VERSION = 2   # of a cached record: another version's choices were judged by other times
 DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "superintervals_amd", "tune.json")
 KNOBS = ("tile", "count_wgs", "fill_wgs", "count_rank", "offsets_rank", "lane_steps", "plan_sync", "ub_tree",
          "plan_skip_low", "heavy_ends32", "range_skip", "ub_learned", "learned_shrink", "long_walk", "long_len")
@@ -98,6 +102,10 @@ def tune(ix, plan_t, nq, offsets_t, idx_t, stream=None, reps=3, tiles=CANDIDATE_
     saved = current()
     count = lambda: ix.count_planned(plan_t, nq, counts, stream=stream)
     fill = lambda: ix.fill_planned(plan_t, nq, offsets_t, idx_t, stream=stream)
+    # the plan's flags: word 4 says whether it holds lower bounds, as it does exactly where no interval
+    # has start > end (with range_skip, the fills the sweep answers)
+    swept = bool(saved["range_skip"]) and int(plan_t.view(torch.uint8)[16:20].view(torch.int32).item()) == 1
+    fill_wgs = (saved["fill_wgs"],) if swept else wgs
     results = []
     try:
         # the tile and the workgroup counts are judged on the walk form of count (the rank
@@ -105,14 +113,15 @@ def tune(ix, plan_t, nq, offsets_t, idx_t, stream=None, reps=3, tiles=CANDIDATE_
         apply({"count_rank": 0})
         for tile in tiles:
             for cw in wgs:
-                for fw in wgs:
+                for fw in fill_wgs:
                     apply({"tile": tile, "count_wgs": cw, "fill_wgs": fw})
                     tc, tf = _time_ms(count, reps, stream), _time_ms(fill, reps, stream)
                     results.append({"tile": tile, "count_wgs": cw, "fill_wgs": fw, "count_ms": tc, "fill_ms": tf})
                     if verbose:
                         print("tune tile=%d count_wgs=%d fill_wgs=%d: count %.3f ms fill %.3f ms"
                               % (tile, cw, fw, tc, tf), flush=True)
-        # count and fill share the tile; pick the tile by their sum, the wgs of each by its own time
+        # count and fill share the tile; pick the tile by their sum (of the count alone when the fill is
+        # the sweep), the wgs of each by its own time
         by_tile = {}
         for r in results:
             c = by_tile.setdefault(r["tile"], {"count": r, "fill": r})
@@ -120,20 +129,23 @@ def tune(ix, plan_t, nq, offsets_t, idx_t, stream=None, reps=3, tiles=CANDIDATE_
                 c["count"] = r
             if r["fill_ms"] < c["fill"]["fill_ms"]:
                 c["fill"] = r
-        tile = min(by_tile, key=lambda t: by_tile[t]["count"]["count_ms"] + by_tile[t]["fill"]["fill_ms"])
+        tile = min(by_tile, key=lambda t: by_tile[t]["count"]["count_ms"] +
+                   (0.0 if swept else by_tile[t]["fill"]["fill_ms"]))
         best = {"tile": tile, "count_wgs": by_tile[tile]["count"]["count_wgs"],
                 "fill_wgs": by_tile[tile]["fill"]["fill_wgs"],
                 "count_ms": by_tile[tile]["count"]["count_ms"], "fill_ms": by_tile[tile]["fill"]["fill_ms"]}
         apply(knobs_of(best))
-        # the lane step budget (shared by the count walk and the fills), by the fill's time
+        # the lane step budget (shared by the count walk and the fills that walk), by the fill's time,
+        # or by the count walk's when the fill is the sweep
+        judged, what = (count, "count_ms") if swept else (fill, "fill_ms")
         for ls in lane_steps:
             apply({"lane_steps": ls})
-            tf = _time_ms(fill, reps, stream)
-            results.append(dict(knobs_of(best), lane_steps=ls, fill_ms=tf))
+            tm = _time_ms(judged, reps, stream)
+            results.append(dict(knobs_of(best), lane_steps=ls, **{what: tm}))
             if verbose:
-                print("tune lane_steps=%d: fill %.3f ms" % (ls, tf), flush=True)
-            if "lane_steps" not in best or tf < best["fill_ms"]:
-                best["lane_steps"], best["fill_ms"] = ls, tf
+                print("tune lane_steps=%d: %s %.3f ms" % (ls, what[:-3], tm), flush=True)
+            if "lane_steps" not in best or tm < best[what]:
+                best["lane_steps"], best[what] = ls, tm
         apply({"lane_steps": best["lane_steps"]})
         # the count's form: the walk (best for short lists) or the rank form (O(log n))
         for cr in (0, 1):
@@ -181,12 +193,12 @@ def load_or_tune(ix, plan_t, nq, offsets_t, idx_t, hits, cache=DEFAULT_CACHE, st
     """Apply cached choices for this workload signature, tuning (and caching) if absent."""
     sig = signature(ix.dtype.itemsize, ix.n, nq, hits)
     table = _load(cache)
-    if not retune and sig in table:
+    if not retune and sig in table and table[sig].get("version") == VERSION:
         apply(knobs_of(table[sig]))
         return dict(table[sig], cached=True, signature=sig)
     t0 = time.perf_counter()
     best, _ = tune(ix, plan_t, nq, offsets_t, idx_t, stream=stream, qs_t=qs_t, qe_t=qe_t, verbose=verbose)
-    best = dict(best, tuned_s=round(time.perf_counter() - t0, 2))
+    best = dict(best, version=VERSION, tuned_s=round(time.perf_counter() - t0, 2))
     table[sig] = best
     try:
         _save(cache, table)

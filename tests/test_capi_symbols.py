@@ -67,6 +67,59 @@ def test_tuning_knobs_round_trip():
     assert autotune.current() == saved
 
 
+def test_tuner_judges_by_what_reads_a_knob(monkeypatch, tmp_path):
+    """Where fills are the sweep, which reads neither tile nor workgroups nor step budget, these are
+    judged by the count walk's time alone, whatever the fill's noise says, and fill_wgs stays;
+    where fills walk (an index with start > end: no lower bounds in the plan; or range_skip 0), the
+    fill's time counts as well.  Times are made up here; nothing runs on a GPU."""
+    import torch
+    from superintervals_amd import autotune
+
+    class Index:
+        dtype, n = __import__("numpy").dtype("int32"), 1000
+
+        def count_planned(self, *a, **k):
+            return "count"
+
+        def fill_planned(self, *a, **k):
+            return "fill"
+
+    timed = []
+
+    def time_ms(fn, reps, stream):
+        now = autotune.current()
+        timed.append((fn(), now["fill_wgs"]))
+        if fn() == "count":   # best at tile 2048, budget 64
+            return 1.0 + 0.1 * abs(now["tile"] - 2048) / 1024 + 0.1 * (now["lane_steps"] != 64) - 0.5 * now["count_rank"]
+        # best at tile 512, one workgroup, budget 1024
+        return 5.0 + abs(now["tile"] - 512) / 1024 + (now["fill_wgs"] != 1) + (now["lane_steps"] != 1024)
+
+    monkeypatch.setattr(autotune, "_time_ms", time_ms)
+    saved = autotune.current()
+    off, idx = torch.zeros(9, dtype=torch.int64), torch.zeros(4, dtype=torch.int32)
+    try:
+        for lower_bounds, range_skip, swept in ((1, 1, True), (0, 1, False), (1, 0, False)):
+            autotune.apply(dict(saved, range_skip=range_skip, fill_wgs=3))
+            plan = torch.zeros(256, dtype=torch.uint8)
+            plan[16] = lower_bounds
+            timed.clear()
+            best, _ = autotune.tune(Index(), plan, 8, off, idx, stream="none")
+            want = (2048, 64, 3) if swept else (512, 1024, 1)
+            assert (best["tile"], best["lane_steps"], best["fill_wgs"]) == want
+            assert all(autotune.current()[k] == v for k, v in autotune.knobs_of(best).items())
+            assert not swept or {w for _, w in timed} == {3}
+        # a record judged the old way is not used again
+        cache = str(tmp_path / "tune.json")
+        sig = autotune.signature(4, 1000, 8, 80)
+        autotune._save(cache, {sig: {"tile": 4096, "lane_steps": 1024}})
+        rec = autotune.load_or_tune(Index(), plan, 8, off, idx, 80, cache=cache, stream="none")
+        assert not rec["cached"] and rec["tile"] == 512
+        rec = autotune.load_or_tune(Index(), plan, 8, off, idx, 80, cache=cache, stream="none")
+        assert rec["cached"] and rec["tile"] == 512
+    finally:
+        autotune.apply(saved)
+
+
 def _run_host_program(name, tmp_path):
     """Builds and runs a program of tests/cpp that brings its own HIP calls (no GPU)."""
     import subprocess
