@@ -2064,24 +2064,42 @@ int launch_grouped(const siIndex* ix, const S* qs, const S* qe, size_t nq, bool 
     return SI_OK;
 }
 
-// count() through the tables.  Grouped, from GROUP_FROM queries and 4 MB of starts on:
-// int32, 10M intervals: 10M queries 0.97 ms ungrouped, 0.56 grouped (through the sorted plan 0.87),
-// 2M 189 and 104 us, 1M 93 and 73, 500K 46 and 57; int64: 1M 135 and 98, 500K 66 and 77.  1M int32
-// intervals (4 MB): 2M queries 88 and 85, 800K 35 and 54.  100K: 10M queries 236 and 270.
+// Where grouping pays.  Each line is where calls back to back and calls that are waited for one by
+// one (which pay some 30 us and more for the copies' memory, hipMallocAsync) gain together what they
+// lose; us of both, ungrouped and grouped.
+//
+// count: 10M int32 intervals: 10M queries 962 and 965, 558 and 625; 1M 94 and 96, 66 and 95.  2M: 2M
+// queries 135 and 137, 82 and 111; 1M 66 and 68, 57 and 86.  1.05M: 3M queries 147 and 149, 101 and
+// 135; 1.4M 68 and 70, 61 and 97; 800K 39 and 41, 51 and 85.  So the more queries the smaller the
+// index.  40M intervals: 1M 106 and 108, 110 and 170; 4M 417 and 422, 314 and 375.  int64, the same bytes
+// of starts: 1M intervals: 1.4M queries 127 and 129, 76 and 109.  100K int32: 10M queries 236, 270.
 constexpr size_t GROUP_FROM = 3u << 18;
 constexpr size_t GROUP_BYTES = (size_t)4 << 20;
-// has_overlaps reads the ends at one place where count searches them: int32, 10M intervals: 4M queries
-// 230 us ungrouped, 134 grouped, 1.5M 87 and 66, 800K 47 and 47; 1.1M intervals: 2M 57 and 63.
-constexpr size_t ANY_GROUP_FROM = (size_t)1 << 20;
-constexpr size_t ANY_GROUP_BYTES = (size_t)8 << 20;
-// coverage reads up to 24 lines a query, which neighbours in a group share in the L1: 1M intervals:
-// 1M queries 132 us ungrouped, 86 grouped, 400K 54 and 50, 200K 31 and 36; 10M intervals: 1M 325
-// and 137; 100K intervals: 1M 95 and 73.
-constexpr size_t COVERAGE_GROUP_FROM = 3u << 17;
-constexpr size_t COVERAGE_GROUP_BYTES = (size_t)256 << 10;
+constexpr size_t GROUP_PRODUCT = (size_t)9 << 40;   // queries x bytes of starts
+constexpr size_t GROUP_WIDE_BYTES = (size_t)96 << 20, GROUP_WIDE_FROM = 1u << 21;
+inline bool group_counts(size_t nq, size_t bytes) {
+    return nq >= GROUP_FROM && bytes >= GROUP_BYTES && nq >= GROUP_PRODUCT / bytes &&
+           (bytes <= GROUP_WIDE_BYTES || nq >= GROUP_WIDE_FROM);
+}
+// has_overlaps reads the ends at one place where count searches them, so it gains less, with int64
+// coordinates nothing (5M intervals: 4M queries 254 and 255, 184 and 340; 20M: 288 and 290, 323 and
+// 500).  int32, 10M intervals: 4M queries 231 and 233, 145 and 190; 1.1M 65 and 66, 58 and 101.  2.1M: 4M 160
+// and 162, 120 and 173; 1.1M 45 and 47, 52 and 99.  32M: 4M 259 and 260, 244 and 304.
+constexpr size_t ANY_GROUP_FROM = 7u << 18;
+constexpr size_t ANY_GROUP_BYTES = (size_t)8 << 20, ANY_GROUP_MOST = (size_t)96 << 20;
+inline bool group_any(size_t nq, size_t bytes, size_t width) {
+    return width == 4 && nq >= ANY_GROUP_FROM && bytes >= ANY_GROUP_BYTES && bytes <= ANY_GROUP_MOST;
+}
+// coverage reads up to 24 lines a query, which neighbours in a group share in the L1: 10M intervals: 400K
+// queries 124 and 126, 89 and 135.  1M: 1M queries 149 and 151, 99 and 127; 600K 90 and 93, 71 and
+// 129.  100K: 2M queries 174 and 178, 120 and 156; 1M 89 and 91, 75 and 132.
+inline bool group_coverage(size_t nq, size_t bytes) {
+    return bytes >= ((size_t)256 << 10) &&
+           nq >= (bytes >= ((size_t)8 << 20) ? 3u << 17 : bytes >= ((size_t)2 << 20) ? 3u << 18 : 5u << 18);
+}
 template <typename S>
 int launch_count_table(const siIndex* ix, const S* qs, const S* qe, size_t nq, uint32_t* counts, hipStream_t st) {
-    const bool group = nq >= GROUP_FROM && ix->n * sizeof(S) >= GROUP_BYTES;
+    const bool group = group_counts(nq, ix->n * sizeof(S));
     return launch_grouped<S>(ix, qs, qe, nq, group, st, [&](const S* s, const S* e, const uint32_t* order, unsigned g) {
         k_count_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), (const S*)ix->d_ends_sorted, ix->ubt.view<S>(),
                                                   ix->ebt.view<S>(), s, e, order, nq, counts);
@@ -2715,7 +2733,7 @@ SI_EXPORT int siHasOverlaps(const siIndex* ix, const void* qs, const void* qe, s
     hipStream_t st = (hipStream_t)stream;
     return DISPATCH_S(ix, ([&]() -> int {
         if (g_tune.ub_tree && ix->ubt.ok) {
-            const bool group = nq >= ANY_GROUP_FROM && ix->n * sizeof(S) >= ANY_GROUP_BYTES;
+            const bool group = group_any(nq, ix->n * sizeof(S), sizeof(S));
             return launch_grouped<S>(ix, (const S*)qs, (const S*)qe, nq, group, st,
                                      [&](const S* s, const S* e, const uint32_t* order, unsigned g) {
                 k_has_overlaps_table<S><<<g, Q_THREADS, 0, st>>>(ix->view<S>(), ix->ubt.view<S>(), s, e, order, nq, out);
@@ -2977,7 +2995,7 @@ SI_EXPORT int siCoverage(const siIndex* ix, const void* qs, const void* qe, size
     if (!qs || !qe) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
     if (rank_exact(ix) && ix->ubt.ok) {
-        const bool group = nq >= COVERAGE_GROUP_FROM && ix->n * 4 >= COVERAGE_GROUP_BYTES;
+        const bool group = group_coverage(nq, ix->n * 4);
         return launch_grouped<int32_t>(ix, (const int32_t*)qs, (const int32_t*)qe, nq, group, st,
                                        [&](const int32_t* s, const int32_t* e, const uint32_t* order, unsigned g) {
             k_coverage_rank<<<g, Q_THREADS, 0, st>>>(

@@ -1792,3 +1792,53 @@ def test_grouped_forms(sia, orc, dtype, nq):
             some = np.concatenate([np.arange(200), rng.integers(0, nq, 3000), [nq - 1]])
             assert [int(cov[k]) for k in some] == [int(orc.coverage(oix, qs[k], qe[k])[1]) for k in some]
         ix.close()
+
+
+@pytest.mark.parametrize("what,dtype,n,first", [
+    ("count", np.int32, 1_100_000, 2_249_001), ("count", np.int64, 1_100_000, 1_124_500),
+    ("count", np.int32, 25_200_000, 2_097_152), ("any", np.int32, 2_100_000, 1_835_008),
+    ("coverage", np.int32, 100_000, 1_310_720), ("coverage", np.int32, 600_000, 786_432)])
+def test_grouping_begins(sia, orc, what, dtype, n, first):
+    """count, has_overlaps and coverage at the batch size from which queries are grouped on an index of
+    n intervals, and one below it: all of the results from sorted coordinates (covered lengths of
+    some queries from the oracle), queries with start > end and at the ends of the range among them,
+    nothing past them written."""
+    import torch
+    print(f"[gpu] grouping begins {what} {np.dtype(dtype).name} n={n} nq={first}", flush=True)
+    rng = np.random.default_rng(n)
+    s = rng.integers(-1000, 20 * n, n)
+    e = s + rng.integers(0, 60, n)
+    qs = rng.integers(-5000, 20 * n + 5000, first)
+    qe = qs + rng.integers(0, 90, first)
+    info = np.iinfo(dtype)
+    qe[:20] = qs[:20] - rng.integers(1, 90, 20)
+    qs[20:24], qe[20:24] = [info.min, info.min, info.max, 7], [info.min, info.max, info.max, info.min]
+    o = np.lexsort((-e, s))
+    s, e = s[o].astype(dtype), e[o].astype(dtype)
+    qs, qe = qs.astype(dtype), qe.astype(dtype)
+    ix = sia.DeviceIndex(dtype).build(s, e, None, start_sorted=True, end_sorted=True)
+    last = np.searchsorted(s, qe, side="right")
+    counts = last - np.searchsorted(np.sort(e), qs)
+    for k in range(24):
+        counts[k] = np.count_nonzero(e[:last[k]] >= qs[k])
+    any_ = (last > 0) & (e[np.maximum(last - 1, 0)] >= qs)
+    oix = orc.build_index(s, e) if what == "coverage" else None
+    lib, check = sia._native.lib, sia._native.check
+    tqs, tqe = torch.from_numpy(qs).cuda(), torch.from_numpy(qe).cuda()
+    for nq in (first - 1, first):
+        out = [torch.full((first + 9,), 5, dtype=torch.uint8 if what == "any" else torch.int32, device="cuda") for _ in range(2)]
+        if what == "count":
+            check(lib.siCount(ix.handle, tqs.data_ptr(), tqe.data_ptr(), nq, out[0].data_ptr(), None), "siCount")
+        elif what == "any":
+            check(lib.siHasOverlaps(ix.handle, tqs.data_ptr(), tqe.data_ptr(), nq, out[0].data_ptr(), None), "siHasOverlaps")
+        else:
+            check(lib.siCoverage(ix.handle, tqs.data_ptr(), tqe.data_ptr(), nq, out[0].data_ptr(), out[1].data_ptr(), None),
+                  "siCoverage")
+        torch.cuda.synchronize()
+        got, cov = (x.cpu().numpy() for x in out)
+        assert np.array_equal(got[:nq], any_[:nq] if what == "any" else counts[:nq]) and np.all(got[nq:] == 5)
+        if what == "coverage":
+            assert np.all(cov[nq:] == 5)
+            some = np.concatenate([np.arange(100), rng.integers(0, nq, 1000), [nq - 1]])
+            assert [int(cov[k]) for k in some] == [int(orc.coverage(oix, qs[k], qe[k])[1]) for k in some]
+    ix.close()
