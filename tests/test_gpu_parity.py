@@ -1842,3 +1842,58 @@ def test_grouping_begins(sia, orc, what, dtype, n, first):
             some = np.concatenate([np.arange(100), rng.integers(0, nq, 1000), [nq - 1]])
             assert [int(cov[k]) for k in some] == [int(orc.coverage(oix, qs[k], qe[k])[1]) for k in some]
     ix.close()
+
+
+@pytest.mark.parametrize("form", ["range_skip 0", "start > end"])
+@pytest.mark.parametrize("lane_steps", [1, 3, 17])
+@pytest.mark.parametrize("kind", ["int32", "int64", "int64 far", "long list", "no long list"])
+def test_fills_that_park_walks(sia, orc, kind, lane_steps, form):
+    """Fills by the block walk (range_skip = 0, or an index that holds intervals with start > end), whose
+    lanes park what exceeds lane_steps for the wave-cooperative kernel: with 32-bit ends, without
+    (ends 2^40 apart), through the long list and not, in both orders and for the values.  The plan says
+    that walks were parked."""
+    import torch
+    from superintervals_amd import autotune
+    print(f"[gpu] fills that park walks {kind} lane_steps={lane_steps} {form}", flush=True)
+    dtype = np.int32 if kind == "int32" else np.int64
+    rng = np.random.default_rng(lane_steps)
+    n, nq = 120_000, 5_000
+    s = rng.integers(0, 3_000_000, n)
+    long_ = rng.random(n) < 0.05
+    e = s + np.where(long_, rng.integers(20_000, 400_000, n), rng.integers(0, 300, n))
+    if kind == "int64 far":
+        s[-50:] += np.int64(1) << 40
+        e[-50:] += np.int64(1) << 40
+    if form == "start > end":
+        e[::400] = s[::400] - rng.integers(1, 50, n // 400)
+    qs = rng.integers(-100, 3_000_000, nq)
+    qe = qs + np.where(rng.random(nq) < 0.9, rng.integers(0, 2000, nq), rng.integers(-300, 80_000, nq))
+    s, e, qs, qe = (x.astype(dtype) for x in (s, e, qs, qe))
+    vals = rng.integers(-9, 9, n).astype(np.int32)
+    saved = autotune.current()
+    try:
+        autotune.apply({"long_len": -1 if kind == "no long list" else 4096 if kind == "long list" else 0})
+        ix = _dev_index(sia, s, e, vals)
+        oix = orc.build_index(s, e, vals)
+        autotune.apply(dict(saved, lane_steps=lane_steps, range_skip=int(form != "range_skip 0")))
+        tqs, tqe = torch.from_numpy(qs).cuda(), torch.from_numpy(qe).cuda()
+        plan = torch.empty(ix.plan_bytes(nq), dtype=torch.uint8, device="cuda")
+        off = torch.empty(nq + 1, dtype=torch.int64, device="cuda")
+        ix.plan_device(tqs, tqe, plan)
+        ix.offsets_planned(plan, nq, off)
+        for order, mode in (("desc", 0), ("vector", 1), ("values", 0)):
+            woff, widx = orc.search_batch(oix, qs, qe, mode=mode)
+            assert np.array_equal(off.cpu().numpy(), woff)
+            out = torch.full((int(woff[-1]) + 64,), -77, dtype=torch.int32, device="cuda")
+            if order == "values":
+                ix.values_fill_planned(plan, nq, off, out)
+            else:
+                ix.fill_planned(plan, nq, off, out, order=order)
+            torch.cuda.synchronize()
+            assert int(plan[4:8].view(torch.int32).item()) > 100, "no walks were parked"
+            got, want = out.cpu().numpy(), oix["data"][widx] if order == "values" else widx
+            assert np.array_equal(got[:len(want)], want), order
+            assert np.all(got[len(want):] == -77)
+    finally:
+        autotune.apply(saved)
+    ix.close()
