@@ -1897,3 +1897,39 @@ def test_fills_that_park_walks(sia, orc, kind, lane_steps, form):
     finally:
         autotune.apply(saved)
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("nq", [2048 * 56, 2048 * 56 + 1])
+def test_plan_sort_where_its_scan_begins(sia, dtype, nq):
+    """The plan's sort on both sides of the size up to which its scatter adds the tiles' counts up itself
+    (56 tiles of 2048)."""
+    test_plan_sort_around_the_scan_free_size(sia, dtype, nq)
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_sweep_of_full_chunks(sia, orc, dtype):
+    """A batch that gives every wave of the sweep its largest chunk (256 queries), with queries that
+    more than 256 intervals hold (spans of four batches in the shared lists) among queries of few
+    hits: both orders and the values against the oracle."""
+    print(f"[gpu] sweep of full chunks {np.dtype(dtype).name}", flush=True)
+    rng = np.random.default_rng(3)
+    n, nq = 200_000, 2_200_003
+    hot = 20_000
+    s = rng.integers(0, 5_000_000, n)
+    s[:n // 10] = rng.integers(0, hot, n // 10)
+    e = s + np.where(s < hot, rng.integers(1, 1200, n), rng.integers(0, 90, n))
+    qs = rng.integers(0, 5_000_000, nq)
+    qs[::40] = rng.integers(0, hot, len(qs[::40]))
+    qe = qs + rng.integers(0, 60, nq)
+    qe[7::1001] = qs[7::1001] - 30
+    s, e, qs, qe = (x.astype(dtype) for x in (s, e, qs, qe))
+    vals = (np.arange(n, dtype=np.int64) * 7 % 1_000_003).astype(np.int32)
+    ix, oix = _dev_index(sia, s, e, vals), orc.build_index(s, e, vals)
+    assert (orc.count_batch(oix, qs, qe) > 300).sum() > 20_000
+    for order, mode in (("desc", 0), ("vector", 1), ("values", 0)):
+        off, out = ix.search(qs, qe, values=True) if order == "values" else ix.search(qs, qe, order=order)
+        woff, widx = orc.search_batch(oix, qs, qe, mode=mode)
+        assert np.array_equal(off, woff)
+        assert np.array_equal(out, oix["data"][widx] if order == "values" else widx), order
+    ix.close()
