@@ -4,11 +4,10 @@ The kernels' results never depend on these choices (tile size, resident workgrou
 CU for the count and the fill pass, the per-lane step budget before a long walk is
 parked for the one-wave-per-query kernel, walk or rank form of the count); only their
 speed does.  tune() times every candidate on the caller's own index and planned batch
-with HIP events, each by the kernels that read it.  The fill of an index without start >
-end intervals is the sweep over the query starts (range_skip = 1), which reads neither the
-tile nor the workgroups nor the step budget: there the tile, the count's workgroups and the
-budget are judged by the walk form of the count alone, and fill_wgs is left as it is.  Where
-fills walk, first tile x workgroups by count + fill, then the budget by the fill's time.
+with HIP events, each by the kernels that read it.  Most fills are the sweep over the query
+starts, which reads neither the tile nor the workgroups nor the step budget: there the tile,
+the count's workgroups and the budget are judged by the walk form of the count alone, and
+fill_wgs is left as it is.  Where the fill walks, first tile x workgroups by count + fill, then the budget by the fill's time.
 Then the count form by the count's time and, given the queries, the plan's constant-digit
 check by the plan's and the unsorted low end digit by plan + fill.  Results are
 cached per workload signature (coordinate width, log2 of the index size, log2 of the
@@ -102,9 +101,8 @@ def tune(ix, plan_t, nq, offsets_t, idx_t, stream=None, reps=3, tiles=CANDIDATE_
     saved = current()
     count = lambda: ix.count_planned(plan_t, nq, counts, stream=stream)
     fill = lambda: ix.fill_planned(plan_t, nq, offsets_t, idx_t, stream=stream)
-    # the plan's flags: word 4 says whether it holds lower bounds, as it does exactly where no interval
-    # has start > end (with range_skip, the fills the sweep answers)
-    swept = bool(saved["range_skip"]) and int(plan_t.view(torch.uint8)[16:20].view(torch.int32).item()) == 1
+    fill()   # word 2 of the plan says who answered it: 1 the sweep, 0 the walk
+    swept = int(plan_t.view(torch.uint8)[8:12].view(torch.int32).item()) == 1
     fill_wgs = (saved["fill_wgs"],) if swept else wgs
     results = []
     try:

@@ -59,7 +59,8 @@ struct HeavyEntry;
 template <typename S>
 struct PlanView {
     uint32_t* counter;   // [0] tiles taken, [1] heavy entries written (by the sweep: 1 when there
-                         // are any), [3] set by a fill pass
+                         // are any), [2] 1 when the sweep answers a fill pass, 0 when the block
+                         // walk does, [3] set by a fill pass
                          // when a query's hits differ from its offsets, [4] 1 when the plan
                          // holds lower_bound positions (lb), [5] 1 when it holds the counts
                          // (cnt), [8 + c] entries taken from chunk c of the heavy list
@@ -750,6 +751,7 @@ __global__ __launch_bounds__(T_THREADS) SI_WALK_OCCUPANCY void k_walk(IndexView<
     const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
     // the guaranteed runs need the plan's lower_bound positions
     use_lb = use_lb && __builtin_amdgcn_readfirstlane(pv.counter[4]) != 0u;
+    if (MODE != W_COUNT && __builtin_amdgcn_readfirstlane(pv.counter[2]) != 0u) return;   // the sweep answers
     EmitSlot* const my_emit = s_emit + (MODE == W_COUNT ? 0u : (threadIdx.x / WAVE) * (WAVE + 1));
     if (MODE != W_COUNT) my_emit[lane].kv = 0u;   // emission slots start free (own wave's)
     // segments held from the previous steps (emission runs every EMIT_EVERY steps)
@@ -1406,10 +1408,17 @@ struct EntryDeal {
     }
 };
 
-// Clears the counters a walk launch uses (tiles, heavy list, mismatch flag, chunk counters).
-__global__ void k_walk_counters_reset(uint32_t* __restrict__ c) {
+// Clears the counters a walk or fill launch uses (tiles, heavy list, mismatch flag, chunk counters).
+// swept: who answers a fill (counter [2]).  With `offsets` the batch says: the walk when it has
+// [few, many) hits.
+__global__ void k_walk_counters_reset(uint32_t* __restrict__ c, uint32_t swept, const uint64_t* __restrict__ offsets,
+                                      uint32_t nq, uint64_t few, uint64_t many) {
     const uint32_t i = threadIdx.x;
-    if (i < 4u || (i >= 8u && i < 8u + HEAVY_CHUNKS)) c[i] = 0u;
+    if (offsets) {
+        const uint64_t hits = offsets[nq] - offsets[0];
+        swept = hits >= few && hits < many ? 0u : 1u;
+    }
+    if (i < 4u || (i >= 8u && i < 8u + HEAVY_CHUNKS)) c[i] = i == 2u ? swept : 0u;
 }
 
 template <typename S, int MODE, bool MULTI = false>
@@ -1425,6 +1434,7 @@ __global__ __launch_bounds__(Q_THREADS) void k_walk_heavy(IndexView<S> ix, TreeD
     const int lane = lane_id();
     const uint32_t nheavy = __builtin_amdgcn_readfirstlane(pv.counter[1]);
     if (nheavy == 0) return;   // nothing parked: no wave touches the shared counters
+    if (MODE != W_COUNT && __builtin_amdgcn_readfirstlane(pv.counter[2]) != 0u) return;   // (the sweep's entries)
     constexpr uint32_t WAVES = Q_THREADS / WAVE;
     EntryDeal deal(pv.counter + 8, nheavy, (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x / WAVE * gridDim.x + blockIdx.x)),
                    gridDim.x * WAVES);
@@ -2373,6 +2383,20 @@ int launch_sweep_shared(const siIndex* ix, const PlanView<S>& pv, size_t nq, uin
     return SI_OK;
 }
 
+// The sweep costs what a window and a list cost, for however few hits, the block walk (k_walk, a lane
+// a query) little for a query of few and more the more there are.  So a large batch's fill is launched
+// both ways, and the batch's hits, which only the device knows, say which one runs: the walk for
+// [walk_few, walk_many) hits a query; the other way's kernels end at once, 4 us in all.  us swept and
+// walked, descending order, int32: 2.5M queries on 3M intervals with 0.06 hits 128 and 85, with 12
+// (most in the run) 198 and 150, with 25 252 and 213, with 50 308 and 329; lognormal lengths: 1M on
+// 1M with 12 hits 97 and 95, on 1.5M with 18 106 and 113; 6M on 30K with 2 hits 215 and 217, 6
+// hits 458 and 347.  Vector order: 1M on 1M with 12 hits 126 and 100, on 2M with 24 138 and 136;
+// values 129 and 97, 159 and 138, on 3M with 37 175 and 243.  Smaller batches, and smaller ones still
+// where the queries lie closer than the intervals, would pay more for the second launch than they gain.
+inline bool walk_too(size_t nq, size_t n) { return nq >= ((size_t)1 << 20) || (nq >= ((size_t)1 << 19) && nq < 4 * n); }
+inline uint64_t walk_few(int mode, size_t nq, size_t n) { return nq >= (mode == W_DESC ? n : 4 * n) ? 6u : 0u; }
+constexpr uint64_t walk_many(int mode) { return mode == W_DESC ? 16u : mode == W_VECTOR ? 22u : 28u; }
+
 template <typename S, int MODE>
 int launch_walk(const siIndex* ix, void* plan, size_t nq, uint32_t* counts, uint64_t* counts64,
                 const uint64_t* offsets, uint32_t* out_idx, int32_t* out_val, hipStream_t st,
@@ -2386,30 +2410,29 @@ int launch_walk(const siIndex* ix, void* plan, size_t nq, uint32_t* counts, uint
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
         cus = std::max(cus, 1);
     }
-    k_walk_counters_reset<<<1, 64, 0, st>>>(pv.counter);
+    // An index with start > end (whose run [lower_bound, upper_bound] may hold misses) and range_skip =
+    // 0 take the line walk.  Other fills are swept, or, in large batches, what the batch's hits say.
+    const bool sweep = MODE != W_COUNT && range_skip_on(ix), either = sweep && walk_too(nq, ix->n);
+    k_walk_counters_reset<<<1, 64, 0, st>>>(pv.counter, sweep, either ? offsets : nullptr, (uint32_t)nq,
+                                            walk_few(MODE, nq, ix->n) * nq, walk_many(MODE) * nq);
     LAUNCH_CHECK();
-    bool swept = false;
     if constexpr (MODE != W_COUNT) {
-        // the sweep answers every query of an index without start > end; the line walk is for the
-        // others (the run [lower_bound, upper_bound] may hold misses there) and for range_skip = 0
-        swept = range_skip_on(ix);
-        if (swept) {
+        if (sweep) {
             const uint32_t chunk = sweep_chunk(nq, cus);
             k_sweep<S, MODE><<<grid_for(nq, chunk * SW_WAVES), SW_THREADS, 0, st>>>(
-                ix->view<S>(), ix->tree<S>(), nullptr, pv, (uint32_t)nq, chunk, offsets,
+                ix->view<S>(), ix->tree<S>(), nullptr, pv, (uint32_t)nq, chunk, either, offsets,
                 MODE == W_VALUES ? (uint32_t*)out_val : out_idx, ix->d_values, cap);
             LAUNCH_CHECK();
-            return launch_sweep_shared<S, MODE>(ix, pv, nq, chunk, cus, offsets, out_idx, out_val, cap, st);
+            const int rc = launch_sweep_shared<S, MODE>(ix, pv, nq, chunk, cus, offsets, out_idx, out_val, cap, st);
+            if (rc || !either) return rc;
         }
     }
-    if (!swept) {
-        uint32_t tile = 0, ntiles = 0;
-        unsigned grid = 0;
-        walk_shape<S, MODE>(nq, &tile, &ntiles, &grid);
-        k_walk<S, MODE><<<grid, T_THREADS, 0, st>>>(
-            ix->view<S>(), pv, (uint32_t)nq, tile, ntiles, g_tune.lane_steps, range_skip_on(ix), pv.counter, counts,
-            counts64, offsets, out_idx, ix->d_values, out_val, cap, nullptr, MultiTiles{nullptr, nullptr, nullptr, 0u});
-    }
+    uint32_t tile = 0, ntiles = 0;
+    unsigned grid = 0;
+    walk_shape<S, MODE>(nq, &tile, &ntiles, &grid);
+    k_walk<S, MODE><<<grid, T_THREADS, 0, st>>>(
+        ix->view<S>(), pv, (uint32_t)nq, tile, ntiles, g_tune.lane_steps, range_skip_on(ix), pv.counter, counts,
+        counts64, offsets, out_idx, ix->d_values, out_val, cap, nullptr, MultiTiles{nullptr, nullptr, nullptr, 0u});
     LAUNCH_CHECK();
     // parked (heavy) walks: one wave each, resident grid, exits at once when none were parked
     IndexView<S> hv = ix->view<S>();
@@ -3244,8 +3267,6 @@ int launch_walk_multi(const siSetTable* tb, void* plan, size_t nq, const uint64_
         cus = std::max(cus, 1);
         per = std::max(per, 1);
     }
-    k_walk_counters_reset<<<1, 64, 0, st>>>(pv.counter);
-    LAUNCH_CHECK();
     const SetView<int32_t>* sets = (const SetView<int32_t>*)tb->d_views;
     // The sweep leaves every query of a set with start > end to the wave-cooperative kernel, the lane
     // walk answers them itself: a table that holds such a set takes the walk (8 sets of 1M intervals
@@ -3253,6 +3274,8 @@ int launch_walk_multi(const siSetTable* tb, void* plan, size_t nq, const uint64_
     // 1000 queries on 4 sets: 68 us and 10).
     bool walk = false;
     for (const siIndex* ix : tb->sets) walk |= ix && !rank_exact(ix);
+    k_walk_counters_reset<<<1, 64, 0, st>>>(pv.counter, walk ? 0u : 1u, nullptr, 0u, 0u, 0u);
+    LAUNCH_CHECK();
     if (walk) {
         const int wgs = (g_tune.fill_wgs > 0) ? std::min(g_tune.fill_wgs, per) : per;
         const uint32_t tile = multi_tile();
@@ -3267,7 +3290,7 @@ int launch_walk_multi(const siSetTable* tb, void* plan, size_t nq, const uint64_
     } else {
         const uint32_t chunk = sweep_chunk(nq, cus), span = shared_span(nq, chunk, cus, MODE);
         k_sweep<int32_t, MODE, true><<<grid_for(nq, chunk * SW_WAVES), SW_THREADS, 0, st>>>(
-            IndexView<int32_t>{}, TreeDesc<int32_t>{}, sets, pv, (uint32_t)nq, chunk, offsets, out_idx, nullptr, cap);
+            IndexView<int32_t>{}, TreeDesc<int32_t>{}, sets, pv, (uint32_t)nq, chunk, false, offsets, out_idx, nullptr, cap);
         LAUNCH_CHECK();
         k_sweep_shared<int32_t, MODE, true><<<shared_grid(nq, span, cus, sh_wgs<int32_t>(MODE)), SH_THREADS, 0, st>>>(
             IndexView<int32_t>{}, TreeDesc<int32_t>{}, UbTree<int32_t>{}, BucketView<int32_t>{}, LongView<int32_t>{}, sets, pv,

@@ -543,13 +543,15 @@ __device__ __forceinline__ void sweep_queries(const IndexView<S>& ix, const Tree
 
 // One wave per chunk of `chunk` consecutive sorted queries.  MODE: W_DESC, W_VECTOR or W_VALUES.
 // A chunk's heavy entries lie at its first query's place, their number in the first one's pad.
+// either: the plan's counters say whether the sweep answers.
 // MULTI: the plan's queries are sorted by their set (pv.set), a chunk's are answered set by set.
 template <typename S, int MODE, bool MULTI = false>
 __global__ __launch_bounds__(SW_THREADS) void k_sweep(IndexView<S> ix, TreeDesc<S> td, const SetView<S>* __restrict__ sets,
-                                                      PlanView<S> pv, uint32_t nq, uint32_t chunk,
+                                                      PlanView<S> pv, uint32_t nq, uint32_t chunk, bool either,
                                                       const uint64_t* __restrict__ offsets,
                                                       uint32_t* __restrict__ out, const int32_t* __restrict__ vals,
                                                       uint64_t cap) {
+    if (either && uniform(pv.counter[2]) == 0u) return;   // the block walk answers
     __shared__ S s_end[SW_WAVES][SW_CAP];
     __shared__ uint32_t s_pay[SW_WAVES][SW_CAP];
     __shared__ uint32_t s_key[SW_WAVES][SW_CHUNK];
@@ -652,7 +654,7 @@ __global__ __launch_bounds__(SH_THREADS) __attribute__((amdgpu_waves_per_eu(sh_w
     __shared__ uint32_t q_top[WAVE], q_p0[WAVE], q_j[WAVE], q_left[WAVE], q_room[WAVE], q_bound[WAVE];
     __shared__ uint32_t q_cur[WAVE], q_set[MULTI ? WAVE : 1];
     __shared__ uint32_t w_tot[2][SH_WAVES], s_n, s_work;
-    if (uniform(pv.counter[1]) == 0u) return;   // nothing was left
+    if (uniform(pv.counter[1]) == 0u || uniform(pv.counter[2]) == 0u) return;   // nothing was left (by the sweep)
     const int lane = lane_id();
     const uint32_t wv = uniform(threadIdx.x / WAVE);
     EntryDeal deal(pv.counter + 8, (nq + span - 1u) / span, blockIdx.x, gridDim.x);

@@ -68,10 +68,9 @@ def test_tuning_knobs_round_trip():
 
 
 def test_tuner_judges_by_what_reads_a_knob(monkeypatch, tmp_path):
-    """Where fills are the sweep, which reads neither tile nor workgroups nor step budget, these are
+    """Where the fill is the sweep, which reads neither tile nor workgroups nor step budget, these are
     judged by the count walk's time alone, whatever the fill's noise says, and fill_wgs stays;
-    where fills walk (an index with start > end: no lower bounds in the plan; or range_skip 0), the
-    fill's time counts as well.  Times are made up here; nothing runs on a GPU."""
+    where it walks (as the plan says after a fill), the fill's time counts as well.  Times are made up here; nothing runs on a GPU."""
     import torch
     from superintervals_amd import autotune
 
@@ -81,7 +80,8 @@ def test_tuner_judges_by_what_reads_a_knob(monkeypatch, tmp_path):
         def count_planned(self, *a, **k):
             return "count"
 
-        def fill_planned(self, *a, **k):
+        def fill_planned(self, plan, *a, **k):
+            plan[8] = self.swept
             return "fill"
 
     timed = []
@@ -98,10 +98,10 @@ def test_tuner_judges_by_what_reads_a_knob(monkeypatch, tmp_path):
     saved = autotune.current()
     off, idx = torch.zeros(9, dtype=torch.int64), torch.zeros(4, dtype=torch.int32)
     try:
-        for lower_bounds, range_skip, swept in ((1, 1, True), (0, 1, False), (1, 0, False)):
-            autotune.apply(dict(saved, range_skip=range_skip, fill_wgs=3))
+        for swept in (True, False):
+            autotune.apply(dict(saved, fill_wgs=3))
             plan = torch.zeros(256, dtype=torch.uint8)
-            plan[16] = lower_bounds
+            Index.swept = int(swept)
             timed.clear()
             best, _ = autotune.tune(Index(), plan, 8, off, idx, stream="none")
             want = (2048, 64, 3) if swept else (512, 1024, 1)

@@ -1920,16 +1920,99 @@ def test_sweep_of_full_chunks(sia, orc, dtype):
     s[:n // 10] = rng.integers(0, hot, n // 10)
     e = s + np.where(s < hot, rng.integers(1, 1200, n), rng.integers(0, 90, n))
     qs = rng.integers(0, 5_000_000, nq)
-    qs[::40] = rng.integers(0, hot, len(qs[::40]))
+    qs[::1000] = rng.integers(0, hot, len(qs[::1000]))
     qe = qs + rng.integers(0, 60, nq)
     qe[7::1001] = qs[7::1001] - 30
     s, e, qs, qe = (x.astype(dtype) for x in (s, e, qs, qe))
     vals = (np.arange(n, dtype=np.int64) * 7 % 1_000_003).astype(np.int32)
     ix, oix = _dev_index(sia, s, e, vals), orc.build_index(s, e, vals)
-    assert (orc.count_batch(oix, qs, qe) > 300).sum() > 20_000
+    counts = orc.count_batch(oix, qs, qe)
+    assert (counts > 300).sum() > 8_000 and counts.mean() < 6   # (the sweep's: many queries of few hits)
     for order, mode in (("desc", 0), ("vector", 1), ("values", 0)):
         off, out = ix.search(qs, qe, values=True) if order == "values" else ix.search(qs, qe, order=order)
         woff, widx = orc.search_batch(oix, qs, qe, mode=mode)
         assert np.array_equal(off, woff)
         assert np.array_equal(out, oix["data"][widx] if order == "values" else widx), order
+    ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_fills_by_the_hits_of_the_batch(sia, orc, dtype):
+    """A large batch's fill is the walk or the sweep by its hits, which only the device knows: batches
+    of 2, 5 (on few intervals), 12, 20, 26 and 40 hits a query in each order say in the plan which one
+    it was, and both give the oracle's lists, inverted queries and a capacity below the total included; a
+    captured fill follows the hits of each replay."""
+    import torch
+    print(f"[gpu] fills by hits {np.dtype(dtype).name}", flush=True)
+    rng = np.random.default_rng(8)
+    nq = 1 << 20
+    few = {"desc": (6, 16), "vector": (6, 22), "values": (6, 28)}
+    for n, batches in ((200_000, (2, 5, 12, 20, 26, 40)), (1_500_000, (2, 12, 40))):
+        span = 20 * n
+        s = rng.integers(0, span, n)
+        e = s + rng.integers(0, 21, n)                       # half an interval holds a point
+        vals = rng.integers(-9, 9, n).astype(np.int32)
+        ix, oix = _dev_index(sia, s.astype(dtype), e.astype(dtype), vals), orc.build_index(s.astype(dtype), e.astype(dtype), vals)
+        dev = lambda x: torch.from_numpy(x).cuda()
+        plan = torch.empty(ix.plan_bytes(nq), dtype=torch.uint8, device="cuda")
+        off = torch.empty(nq + 1, dtype=torch.int64, device="cuda")
+        for hits in batches:
+            qs = rng.integers(0, span, nq)
+            qe = qs + rng.integers(0, int(40 * (hits - 0.5)), nq)
+            qe[::5003] = qs[::5003] - 7
+            qs, qe = qs.astype(dtype), qe.astype(dtype)
+            ix.plan_device(dev(qs), dev(qe), plan)
+            ix.offsets_planned(plan, nq, off)
+            for order, mode in (("desc", 0), ("vector", 1), ("values", 0)):
+                woff, widx = orc.search_batch(oix, qs, qe, mode=mode)
+                mean = woff[-1] / nq
+                lo, hi = few[order]
+                lo = lo if nq >= (n if order == "desc" else 4 * n) else 0
+                want = oix["data"][widx] if order == "values" else widx
+                for capacity in (int(woff[-1]), int(woff[-1]) * 2 // 3):
+                    out = torch.full((len(want) + 64,), -77, dtype=torch.int32, device="cuda")
+                    if order == "values":
+                        sia._native.check(sia._native.lib.siSearchValuesFillPlannedBounded(
+                            ix.handle, plan.data_ptr(), nq, off.data_ptr(), out.data_ptr(), capacity, None), "fill")
+                    else:
+                        ix.fill_planned(plan, nq, off, out, order=order, capacity=capacity)
+                    torch.cuda.synchronize()
+                    assert int(plan[8:12].view(torch.int32).item()) == int(not lo <= mean < hi), (n, hits, order)
+                    got = out.cpu().numpy()
+                    assert np.array_equal(got[:capacity], want[:capacity]) and np.all(got[capacity:] == -77), (n, hits, order)
+        ix.close()
+    # one captured graph, replayed for batches of either kind
+    n = 300_000
+    s = rng.integers(0, 20 * n, n)
+    e = s + rng.integers(0, 21, n)
+    s, e = s.astype(dtype), e.astype(dtype)
+    ix, oix = _dev_index(sia, s, e), orc.build_index(s, e)
+    tqs, tqe = torch.zeros(nq, dtype=torch.int32 if dtype == np.int32 else torch.int64, device="cuda"), None
+    tqe = torch.zeros_like(tqs)
+    out = torch.empty(60 * nq, dtype=torch.int32, device="cuda")
+    g, st = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    from superintervals_amd import autotune
+    saved = autotune.current()
+    try:
+        autotune.apply({"plan_sync": 0})
+        with torch.cuda.graph(g, stream=st):
+            ix.plan_device(tqs, tqe, plan, stream=st)
+            ix.offsets_planned(plan, nq, off, stream=st)
+            ix.fill_planned(plan, nq, off, out, capacity=out.numel(), stream=st)
+        for hits, swept in ((12, 0), (40, 1), (8, 0), (3, 1), (10, 0)):
+            qs = rng.integers(0, 20 * n, nq)
+            qe = qs + rng.integers(0, int(40 * (hits - 0.5)), nq)
+            qs, qe = qs.astype(dtype), qe.astype(dtype)
+            tqs.copy_(dev(qs))
+            tqe.copy_(dev(qe))
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            woff, widx = orc.search_batch(oix, qs, qe, mode=0)
+            assert np.array_equal(off.cpu().numpy(), woff) and np.array_equal(out[:len(widx)].cpu().numpy(), widx)
+            assert int(plan[8:12].view(torch.int32).item()) == swept, hits
+            _ = (out[:1000].to(torch.int64) * 3).sum().item()   # eager work between replays
+    finally:
+        autotune.apply(saved)
+    del g
     ix.close()
