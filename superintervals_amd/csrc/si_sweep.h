@@ -253,11 +253,22 @@ __device__ __forceinline__ void sweep_emit(SweepGroup<S>& g, uint64_t todo, int 
         {
             const __amdgpu_buffer_rsrc_t rs =
                 __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(at), (short)0, (int)(w * 4u), 0x00020000);
-            for (uint32_t x = 0; x < w; x += WAVE) {
-                // (lanes past the run read a value too: position 0's)
-                const uint32_t v = VALUES ? (uint32_t)vals[x + (uint32_t)lane < w ? p : 0u] : p;
-                __builtin_amdgcn_raw_buffer_store_b32(v, rs, lane4 + x * 4u, 0, 0);
-                p += (MODE == W_VECTOR) ? (uint32_t)WAVE : 0u - (uint32_t)WAVE;
+            if (VALUES) {
+                // two loads before their stores, as a load waits for the stores before it (2.5M queries on 3M int32
+                // intervals that start at 60K places, 75 hits each: 594 us one by one, 541; the walk 466)
+                for (uint32_t x = 0; x < w; x += 2u * WAVE) {
+                    // (lanes past the run read a value too: position 0's)
+                    const uint32_t a = (uint32_t)vals[x + (uint32_t)lane < w ? p : 0u];
+                    const uint32_t b = (uint32_t)vals[x + (uint32_t)lane + WAVE < w ? p - (uint32_t)WAVE : 0u];
+                    __builtin_amdgcn_raw_buffer_store_b32(a, rs, lane4 + x * 4u, 0, 0);
+                    __builtin_amdgcn_raw_buffer_store_b32(b, rs, lane4 + (x + WAVE) * 4u, 0, 0);
+                    p -= 2u * (uint32_t)WAVE;
+                }
+            } else {
+                for (uint32_t x = 0; x < w; x += WAVE) {
+                    __builtin_amdgcn_raw_buffer_store_b32(p, rs, lane4 + x * 4u, 0, 0);
+                    p += (MODE == W_VECTOR) ? (uint32_t)WAVE : 0u - (uint32_t)WAVE;
+                }
             }
         }
         if (NB >= 0) {
