@@ -2791,11 +2791,12 @@ SI_EXPORT int siGatherKeys(const siIndex* ix, const uint32_t* idx, size_t n, voi
 
 // Intersection pieces (superintervals.hpp:1158-1174): hit j of query k (search_idxs
 // vector order) gives [max(a_s, b_s), min(a_e, b_e)] with A's data (the default combine)
-// and B's.  The grid's waves share the hits evenly, whatever query they belong to: a wave finds
-// the query of its first hit, then holds 64 queries at a time (a lane each, and in LDS for the hits
+// and B's.  The grid's waves share queries and hits together evenly, whatever query a hit belongs to (by
+// hits alone, a wave went past thousands of queries without any: 200K queries with 0.02 hits each
+// 159 us, so 5.8, one thread per query 5.2): a wave finds the query of its first hit, then holds 64 queries at a time (a lane each, and in LDS for the hits
 // to look up) and goes through the hits PC_HITS at a time, which mark where a query's hits
 // begin; ballots of the marks number the others.  200K queries with 12 hits each on 1M int32
-// intervals: 30 us, 1.6 TB/s of hits and pieces, bound by the launch and a few dependent reads a
+// intervals: 27 us, 1.8 TB/s of hits and pieces, bound by the launch and a few dependent reads a
 // wave (one thread per query, every store to lines of its own: 421 us).  2 and 8 hits: the same.
 constexpr int PC_WAVES = Q_THREADS / WAVE;
 constexpr int PC_ITEMS = 4;                          // hits per lane and step
@@ -2817,24 +2818,39 @@ __global__ __launch_bounds__(Q_THREADS) void k_intersect_pieces(IndexView<S> ix,
     uint8_t* const mark = reinterpret_cast<uint8_t*>(l_mark[wv]);
     const uint64_t first = off[0], total = off[na] - first;
     const uint64_t waves = (uint64_t)gridDim.x * PC_WAVES, w = (uint64_t)blockIdx.x * PC_WAVES + wv;
-    const uint64_t per = ((total + waves - 1u) / waves + PC_HITS - 1u) / PC_HITS * PC_HITS;
-    if (w * per >= total) return;
-    uint64_t j = first + w * per;
-    const uint64_t stop = first + min(w * per + per, total);
-    // the last query with off <= j, 64 samples a step
+    // query k lies at off[k] + k of the joint order, its hits follow it
+    const uint64_t all = first + total + na, even = max((total + na + waves - 1u) / waves, (uint64_t)WAVE);
+    // where hits outnumber queries, more for a wave's start, and parts that begin at whole lines of the
+    // output (200K queries with 12 hits: 32 us, so 27)
+    const bool dense = total > 2 * (uint64_t)na;
+    const uint64_t per = dense ? (even + PC_HITS - 1u) / PC_HITS * PC_HITS : even;
+    const uint64_t at0 = first + w * per, stop = min(at0 + per, all);
+    if (at0 >= all) return;
+    // the last query at or before at0, 64 samples a step
     size_t k0 = 0;
     for (size_t n = na; n > 1;) {
         const size_t step = (n + WAVE - 1) / WAVE, i = (size_t)lane * step;
-        const uint64_t m = __builtin_amdgcn_ballot_w64(i < n && off[k0 + i] <= j);   // (a prefix of the lanes, not empty)
+        const uint64_t m = __builtin_amdgcn_ballot_w64(i < n && off[k0 + i] + (k0 + i) <= at0);   // (a prefix of the lanes, not empty)
         const size_t at = (size_t)(63 - __builtin_clzll(m)) * step;
         k0 += at;
         n = min(step, n - at);
     }
-    while (j < stop) {
+    const auto line = [&](uint64_t x) { return min(dense ? (x + 63u) & ~(uint64_t)63u : x, first + total); };
+    uint64_t j = w ? line(at0 - k0) : first, last = ~(uint64_t)0;   // the part: hits [j, last)
+    while (j < last) {
         // queries k0 .. k0 + 63
         const size_t k = min(k0 + (size_t)lane, na);
         const uint64_t o0 = off[k], o1 = off[min(k + 1, na)];
-        const uint64_t end = off[min(k0 + (size_t)WAVE, na)], to = min(end, stop);
+        const uint64_t end = off[min(k0 + (size_t)WAVE, na)];
+        if (last == ~(uint64_t)0 && (k0 + WAVE >= na || end + (k0 + WAVE) > stop)) {   // the last query at or before stop is here
+            const uint64_t m = __builtin_amdgcn_ballot_w64(k < na && o0 + k <= stop);
+            last = stop < all ? line(stop - (k0 + (size_t)(63 - __builtin_clzll(m)))) : first + total;
+        }
+        const uint64_t to = min(end, last);
+        if (j >= to) {   // (no hits of the part's)
+            k0 += WAVE;
+            continue;
+        }
         const uint64_t some = __builtin_amdgcn_ballot_w64(o1 > o0);
         wave_lds_sync();
         if (k < na) {
@@ -2844,7 +2860,7 @@ __global__ __launch_bounds__(Q_THREADS) void k_intersect_pieces(IndexView<S> ix,
         }
         if (o1 > o0) l_lane[wv][lanes_below(some)] = (uint8_t)lane;
         while (j < to) {
-            const uint32_t n = (uint32_t)min((uint64_t)PC_HITS, to - j);
+            const uint32_t n = (uint32_t)min((uint64_t)(PC_HITS - (uint32_t)(j & 63u)), to - j);
             uint32_t rank = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(o1 > o0 && o0 <= j)) - 1u;   // of j's query
             l_mark[wv][lane] = 0u;
             wave_lds_sync();

@@ -300,3 +300,49 @@ def test_intersection_pieces_balanced(sia, dtype, na):
             assert np.all(got[total:] == -77) and np.all(got[:o0] == -77)
             assert np.array_equal(got[o0:total], want[i][o0:]) if i != skip else np.all(got == -77), (i, skip, k0)
     ix.close()
+
+
+@pytest.mark.parametrize("na", [1, 2, 64, 65, 4097, 300_001])
+@pytest.mark.parametrize("counts", ["few", "last", "first", "two each", "two each and one", "three each", "one of many"])
+def test_intersection_pieces_share_queries_and_hits(sia, na, counts):
+    """Pieces for lists of every kind of share: next to no hits, all of them with the last or the first
+    query, as many as parts that begin anywhere still take (two a query) and one more, lists that
+    begin past the output's start; every piece once, nothing else written."""
+    import torch
+    print(f"[gpu] intersection pieces na={na} {counts}", flush=True)
+    rng = np.random.default_rng(na)
+    c = np.zeros(na, np.int64)
+    if counts == "few":
+        c[rng.integers(0, na, max(1, na // 300))] = 1
+    elif counts in ("last", "first"):
+        c[-1 if counts == "last" else 0] = 1000
+    elif counts == "one of many":
+        c[:] = 5
+        c[na // 2] = 100_000
+    else:
+        c[:] = 3 if counts == "three each" else 2
+        c[rng.permutation(na)[: na // 2]] += 1
+        c[:] = np.where(c == c.max(), c - 1, c) if counts != "three each" else c
+        c[-1] += 2 * na - c.sum() if counts == "two each" else 2 * na + 1 - c.sum() if counts == "two each and one" else 0
+    s = np.arange(5000, dtype=np.int32) * 3
+    e = s + rng.integers(0, 50, 5000).astype(np.int32)
+    vals = rng.integers(-9, 9, 5000).astype(np.int32)
+    ix = sia.DeviceIndex(np.int32).build(s, e, vals)
+    e, vals = (ix.download(values=True)[k] for k in ("ends", "values"))
+    a_s = rng.integers(0, 15_000, na).astype(np.int32)
+    a_e, ad = a_s + 40, rng.integers(-9, 9, na).astype(np.int32)
+    for begin in (0, 77):
+        off = np.concatenate([[0], np.cumsum(c)]) + begin
+        idx = rng.integers(0, 5000, off[-1] + 1).astype(np.int32)
+        k, h = np.repeat(np.arange(na), c), idx[begin:off[-1]]
+        want = [np.maximum(a_s[k], s[h]), np.minimum(a_e[k], e[h]), ad[k], vals[h]]
+        t = [torch.from_numpy(x).cuda() for x in (a_s, a_e, ad, off, idx)]
+        outs = [torch.full((int(off[-1]) + 70,), -77, dtype=torch.int32, device="cuda") for _ in range(4)]
+        sia._native.check(sia._native.lib.siIntersectPieces(ix.handle, *(x.data_ptr() for x in t[:3]), na, t[3].data_ptr(),
+                                                            t[4].data_ptr(), *(o.data_ptr() for o in outs), None), "pieces")
+        torch.cuda.synchronize()
+        for o, w in zip(outs, want):
+            got = o.cpu().numpy()
+            assert np.array_equal(got[begin:off[-1]], w)
+            assert np.all(got[:begin] == -77) and np.all(got[off[-1]:] == -77)
+    ix.close()
