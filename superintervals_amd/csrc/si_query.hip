@@ -2261,7 +2261,9 @@ __device__ __forceinline__ uint32_t sum_below(const int32_t* __restrict__ v, con
 // that start by e and do not end before s; the A - B of them that start in (s, e] add their own
 // start, the others s, to the sum of max(start, s), and the D - C that end in [s, e) their own
 // end, the others e, to the sum of min(end, e): four table searches and four line sums in place of
-// a walk over the hits (1M queries on 1M intervals, 12 hits each: 0.47 ms before).  All sums are
+// a walk over the hits (1M queries on 1M intervals, 12 hits each: 0.47 ms before).  A and C go first: a
+// query without hits needs no more (1M queries with 0.02 hits on 100K: all four together 95 us, two
+// first 33, the walk 53; with 12 hits 91 and 90, the walk 169; 350K on 1M 49 and 54, 129).  All sums are
 // modulo 2^32, as the walk's int32 arithmetic.  Queries with s > e take the walk.
 __global__ __launch_bounds__(Q_THREADS) void k_coverage_rank(IndexView<int32_t> ix, const int32_t* __restrict__ ends_sorted,
                                                              BucketView<int32_t> ts, BucketView<int32_t> te,
@@ -2277,18 +2279,23 @@ __global__ __launch_bounds__(Q_THREADS) void k_coverage_rank(IndexView<int32_t> 
     uint32_t c, acc;
     if (s <= e) {
         const bool s1 = s != INT32_MIN, e1 = e != INT32_MIN;   // s - 1, e - 1 exist
-        const BucketView<int32_t> t[4] = {ts, ts, te, te};
-        const int32_t* const v[4] = {ix.starts, ix.starts, ends_sorted, ends_sorted};
-        const int32_t x[4] = {e, s, s1 ? s - 1 : s, e1 ? e - 1 : e};
-        uint32_t r[4];
-        bucket_ranks<int32_t, 4>(t, v, ix.n, x, r);
-        const uint32_t A = r[0], B = r[1], C = s1 ? r[2] : 0u, D = e1 ? r[3] : 0u;
+        const BucketView<int32_t> t[2] = {ts, te};
+        const int32_t* const v[2] = {ix.starts, ends_sorted};
+        const int32_t xc[2] = {e, s1 ? s - 1 : s}, xl[2] = {s, e1 ? e - 1 : e};
+        uint32_t r[2];
+        bucket_ranks<int32_t, 2>(t, v, ix.n, xc, r);
+        const uint32_t A = r[0], C = s1 ? r[1] : 0u;
         c = A - C;
-        const uint32_t* const es = line_sums + lines;
-        const uint32_t smax = sum_below(ix.starts, line_sums, A) - sum_below(ix.starts, line_sums, B) +
-                              (uint32_t)s * (c - (A - B));
-        const uint32_t smin = sum_below(ends_sorted, es, D) - sum_below(ends_sorted, es, C) + (uint32_t)e * (c - (D - C));
-        acc = smin - smax;
+        acc = 0;
+        if (c) {
+            bucket_ranks<int32_t, 2>(t, v, ix.n, xl, r);
+            const uint32_t B = r[0], D = e1 ? r[1] : 0u;
+            const uint32_t* const es = line_sums + lines;
+            const uint32_t smax = sum_below(ix.starts, line_sums, A) - sum_below(ix.starts, line_sums, B) +
+                                  (uint32_t)s * (c - (A - B));
+            const uint32_t smin = sum_below(ends_sorted, es, D) - sum_below(ends_sorted, es, C) + (uint32_t)e * (c - (D - C));
+            acc = smin - smax;
+        }
     } else {
         coverage_walk(ix, s, e, &c, &acc);
     }
