@@ -381,9 +381,10 @@ struct BuildInfo {
     unsigned long long inverted;   // intervals with start > end
     long long end_lo, end_hi;      // smallest and largest end
     uint32_t long_run;             // 1: a run of equal starts longer than TIE_RUN was left as it was
-    uint32_t crowded[2];           // sampled keys in crowded buckets of the starts' and the sorted ends' tables
+    uint32_t crowded[2][3];        // sampled keys in crowded buckets (CROWD) of the starts' and the sorted ends' tables
     uint32_t gaps[2];              // long gaps of the two tables (BucketGap)
     uint32_t unsorted;             // 1: a start is below the one before it
+    uint32_t pad;
     long long start_lo, start_hi;  // smallest and largest start
 };
 
@@ -617,7 +618,7 @@ struct BucketGap {
     uint32_t from, to, value;   // tab[from .. to) = value
 };
 constexpr uint32_t GAP_WAVE = 4096;       // most entries a wave fills by itself
-constexpr uint32_t CROWD = 4096;          // keys of a crowded bucket
+__device__ constexpr uint32_t CROWD[3] = {32, 256, 4096};   // keys of a crowded bucket, three degrees
 constexpr uint32_t CROWD_STEP = 64;       // every 64th key is sampled
 
 // tab[b] = i for the buckets b above key i - 1's up to key i's, and n above the last key's.
@@ -631,8 +632,9 @@ __global__ __launch_bounds__(256) void k_bucket_table(const S* __restrict__ v, u
     if (i < n) {
         hi = (uint32_t)bucket_of(t, v[i]) + 1u;
         lo = i ? (uint32_t)bucket_of(t, v[i - 1]) + 1u : 0u;
-        // (a bucket of more than CROWD keys holds key i + CROWD too, for most of its keys)
-        if (i % CROWD_STEP == 0 && n - i > CROWD && bucket_of(t, v[i + CROWD]) + 1u == hi) atomicAdd(crowded, 1u);
+        // (a bucket of more than CROWD keys holds key i + CROWD too, for half of them from twice as many on)
+        for (int d = 0; d < 3 && i % CROWD_STEP == 0 && n - i > CROWD[d] && bucket_of(t, v[i + CROWD[d]]) + 1u == hi; ++d)
+            atomicAdd(&crowded[d], 1u);
     } else if (i == n) {
         lo = (uint32_t)bucket_of(t, v[n - 1]) + 1u;
         hi = nb + 1u;
@@ -818,7 +820,7 @@ int build_bucket_table(const S* keys, size_t n, int64_t lo, int64_t hi, BucketTa
     BucketGap* const gaps = scratch.take<BucketGap>(bucket_gaps(n));
     const BucketView<S> v{t.d_tab, (S)lo, (S)hi, t.shift};
     k_bucket_table<S><<<grid_for(n + 1, 256), 256, 0, st>>>(keys, (uint32_t)n, v, nb, t.d_tab, gaps, &info->gaps[which],
-                                                            &info->crowded[which]);
+                                                            info->crowded[which]);
     LAUNCH_CHECK();
     if (nb > GAP_WAVE) {
         k_bucket_gaps<<<64, 256, 0, st>>>(gaps, &info->gaps[which], t.d_tab);
@@ -1208,9 +1210,10 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     HIP_TRY(hipStreamSynchronize(st));
     // A search in a bucket of m keys takes about log2(m) - 2 reads after the table's, one through the
     // 64-ary tree 14 (n > 4095 x 64): the tables are used unless half of the keys share a bucket
-    // with more than 4096 others.
-    const uint32_t half = (uint32_t)(n / CROWD_STEP / 2);
-    ix->ubt.ok = ix->ebt.ok = !back.info.unsorted && back.info.crowded[0] <= half && back.info.crowded[1] <= half;
+    // with more than 4096 others (what large batches do from 64 on: count_by_plan, bound_by_tree).
+    const auto half = [&](int d) { return std::max(back.info.crowded[0][d], back.info.crowded[1][d]) > n / CROWD_STEP / 2; };
+    ix->ubt.ok = ix->ebt.ok = !back.info.unsorted && !half(2);
+    ix->ubt.busy = ix->ebt.busy = half(1) ? 2 : half(0) ? 1 : 0;
     ix->built = true;
     ix->last_build_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

@@ -59,11 +59,13 @@ struct KeyTree {
 struct BucketTable {
     uint32_t* d_tab = nullptr;
     bool ok = false;          // false: too many keys share a bucket, the search trees are used
+    int busy = 0;             // 1, 2: half of the keys share a bucket with more than 64, 512 others or so
     int64_t lo = 0, hi = 0;
     uint32_t shift = 0;
     void release() {
         d_tab = nullptr;
         ok = false;
+        busy = 0;
     }
     template <typename S>
     BucketView<S> view() const { return BucketView<S>{ok ? d_tab : nullptr, (S)lo, (S)hi, shift}; }

@@ -2107,6 +2107,19 @@ inline bool group_coverage(size_t nq, size_t bytes) {
     return bytes >= ((size_t)256 << 10) &&
            nq >= (bytes >= ((size_t)8 << 20) ? 3u << 17 : bytes >= ((size_t)2 << 20) ? 3u << 18 : 5u << 18);
 }
+// Large batches on large indexes whose intervals lie in few of the buckets (one far off stretches them) count
+// through the sorted plan, whose neighbours read the same keys: 4M queries on 10M int64 intervals with 64 keys
+// in a bucket 798 us, through the plan 652, with 512 1627 and 649, with 32 549 and 653; 10M int32, 128: 785
+// and 478; 1M int64, 512: 832 and 554, 128: 417 and 546; 100K, 3500: 304 and 351.
+inline bool count_by_plan(int busy, size_t nq, size_t bytes) {
+    return nq >= 1000000 && (bytes >= ((size_t)32 << 20) ? busy >= 1 : bytes >= ((size_t)4 << 20) && busy >= 2);
+}
+// upper_bound goes through the search tree where buckets are busy: 4M int64 queries on 10M intervals with 64 keys
+// in a bucket 457 us, through the tree 366, with 16 381 and 373; 1M, 128: 205 and 228, 3500: 271 and 229; 100K,
+// 64: 136 and 115; int32, 10M, 128: 383 and 341; 1M, 128: 128 and 190; 100K, 64: 97 and 110, 512: 133 and 111.
+inline bool bound_by_tree(int busy, size_t bytes) {
+    return busy >= 2 || (busy == 1 && (bytes >= ((size_t)32 << 20) || bytes < ((size_t)2 << 20)));
+}
 template <typename S>
 int launch_count_table(const siIndex* ix, const S* qs, const S* qe, size_t nq, uint32_t* counts, hipStream_t st) {
     const bool group = group_counts(nq, ix->n * sizeof(S));
@@ -2669,7 +2682,8 @@ SI_EXPORT int siCount(const siIndex* ix, const void* qs, const void* qe, size_t 
         const uintptr_t a = (uintptr_t)counts, b = (uintptr_t)q;
         return a < b + nq * ix->cb && b < a + nq * 4;
     };
-    if (g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF && !over(qs) && !over(qe))
+    if (g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF && !over(qs) && !over(qe) &&
+        !count_by_plan(ix->ubt.busy, nq, ix->n * ix->cb))
         return DISPATCH_S(ix, (launch_count_table<S>(ix, (const S*)qs, (const S*)qe, nq, counts, st)));
     ScopedPlan P(st);
     const size_t pb = siPlanBytes(ix, nq);
@@ -2738,7 +2752,7 @@ SI_EXPORT int siUpperBound(const siIndex* ix, const void* xs, size_t n, uint32_t
     if (n == 0) return SI_OK;
     if (!xs || !out) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
-    if (g_tune.ub_tree && ix->ubt.ok)
+    if (g_tune.ub_tree && ix->ubt.ok && !bound_by_tree(ix->ubt.busy, ix->n * ix->cb))
         return DISPATCH_S(ix, ([&]() -> int {
             k_upper_bound_table<S><<<grid_for(n, Q_THREADS), Q_THREADS, 0, st>>>((const S*)ix->d_starts, (uint32_t)ix->n,
                                                                                  ix->ubt.view<S>(), (const S*)xs, n, out);

@@ -2016,3 +2016,47 @@ def test_fills_by_the_hits_of_the_batch(sia, orc, dtype):
         autotune.apply(saved)
     del g
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+@pytest.mark.parametrize("n,keys", [(100_000, 40), (100_000, 100), (100_000, 1000), (1_200_000, 100), (1_200_000, 1000),
+                                    (9_000_000, 100)])
+def test_busy_buckets(sia, orc, dtype, n, keys):
+    """Indexes most of whose intervals share a bucket with about `keys` others, as one interval far off
+    makes them (few, busy, very busy: large counts through the plan, upper_bound through the tree):
+    upper_bound, count, has_overlaps and coverage for batches below and above a million queries."""
+    import torch
+    print(f"[gpu] busy buckets {np.dtype(dtype).name} n={n} keys={keys}", flush=True)
+    rng = np.random.default_rng(n + keys)
+    span = 2 * n
+    s = rng.integers(0, span, n)
+    s[n // 2] = min(span * keys // 4, 2**31 - 50)
+    e = s + rng.integers(0, 9, n)
+    o = np.lexsort((-e, s))
+    s, e = s[o].astype(dtype), e[o].astype(dtype)
+    ix = sia.DeviceIndex(dtype).build(s, e, None, start_sorted=True, end_sorted=True)
+    by_end = np.sort(e)
+    lib, check = sia._native.lib, sia._native.check
+    for nq in (5000, 999_999, 1_000_001):
+        qs = rng.integers(-50, span + 50, nq)
+        qe = qs + rng.integers(0, 20, nq)
+        qs[:3] = int(s[-1]) + np.array([-1, 0, 60])
+        qe[:3] = qs[:3] + 1
+        qs, qe = qs.astype(dtype), qe.astype(dtype)
+        t = [torch.from_numpy(x).cuda() for x in (qs, qe)]
+        out = torch.full((nq + 8,), 5, dtype=torch.int32, device="cuda")
+        any_ = torch.full((nq + 8,), 5, dtype=torch.uint8, device="cuda")
+        last = np.searchsorted(s, qe, side="right")
+        check(lib.siUpperBound(ix.handle, t[1].data_ptr(), nq, out.data_ptr(), None), "siUpperBound")
+        assert np.array_equal(out[:nq].cpu().numpy(), last - 1) and bool((out[nq:] == 5).all())
+        check(lib.siCount(ix.handle, t[0].data_ptr(), t[1].data_ptr(), nq, out.data_ptr(), None), "siCount")
+        counts = last - np.searchsorted(by_end, qs)
+        assert np.array_equal(out[:nq].cpu().numpy(), counts) and bool((out[nq:] == 5).all())
+        check(lib.siHasOverlaps(ix.handle, t[0].data_ptr(), t[1].data_ptr(), nq, any_.data_ptr(), None), "siHasOverlaps")
+        assert np.array_equal(any_[:nq].cpu().numpy(), (last > 0) & (e[np.maximum(last - 1, 0)] >= qs))
+        if dtype == np.int32 and n <= 1_200_000:
+            c, v = ix.coverage(qs[:2000], qe[:2000])
+            oix = orc.build_index(s, e) if nq == 5000 else oix
+            want = [orc.coverage(oix, a, b) for a, b in zip(qs[:300], qe[:300])]
+            assert np.array_equal(c, counts[:2000]) and np.array_equal(v[:300], [w[1] for w in want])
+    ix.close()
