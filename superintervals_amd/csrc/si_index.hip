@@ -600,17 +600,6 @@ __global__ __launch_bounds__(256) void k_line_sums(const int32_t* __restrict__ a
     out[k] = sum;
 }
 
-template <typename S>
-__global__ void k_ranges(const S* __restrict__ starts, const S* __restrict__ sorted, size_t n,
-                         BuildInfo* __restrict__ info) {
-    if (threadIdx.x == 0) {
-        info->start_lo = (long long)starts[0];
-        info->start_hi = (long long)starts[n - 1];
-        info->end_lo = (long long)sorted[0];
-        info->end_hi = (long long)sorted[n - 1];
-    }
-}
-
 // ---- bucket tables (BucketView) ----------------------------------------------------------
 // Entries of a table between the buckets of two neighbouring keys that are too many for one
 // wave; filled by k_bucket_gaps.
@@ -618,23 +607,62 @@ struct BucketGap {
     uint32_t from, to, value;   // tab[from .. to) = value
 };
 constexpr uint32_t GAP_WAVE = 4096;       // most entries a wave fills by itself
-__device__ constexpr uint32_t CROWD[3] = {32, 256, 4096};   // keys of a crowded bucket, three degrees
-constexpr uint32_t CROWD_STEP = 64;       // every 64th key is sampled
+
+// At most max(n / 4, 1) buckets of a power of two of values over a span: its exponent.
+__host__ __device__ inline uint32_t bucket_shift(uint64_t span, uint64_t n) {
+    const uint64_t most = n / 4 ? n / 4 : 1;
+    uint32_t shift = 0;
+    while ((span >> shift) >= most && shift < 63) ++shift;
+    return shift;
+}
+
+// The ranges of the sorted starts and ends, and how crowded their buckets will be: of CROWD_SAMPLE keys
+// those that share one with the CROWD-th key after them, three degrees (in a bucket of m keys m - CROWD do,
+// half from twice as many on).  One workgroup, before the tables: counted by the kernel that fills them, an
+// atomic a sample, 10M intervals in 20 clusters took 5.5 ms to build, so 2.6.
+__device__ constexpr uint32_t CROWD[3] = {32, 256, 4096};
+constexpr uint32_t CROWD_SAMPLE = 512;   // (4096: 40 us, the misses of one CU)
+template <typename S>
+__global__ __launch_bounds__(CROWD_SAMPLE) void k_ranges(const S* __restrict__ starts, const S* __restrict__ sorted, size_t n,
+                                                 BuildInfo* __restrict__ info) {
+    __shared__ uint32_t s_c[2][3];
+    if (threadIdx.x < 6) s_c[threadIdx.x / 3][threadIdx.x % 3] = 0;
+    __syncthreads();
+    for (int which = 0; which < 2; ++which) {
+        const S* const v = which ? sorted : starts;
+        const S lo = v[0], hi = v[n - 1];
+        const BucketView<S> t{nullptr, lo, hi, bucket_shift((uint64_t)hi - (uint64_t)lo, n)};
+        if (threadIdx.x == 0) {
+            (which ? info->end_lo : info->start_lo) = (long long)lo;
+            (which ? info->end_hi : info->start_hi) = (long long)hi;
+        }
+        const size_t i = (uint64_t)threadIdx.x * n / CROWD_SAMPLE;
+        const uint64_t b = bucket_of(t, v[i]);
+        bool with[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) with[d] = n - i > CROWD[d] && bucket_of(t, v[i + (n - i > CROWD[d] ? CROWD[d] : 0u)]) == b;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const uint64_t m = __ballot(with[d]);
+            if (lane_id() == 0 && m) atomicAdd(&s_c[which][d], (uint32_t)__popcll(m));
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) info->crowded[threadIdx.x / 3][threadIdx.x % 3] = s_c[threadIdx.x / 3][threadIdx.x % 3];
+}
 
 // tab[b] = i for the buckets b above key i - 1's up to key i's, and n above the last key's.
 template <typename S>
 __global__ __launch_bounds__(256) void k_bucket_table(const S* __restrict__ v, uint32_t n, BucketView<S> t, uint32_t nb,
                                                       uint32_t* __restrict__ tab, BucketGap* __restrict__ gaps,
-                                                      uint32_t* __restrict__ ngaps, uint32_t* __restrict__ crowded) {
+                                                      uint32_t* __restrict__ ngaps, const uint32_t* __restrict__ unsorted) {
+    if (*unsorted) return;   // a key may lie in no bucket: the searches go through the trees
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;   // n included: the entries past the last key
     const int lane = lane_id();
     uint32_t lo = 0, hi = 0;   // entries [lo, hi) are i
     if (i < n) {
         hi = (uint32_t)bucket_of(t, v[i]) + 1u;
         lo = i ? (uint32_t)bucket_of(t, v[i - 1]) + 1u : 0u;
-        // (a bucket of more than CROWD keys holds key i + CROWD too, for half of them from twice as many on)
-        for (int d = 0; d < 3 && i % CROWD_STEP == 0 && n - i > CROWD[d] && bucket_of(t, v[i + CROWD[d]]) + 1u == hi; ++d)
-            atomicAdd(&crowded[d], 1u);
     } else if (i == n) {
         lo = (uint32_t)bucket_of(t, v[n - 1]) + 1u;
         hi = nb + 1u;
@@ -806,21 +834,19 @@ constexpr size_t bucket_gaps(size_t n) { return bucket_entries(n) / GAP_WAVE + 2
 
 // Bucket table over n sorted keys in [lo, hi]: at most n / 4 buckets of a power of two of values.
 // scratch holds bucket_gaps(n) entries.  Whether the table is used (t.ok) is left to the caller,
-// who reads the crowded sample back.
+// who has read the crowded samples back (k_ranges).
 template <typename S>
 int build_bucket_table(const S* keys, size_t n, int64_t lo, int64_t hi, BucketTable& t, BuildInfo* info, int which,
                        Carver scratch, hipStream_t st) {
     t.lo = lo;
     t.hi = hi;
     const uint64_t span = (uint64_t)hi - (uint64_t)lo;
-    const uint64_t most = std::max<uint64_t>(n / 4, 1);
-    t.shift = 0;
-    while ((span >> t.shift) >= most && t.shift < 63) ++t.shift;
+    t.shift = bucket_shift(span, n);
     const uint32_t nb = (uint32_t)(span >> t.shift) + 1u;
     BucketGap* const gaps = scratch.take<BucketGap>(bucket_gaps(n));
     const BucketView<S> v{t.d_tab, (S)lo, (S)hi, t.shift};
     k_bucket_table<S><<<grid_for(n + 1, 256), 256, 0, st>>>(keys, (uint32_t)n, v, nb, t.d_tab, gaps, &info->gaps[which],
-                                                            info->crowded[which]);
+                                                            &info->unsorted);
     LAUNCH_CHECK();
     if (nb > GAP_WAVE) {
         k_bucket_gaps<<<64, 256, 0, st>>>(gaps, &info->gaps[which], t.d_tab);
@@ -1099,8 +1125,8 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
             if (rc != SI_OK) return rc;
             known = sizeof(S) == 4;
         }
-        // ---- ends in ascending order, for the rank form of count
-        {
+        // ---- ends in ascending order, for the rank form of count (whatever the order within equal starts)
+        if (!full) {
             using K = typename std::conditional<sizeof(S) == 4, uint32_t, uint64_t>::type;
             const K* raw = (const K*)ix->d_ends;
             if (!known) {
@@ -1115,33 +1141,12 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
             } else {   // all ends equal
                 HIP_TRY(hipMemcpyAsync(ix->d_ends_sorted, ix->d_ends, nb, hipMemcpyDeviceToDevice, st));
             }
-            k_ranges<S><<<1, 64, 0, st>>>((const S*)ix->d_starts, (const S*)ix->d_ends_sorted, n, info);
+            k_ranges<S><<<1, CROWD_SAMPLE, 0, st>>>((const S*)ix->d_starts, (const S*)ix->d_ends_sorted, n, info);
             LAUNCH_CHECK();
         }
-        // ---- branch and exits, through the 16-ary max tree
-        {
-            Carver m;
-            m.base = (char*)scratch.p;
-            m.used = shared_from;
-            Max16<S> t;
-            t.lv[0] = (const S*)ix->d_ends;
-            t.n = 1;
-            size_t sz = npad;
-            while (sz > 16 && t.n < MAX_LEVELS) {
-                const size_t up = (sz + 15) / 16, pad = (up + 15) & ~(size_t)15;
-                S* const lv = m.take<S>(pad);
-                k_max16<S><<<grid_for(pad, 256), 256, 0, st>>>(t.lv[t.n - 1], (uint32_t)up, (uint32_t)pad, lv);
-                LAUNCH_CHECK();
-                t.lv[t.n++] = lv;
-                sz = up;
-            }
-            for (int l = t.n; l < MAX_LEVELS; ++l) t.lv[l] = nullptr;
-            k_branch_exit<S><<<grid_for(npad / 16, 256), 256, 0, st>>>(t, (const S*)ix->d_starts, (uint32_t)n,
-                                                                       (uint32_t)(npad / 16), ix->d_branch, ix->d_exit,
-                                                                       info);
-            LAUNCH_CHECK();
-        }
-        // ---- the lengths the long list's threshold is chosen from, and the one read-back
+        // ---- the lengths the long list's threshold is chosen from, and the one read-back (before the
+        // stages that another sort would have to repeat: 10M int32 intervals with one run of 50 equal
+        // starts 2.9 ms with them in between, so 2.5, without such a run 1.4)
         const bool sample = n >= LONG_FROM && si_tune_long_len() == 0;
         if (sample) {
             k_len_sample<S><<<grid_for(LEN_SAMPLE, 256), 256, 0, st>>>((const S*)ix->d_starts, (const S*)ix->d_ends,
@@ -1152,16 +1157,35 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
         HIP_TRY(hipStreamSynchronize(st));
         if (presorted || full || !back.info.long_run) break;
         // runs of equal starts too long to mend: sort by (start, end)
-        k_zero_u32<<<1, 64, 0, st>>>((uint32_t*)info, sizeof(BuildInfo) / 4);
+    }
+    // ---- branch and exits, through the 16-ary max tree
+    {
+        Carver m;
+        m.base = (char*)scratch.p;
+        m.used = shared_from;
+        Max16<S> t;
+        t.lv[0] = (const S*)ix->d_ends;
+        t.n = 1;
+        size_t sz = npad;
+        while (sz > 16 && t.n < MAX_LEVELS) {
+            const size_t up = (sz + 15) / 16, pad = (up + 15) & ~(size_t)15;
+            S* const lv = m.take<S>(pad);
+            k_max16<S><<<grid_for(pad, 256), 256, 0, st>>>(t.lv[t.n - 1], (uint32_t)up, (uint32_t)pad, lv);
+            LAUNCH_CHECK();
+            t.lv[t.n++] = lv;
+            sz = up;
+        }
+        for (int l = t.n; l < MAX_LEVELS; ++l) t.lv[l] = nullptr;
+        k_branch_exit<S><<<grid_for(npad / 16, 256), 256, 0, st>>>(t, (const S*)ix->d_starts, (uint32_t)n,
+                                                                   (uint32_t)(npad / 16), ix->d_branch, ix->d_exit,
+                                                                   info);
         LAUNCH_CHECK();
     }
-    // intervals with start > end (queries on such an index take the walk, see siIndex)
-    ix->n_inverted = (size_t)back.info.inverted;
     int rc = build_max_tree<S>((const S*)ix->d_ends, ix->nlev, ix->lvl_off, ix->lvl_size, (S*)ix->d_tree, st);
     if (rc == SI_OK) rc = build_key_tree<S>((const S*)ix->d_starts, shape, ix->ub, st);        // upper_bound
     if (rc == SI_OK) rc = build_key_tree<S>((const S*)ix->d_ends_sorted, shape, ix->eb, st);   // rank count
     if (rc != SI_OK) return rc;
-    if (!back.info.unsorted) {   // (else a key may lie in no bucket: the searches go through the trees)
+    {
         Carver m;
         m.base = (char*)scratch.p;
         m.used = shared_from;
@@ -1208,10 +1232,12 @@ int build_impl(siIndex* ix, const void* starts, const void* ends, const int32_t*
     }
     HIP_TRY(hipMemcpyAsync(&back.info, info, sizeof(BuildInfo), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    // intervals with start > end (queries on such an index take the walk, see siIndex)
+    ix->n_inverted = (size_t)back.info.inverted;
     // A search in a bucket of m keys takes about log2(m) - 2 reads after the table's, one through the
     // 64-ary tree 14 (n > 4095 x 64): the tables are used unless half of the keys share a bucket
     // with more than 4096 others (what large batches do from 64 on: count_by_plan, bound_by_tree).
-    const auto half = [&](int d) { return std::max(back.info.crowded[0][d], back.info.crowded[1][d]) > n / CROWD_STEP / 2; };
+    const auto half = [&](int d) { return std::max(back.info.crowded[0][d], back.info.crowded[1][d]) > CROWD_SAMPLE / 2; };
     ix->ubt.ok = ix->ebt.ok = !back.info.unsorted && !half(2);
     ix->ubt.busy = ix->ebt.busy = half(1) ? 2 : half(0) ? 1 : 0;
     ix->built = true;
