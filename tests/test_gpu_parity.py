@@ -2023,8 +2023,9 @@ def test_fills_by_the_hits_of_the_batch(sia, orc, dtype):
                                     (9_000_000, 100)])
 def test_busy_buckets(sia, orc, dtype, n, keys):
     """Indexes most of whose intervals share a bucket with about `keys` others, as one interval far off
-    makes them (few, busy, very busy: large counts through the plan, upper_bound through the tree):
-    upper_bound, count, has_overlaps and coverage for batches below and above a million queries."""
+    makes them (few, busy, very busy: large counts through the plan, upper_bound and single queries
+    through the trees): upper_bound, count, has_overlaps and coverage for batches below and above a
+    million queries, and single queries."""
     import torch
     print(f"[gpu] busy buckets {np.dtype(dtype).name} n={n} keys={keys}", flush=True)
     rng = np.random.default_rng(n + keys)
@@ -2054,6 +2055,11 @@ def test_busy_buckets(sia, orc, dtype, n, keys):
         assert np.array_equal(out[:nq].cpu().numpy(), counts) and bool((out[nq:] == 5).all())
         check(lib.siHasOverlaps(ix.handle, t[0].data_ptr(), t[1].data_ptr(), nq, any_.data_ptr(), None), "siHasOverlaps")
         assert np.array_equal(any_[:nq].cpu().numpy(), (last > 0) & (e[np.maximum(last - 1, 0)] >= qs))
+        for k in range(30) if nq == 5000 else ():
+            a, b = qs[k:k + 1], qe[k:k + 1]
+            hits = np.flatnonzero(e[:last[k]] >= a[0])[::-1]
+            assert ix.count(a, b)[0] == counts[k] and ix.upper_bound(b)[0] == np.uint32(last[k] - 1)
+            assert np.array_equal(ix.search(a, b)[1].astype(np.int64), hits)
         if dtype == np.int32 and n <= 1_200_000:
             c, v = ix.coverage(qs[:2000], qe[:2000])
             oix = orc.build_index(s, e) if nq == 5000 else oix
