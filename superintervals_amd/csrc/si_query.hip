@@ -2413,8 +2413,8 @@ int launch_sweep_shared(const siIndex* ix, const PlanView<S>& pv, size_t nq, uin
 // hits 458 and 347.  Vector order: 1M on 1M with 12 hits 126 and 100, on 2M with 24 138 and 136;
 // values 129 and 97, 159 and 138, on 3M with 37 175 and 243.  Smaller batches, and smaller ones still
 // where the queries lie closer than the intervals, would pay more for the second launch than they gain.
-inline bool walk_too(size_t nq, size_t n) { return nq >= ((size_t)1 << 20) || (nq >= ((size_t)1 << 19) && nq < 4 * n); }
-inline uint64_t walk_few(int mode, size_t nq, size_t n) { return nq >= (mode == W_DESC ? n : 4 * n) ? 6u : 0u; }
+inline bool walk_too(size_t nq, size_t n) { return nq >= (3u << 18) || (nq >= (1u << 19) && nq < 4 * n); }
+inline uint64_t walk_few(int mode, size_t nq, size_t n) { return nq >= (mode == W_DESC ? n : 3 * n) ? 6u : 0u; }
 constexpr uint64_t walk_many(int mode) { return mode == W_DESC ? 16u : mode == W_VECTOR ? 22u : 28u; }
 
 template <typename S, int MODE>

@@ -1967,7 +1967,7 @@ def test_fills_by_the_hits_of_the_batch(sia, orc, dtype):
                 woff, widx = orc.search_batch(oix, qs, qe, mode=mode)
                 mean = woff[-1] / nq
                 lo, hi = few[order]
-                lo = lo if nq >= (n if order == "desc" else 4 * n) else 0
+                lo = lo if nq >= (n if order == "desc" else 3 * n) else 0
                 want = oix["data"][widx] if order == "values" else widx
                 for capacity in (int(woff[-1]), int(woff[-1]) * 2 // 3):
                     out = torch.full((len(want) + 64,), -77, dtype=torch.int32, device="cuda")
