@@ -2682,12 +2682,19 @@ SI_EXPORT int siCount(const siIndex* ix, const void* qs, const void* qe, size_t 
         const uintptr_t a = (uintptr_t)counts, b = (uintptr_t)q;
         return a < b + nq * ix->cb && b < a + nq * 4;
     };
-    if (g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF && !over(qs) && !over(qe) &&
-        !count_by_plan(ix->ubt.busy, nq, ix->n * ix->cb))
-        return DISPATCH_S(ix, (launch_count_table<S>(ix, (const S*)qs, (const S*)qe, nq, counts, st)));
+    const bool table = g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF &&
+                       !over(qs) && !over(qe);
     ScopedPlan P(st);
     const size_t pb = siPlanBytes(ix, nq);
-    if ((rc = P.alloc(pb))) return rc;
+    bool by_plan = !table;
+    if (table && count_by_plan(ix->ubt.busy, nq, ix->n * ix->cb)) {   // (not in a captured stream, nor without memory for it)
+        hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+        by_plan = hipStreamIsCapturing(st, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
+                  P.alloc(pb, false) == SI_OK;
+        if (!by_plan) (void)hipGetLastError();
+    }
+    if (!by_plan) return DISPATCH_S(ix, (launch_count_table<S>(ix, (const S*)qs, (const S*)qe, nq, counts, st)));
+    if (!P.p && (rc = P.alloc(pb))) return rc;
     if ((rc = siPlanQueries(ix, qs, qe, nq, P.p, pb, stream))) return rc;
     return siCountPlanned(ix, P.p, nq, counts, stream);
 }

@@ -2066,3 +2066,43 @@ def test_busy_buckets(sia, orc, dtype, n, keys):
             want = [orc.coverage(oix, a, b) for a, b in zip(qs[:300], qe[:300])]
             assert np.array_equal(c, counts[:2000]) and np.array_equal(v[:300], [w[1] for w in want])
     ix.close()
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.int64])
+def test_busy_buckets_counted_in_a_graph(sia, dtype):
+    """A large count over busy buckets takes the sorted plan, which reads back which digits vary; a
+    captured one takes the tables, which need neither that nor memory: three replays over new queries,
+    with eager counts between them."""
+    import torch
+    print(f"[gpu] busy buckets in a graph {np.dtype(dtype).name}", flush=True)
+    rng = np.random.default_rng(8)
+    n, nq, keys = 1_200_000, 1_000_001, 1000
+    s = rng.integers(0, 2 * n, n)
+    s[n // 2] = min(2 * n * keys // 4, 2**31 - 50)
+    e = s + rng.integers(0, 9, n)
+    o = np.lexsort((-e, s))
+    s, e = s[o].astype(dtype), e[o].astype(dtype)
+    ix = sia.DeviceIndex(dtype).build(s, e, None, start_sorted=True, end_sorted=True)
+    by_end = np.sort(e)
+    lib, check = sia._native.lib, sia._native.check
+    t = [torch.zeros(nq, dtype=torch.int32 if dtype == np.int32 else torch.int64, device="cuda") for _ in range(2)]
+    out = torch.zeros(nq, dtype=torch.int32, device="cuda")
+    eager = torch.zeros(nq, dtype=torch.int32, device="cuda")
+    g, st = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(g, stream=st):
+        check(lib.siCount(ix.handle, t[0].data_ptr(), t[1].data_ptr(), nq, out.data_ptr(), st.cuda_stream), "siCount")
+    for _ in range(3):
+        qs = rng.integers(-50, 2 * n + 50, nq)
+        qe = qs + rng.integers(0, 20, nq)
+        qs, qe = qs.astype(dtype), qe.astype(dtype)
+        t[0].copy_(torch.from_numpy(qs))
+        t[1].copy_(torch.from_numpy(qe))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        want = np.searchsorted(s, qe, side="right") - np.searchsorted(by_end, qs)
+        assert np.array_equal(out.cpu().numpy(), want)
+        check(lib.siCount(ix.handle, t[0].data_ptr(), t[1].data_ptr(), nq, eager.data_ptr(), None), "siCount")
+        assert np.array_equal(eager.cpu().numpy(), want)
+    del g
+    ix.close()
