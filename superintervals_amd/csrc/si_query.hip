@@ -2677,10 +2677,11 @@ SI_EXPORT int siCount(const siIndex* ix, const void* qs, const void* qe, size_t 
     if (nq == 0) return SI_OK;
     if (!qs || !qe || !counts) return si_set_error(SI_ERR_ARG, "null buffer");
     hipStream_t st = (hipStream_t)stream;
-    // (counts over the queries' own arrays: the plan reads all of these before it writes one)
+    // (counts over the queries' own arrays: the plan reads all of these before it writes one; the tables
+    // read a query before they write the word it lies in)
     const auto over = [&](const void* q) {
         const uintptr_t a = (uintptr_t)counts, b = (uintptr_t)q;
-        return a < b + nq * ix->cb && b < a + nq * 4;
+        return a < b + nq * ix->cb && b < a + nq * 4 && !(a == b && ix->cb == 4);
     };
     const bool table = g_tune.count_rank && g_tune.ub_tree && rank_exact(ix) && ix->ubt.ok && nq < (size_t)0x7FFFFFFF &&
                        !over(qs) && !over(qe);

@@ -2106,3 +2106,37 @@ def test_busy_buckets_counted_in_a_graph(sia, dtype):
         assert np.array_equal(eager.cpu().numpy(), want)
     del g
     ix.close()
+
+
+@pytest.mark.parametrize("place", ["starts", "ends"])
+def test_count_in_place_in_a_graph(sia, place):
+    """int32 counts written over their own queries' starts or ends, each over the word it came from: as
+    without, a captured call needs no plan, whose read-back a captured stream refuses."""
+    import torch
+    print(f"[gpu] count in place in a graph {place}", flush=True)
+    rng = np.random.default_rng(9)
+    n, nq = 20_000, (1 << 22) + 77
+    s = np.sort(rng.integers(0, 1_000_000, n)).astype(np.int32)
+    e = s + rng.integers(0, 400, n).astype(np.int32)
+    ix = sia.DeviceIndex(np.int32).build(s, e, None, start_sorted=True, end_sorted=False)
+    by_end = np.sort(e)
+    lib, check = sia._native.lib, sia._native.check
+    t = [torch.zeros(nq, dtype=torch.int32, device="cuda") for _ in range(2)]
+    out = t[0 if place == "starts" else 1]
+    g, st = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.graph(g, stream=st):
+        check(lib.siCount(ix.handle, t[0].data_ptr(), t[1].data_ptr(), nq, out.data_ptr(), st.cuda_stream), "siCount")
+    for replay in (True, True, False, True):
+        qs = rng.integers(-50, 1_000_050, nq).astype(np.int32)
+        qe = qs + rng.integers(0, 3000, nq).astype(np.int32)
+        t[0].copy_(torch.from_numpy(qs))
+        t[1].copy_(torch.from_numpy(qe))
+        torch.cuda.synchronize()
+        if replay:
+            g.replay()
+        else:
+            check(lib.siCount(ix.handle, t[0].data_ptr(), t[1].data_ptr(), nq, out.data_ptr(), None), "siCount")
+        torch.cuda.synchronize()
+        assert np.array_equal(out.cpu().numpy(), np.searchsorted(s, qe, side="right") - np.searchsorted(by_end, qs))
+    del g
+    ix.close()
