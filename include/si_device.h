@@ -67,7 +67,9 @@ const char* siVersion(void);
  * Returns NULL on failure. */
 siIndex* siIndexCreate(int coord_bytes);
 
-/* Free the index and its device memory. */
+/* Free the index and its device memory.  While an index exists the library keeps blocks of device
+ * memory that it is done with, at most 2 GiB in all, for its next builds and host-buffer calls; they
+ * are freed when an allocation of the library finds no memory, and with the last index. */
 void siIndexDestroy(siIndex* ix);
 
 /* Build the index from n intervals (end-inclusive), replacing any previous
@@ -118,18 +120,23 @@ double siIndexLastBuildMs(const siIndex* ix);
 
 /* ---- Launch tuning ----------------------------------------------------------
  * Process-wide launch choices of the walk kernels (results never depend on them):
- *   "tile"       sorted queries per workgroup tile (64 .. 2^20, default 1024)
- *   "count_wgs"  resident workgroups per CU in the count pass (0 = occupancy limit)
- *   "fill_wgs"   resident workgroups per CU in the fill passes (0 = occupancy limit)
+ *   "tile"       sorted queries per workgroup tile of the block walk (64 .. 2^20, default 1024).
+ *                The count in walk form walks, and the fills that the sweep over the query starts
+ *                does not answer: indexes and set tables that hold an interval with start > end,
+ *                "range_skip" = 0, and large batches of few hits a query
+ *   "count_wgs"  resident workgroups per CU in the count's walk (0 = occupancy limit)
+ *   "fill_wgs"   resident workgroups per CU in the fills that walk (0 = occupancy limit)
  *   "count_rank"   1 (default): siCount* use the rank form (upper_bound + 1 - #{ends < s},
- *                  exact for s <= e; inverted queries walk); 0: the walk
+ *                  exact for s <= e; inverted queries walk), siCount* from two table searches
+ *                  a query without a plan where that is faster; 0: the walk
  *   "offsets_rank" 1 (default): siSearchOffsets* count with the rank form; 0: the walk
- *   "lane_steps"   line steps a lane spends on one query before the walk is parked for
- *                  the wave-cooperative kernel (1 .. 2^30, default 256)
+ *   "lane_steps"   line steps a lane of the block walk spends on one query before the walk is
+ *                  parked for the wave-cooperative kernel (1 .. 2^30, default 256)
  *   "ub_tree"      1 (default): siUpperBound, the plan's upper_bound and the rank-form
- *                  count descend 64-ary trees of first keys (top level of at most 4096
- *                  keys in Eytzinger order in LDS, then one 64-key node per level) over
- *                  the starts / the sorted ends; 0: plain halving
+ *                  count search the bucket tables over the starts / the sorted ends, or,
+ *                  where intervals crowd a few of the buckets, 64-ary trees of first keys
+ *                  (top level of at most 4095 keys in Eytzinger order in LDS, then one
+ *                  64-key node per level); 0: plain halving
  *   "plan_sync"    1 (default): siPlanQueries of a large batch (more than 8192 int64
  *                  queries, or 4M int32 ones) reads back once which key bits vary to skip
  *                  constant digits (one stream synchronisation); 0: it sorts every digit
@@ -159,8 +166,8 @@ int64_t siTuneGet(const char* name);   /* -1 for an unknown name */
  * neighbouring lanes.  A plan is a caller-owned device buffer of siPlanBytes bytes;
  * it is valid for the index and queries it was made from until the index is rebuilt.
  * Calls that share one plan must be ordered on one stream (they reuse its scratch).
- * siPlanQueries synchronises the stream once (radix pass selection) unless the tuning
- * knob "plan_sync" is 0. */
+ * siPlanQueries synchronises the stream once (radix pass selection) for a large batch
+ * unless the tuning knob "plan_sync" is 0. */
 size_t siPlanBytes(const siIndex* ix, size_t nq);
 
 int siPlanQueries(const siIndex* ix, const void* qs, const void* qe, size_t nq, void* plan,
@@ -230,7 +237,10 @@ int siSearchNoAlloc(const siIndex* ix, const void* qs, const void* qe, size_t nq
  * its index (calls on a table whose index was rebuilt since it was put return
  * SI_ERR_NOT_BUILT), and do not destroy an index while batches that use it are in flight.
  * Both calls are stream-ordered with no host read-back, so they can be captured in a graph;
- * calls that share one plan must be ordered on one stream. */
+ * calls that share one plan must be ordered on one stream.  A table whose sets hold no interval
+ * with start > end fills by the sweep over the query starts, another by the block walk; a graph
+ * keeps the way it was captured with when sets are put afterwards.  Its results stay exact, its
+ * time may be up to twice the other way's, or a tenth of it. */
 typedef struct siSetTable siSetTable;
 
 /* A table of max_sets slots (1 .. 4095) for indexes of coord_bytes (4: int32 only). */

@@ -37,7 +37,7 @@ struct IndexView {
     const S* __restrict__ starts;
     const S* __restrict__ ends;
     const uint32_t* __restrict__ branch;
-    const uint32_t* __restrict__ exitp;   // line exit target of each position (see k_exit)
+    const uint32_t* __restrict__ exitp;   // line exit target of each position (see k_branch_exit)
     const uint32_t* __restrict__ ends32;  // ends - ends32_base, or null
     int64_t ends32_base;
     uint32_t n;

@@ -18,7 +18,8 @@
 //     the wave grabs from the tile's LDS counter, so lanes stay busy however uneven
 //     the hit counts are.  counts[q] / offsets are written in input order.
 //  3. Fill: a sweep over the query starts writes each query's positions at its CSR offset
-//     (si_sweep.h); the walk kernel of the count does on an index with start > end intervals.
+//     (si_sweep.h); the walk kernel of the count does on an index with start > end intervals,
+//     and in large batches of few hits a query (walk_too).
 //
 // The walk is the reference's backward superset walk taken one aligned 64-byte line of
 // ends at a time.  In the line [b0, b0 + W) holding the current position cur, every
@@ -29,7 +30,7 @@
 // there; that chain's first element below b0 is the nearest j < b0 with
 // ends[j] >= max(ends[b0..x]), which is branch[a] for the leftmost maximum a of
 // ends[b0..x].  That target depends on x only, so the build stores it per position
-// (exitp[x], see si_index.hip k_exit).  One line load and at most one exitp load replace
+// (exitp[x], see si_index.hip k_branch_exit).  One line load and at most one exitp load replace
 // the reference's per-element steps while visiting the same hits in the same order.
 #include <hip/hip_runtime.h>
 
@@ -3313,10 +3314,13 @@ int launch_walk_multi(const siSetTable* tb, void* plan, size_t nq, const uint64_
         per = std::max(per, 1);
     }
     const SetView<int32_t>* sets = (const SetView<int32_t>*)tb->d_views;
-    // The sweep leaves every query of a set with start > end to the wave-cooperative kernel, the lane
-    // walk answers them itself: a table that holds such a set takes the walk (8 sets of 1M intervals
-    // each, every 1000th inverted, 1M queries: 0.44 ms, swept 41 ms; none inverted: 0.43 and 0.30;
-    // 1000 queries on 4 sets: 68 us and 10).
+    // The sweep leaves every query of a set with start > end to k_sweep_shared, the lane walk answers
+    // them itself: a table that holds such a set takes the walk, which large batches of few hits want
+    // most (us, walked and swept: 3M queries of 3 hits on two sets of 3M 866 and 1330, vector order 884
+    // and 1947; wide queries, vector order, 4454 and 7227; 60 sets of 300 142 and 197).  Small ones
+    // would rather be swept (1000 queries on 4 sets of 100K 155 and 49; 1M on 8 of 1M 832 and 734), and
+    // so would sets of which some intervals are long (1 %: 14136 and 1310).  A graph keeps the way it
+    // was captured with, whatever is put afterwards; both are exact for any set.
     bool walk = false;
     for (const siIndex* ix : tb->sets) walk |= ix && !rank_exact(ix);
     k_walk_counters_reset<<<1, 64, 0, st>>>(pv.counter, walk ? 0u : 1u, nullptr, 0u, 0u, 0u);
@@ -3359,7 +3363,7 @@ SI_EXPORT siSetTable* siSetTableCreate(int coord_bytes, uint32_t max_sets) {
         si_set_error(SI_ERR_UNSUPPORTED, "set tables hold int32 indexes");
         return nullptr;
     }
-    if (max_sets < 1 || max_sets > 4095) {   // the key kernel's per-slot histogram lives in LDS
+    if (max_sets < 1 || max_sets > 4095) {   // (two digits of the sort hold a slot, k_multi_tiles takes four a thread)
         si_set_error(SI_ERR_ARG, "max_sets must be in [1, 4095]");
         return nullptr;
     }
